@@ -91,6 +91,21 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
       rowsec[si][dir] = rowtw[si][dir].empty() ? -1 : (int)secs.size();
       if (!rowtw[si][dir].empty()) secs.push_back({rowtw[si][dir].data(), rowtw[si][dir].size() * 8, 0});
     }
+  FusedTables F;
+  build_fused_tables(H, &F);
+  const int fsec = (int)secs.size();
+  secs.push_back({F.tw[0].data(), F.tw[0].size() * 8, 0});
+  secs.push_back({F.tw[1].data(), F.tw[1].size() * 8, 0});
+  secs.push_back({F.lc.data(), F.lc.size() * 8, 0});
+  secs.push_back({F.lc_key.data(), F.lc_key.size() * 8, 0});
+  secs.push_back({F.lc_up.data(), F.lc_up.size() * 8, 0});
+  secs.push_back({F.bq.data(), F.bq.size() * 8, 0});
+  secs.push_back({F.mu_w.data(), F.mu_w.size(), 0});
+  secs.push_back({F.md_w.data(), F.md_w.size(), 0});
+  secs.push_back({F.mu_out.data(), F.mu_out.size() * sizeof(ConvOut), 0});
+  secs.push_back({F.md_out.data(), F.md_out.size() * sizeof(ConvOut), 0});
+  secs.push_back({F.scr.data(), F.scr.size() * 8, 0});
+  secs.push_back({F.scr_thr.data(), F.scr_thr.size() * 8, 0});
   const int nsec = (int)secs.size();
   size_t total = 0;
   for (int i = 0; i < nsec; ++i) {
@@ -138,6 +153,22 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
   for (int si = 0; si < 3; ++si)
     for (int dir = 0; dir < 2; ++dir)
       D.tw_row[si][dir] = rowsec[si][dir] < 0 ? nullptr : (const uint64_t*)(b + secs[rowsec[si][dir]].off);
+  FusedDev& Z = D.fz;
+  Z.tw[0] = (const uint64_t*)(b + secs[fsec].off);
+  Z.tw[1] = (const uint64_t*)(b + secs[fsec + 1].off);
+  Z.lc = (const uint64_t*)(b + secs[fsec + 2].off);
+  Z.lc_key = (const uint64_t*)(b + secs[fsec + 3].off);
+  Z.lc_up = (const uint64_t*)(b + secs[fsec + 4].off);
+  Z.bq = (const uint64_t*)(b + secs[fsec + 5].off);
+  Z.mu_w = (const uint8_t*)(b + secs[fsec + 6].off);
+  Z.md_w = (const uint8_t*)(b + secs[fsec + 7].off);
+  Z.mu_out = (const ConvOut*)(b + secs[fsec + 8].off);
+  Z.md_out = (const ConvOut*)(b + secs[fsec + 9].off);
+  Z.scr = (const double*)(b + secs[fsec + 10].off);
+  Z.scr_thr = (const double*)(b + secs[fsec + 11].off);
+  Z.mu_stride = F.mu_stride;
+  Z.mu_kb = F.mu_kb;
+  Z.md_kb = F.md_kb;
   *out = h;
   return AOA_OK;
 }
@@ -453,54 +484,21 @@ extern "C" size_t aoa_workspace_bytes(const aoa_params* h, int level) {
 static int keyswitch_core(const aoa_params* h, hipStream_t st, uint64_t* out0, uint64_t* out1,
                           const uint64_t* add0, const uint64_t* d, const uint64_t* kb, const uint64_t* ka,
                           int level, uint64_t* ws) {
-  const DevParams& P = h->dev;
-  const size_t N = (size_t)P.N;
-  const int L = level + 1, K = P.K;
-  uint64_t* X = ws;
-  uint64_t* P0 = X + (size_t)(L + K) * N;
-  uint64_t* P1 = P0 + (size_t)(L + K) * N;
-  // ModUp: special limbs of X from d
-  launch_modup(P, d, X + (size_t)L * N, level, st);
-  // X_Q = NTT(d) (out of place), X_B = NTT(X_B)
-  LimbMap mq;
-  std::memset(&mq, 0, sizeof(mq));
-  mq.base[0] = X;
-  mq.src[0] = d;
-  mq.nlimbs = L;
-  mq.qlimbs = L;
-  mq.npolys = 1;
-  if (ntt_forward(P, mq, 0, st)) return fail(AOA_ERR_UNSUPPORTED, "no NTT split");
-  LimbMap mb;
-  std::memset(&mb, 0, sizeof(mb));
-  mb.base[0] = X + (size_t)L * N;
-  mb.nlimbs = K;
-  mb.qlimbs = 0;
-  mb.npolys = 1;
-  if (ntt_forward(P, mb, 0, st)) return fail(AOA_ERR_UNSUPPORTED, "no NTT split");
-  // P_y = INTT(X * key_y)
-  LimbMap mk;
-  std::memset(&mk, 0, sizeof(mk));
-  mk.base[0] = P0;
-  mk.base[1] = P1;
-  mk.src[0] = X;
-  mk.nlimbs = L + K;
-  mk.qlimbs = L;
-  mk.npolys = 2;
-  if (ntt_inverse(P, mk, 0, kb, ka, st)) return fail(AOA_ERR_UNSUPPORTED, "no NTT split");
-  ModDownArgs a;
-  std::memset(&a, 0, sizeof(a));
-  a.inQ[0] = P0;
-  a.inQ[1] = P1;
-  a.inB[0] = P0 + (size_t)L * N;
-  a.inB[1] = P1 + (size_t)L * N;
-  a.add[0] = add0;
-  a.out[0] = out0;
-  a.out[1] = out1;
-  a.npolys = 2;
-  a.level = level;
-  a.rescale = 0;
-  launch_moddown(P, a, st);
-  return AOA_OK;
+  const size_t N = (size_t)h->dev.N;
+  const int L = level + 1, K = h->dev.K;
+  FzItem it{};
+  it.d = d;
+  it.kb = kb;
+  it.ka = ka;
+  it.XQ = ws;
+  it.X = ws + (size_t)L * N;
+  it.P0 = it.XQ + (size_t)(L + K) * N;
+  it.P1 = it.P0 + (size_t)(L + K) * N;
+  it.add0 = add0;
+  it.out0 = out0;
+  it.out1 = out1;
+  it.level = level;
+  return fz_switch(h->dev, it, st) ? fail(AOA_ERR_UNSUPPORTED, "no NTT split") : AOA_OK;
 }
 
 extern "C" int aoa_keyswitch(const aoa_params* h, void* stream, uint64_t* out0, uint64_t* out1,
@@ -526,73 +524,25 @@ int aoa::hommul_core(const aoa_params* h, void* stream, uint64_t* c3_0, uint64_t
   if (level < 0 || level >= h->host.k) return fail(AOA_ERR_ARG, "level out of range");
   if (ws_bytes < aoa_workspace_bytes(h, level)) return fail(AOA_ERR_WORKSPACE, "workspace too small");
   const DevParams& P = h->dev;
-  hipStream_t st = (hipStream_t)stream;
   const size_t N = (size_t)P.N;
   const int L = level + 1, K = P.K;
-  uint64_t* X = (uint64_t*)ws;            // L+K: d2 (NTT) | special limbs
-  uint64_t* D0 = X + (size_t)(L + K) * N;  // L
-  uint64_t* D1 = D0 + (size_t)L * N;       // L
-  uint64_t* D2 = D1 + (size_t)L * N;       // L: d2 in the coefficient domain
-  uint64_t* P0 = D2 + (size_t)L * N;       // L+K
-  uint64_t* P1 = P0 + (size_t)(L + K) * N; // L+K
-  // With two-pass transforms d0 and d1 stay in the NTT domain and join the
-  // key products as (B mod q) d0, (B mod q) d1: ModDown is linear in its Q
-  // limbs and its special-limb sum does not see them, so
-  // ModDown(X + B d) = ModDown(X) + d residue for residue, and only d2 is
-  // transformed back.  The single-workgroup transform (N <= 4096) keeps the
-  // additions in ModDown.
-  const bool fold = (P.ntt_n1 ? P.ntt_n1 : ntt_default_n1(P.N)) != P.N;
-  launch_tensor(P, D0, D1, X, a0, a1, b0, b1, L, st);
-  LimbMap mi;
-  std::memset(&mi, 0, sizeof(mi));
-  if (fold) {
-    mi.base[0] = D2;
-    mi.src[0] = X;
-    mi.npolys = 1;
-  } else {
-    mi.base[0] = D0;
-    mi.base[1] = D1;
-    mi.base[2] = D2;
-    mi.src[0] = D0;
-    mi.src[1] = D1;
-    mi.src[2] = X;
-    mi.npolys = 3;
-  }
-  mi.nlimbs = L;
-  mi.qlimbs = L;
-  if (ntt_inverse(P, mi, 0, nullptr, nullptr, st)) return fail(AOA_ERR_UNSUPPORTED, "no NTT split");
-  launch_modup(P, D2, X + (size_t)L * N, level, st);
-  LimbMap mb;
-  std::memset(&mb, 0, sizeof(mb));
-  mb.base[0] = X + (size_t)L * N;
-  mb.nlimbs = K;
-  mb.qlimbs = 0;
-  mb.npolys = 1;
-  if (ntt_forward(P, mb, 0, st)) return fail(AOA_ERR_UNSUPPORTED, "no NTT split");
-  LimbMap mk;
-  std::memset(&mk, 0, sizeof(mk));
-  mk.base[0] = P0;
-  mk.base[1] = P1;
-  mk.src[0] = X;
-  mk.nlimbs = L + K;
-  mk.qlimbs = L;
-  mk.npolys = 2;
-  if (ntt_inverse(P, mk, 0, evk_b, evk_a, st, fold ? D0 : nullptr, fold ? D1 : nullptr))
-    return fail(AOA_ERR_UNSUPPORTED, "no NTT split");
-  ModDownArgs a;
-  std::memset(&a, 0, sizeof(a));
-  a.inQ[0] = P0;
-  a.inQ[1] = P1;
-  a.inB[0] = P0 + (size_t)L * N;
-  a.inB[1] = P1 + (size_t)L * N;
-  a.add[0] = fold ? nullptr : D0;
-  a.add[1] = fold ? nullptr : D1;
-  a.out[0] = c3_0;
-  a.out[1] = c3_1;
-  a.npolys = 2;
-  a.level = level;
-  a.rescale = rescale;
-  launch_moddown(P, a, st);
+  // d2 after its inverse rows (L limbs), the special limbs (K), the key products (L + K each)
+  FzItem it{};
+  it.a0 = a0;
+  it.a1 = a1;
+  it.b0 = b0;
+  it.b1 = b1;
+  it.kb = evk_b;
+  it.ka = evk_a;
+  it.D = (uint64_t*)ws;
+  it.X = it.D + (size_t)L * N;
+  it.P0 = it.X + (size_t)K * N;
+  it.P1 = it.P0 + (size_t)(L + K) * N;
+  it.out0 = c3_0;
+  it.out1 = c3_1;
+  it.level = level;
+  it.rescale = rescale;
+  if (fz_mul(P, it, (hipStream_t)stream)) return fail(AOA_ERR_UNSUPPORTED, "no NTT split");
   return check_launch(rescale ? "aoa_hommul_relin_rescale" : "aoa_hommul_relin");
 }
 

@@ -54,6 +54,7 @@ __device__ __forceinline__ int xcd_chunk_id(unsigned w, unsigned n) {
 // One field of a DevPrime at a wave-uniform index, as a scalar load.
 __device__ __forceinline__ uint64_t ld_prime_p(const DevPrime* base, int i) { return as_const(&base[i].p)[0]; }
 __device__ __forceinline__ int ld_prime_nb(const DevPrime* base, int i) { return (int)as_const(&base[i].nb)[0]; }
+__device__ __forceinline__ uint32_t ld_prime_field(const DevPrime* base, int i) { return as_const(&base[i].field)[0]; }
 __device__ __forceinline__ DevPrime ld_prime(const DevPrime* base, int i) {
   constexpr int W = (int)(sizeof(DevPrime) / 8);
   const cptr<uint64_t> w = as_const(reinterpret_cast<const uint64_t*>(base + i));
@@ -146,6 +147,22 @@ struct AutoDesc {
   uint64_t ginv;           // inverse Galois element mod 2N
   int prime;
   int pad;
+};
+
+// One HomMul (a0 set) or key switching of the fused kernels (fused.hip).
+// Limb-major buffers, stride N; P0 and P1 hold level + 1 + K limbs.
+struct FzItem {
+  const uint64_t *a0, *a1, *b0, *b1;  // HomMul's operands (NTT domain)
+  const uint64_t* d;                  // key switching's input (coefficient domain)
+  const uint64_t *kb, *ka;            // switching key, limb of prime r at + r N
+  uint64_t* D;                        // HomMul: d2 after the inverse rows (level + 1 limbs)
+  uint64_t* XQ;                       // key switching: the input's forward columns (level + 1 limbs)
+  uint64_t* X;                        // the special limbs' forward columns (K limbs)
+  uint64_t *P0, *P1;                  // key products after the inverse rows
+  const uint64_t *add0, *add1;        // added to the result (coefficient domain), or null
+  uint64_t *out0, *out1;
+  int level;
+  int rescale;
 };
 
 __device__ __forceinline__ tw2 load_tw(const uint64_t* table, size_t idx) {

@@ -1,0 +1,477 @@
+// Column kernels of the fused key switching (fused.hpp): the column stages of
+// both transforms with the basis conversion between or after them.
+#include "fused.hpp"
+
+namespace aoa {
+
+
+// Sums of basis conversions run as products of signed bytes on the matrix
+// cores: input byte s of residue i against the digits of 256^s c_ij mod q_j
+// (FusedDev::mu_w, md_w).
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+constexpr int FZ_COLS = 8;               // columns of a tile: 64-byte row segments
+constexpr int FZ_TILE = 16 * FZ_COLS;    // coefficients of a tile
+constexpr int FZ_PITCH = FZ_TILE + 8;    // LDS words between limbs (limbs of a wave on different banks)
+constexpr int FZ_THREADS = 512;
+
+__device__ __forceinline__ int up8(int x) { return (x + 7) & ~7; }
+
+// Orders a wave's LDS accesses: the four threads of a column are lanes of one
+// wave, whose LDS instructions run in order, so an exchange between them needs
+// no barrier.
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// A column's values between its two pairs of stages, through its place in LDS:
+// from rows 4q + k to q + 4k, or back.
+template <bool TO_A, class F>
+__device__ __forceinline__ void col_turn(const F& f, typename F::V (&x)[4], uint64_t* t, int q) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) t[(TO_A ? 4 * q + k : q + 4 * k) * FZ_COLS] = f.raw(x[k]);
+  wave_order();
+#pragma unroll
+  for (int k = 0; k < 4; ++k) x[k] = f.raw_in(t[(TO_A ? q + 4 * k : 4 * q + k) * FZ_COLS]);
+}
+
+// ------------------------------------------------- conversions by matrix --
+// One step of 8 inputs per instruction: lane (n, g) holds the bytes of inputs
+// 8 kb + 2 g and + 1 of coefficient n, and of the same inputs' constants for
+// output row n; byte - 128 as the signed digit (ConvOut::off makes up for it).
+template <int T, int NB>
+__device__ __forceinline__ void conv_acc(v4i (&acc)[T][NB], const uint8_t* W, int kbs, int kbn, const uint64_t* tl, int nb0,
+                                         int lane) {
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[t][b] = v4i{0, 0, 0, 0};
+  const v4i* w = reinterpret_cast<const v4i*>(W) + lane;
+  const int n = lane & 15, g = lane >> 4;
+  for (int kb = 0; kb < kbn; ++kb) {
+    v4i in[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const uint64_t* q = tl + (8 * kb + 2 * g) * FZ_PITCH + (nb0 + b) * 16 + n;
+      const uint64_t v0 = q[0] ^ 0x8080808080808080ull, v1 = q[FZ_PITCH] ^ 0x8080808080808080ull;
+      in[b] = v4i{(int)(uint32_t)v0, (int)(v0 >> 32), (int)(uint32_t)v1, (int)(v1 >> 32)};
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const v4i a = w[(size_t)(t * kbs + kb) * 64];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[t][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, in[b], acc[t][b], 0, 0, 0);
+    }
+  }
+}
+
+// The sum modulo o.p in [0, 1.3 p) from its digit columns (component r).  The
+// columns stay below 2^23 (at most 65 x 7 bytes), pairs of them fit 32 bits.
+template <int T, int NB>
+__device__ __forceinline__ uint64_t conv_join(const v4i (&acc)[T][NB], int b, int r, const ConvOut& o) {
+  auto S = [&](int t) -> int { return t < T ? acc[t < T ? t : 0][b][r] : 0; };
+  const int A01 = S(0) + (S(1) << 8), A23 = S(2) + (S(3) << 8), A45 = S(4) + (S(5) << 8), A67 = S(6) + (S(7) << 8);
+  float f = __builtin_fmaf((float)A45, o.c_32, __builtin_fmaf((float)A23, o.c_16, o.c_b));
+  uint64_t v = o.off + (uint64_t)((int64_t)A01 + (int64_t)A23 * 65536);
+  uint32_t hi = (uint32_t)A45;
+  if (T > 6) {
+    f = __builtin_fmaf((float)A67, o.c_48, f);
+    hi += (uint32_t)A67 << 16;
+  }
+  v += (uint64_t)hi << 32;
+  return v - (uint64_t)(uint32_t)f * o.p;
+}
+
+__device__ __forceinline__ ConvOut ld_conv(const ConvOut* t) {
+  ConvOut o;
+  const uint4* s = reinterpret_cast<const uint4*>(t);
+  uint4 v[2] = {s[0], s[1]};
+  __builtin_memcpy(&o, v, sizeof(o));
+  return o;
+}
+
+// ------------------------------------------------------------------ ModUp --
+// MUL: the item's D (inverse rows of d2) is brought to coefficients; otherwise
+// the item's d holds coefficients, whose Q limbs also start their forward NTT
+// here.  v_i = x_i (Q_l/q_i)^-1 into LDS, the conversion, the forward columns
+// of the special limbs.
+template <class F, bool MUL>
+__device__ __forceinline__ void up_in(const DevParams& P, const FzItem& it, int i, int M, int col, int q, int c,
+                                      uint64_t* tl) {
+  const DevPrime dp = P.primes[i];
+  const F f(dp);
+  const uint64_t* src = glob(MUL ? it.D : it.d) + (size_t)i * P.N + col;
+  uint64_t* t = tl + i * FZ_PITCH + c;
+  typename F::V x[4];
+  if constexpr (MUL) {
+    const uint64_t* T = P.fz.tw[1] + (size_t)i * P.N * 2;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[k] = f.raw_in(src[(size_t)(4 * q + k) * M]);
+    col_inv_b(f, x, T, q);
+    col_turn<true>(f, x, t, q);
+    col_inv_a(f, x, T, P.fz.lc_up + 4 * ((size_t)it.level * P.k + i));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) t[(q + 4 * k) * FZ_COLS] = f.out_last(x[k]);
+  } else {
+    const uint64_t* T = P.fz.tw[0] + (size_t)i * P.N * 2;
+    const tw2 w = reinterpret_cast<const tw2*>(P.inv_qhat)[(size_t)it.level * P.k + i];
+    uint64_t v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint64_t u = src[(size_t)(q + 4 * k) * M];
+      v[k] = mul_shoup(u, w.w, w.q, dp.p);
+      x[k] = f.in(u);
+    }
+    col_fwd_a(f, x, T);
+    col_turn<false>(f, x, t, q);
+    wave_order();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) t[(q + 4 * k) * FZ_COLS] = v[k];
+    col_fwd_b(f, x, T, q);
+    uint64_t* dst = glob(it.XQ) + (size_t)i * P.N + col;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) dst[(size_t)(4 * q + k) * M] = f.raw(x[k]);
+  }
+}
+
+template <class F>
+__device__ __forceinline__ void up_out(const DevParams& P, const FzItem& it, int j, int M, int col, int q, int c,
+                                       uint64_t* tl) {
+  const F f(P.primes[P.k + j]);
+  const uint64_t* T = P.fz.tw[0] + (size_t)(P.k + j) * P.N * 2;
+  typename F::V x[4];
+  uint64_t* t = tl + j * FZ_PITCH + c;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) x[k] = f.in(t[(q + 4 * k) * FZ_COLS]);
+  col_fwd_a(f, x, T);
+  col_turn<false>(f, x, t, q);
+  col_fwd_b(f, x, T, q);
+  uint64_t* dst = glob(it.X) + (size_t)j * P.N + col;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) dst[(size_t)(4 * q + k) * M] = f.raw(x[k]);
+}
+
+// Special limbs 16 jb.. of coefficients 16 nb0..: the conversion into LDS.
+template <int T, int NB>
+__device__ __forceinline__ void up_conv(const DevParams& P, const FzItem& it, int jb, int nb0, const uint64_t* tl,
+                                        uint64_t* to, int lane) {
+  const FusedDev& Z = P.fz;
+  v4i acc[T][NB];
+  const uint8_t* W = Z.mu_w + (size_t)it.level * Z.mu_stride + (size_t)jb * T * Z.mu_kb * 1024;
+  conv_acc<T, NB>(acc, W, Z.mu_kb, (it.level + 8) / 8, tl, nb0, lane);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int j = jb * 16 + 4 * (lane >> 4) + r;
+    if (j < P.K) {
+      const ConvOut o = ld_conv(Z.mu_out + (size_t)it.level * P.K + j);
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        to[j * FZ_PITCH + (nb0 + b) * 16 + (lane & 15)] = conv_join<T, NB>(acc, b, r, o);
+    }
+  }
+}
+
+template <bool MUL, bool ARG>
+__global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_fz_up(DevParams P, FzItem arg,
+                                                                                                  const FzItem* items) {
+  extern __shared__ uint64_t fz_lds[];
+  const int M = P.N / 16, per = M / FZ_COLS;
+  const int w = xcd_chunk_id(blockIdx.x, gridDim.x);
+  const FzItem it = fz_item<ARG>(arg, items, w / per);
+  const int col0 = (w % per) * FZ_COLS, L = it.level + 1;
+  uint64_t* to = fz_lds + up8(L) * FZ_PITCH;
+  for (int t = threadIdx.x; t < L * 32; t += FZ_THREADS) {
+    const int i = t / 32, q = t / FZ_COLS % 4, c = t % FZ_COLS;
+#define CALL(F) up_in<F, MUL>(P, it, i, M, col0 + c, q, c, fz_lds)
+    switch (P.primes[i].field) {
+      case FIELD_FP64: CALL(FieldFp64); break;
+      case FIELD_LAZY: CALL(FieldLazy); break;
+      default: CALL(FieldStrict); break;
+    }
+#undef CALL
+  }
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int units = ((P.K + 15) / 16) * 4;
+  const bool fp = ld_prime_field(P.primes, P.k) == FIELD_FP64;
+  for (int u = wave; u < units; u += FZ_THREADS / 64) {
+    if (fp)
+      up_conv<6, 2>(P, it, u / 4, (u % 4) * 2, fz_lds, to, lane);
+    else
+      up_conv<7, 2>(P, it, u / 4, (u % 4) * 2, fz_lds, to, lane);
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < P.K * 32; t += FZ_THREADS) {
+    const int j = t / 32, q = t / FZ_COLS % 4, c = t % FZ_COLS;
+    if (fp)
+      up_out<FieldFp64>(P, it, j, M, col0 + c, q, c, to);
+    else
+      up_out<FieldLazy>(P, it, j, M, col0 + c, q, c, to);
+  }
+}
+
+// ---------------------------------------------------------------- ModDown --
+template <class F>
+__device__ __forceinline__ void down_in(const DevParams& P, const uint64_t* src, int pr, int M, int q, uint64_t* t) {
+  const F f(P.primes[pr]);
+  const uint64_t* T = P.fz.tw[1] + (size_t)pr * P.N * 2;
+  typename F::V x[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) x[k] = f.raw_in(src[(size_t)(4 * q + k) * M]);
+  col_inv_b(f, x, T, q);
+  col_turn<true>(f, x, t, q);
+  col_inv_a(f, x, T, P.fz.lc_key + 4 * (size_t)pr);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) t[(q + 4 * k) * FZ_COLS] = f.out_last(x[k]);
+}
+
+// ref(a c) - (a c mod q) mod q of one product, c = (B/b_j) mod q_i: what the
+// reference's reduction of it deviates by.
+__device__ __forceinline__ uint64_t down_deviation(const DevParams& P, uint64_t a, int i, int j) {
+  const DevPrime dq = ld_prime(P.primes, i);
+  const tw2 w = ld_tw2(reinterpret_cast<const tw2*>(P.bhat_mod_q) + (size_t)i * P.K, j);
+  const uint64_t x = mul_shoup(a, w.w, w.q, dq.p);
+  const uint64_t f = ref_barrett(mulhi64(a, w.w), a * w.w, dq.p, dq.mu, (int)dq.nb);
+  return sub_mod(f, x, dq.p);
+}
+
+// Looks for the products a_j c_ij of the limbs i = g + 4 n, n0 <= n < n0 + NL,
+// whose remainder may lie in the reference's deviation window and takes what
+// they deviate by off x_i.  frac(a c / q) = frac(al c/q + ah frac(2^28 c/q)),
+// a = al + ah 2^28, in two FP64 multiply-adds onto 1.5 2^36 + 2^-15, which leaves
+// its first 16 bits (one unit off at most, two units added) in the low half
+// word; the least of a term's NL halves is compared with the widest window.
+// About one wave in a hundred looks closer: to 2^-22 (bias 2^-21, bound 2^-20
+// more), then with the exact formulas.
+template <int NL>
+__device__ __forceinline__ void down_screen(const DevParams& P, const uint64_t* aux, uint64_t* xq, int g, int n0, int c) {
+  const cptr<double> tab = as_const(P.fz.scr) + (g * 16 + n0) * 2;
+  const cptr<double> thr = as_const(P.fz.scr_thr) + g + 4 * n0;
+  double widest = thr[0];
+#pragma unroll
+  for (int n = 1; n < NL; ++n) widest = __builtin_fmax(widest, thr[4 * n]);
+  const uint32_t bound = min((uint32_t)(widest * 65536.0) + 4, 65535u);
+  for (int j = 0; j < P.K; ++j) {
+    const uint64_t a = aux[j * FZ_PITCH + c];
+    const double al = (double)((uint32_t)a & ((1u << 28) - 1)), ah = (double)(uint32_t)(a >> 28);
+    const cptr<double> e = tab + (size_t)j * 128;
+    uint16_t least = 65535;
+#pragma unroll
+    for (int n = 0; n < NL; ++n) {
+      const double s = __builtin_fma(ah, e[2 * n + 1], __builtin_fma(al, e[2 * n], 103079215104.000030517578125));
+      const uint16_t h = (uint16_t)(uint32_t)__double_as_longlong(s);
+      least = h < least ? h : least;
+    }
+    if (__builtin_amdgcn_ballot_w64(least <= bound)) {
+#pragma unroll 1
+      for (int n = 0; n < NL; ++n) {
+        const double s = __builtin_fma(ah, e[2 * n + 1], __builtin_fma(al, e[2 * n], 4.76837158203125e-07));
+        if (__builtin_amdgcn_fract(s) < thr[4 * n]) {
+          const int i = g + 4 * (n0 + n);
+          uint64_t* x = xq + i * FZ_PITCH + c;
+          *x = sub_mod(*x, down_deviation(P, a, i, j), ld_prime_p(P.primes, i));
+        }
+      }
+    }
+  }
+}
+
+// The rescale's dropped limb `level` (a prime below 2^57): the conversion's sum
+// over j in [j0, j1), with the deviating products as the reference reduces
+// them, in [0, 5 q) (as moddown_conv in rns.hip).
+__device__ __forceinline__ uint64_t down_top(const DevParams& P, const uint64_t* aux, int level, int j0, int j1, int c) {
+  constexpr uint32_t M28 = (1u << 28) - 1;
+  constexpr int TW = (int)(sizeof(MdTerm) / 4);
+  const cptr<uint32_t> terms = as_const(P.md_terms) + (size_t)level * TW;
+  const uint32_t thr = as_const(P.md_thr)[level];
+  uint64_t s0 = 0, s2 = 0, sm = 0;
+  for (int j = j0; j < j1; ++j) {
+    const uint64_t a = aux[j * FZ_PITCH + c];
+    const uint32_t a0 = (uint32_t)a, a1 = (uint32_t)(a >> 32);
+    const uint32_t al = a0 & M28, ah = (uint32_t)(a >> 28);
+    const cptr<uint32_t> e = terms + (size_t)j * P.k * TW;
+    s0 += (uint64_t)al * e[0];
+    s2 += (uint64_t)ah * e[1];
+    sm += (uint64_t)(al + ah) * e[2];
+    if (!P.moddown_exact && moddown_screen(a0, a1, e[3], e[4], e[5]) <= thr) {
+      const uint64_t d = down_deviation(P, a, level, j);
+      s0 += d;
+      sm += d;
+    }
+  }
+  return reduce_sums_lazy(s0, sm - s0 - s2, s2, ld_prime_p(P.primes, level), as_const(P.md_red)[2 * level],
+                          ld_prime_nb(P.primes, level));
+}
+
+// Limbs 16 ib.. of coefficients 16 nb0..: the conversion and the result,
+// (x_i - sum) B^-1 (+ add_i), or with the rescale, whose dropped limb is input
+// K of the sum, (x_i - sum) B^-1 q_l^-1.
+template <int T, int NB>
+__device__ __forceinline__ void down_out(const DevParams& P, const FzItem& it, const uint64_t* add, uint64_t* out, int ib,
+                                         int nb0, int lout, const uint64_t* aux, const uint64_t* xq, int M, int col0,
+                                         int lane) {
+  const FusedDev& Z = P.fz;
+  v4i acc[T][NB];
+  conv_acc<T, NB>(acc, Z.md_w + (size_t)ib * 8 * Z.md_kb * 1024, Z.md_kb, Z.md_kb, aux, nb0, lane);
+  const tw2* fin = it.rescale ? reinterpret_cast<const tw2*>(P.md_fin) + (size_t)it.level * P.k
+                              : reinterpret_cast<const tw2*>(P.inv_b_mod_q);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int i = ib * 16 + 4 * (lane >> 4) + r;
+    if (i < lout) {
+      const ConvOut o = ld_conv(Z.md_out + i);
+      const tw2 w = fin[i];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const int n = (nb0 + b) * 16 + (lane & 15);
+        uint64_t v = conv_join<T, NB>(acc, b, r, o);
+        if constexpr (T == 8) {
+          v = v >= o.p ? v - o.p : v;
+          v = mul_shoup(xq[i * FZ_PITCH + n] + (o.p - v), w.w, w.q, o.p);
+        } else {  // primes below 2^56
+          v = shoup4(xq[i * FZ_PITCH + n] + (2 * o.p - v), w.w, w.q, 0 - o.p);
+          v = v >= 2 * o.p ? v - 2 * o.p : v;
+          v = v >= o.p ? v - o.p : v;
+        }
+        const size_t at = (size_t)i * P.N + (size_t)(n / FZ_COLS) * M + col0 + n % FZ_COLS;
+        if (add) v = add_mod(v, add[at], o.p);
+        out[at] = v;
+      }
+    }
+  }
+}
+
+__host__ __device__ inline int down_aux_rows(int K) { return (K + 8) & ~7; }
+
+template <bool ARG>
+__global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_fz_down(DevParams P, FzItem arg,
+                                                                                                const FzItem* items) {
+  extern __shared__ uint64_t fz_lds[];  // special limbs (and the dropped limb), Q limbs, partial sums [4][128]
+  const int M = P.N / 16, per = M / FZ_COLS, K = P.K;
+  const int w = xcd_chunk_id(blockIdx.x, gridDim.x);
+  const FzItem it = fz_item<ARG>(arg, items, w / (2 * per));
+  const int y = (w / per) & 1, col0 = (w % per) * FZ_COLS, L = it.level + 1;
+  const int rescale = it.rescale, lout = rescale ? it.level : L;
+  const uint64_t* p = glob(y ? it.P1 : it.P0) + col0;
+  uint64_t* aux = fz_lds;
+  uint64_t* xq = aux + down_aux_rows(K) * FZ_PITCH;
+  uint64_t* part = xq + up8(L) * FZ_PITCH;
+  // inverse columns: Q limbs, then from a wave boundary the special limbs
+  const int L2 = (L + 1) & ~1;
+  for (int t = threadIdx.x; t < (L2 + K) * 32; t += FZ_THREADS) {
+    const int m = t / 32, q = t / FZ_COLS % 4, c = t % FZ_COLS;
+    if (m < L2) {
+      if (m < L) {
+#define CALL(F) down_in<F>(P, p + (size_t)m * P.N + c, m, M, q, xq + m * FZ_PITCH + c)
+        switch (P.primes[m].field) {
+          case FIELD_FP64: CALL(FieldFp64); break;
+          case FIELD_LAZY: CALL(FieldLazy); break;
+          default: CALL(FieldStrict); break;
+        }
+#undef CALL
+      }
+    } else {
+      const int j = m - L2;
+      const uint64_t* s = p + (size_t)(L + j) * P.N + c;
+      if (P.primes[P.k].field == FIELD_FP64)
+        down_in<FieldFp64>(P, s, P.k + j, M, q, aux + j * FZ_PITCH + c);
+      else
+        down_in<FieldLazy>(P, s, P.k + j, M, q, aux + j * FZ_PITCH + c);
+    }
+  }
+  if (!rescale && threadIdx.x < FZ_TILE) aux[K * FZ_PITCH + threadIdx.x] = 0;
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int g = wave >> 1, c = (wave & 1) * 64 + lane;
+  if (rescale) {
+    const int jq = (K + 3) / 4, j0 = g * jq, j1 = min(K, j0 + jq);
+    part[g * FZ_TILE + c] = j1 > j0 ? down_top(P, aux, it.level, j0, j1, c) : 0;
+  }
+  if (!P.moddown_exact) {
+    int n = 0;
+    const int nl = (lout - g + 3) / 4;  // limbs g, g + 4, ... below lout
+    for (; nl - n >= 8; n += 8) down_screen<8>(P, aux, xq, g, n, c);
+    if (nl - n >= 4) {
+      down_screen<4>(P, aux, xq, g, n, c);
+      n += 4;
+    }
+    if (nl - n >= 2) {
+      down_screen<2>(P, aux, xq, g, n, c);
+      n += 2;
+    }
+    if (nl - n >= 1) down_screen<1>(P, aux, xq, g, n, c);
+  }
+  __syncthreads();
+  if (rescale) {
+    if (threadIdx.x < FZ_TILE) {
+      const int l = it.level;
+      const uint64_t q = ld_prime_p(P.primes, l), q5 = as_const(P.md_red)[2 * l + 1];
+      uint64_t s = 0;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) s = add_mod(s, part[t * FZ_TILE + threadIdx.x], q5);
+      const tw2 bi = ld_tw2(reinterpret_cast<const tw2*>(P.inv_b_mod_q), l);
+      aux[K * FZ_PITCH + threadIdx.x] = mul_shoup(xq[l * FZ_PITCH + threadIdx.x] + q5 - s, bi.w, bi.q, q);
+    }
+    __syncthreads();
+  }
+  const uint64_t* add = glob(y ? it.add1 : it.add0);
+  uint64_t* out = glob(y ? it.out1 : it.out0);
+  const int units = ((lout + 15) / 16) * 4;
+  for (int u = wave; u < units; u += FZ_THREADS / 64) {
+    const int ib = u / 4, nb0 = (u % 4) * 2, nb = ld_prime_nb(P.primes, ib * 16);
+    if (nb > 56)
+      down_out<8, 2>(P, it, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
+    else if (nb > 48)
+      down_out<7, 2>(P, it, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
+    else
+      down_out<6, 2>(P, it, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
+  }
+}
+
+// ---------------------------------------------------------------- launch ---
+
+template <bool ARG>
+static void fz_up(const DevParams& P, const FzItem& arg, const FzItem* items, int n, int max_level, bool mul,
+                  hipStream_t st) {
+  const size_t lds = (size_t)(((max_level + 8) & ~7) + P.K) * FZ_PITCH * 8;
+  const dim3 grid((unsigned)(n * (P.N / FZ_TILE)));
+  if (mul)
+    k_fz_up<true, ARG><<<grid, FZ_THREADS, lds, st>>>(P, arg, items);
+  else
+    k_fz_up<false, ARG><<<grid, FZ_THREADS, lds, st>>>(P, arg, items);
+}
+
+template <bool ARG>
+static void fz_down(const DevParams& P, const FzItem& arg, const FzItem* items, int n, int max_level, hipStream_t st) {
+  const size_t lds = ((size_t)(down_aux_rows(P.K) + ((max_level + 8) & ~7)) * FZ_PITCH + 4 * FZ_TILE) * 8;
+  k_fz_down<ARG><<<dim3((unsigned)(2 * n * (P.N / FZ_TILE))), FZ_THREADS, lds, st>>>(P, arg, items);
+}
+
+void fz_up_item(const DevParams& P, const FzItem& it, bool mul, hipStream_t st) {
+  fz_up<true>(P, it, nullptr, 1, it.level, mul, st);
+}
+void fz_down_item(const DevParams& P, const FzItem& it, hipStream_t st) { fz_down<true>(P, it, nullptr, 1, it.level, st); }
+void fz_up_desc(const DevParams& P, const FzItem* items, int n, int max_level, bool mul, hipStream_t st) {
+  fz_up<false>(P, FzItem{}, items, n, max_level, mul, st);
+}
+void fz_down_desc(const DevParams& P, const FzItem* items, int n, int max_level, hipStream_t st) {
+  fz_down<false>(P, FzItem{}, items, n, max_level, st);
+}
+
+int fz_mul(const DevParams& P, const FzItem& it, hipStream_t st) {
+  if (fz_rows_item(P, it, st)) return -1;
+  fz_up_item(P, it, true, st);
+  if (fz_key_item(P, it, st)) return -1;
+  fz_down_item(P, it, st);
+  return 0;
+}
+
+int fz_switch(const DevParams& P, const FzItem& it, hipStream_t st) {
+  fz_up_item(P, it, false, st);
+  if (fz_key_item(P, it, st)) return -1;
+  fz_down_item(P, it, st);
+  return 0;
+}
+
+}  // namespace aoa

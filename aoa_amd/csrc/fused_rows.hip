@@ -1,0 +1,242 @@
+// Row kernels of the fused key switching (fused.hpp): the forward and inverse
+// row stages with the products between them.
+#include <type_traits>
+
+#include "fused.hpp"
+
+namespace aoa {
+
+#define FZ_FIELD(pr_, CALL)                            \
+  switch (ld_prime_field(P.primes, pr_)) {             \
+    case FIELD_FP64: CALL(FieldFp64); break;           \
+    case FIELD_LAZY: CALL(FieldLazy); break;           \
+    default: CALL(FieldStrict); break;                 \
+  }
+
+// Values per thread: four (two stages a round) up to rows of 1024, so that a
+// small call's few rows spread over many waves; eight above.
+template <int LOGM>
+using RowOf = Row<LOGM, (LOGM <= 10 ? 2 : 3)>;
+
+template <int LOGM>
+struct RowId {
+  using G = RowOf<LOGM>;
+  int s, row;
+  uint32_t off;   // byte offset of the thread's first strided element in its limb
+  uint32_t poff;  // of its first packed one
+  uint64_t* L;
+  __device__ __forceinline__ RowId(int tile, uint64_t* lds) {
+    const int rl = G::ROWS == 1 ? 0 : threadIdx.x / G::TS;
+    s = G::ROWS == 1 ? threadIdx.x : threadIdx.x % G::TS;
+    row = tile * G::ROWS + rl;
+    off = (row * G::M + s) * 8;
+    poff = (row * G::M + s * G::V) * 8;
+    L = lds + rl * G::PITCH;
+  }
+};
+
+// The inverse rows of x (packed) and the store.
+template <class F, int LOGM>
+__device__ __forceinline__ void rows_out(const F& f, typename F::V (&x)[RowOf<LOGM>::V], const uint64_t* T, uint64_t* dst,
+                                         const RowId<LOGM>& id) {
+  using G = RowOf<LOGM>;
+  constexpr int LV = LOGM <= 10 ? 2 : 3;
+  const RoundTw<LOGM, LV, G::ROUNDS - 1, F> t(f, T, id.row, id.s);
+  row_inv_from<LOGM, LV, G::ROUNDS - 1>(f, x, t, T, id.row, id.s, id.L);
+#pragma unroll
+  for (int k = 0; k < G::V; ++k) put_byte(dst, id.off + G::TS * 8 * k, f.raw(x[k]));
+}
+
+// ------------------------------------------------------ d2 = a b, its rows --
+template <class F, int LOGM>
+__device__ __forceinline__ void rows_body(const DevParams& P, const uint64_t* a, const uint64_t* b, uint64_t* dst, int pr,
+                                          int tile, uint64_t* lds) {
+  using G = RowOf<LOGM>;
+  constexpr int LV = LOGM <= 10 ? 2 : 3;
+  const F f(ld_prime(P.primes, pr));
+  const uint64_t* T = P.fz.tw[1] + (size_t)pr * P.N * 2;
+  const RowId<LOGM> id(tile, lds);
+  typename F::V x[G::V];
+#pragma unroll
+  for (int k = 0; k < G::V; ++k) {
+    const uint32_t o = id.off + G::TS * 8 * k;
+    x[k] = f.key(f.in(at_byte<uint64_t>(a, o)), at_byte<uint64_t>(b, o));
+  }
+  row_turn<LOGM, LV, 0, G::ROUNDS - 1>(f, x, id.s, id.L);
+  rows_out<F, LOGM>(f, x, T, dst, id);
+}
+
+template <int LOGM, bool ARG>
+__global__ __launch_bounds__(RowOf<LOGM>::THREADS) void k_fz_rows(DevParams P, FzItem arg, const FzItem* items,
+                                                                  const uint32_t* list) {
+  __shared__ uint64_t lds[RowOf<LOGM>::LDS];
+  constexpr int per = 16 / RowOf<LOGM>::ROWS;
+  const uint32_t e = fz_entry<ARG>(list, blockIdx.x / per);
+  const FzItem it = fz_item<ARG>(arg, items, e >> 8);
+  const int i = (int)(e & 255), tile = blockIdx.x % per;
+  const size_t o = (size_t)i * P.N;
+  const uint64_t *a = glob(it.a1) + o, *b = glob(it.b1) + o;
+  uint64_t* d = glob(it.D) + o;
+#define CALL(F) rows_body<F, LOGM>(P, a, b, d, i, tile, lds)
+  FZ_FIELD(i, CALL)
+#undef CALL
+}
+
+// ---------------------------------------------------------- key products --
+// Limb m of an item: Q limbs 0..level, then the special limbs.  HomMul's Q
+// limbs take their NTT-domain input d2 and addends d0, d1 from the operands;
+// other limbs come as forward columns and take the forward rows here, once for
+// both key halves.  y0..y1: the key halves of this workgroup.
+
+// A zero that the compiler does not see through: what depends on it is formed
+// again for each key half instead of staying in registers from one to the next.
+__device__ __forceinline__ uint32_t opaque_zero() {
+  uint32_t z = 0;
+  asm volatile("" : "+s"(z));
+  return z;
+}
+
+template <class F, int LOGM>
+__device__ __forceinline__ void key_body_tensor(const DevParams& P, const FzItem& it, int m, int tile, int y0, int y1,
+                                                uint64_t* lds) {
+  using G = RowOf<LOGM>;
+  constexpr int LV = LOGM <= 10 ? 2 : 3;
+  const F f(ld_prime(P.primes, m));
+  const uint64_t* T = P.fz.tw[1] + (size_t)m * P.N * 2;
+  const RowId<LOGM> id(tile, lds);
+  const size_t o = (size_t)m * P.N;
+  const uint64_t *a0 = glob(it.a0) + o, *a1 = glob(it.a1) + o, *b0 = glob(it.b0) + o, *b1 = glob(it.b1) + o;
+#pragma unroll 1
+  for (int y = y0; y < y1; ++y) {
+    const uint32_t z = opaque_zero(), off = id.off + z;
+    const typename F::W bq = f.tw_u(P.fz.bq + 2 * m, 0);
+    const uint64_t* kp = glob(y ? it.ka : it.kb) + o;
+    typename F::V x[G::V];
+    auto products = [&](auto half) {
+#pragma unroll
+      for (int k = 0; k < G::V; ++k) {
+        const uint32_t i = off + G::TS * 8 * k;
+        x[k] = f.template tensor<half.value>(at_byte<uint64_t>(a0, i), at_byte<uint64_t>(a1, i), at_byte<uint64_t>(b0, i),
+                                             at_byte<uint64_t>(b1, i), at_byte<uint64_t>(kp, i), bq);
+      }
+    };
+    if (y)
+      products(std::integral_constant<int, 1>());
+    else
+      products(std::integral_constant<int, 0>());
+    row_turn<LOGM, LV, 0, G::ROUNDS - 1>(f, x, id.s, id.L);
+    rows_out<F, LOGM>(f, x, T + z, glob(y ? it.P1 : it.P0) + o, id);
+  }
+}
+
+template <class F, int LOGM>
+__device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, int m, int pr, int tile, int y0, int y1,
+                                         uint64_t* lds) {
+  using G = RowOf<LOGM>;
+  constexpr int LV = LOGM <= 10 ? 2 : 3;
+  const F f(ld_prime(P.primes, pr));
+  const int N = P.N, L = it.level + 1;
+  const uint64_t* T = P.fz.tw[1] + (size_t)pr * N * 2;
+  const RowId<LOGM> id(tile, lds);
+  typename F::V x0[G::V];
+  const uint64_t* src = m < L ? glob(it.XQ) + (size_t)m * N : glob(it.X) + (size_t)(m - L) * N;
+#pragma unroll
+  for (int k = 0; k < G::V; ++k) x0[k] = f.raw_in(at_byte<uint64_t>(src, id.off + G::TS * 8 * k));
+  row_fwd<LOGM, LV>(f, x0, P.fz.tw[0] + (size_t)pr * N * 2, id.row, id.s, id.L);
+#pragma unroll
+  for (int k = 0; k < G::V; ++k) x0[k] = f.factor(x0[k]);
+#pragma unroll 1
+  for (int y = y0; y < y1; ++y) {
+    const uint32_t z = opaque_zero();
+    // packed, as the inverse rows begin: a thread's values are 16-byte loads
+    const uint64_t* kp = glob(y ? it.ka : it.kb) + (size_t)pr * N;
+    typename F::V x[G::V];
+#pragma unroll
+    for (int k = 0; k < G::V; k += 2) {
+      const tw2 v = at_byte<tw2>(kp, id.poff + 8 * k);
+      x[k] = f.key(x0[k], v.w);
+      x[k + 1] = f.key(x0[k + 1], v.q);
+    }
+    if (y > y0) __syncthreads();  // the first half's last exchange has been read
+    rows_out<F, LOGM>(f, x, T + z, glob(y ? it.P1 : it.P0) + (size_t)m * N, id);
+  }
+}
+
+// ysplit: one workgroup per key half (the two halves of a tile `n` blocks apart).
+template <int LOGM, bool ARG>
+__global__ __launch_bounds__(RowOf<LOGM>::THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_fz_key(
+    DevParams P, FzItem arg, const FzItem* items, const uint32_t* list, int n, int ysplit) {
+  __shared__ uint64_t lds[RowOf<LOGM>::LDS];
+  constexpr int per = 16 / RowOf<LOGM>::ROWS;
+  const int y = ysplit ? (int)blockIdx.x / n : 0;
+  const int w = ysplit ? (int)blockIdx.x % n : (int)blockIdx.x;
+  const uint32_t e = fz_entry<ARG>(list, w / per);
+  const FzItem it = fz_item<ARG>(arg, items, e >> 8);
+  const int m = (int)(e & 255), L = it.level + 1, pr = m < L ? m : P.k + m - L;
+  const int y0 = y, y1 = ysplit ? y + 1 : 2;
+  if (it.a0 && m < L) {
+#define CALL(F) key_body_tensor<F, LOGM>(P, it, m, w % per, y0, y1, lds)
+    FZ_FIELD(pr, CALL)
+#undef CALL
+  } else {
+#define CALL(F) key_body<F, LOGM>(P, it, m, pr, w % per, y0, y1, lds)
+    FZ_FIELD(pr, CALL)
+#undef CALL
+  }
+}
+
+// ---------------------------------------------------------------- launch ---
+
+static int log2_of(int n) {
+  int g = 0;
+  while ((1 << g) < n) ++g;
+  return g;
+}
+
+#define FZ_DISPATCH_M(CALL)          \
+  switch (log2_of(P.N) - 4) {        \
+    case 7: CALL(7); break;          \
+    case 8: CALL(8); break;          \
+    case 9: CALL(9); break;          \
+    case 10: CALL(10); break;        \
+    case 11: CALL(11); break;        \
+    case 12: CALL(12); break;        \
+    default: return -1;              \
+  }
+
+template <bool ARG>
+static int fz_rows(const DevParams& P, const FzItem& arg, const FzItem* items, const uint32_t* list, int n, hipStream_t st) {
+#define CALL(LM) k_fz_rows<LM, ARG><<<dim3(n * 16 / RowOf<LM>::ROWS), RowOf<LM>::THREADS, 0, st>>>(P, arg, items, list)
+  FZ_DISPATCH_M(CALL)
+#undef CALL
+  return 0;
+}
+
+// One workgroup per key half while both halves together leave the chip
+// partly idle: the forward rows are then done twice, on idle units.
+template <bool ARG>
+static int fz_key(const DevParams& P, const FzItem& arg, const FzItem* items, const uint32_t* list, int n, hipStream_t st) {
+#define CALL(LM)                                                                                                       \
+  {                                                                                                                    \
+    const int blocks = n * 16 / RowOf<LM>::ROWS, ysplit = blocks * (RowOf<LM>::THREADS / 64) <= 2048 ? 1 : 0;          \
+    k_fz_key<LM, ARG><<<dim3(blocks << ysplit), RowOf<LM>::THREADS, 0, st>>>(P, arg, items, list, blocks, ysplit);     \
+  }
+  FZ_DISPATCH_M(CALL)
+#undef CALL
+  return 0;
+}
+
+int fz_rows_item(const DevParams& P, const FzItem& it, hipStream_t st) {
+  return fz_rows<true>(P, it, nullptr, nullptr, it.level + 1, st);
+}
+int fz_key_item(const DevParams& P, const FzItem& it, hipStream_t st) {
+  return fz_key<true>(P, it, nullptr, nullptr, it.level + 1 + P.K, st);
+}
+int fz_rows_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, hipStream_t st) {
+  return fz_rows<false>(P, FzItem{}, items, list, n, st);
+}
+int fz_key_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, hipStream_t st) {
+  return fz_key<false>(P, FzItem{}, items, list, n, st);
+}
+
+}  // namespace aoa

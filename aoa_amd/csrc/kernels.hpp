@@ -24,6 +24,20 @@ int ntt_forward(const DevParams& P, LimbMap m, int N1, hipStream_t st);
 int ntt_inverse(const DevParams& P, LimbMap m, int N1, const uint64_t* key0, const uint64_t* key1,
                 hipStream_t st, const uint64_t* add0 = nullptr, const uint64_t* add1 = nullptr);
 
+// Fused key switching (fused.hip).  fz_mul: HomMul + relinearisation (+ rescale)
+// of one item; fz_switch: key switching of one item.  Workspace in the item.
+int fz_mul(const DevParams& P, const FzItem& it, hipStream_t st);
+int fz_switch(const DevParams& P, const FzItem& it, hipStream_t st);
+int fz_rows_item(const DevParams& P, const FzItem& it, hipStream_t st);
+void fz_up_item(const DevParams& P, const FzItem& it, bool mul, hipStream_t st);
+int fz_key_item(const DevParams& P, const FzItem& it, hipStream_t st);
+void fz_down_item(const DevParams& P, const FzItem& it, hipStream_t st);
+// The same stage by stage over device tables: `list` entries are item << 8 | limb.
+int fz_rows_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, hipStream_t st);
+void fz_up_desc(const DevParams& P, const FzItem* items, int n, int max_level, bool mul, hipStream_t st);
+int fz_key_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, hipStream_t st);
+void fz_down_desc(const DevParams& P, const FzItem* items, int n, int max_level, hipStream_t st);
+
 // out = a op b (out = a*b + c for MULADD) over nlimbs limbs mapped to primes
 // as in LimbMap (qlimbs Q limbs from prime0, then special limbs).
 void launch_encrypt_combine(const DevParams& P, uint64_t* c0, uint64_t* c1, const uint64_t* pkb,

@@ -97,6 +97,10 @@ static std::string select_primes(int k, int kl, int prec, std::vector<aoa_prime_
     if (nb > 56 && (u128)kl * bmax + 2 * (u128)kl > ((u128)1 << nb))
       return "special primes too large for ModDown's sums of a wide Q prime";
   }
+  // The strict butterflies' products fold at bit 63 (FieldStrict): primes
+  // wider than 56 bits are 2^63 - c with c < 2^26.
+  for (const aoa_prime_entry& e : *q)
+    if ((e.p >> 56) && ((uint64_t)1 << 63) - e.p >= ((uint64_t)1 << 26)) return "wide Q primes must be just below 2^63";
   // ModDown's rescale forms q_i + add_i - top with top < q_l for i < l, which
   // needs q_l < q_i: the Q primes decrease (q0 first, then the bucket in
   // decreasing order).
@@ -194,6 +198,9 @@ std::string build_host_params(int N, int k, int kl, int prec, HostParams* out) {
     d.eps = (((uint64_t)1) << d.nb) - p;
     d.r64 = (uint64_t)((((unsigned __int128)1) << 64) % p);
     d.r64_q = shoup_quot(d.r64, p);
+    d.fp = (double)p;
+    d.fpinv = 1.0 / (double)p;
+    d.field = field_of((int)d.nb);
     P.dprimes.push_back(d);
   }
   for (int j = 0; j < kl; ++j)

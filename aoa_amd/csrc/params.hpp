@@ -41,7 +41,17 @@ struct DevPrime {
   // ModUp must reduce those residues before multiplying (q0 is checked
   // separately).
   uint32_t modup_reduce;
+  // Arithmetic of the row / column transforms and key products (fields.hpp):
+  // p and 1/p rounded to FP64, and which of the forms the prime takes.
+  double fp, fpinv;
+  uint32_t field;
+  uint32_t pad;
 };
+
+// FIELD_STRICT: primes above 2^56 (q0), canonical residues; FIELD_LAZY: below
+// 2^56, lazy 64-bit residues; FIELD_FP64: at most 48 bits, signed FP64 values.
+enum { FIELD_STRICT = 0, FIELD_LAZY = 1, FIELD_FP64 = 2 };
+AOA_HD uint32_t field_of(int nb) { return nb > 56 ? FIELD_STRICT : nb > 48 ? FIELD_LAZY : FIELD_FP64; }
 
 // Pointers into one device allocation holding every table of a parameter set.
 // Passed to kernels by value.
@@ -51,6 +61,38 @@ struct DevPrime {
 constexpr double kGaussSigma = 3.2;
 constexpr int kGaussHalf = 32;
 constexpr int kHammingWeight = 64;
+
+// One output residue of a basis conversion on the matrix cores: the sum of
+// signed byte products V, plus `off`, is a non-negative value congruent to the
+// wanted sum; c_48, c_32 and c_16 (2^48/p, 2^32/p, 2^16/p) weigh V's columns in
+// the FP32 quotient estimate and c_b is its constant part.
+struct ConvOut {
+  uint64_t p;
+  uint64_t off;
+  float c_48, c_32, c_16, c_b;
+};
+
+// Tables of the fused kernels, N = 16 x M with M = N/16 (build_fused_tables).
+struct FusedDev {
+  // [0: forward, 1: inverse]: [k+K][2N] words, entry i psi^(+-brev(i)); a FIELD_FP64
+  // prime's block holds N balanced doubles, another's N (w, quotient) pairs
+  const uint64_t* tw[2];
+  // last inverse stage's two constants, 4 words per entry ((w, quotient) pairs, or two doubles):
+  const uint64_t* lc;      // [k+K]: N^-1, psi^-brev(1) N^-1
+  const uint64_t* lc_key;  // [k+K]: the same, special limbs also times (B/b_j)^-1
+  const uint64_t* lc_up;   // [k][k] (l, i): the same times (Q_l/q_i)^-1
+  const uint64_t* bq;      // [k][2]: B mod q_i (pair, or one double)
+  // ModUp and ModDown as products of signed bytes, in the operand order of
+  // the 16x16x64 matrix instruction: [block of 16 outputs][digit][step of 8 inputs][lane][16]
+  const uint8_t* mu_w;     // per level: mu_stride bytes
+  const uint8_t* md_w;
+  const ConvOut* mu_out;   // [k][K] (l, j)
+  const ConvOut* md_out;   // [k]
+  const double* scr;       // [K][4][16][2]: frac(c/q_i), frac(2^28 c/q_i) for c = (B/b_j) mod q_i, i = g + 4n
+  const double* scr_thr;   // [k]: screen bound of q_i
+  uint32_t mu_stride;      // bytes of mu_w per level
+  int mu_kb, md_kb;        // steps of 8 inputs the layouts hold
+};
 
 struct DevParams {
   int N, logN, k, K;
@@ -98,6 +140,7 @@ struct DevParams {
   // halves of (Q_l/q_i) mod b_j and their sum, row i = k: of
   // (2^56 Q_l/q_0) mod b_j; positions as in build_host_params
   const uint32_t* mu_terms;
+  FusedDev fz;  // tables of the fused key-switching kernels (fused.hip)
 };
 
 // The device layout of the ModDown product constants: MdConst's first six
@@ -135,6 +178,19 @@ struct HostParams {
   std::vector<uint32_t> md_negb;    // k * 4
   std::vector<uint32_t> mu_terms;   // k * (k + 1) * kp * 4
 };
+
+// Host tables behind FusedDev.
+struct FusedTables {
+  std::vector<uint64_t> tw[2], lc, lc_key, lc_up, bq;
+  std::vector<uint8_t> mu_w, md_w;
+  std::vector<ConvOut> mu_out, md_out;
+  std::vector<double> scr, scr_thr;
+  uint32_t mu_stride = 0;
+  int mu_kb = 0, md_kb = 0;
+};
+void build_fused_tables(const HostParams& h, FusedTables* out);
+// Bytes of a prime's balanced digits: 6 up to 48 bits, 7 up to 56, else 8.
+inline int conv_digits(int nb) { return nb <= 48 ? 6 : nb <= 56 ? 7 : 8; }
 
 // Builds every table.  Returns an empty string on success, else the reason
 // (unsupported precision, bucket too small, N not supported by a prime).
