@@ -32,37 +32,30 @@ struct BatchGroup {
   int n_pre_fwd = 0;
   NttDesc* d_pre_inv = nullptr;
   int n_pre_inv = 0;
-  TensorDesc* d_tensor = nullptr;
-  int n_tensor = 0;
   AutoDesc* d_auto = nullptr;
   int n_auto = 0;
-  NttDesc* d_intt3 = nullptr;  // mul: INTT of d0, d1, d2
-  int n_intt3 = 0;
-  NttDesc* d_trow = nullptr;  // mul (N >= 8192): inverse NTT of d2 = a1 b1, the product in its first pass
-  int n_trow = 0, ns_trow = -1;
-  ModUpDesc* d_modup = nullptr;
-  int n_modup = 0;
+  // HomMuls and rotations (fused.hpp): items, HomMuls first, and the limbs of
+  // each stage's launches, item << 8 | limb
+  FzItem* d_items = nullptr;
+  int n_mul = 0, n_rot = 0;
   int max_level = 0;
-  NttDesc* d_fwd = nullptr;  // NTT of ModUp output (and of the rotated c1)
-  int n_fwd = 0;
-  KeyDesc2* d_key2 = nullptr;  // key product + first INTT pass, both key halves
-  int n_key2 = 0;
-  NttDesc* d_keycol = nullptr;  // second INTT pass of the key products
-  int n_keycol = 0;
-  ModDownDesc* d_moddown = nullptr;
-  int n_moddown = 0;
-  // leading descriptors whose prime is 2^61 or above (-1: not a prefix)
-  int ns_key2 = -1;
+  uint32_t* d_rows = nullptr;  // d2 = a1 b1 and its inverse rows
+  uint32_t* d_keyb = nullptr;  // key products of the special limbs
+  uint32_t* d_keyq = nullptr;  // key products of the Q limbs
+  int n_rows = 0, n_keyb = 0, n_keyq = 0;
+  // leading entries of rows and keyq whose prime is above 2^56 (-1: not split)
+  int ns_rows = -1, ns_keyq = -1;
+  int field_q = 0, field_b = 0;  // form of the Q primes after q0, of the special primes
 };
 
 struct BatchLayer {
   std::vector<BatchGroup> groups;
 };
 
-// Workspace limbs of one HomMul item: X (L + K), d0, d1, d2 (L each), P0, P1
-// (L + K each); from N = 8192 up (fused) the tensor product is never stored
-// and X's Q limbs are not needed: X's special limbs (K), d2 (L), P0, P1.
-size_t mul_ws_limbs(int L, int K, bool fused) { return (fused ? 3 : 6) * (size_t)L + 3 * (size_t)K; }
+// Workspace limbs of one HomMul item: d2 after its inverse rows (L), the
+// special limbs (K), P0, P1 (L + K each); of a rotation: the rotated
+// polynomials (L each), the forward columns of the second (L + K), P0, P1.
+size_t mul_ws_limbs(int L, int K) { return 3 * (size_t)L + 3 * (size_t)K; }
 size_t rot_ws_limbs(int L, int K) { return 5 * (size_t)L + 3 * (size_t)K; }
 
 }  // namespace aoa
@@ -96,45 +89,6 @@ static BatchGroup& group_for(aoa_batch* b, const aoa_params* p, const uint64_t* 
   return g;
 }
 
-// Key-switching product descriptors of one item: X (Lq Q limbs at XQ, K
-// special limbs at XB, NTT domain) times both key halves into P0 / P1, one
-// KeyDesc2 per limb for the first inverse pass and one NttDesc per output
-// limb for the second.  A0 / A1 (Lq limbs, NTT domain, or null) join the Q
-// limbs of P0 / P1 times B mod q, so that ModDown adds them (two-pass
-// transforms only).  With c1 / c2 set (HomMul's operands, two-pass
-// transforms) the Q limbs take X = a1 b1 and the adds d0, d1 from the
-// operands in the pass instead (KeyDesc2::ab), and XQ is not read (null).
-static void add_key_descs(std::vector<KeyDesc2>& key2, std::vector<NttDesc>& keycol, const uint64_t* XQ,
-                          const uint64_t* XB, uint64_t* P0, uint64_t* P1, const uint64_t* kb, const uint64_t* ka,
-                          const uint64_t* A0, const uint64_t* A1, int Lq, int K, int k, size_t N,
-                          const uint64_t* const* c1 = nullptr, const uint64_t* const* c2 = nullptr) {
-  for (int m = 0; m < Lq + K; ++m) {
-    const int pr = m < Lq ? m : k + (m - Lq);
-    const size_t o = (size_t)m * N;
-    KeyDesc2 e;
-    e.src = m < Lq ? (XQ ? XQ + o : nullptr) : XB + (size_t)(m - Lq) * N;
-    e.dst[0] = P0 + o;
-    e.dst[1] = P1 + o;
-    e.key[0] = kb + (size_t)pr * N;
-    e.key[1] = ka + (size_t)pr * N;
-    e.add[0] = A0 && m < Lq ? A0 + o : nullptr;
-    e.add[1] = A1 && m < Lq ? A1 + o : nullptr;
-    const bool t = c1 && c2 && m < Lq;
-    e.ab[0] = t ? c1[0] + o : nullptr;
-    e.ab[1] = t ? c1[1] + o : nullptr;
-    e.ab[2] = t ? c2[0] + o : nullptr;
-    e.ab[3] = t ? c2[1] + o : nullptr;
-    e.prime = pr;
-    e.pad = 0;
-    key2.push_back(e);
-  }
-  for (int y = 0; y < 2; ++y)
-    for (int m = 0; m < Lq + K; ++m) {
-      uint64_t* d = (y ? P1 : P0) + (size_t)m * N;
-      keycol.push_back({d, d, nullptr, m < Lq ? m : k + (m - Lq), 0});
-    }
-}
-
 // Workspace bytes (max over layers of the layer's sum) and descriptor bytes.
 void batch_sizes(const aoa_batch* b, size_t* ws_bytes, size_t* desc_bytes) {
   size_t ws = 0, desc = 0;
@@ -144,19 +98,16 @@ void batch_sizes(const aoa_batch* b, size_t* ws_bytes, size_t* desc_bytes) {
       const size_t N = g.params->host.N, K = g.params->host.K;
       for (auto& it : g.muls) {
         const size_t Lq = it.level + 1;
-        s += mul_ws_limbs((int)Lq, (int)K, N >= 8192) * N * 8;
-        desc += Lq * (sizeof(TensorDesc) + 3 * sizeof(NttDesc)) + sizeof(ModUpDesc) +
-                K * sizeof(NttDesc) +
-                (Lq + K) * sizeof(KeyDesc2) + 2 * (Lq + K) * sizeof(NttDesc) + 2 * sizeof(ModDownDesc);
+        s += mul_ws_limbs((int)Lq, (int)K) * N * 8;
+        desc += sizeof(FzItem) + (2 * Lq + K) * sizeof(uint32_t);
       }
       for (auto& it : g.rots) {
         const size_t Lq = it.level + 1;
         s += rot_ws_limbs((int)Lq, (int)K) * N * 8;
-        desc += Lq * (2 * sizeof(AutoDesc) + sizeof(NttDesc)) + sizeof(ModUpDesc) + K * sizeof(NttDesc) +
-                (Lq + K) * sizeof(KeyDesc2) + 2 * (Lq + K) * sizeof(NttDesc) + 2 * sizeof(ModDownDesc);
+        desc += sizeof(FzItem) + 2 * Lq * sizeof(AutoDesc) + (Lq + K) * sizeof(uint32_t);
       }
       for (auto& it : g.ntts) desc += 2 * (size_t)(it.level + 1) * sizeof(NttDesc);
-      desc += 16 * 256;  // per-table alignment slack
+      desc += 8 * 256;  // per-table alignment slack
     }
     ws = std::max(ws, s);
   }
@@ -186,11 +137,9 @@ size_t batch_fill(aoa_batch* b, uint64_t* ws, char* host, char* dev, size_t desc
       const DevParams& P = g.params->dev;
       const size_t N = (size_t)P.N;
       const int k = P.k, K = P.K;
-      std::vector<TensorDesc> tens;
-      std::vector<NttDesc> prefwd, preinv, intt3, fwd, keycol, trow;
-      std::vector<KeyDesc2> key2;
-      std::vector<ModUpDesc> mu;
-      std::vector<ModDownDesc> md;
+      std::vector<NttDesc> prefwd, preinv;
+      std::vector<FzItem> items;
+      std::vector<uint32_t> rows, keyb, keyq;
       std::vector<AutoDesc> au;
       g.max_level = 0;
       for (auto& it : g.ntts)
@@ -199,81 +148,65 @@ size_t batch_fill(aoa_batch* b, uint64_t* ws, char* host, char* dev, size_t desc
             uint64_t* l = it.poly[y] + (size_t)i * N;
             (it.dir == AOA_FORWARD ? prefwd : preinv).push_back({l, l, nullptr, i, 0});
           }
+      auto key_entries = [&](uint32_t item, int Lq) {
+        for (int m = 0; m < Lq; ++m) keyq.push_back(item << 8 | m);
+        for (int m = Lq; m < Lq + K; ++m) keyb.push_back(item << 8 | m);
+      };
       for (auto& it : g.muls) {
         const int lv = it.level, Lq = lv + 1;
+        const uint32_t item = (uint32_t)items.size();
         g.max_level = std::max(g.max_level, lv);
-        const bool fused = P.N >= 8192;
-        // unfused: X (Lq + K), D0, D1, D2, P0, P1; fused: X's special limbs, D2, P0, P1
-        uint64_t* X = fused ? nullptr : w;
-        uint64_t* XB = fused ? w : X + (size_t)Lq * N;
-        uint64_t* D0 = fused ? nullptr : XB + (size_t)K * N;
-        uint64_t* D1 = fused ? nullptr : D0 + (size_t)Lq * N;
-        uint64_t* D2 = fused ? XB + (size_t)K * N : D1 + (size_t)Lq * N;
-        uint64_t* P0 = D2 + (size_t)Lq * N;
-        uint64_t* P1 = P0 + (size_t)(Lq + K) * N;
-        w += mul_ws_limbs(Lq, K, fused) * N;
-        // From N = 8192 up the transforms are two-pass and the tensor product
-        // is never stored: d2 = a1 b1 is formed in the first inverse pass of
-        // d2 (for ModUp), and again with d0 and d1 in the key products' first
-        // pass, where d0, d1 join the Q limbs as B d0, B d1: ModDown is linear
-        // in its Q limbs and its B-limb sum does not see them, so
-        // ModDown(X + B d) = ModDown(X) + d, residue for residue, and d0, d1
-        // need no transform.  Below, a tensor kernel, the single-workgroup
-        // transforms, and the additions in ModDown.
-        for (int i = 0; i < Lq && fused; ++i) {
-          const size_t o = (size_t)i * N;
-          trow.push_back({it.c1[1] + o, D2 + o, it.c2[1] + o, i, 0});
-        }
-        for (int i = 0; i < Lq && !fused; ++i) {
-          const size_t o = (size_t)i * N;
-          TensorDesc t;
-          t.a0 = it.c1[0] + o;
-          t.a1 = it.c1[1] + o;
-          t.b0 = it.c2[0] + o;
-          t.b1 = it.c2[1] + o;
-          t.d0 = D0 + o;
-          t.d1 = D1 + o;
-          t.d2 = X + o;
-          t.prime = i;
-          t.pad = 0;
-          tens.push_back(t);
-          intt3.push_back({D0 + o, D0 + o, nullptr, i, 0});
-          intt3.push_back({D1 + o, D1 + o, nullptr, i, 0});
-          intt3.push_back({X + o, D2 + o, nullptr, i, 0});
-        }
-        mu.push_back({D2, XB, lv, 0});
-        for (int j = 0; j < K; ++j) fwd.push_back({XB + (size_t)j * N, XB + (size_t)j * N, nullptr, k + j, 0});
-        add_key_descs(key2, keycol, X, XB, P0, P1, g.evk_b, g.evk_a, nullptr, nullptr, Lq, K, k, N,
-                      fused ? it.c1 : nullptr, fused ? it.c2 : nullptr);
-        for (int y = 0; y < 2; ++y)
-          md.push_back({y ? P1 : P0, (y ? P1 : P0) + (size_t)Lq * N, fused ? nullptr : (y ? D1 : D0), it.out[y],
-                        lv, 1});
+        FzItem z{};
+        z.a0 = it.c1[0];
+        z.a1 = it.c1[1];
+        z.b0 = it.c2[0];
+        z.b1 = it.c2[1];
+        z.kb = g.evk_b;
+        z.ka = g.evk_a;
+        z.D = w;
+        z.X = z.D + (size_t)Lq * N;
+        z.P0 = z.X + (size_t)K * N;
+        z.P1 = z.P0 + (size_t)(Lq + K) * N;
+        z.out0 = it.out[0];
+        z.out1 = it.out[1];
+        z.level = lv;
+        z.rescale = 1;
+        w += mul_ws_limbs(Lq, K) * N;
+        items.push_back(z);
+        for (int i = 0; i < Lq; ++i) rows.push_back(item << 8 | i);
+        key_entries(item, Lq);
       }
+      g.n_mul = (int)items.size();
       for (auto& it : g.rots) {
         const int lv = it.level, Lq = lv + 1;
+        const uint32_t item = (uint32_t)items.size();
         g.max_level = std::max(g.max_level, lv);
         uint64_t* R0 = w;
         uint64_t* R1 = R0 + (size_t)Lq * N;
-        uint64_t* X = R1 + (size_t)Lq * N;
-        uint64_t* P0 = X + (size_t)(Lq + K) * N;
-        uint64_t* P1 = P0 + (size_t)(Lq + K) * N;
-        w += rot_ws_limbs(Lq, K) * N;
         const uint64_t ginv = galois_inverse(galois_of(it.rot_slots, P.N), P.N);
         for (int i = 0; i < Lq; ++i) {
           const size_t o = (size_t)i * N;
           au.push_back({it.in[0] + o, R0 + o, it.accumulate ? it.in[0] + o : nullptr, ginv, i, 0});
           au.push_back({it.in[1] + o, R1 + o, nullptr, ginv, i, 0});
-          fwd.push_back({R1 + o, X + o, nullptr, i, 0});
         }
-        mu.push_back({R1, X + (size_t)Lq * N, lv, 0});
-        for (int j = 0; j < K; ++j)
-          fwd.push_back({X + (size_t)(Lq + j) * N, X + (size_t)(Lq + j) * N, nullptr, k + j, 0});
-        add_key_descs(key2, keycol, X, X + (size_t)Lq * N, P0, P1, it.rtk_b, it.rtk_a, nullptr, nullptr, Lq, K, k, N);
-        for (int y = 0; y < 2; ++y) {
-          const uint64_t* add = y == 0 ? R0 : (it.accumulate ? it.in[1] : nullptr);
-          md.push_back({y ? P1 : P0, (y ? P1 : P0) + (size_t)Lq * N, add, it.out[y], lv, 0});
-        }
+        FzItem z{};
+        z.d = R1;
+        z.kb = it.rtk_b;
+        z.ka = it.rtk_a;
+        z.XQ = R1 + (size_t)Lq * N;
+        z.X = z.XQ + (size_t)Lq * N;
+        z.P0 = z.X + (size_t)K * N;
+        z.P1 = z.P0 + (size_t)(Lq + K) * N;
+        z.add0 = R0;
+        z.add1 = it.accumulate ? it.in[1] : nullptr;
+        z.out0 = it.out[0];
+        z.out1 = it.out[1];
+        z.level = lv;
+        w += rot_ws_limbs(Lq, K) * N;
+        items.push_back(z);
+        key_entries(item, Lq);
       }
+      g.n_rot = (int)items.size() - g.n_mul;
       // Prime-major order: the limbs of one prime from every item run next
       // to each other, so their workgroups (spread over the XCDs by block
       // index) find that prime's twiddles, and in the key stage its key
@@ -286,57 +219,51 @@ size_t batch_fill(aoa_batch* b, uint64_t* ws, char* host, char* dev, size_t desc
       };
       by_prime(prefwd);
       by_prime(preinv);
-      by_prime(intt3);
-      by_prime(fwd);
-      by_prime(key2);
-      by_prime(keycol);
-      by_prime(trow);
-      // The butterflies of primes of 2^61 and above (the 63-bit q0) are not
-      // lazy; they sort first, and the key stage's first pass over the other
-      // limbs is launched in its lazy-only form (98 instead of 160 registers,
-      // four waves per SIMD instead of three).  The other stages gain nothing
-      // from the split (their occupancy is bound by LDS) and keep one launch.
-      auto strict_prefix = [&](const auto& v) -> int {
-        const std::vector<uint64_t>& pr = g.params->host.primes;
-        int n = 0;
-        while (n < (int)v.size() && pr[v[n].prime] >= (1ull << 61)) ++n;
-        for (size_t t = n; t < v.size(); ++t)
-          if (pr[v[t].prime] >= (1ull << 61)) return -1;
-        return n;
-      };
-      // Small stages (a serving step of a few requests) keep one launch by
-      // default: the split pays only where a launch fills the GPU.  The split
-      // needs the q0 limbs first, i.e. prime-major order.
+      // Q limbs come first in an item, so in each list the entries of one prime
+      // are those of one limb (special limbs: of one place after level + 1)
+      auto prime_of = [&](uint32_t e) { return (int)(e & 255) - (items[e >> 8].level + 1); };
+      if (pm) {
+        auto by_limb = [](uint32_t a, uint32_t b) { return (a & 255) < (b & 255); };
+        std::stable_sort(rows.begin(), rows.end(), by_limb);
+        std::stable_sort(keyq.begin(), keyq.end(), by_limb);
+        std::stable_sort(keyb.begin(), keyb.end(), [&](uint32_t a, uint32_t b) { return prime_of(a) < prime_of(b); });
+      }
+      // The limbs of primes wider than 2^56 (q0), which sort first, take another
+      // form of arithmetic; with them in a launch of their own the others'
+      // launch compiles for its form alone and holds fewer registers.  Small
+      // stages (a serving step of a few requests) keep one launch by default:
+      // the split pays only where a launch fills the GPU.
       constexpr size_t kSplitMin = 256;
-      auto split_at = [&](const auto& v) -> int {
+      auto split_at = [&](const std::vector<uint32_t>& v) -> int {
         if (b->opt.strict_split < 0 || !pm) return -1;
         if (b->opt.strict_split == 0 && v.size() < kSplitMin) return -1;
-        return strict_prefix(v);
+        const auto& dp = g.params->host.dprimes;
+        int n = 0;
+        while (n < (int)v.size() && dp[v[n] & 255].field == FIELD_STRICT) ++n;
+        for (size_t t = n; t < v.size(); ++t)
+          if (dp[v[t] & 255].field != dp[v[n] & 255].field) return -1;  // not in order
+        return n;
       };
-      g.ns_key2 = split_at(key2);
-      g.ns_trow = split_at(trow);
-      g.n_trow = (int)trow.size();
-      g.d_trow = (NttDesc*)(trow.empty() ? nullptr : put(trow.data(), trow.size() * sizeof(NttDesc)));
+      g.field_q = (int)g.params->host.dprimes[k > 1 ? 1 : 0].field;
+      g.field_b = (int)g.params->host.dprimes[k].field;
+      g.ns_rows = split_at(rows);
+      g.ns_keyq = split_at(keyq);
+      g.n_rows = (int)rows.size();
+      g.n_keyb = (int)keyb.size();
+      g.n_keyq = (int)keyq.size();
       g.n_pre_fwd = (int)prefwd.size();
       g.n_pre_inv = (int)preinv.size();
-      g.n_tensor = (int)tens.size();
-      g.n_intt3 = (int)intt3.size();
       g.n_auto = (int)au.size();
-      g.n_fwd = (int)fwd.size();
-      g.n_modup = (int)mu.size();
-      g.n_key2 = (int)key2.size();
-      g.n_keycol = (int)keycol.size();
-      g.n_moddown = (int)md.size();
       g.d_pre_fwd = (NttDesc*)(prefwd.empty() ? nullptr : put(prefwd.data(), prefwd.size() * sizeof(NttDesc)));
       g.d_pre_inv = (NttDesc*)(preinv.empty() ? nullptr : put(preinv.data(), preinv.size() * sizeof(NttDesc)));
-      g.d_tensor = (TensorDesc*)(tens.empty() ? nullptr : put(tens.data(), tens.size() * sizeof(TensorDesc)));
-      g.d_intt3 = (NttDesc*)(intt3.empty() ? nullptr : put(intt3.data(), intt3.size() * sizeof(NttDesc)));
+      g.d_items = (FzItem*)(items.empty() ? nullptr : put(items.data(), items.size() * sizeof(FzItem)));
+      auto put_list = [&](const std::vector<uint32_t>& v) {
+        return (uint32_t*)(v.empty() ? nullptr : put(v.data(), v.size() * sizeof(uint32_t)));
+      };
+      g.d_rows = put_list(rows);
+      g.d_keyb = put_list(keyb);
+      g.d_keyq = put_list(keyq);
       g.d_auto = (AutoDesc*)(au.empty() ? nullptr : put(au.data(), au.size() * sizeof(AutoDesc)));
-      g.d_fwd = (NttDesc*)(fwd.empty() ? nullptr : put(fwd.data(), fwd.size() * sizeof(NttDesc)));
-      g.d_modup = (ModUpDesc*)(mu.empty() ? nullptr : put(mu.data(), mu.size() * sizeof(ModUpDesc)));
-      g.d_key2 = (KeyDesc2*)(key2.empty() ? nullptr : put(key2.data(), key2.size() * sizeof(KeyDesc2)));
-      g.d_keycol = (NttDesc*)(keycol.empty() ? nullptr : put(keycol.data(), keycol.size() * sizeof(NttDesc)));
-      g.d_moddown = (ModDownDesc*)(md.empty() ? nullptr : put(md.data(), md.size() * sizeof(ModDownDesc)));
     }
   }
   return overflow ? 0 : used;
@@ -394,36 +321,28 @@ int batch_enqueue(aoa_batch* b, hipStream_t st, StageTimer* tm) {
         [&](BatchGroup& g) { return ntt_forward_desc(launch_params(b, g), g.d_pre_fwd, g.n_pre_fwd, 0, st); });
     run(AOA_STAGE_PRE_INV, [](BatchGroup& g) { return g.n_pre_inv > 0; },
         [&](BatchGroup& g) { return ntt_inverse_desc(launch_params(b, g), g.d_pre_inv, g.n_pre_inv, 0, st); });
-    run(AOA_STAGE_TENSOR, [](BatchGroup& g) { return g.n_tensor > 0; }, [&](BatchGroup& g) {
-      launch_tensor_desc(launch_params(b, g), g.d_tensor, g.n_tensor, st);
-      return 0;
-    });
     run(AOA_STAGE_AUTOMORPHISM, [](BatchGroup& g) { return g.n_auto > 0; }, [&](BatchGroup& g) {
       launch_automorphism_desc(launch_params(b, g), g.d_auto, g.n_auto, st);
       return 0;
     });
-    run(AOA_STAGE_INTT, [](BatchGroup& g) { return g.n_intt3 > 0 || g.n_trow > 0; }, [&](BatchGroup& g) {
-      // d2 goes to ModUp only, whose Shoup products take [0, 2p)
-      if (g.n_trow > 0 && ntt_inverse_desc(launch_params(b, g), g.d_trow, g.n_trow, 0, st, g.ns_trow, false))
-        return -1;
-      return g.n_intt3 > 0 ? ntt_inverse_desc(launch_params(b, g), g.d_intt3, g.n_intt3, 0, st) : 0;
+    run(AOA_STAGE_INTT, [](BatchGroup& g) { return g.n_rows > 0; }, [&](BatchGroup& g) {
+      return fz_rows_desc(launch_params(b, g), g.d_items, g.d_rows, g.n_rows, g.ns_rows, g.field_q, st);
     });
-    run(AOA_STAGE_MODUP, [](BatchGroup& g) { return g.n_modup > 0; }, [&](BatchGroup& g) {
-      launch_modup_desc(launch_params(b, g), g.d_modup, g.n_modup, g.max_level, st);
+    auto switches = [](BatchGroup& g) { return g.n_mul + g.n_rot > 0; };
+    run(AOA_STAGE_MODUP, switches, [&](BatchGroup& g) {
+      const DevParams P = launch_params(b, g);
+      if (g.n_mul) fz_up_desc(P, g.d_items, g.n_mul, g.max_level, true, st);
+      if (g.n_rot) fz_up_desc(P, g.d_items + g.n_mul, g.n_rot, g.max_level, false, st);
       return 0;
     });
-    run(AOA_STAGE_NTT, [](BatchGroup& g) { return g.n_fwd > 0; },
-        [&](BatchGroup& g) { return ntt_forward_desc(launch_params(b, g), g.d_fwd, g.n_fwd, 0, st); });
-    run(AOA_STAGE_KEY_INTT, [](BatchGroup& g) { return g.n_key2 > 0; }, [&](BatchGroup& g) {
-      // the key products go to ModDown only, which takes [0, 2p) except for q0
-      return ntt_inverse_key2_desc(launch_params(b, g), g.d_key2, g.n_key2, g.d_keycol, g.n_keycol, 0, st, g.ns_key2,
-                                   -1, false);
+    run(AOA_STAGE_NTT, switches, [&](BatchGroup& g) {
+      return fz_key_special_desc(launch_params(b, g), g.d_items, g.d_keyb, g.n_keyb, g.field_b, st);
     });
-    run(AOA_STAGE_MODDOWN, [](BatchGroup& g) { return g.n_moddown > 0; }, [&](BatchGroup& g) {
-      // the key stage above (canon = false) hands over special limbs
-      // already multiplied by (B/b_j)^-1 in its two-pass form
-      const DevParams P = launch_params(b, g);
-      launch_moddown_desc(P, g.d_moddown, g.n_moddown, ntt_key2_bscaled(P, 0), st);
+    run(AOA_STAGE_KEY_INTT, switches, [&](BatchGroup& g) {
+      return fz_key_desc(launch_params(b, g), g.d_items, g.d_keyq, g.n_keyq, g.ns_keyq, g.field_q, st);
+    });
+    run(AOA_STAGE_MODDOWN, switches, [&](BatchGroup& g) {
+      fz_down_desc(launch_params(b, g), g.d_items, g.n_mul + g.n_rot, g.max_level, st);
       return 0;
     });
   }

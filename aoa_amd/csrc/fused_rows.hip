@@ -6,12 +6,18 @@
 
 namespace aoa {
 
-#define FZ_FIELD(pr_, CALL)                            \
-  switch (ld_prime_field(P.primes, pr_)) {             \
-    case FIELD_FP64: CALL(FieldFp64); break;           \
-    case FIELD_LAZY: CALL(FieldLazy); break;           \
-    default: CALL(FieldStrict); break;                 \
+// FIELD: the form of every limb of the launch, or FZ_ANY, which looks it up;
+// a kernel of one form holds fewer registers.
+constexpr int FZ_ANY = -1;
+#define FZ_FIELD(pr_, CALL)                                                            \
+  switch (FIELD == FZ_ANY ? (int)ld_prime_field(P.primes, pr_) : FIELD) {              \
+    case FIELD_FP64: if constexpr (FIELD == FZ_ANY || FIELD == FIELD_FP64) CALL(FieldFp64); break;      \
+    case FIELD_LAZY: if constexpr (FIELD == FZ_ANY || FIELD == FIELD_LAZY) CALL(FieldLazy); break;      \
+    default: if constexpr (FIELD == FZ_ANY || FIELD == FIELD_STRICT) CALL(FieldStrict); break;          \
   }
+
+// Work item of a workgroup: its index, or with P.xcd_chunks the XCD chunk map.
+__device__ __forceinline__ int fz_work(const DevParams& P, int w, int n) { return P.xcd_chunks ? xcd_chunk_id(w, n) : w; }
 
 // Values per thread: four (two stages a round) up to rows of 1024, so that a
 // small call's few rows spread over many waves; eight above.
@@ -66,14 +72,15 @@ __device__ __forceinline__ void rows_body(const DevParams& P, const uint64_t* a,
   rows_out<F, LOGM>(f, x, T, dst, id);
 }
 
-template <int LOGM, bool ARG>
+template <int LOGM, bool ARG, int FIELD>
 __global__ __launch_bounds__(RowOf<LOGM>::THREADS) void k_fz_rows(DevParams P, FzItem arg, const FzItem* items,
                                                                   const uint32_t* list) {
   __shared__ uint64_t lds[RowOf<LOGM>::LDS];
   constexpr int per = 16 / RowOf<LOGM>::ROWS;
-  const uint32_t e = fz_entry<ARG>(list, blockIdx.x / per);
+  const int w = fz_work(P, blockIdx.x, gridDim.x);
+  const uint32_t e = fz_entry<ARG>(list, w / per);
   const FzItem it = fz_item<ARG>(arg, items, e >> 8);
-  const int i = (int)(e & 255), tile = blockIdx.x % per;
+  const int i = (int)(e & 255), tile = w % per;
   const size_t o = (size_t)i * P.N;
   const uint64_t *a = glob(it.a1) + o, *b = glob(it.b1) + o;
   uint64_t* d = glob(it.D) + o;
@@ -162,19 +169,20 @@ __device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, i
   }
 }
 
-// ysplit: one workgroup per key half (the two halves of a tile `n` blocks apart).
-template <int LOGM, bool ARG>
+// ysplit: one workgroup per key half (the two halves of a tile `n` blocks
+// apart).  SPECIAL: every limb is a special one.
+template <int LOGM, bool ARG, int FIELD, bool SPECIAL>
 __global__ __launch_bounds__(RowOf<LOGM>::THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_fz_key(
     DevParams P, FzItem arg, const FzItem* items, const uint32_t* list, int n, int ysplit) {
   __shared__ uint64_t lds[RowOf<LOGM>::LDS];
   constexpr int per = 16 / RowOf<LOGM>::ROWS;
   const int y = ysplit ? (int)blockIdx.x / n : 0;
-  const int w = ysplit ? (int)blockIdx.x % n : (int)blockIdx.x;
+  const int w = fz_work(P, ysplit ? (int)blockIdx.x % n : (int)blockIdx.x, n);
   const uint32_t e = fz_entry<ARG>(list, w / per);
   const FzItem it = fz_item<ARG>(arg, items, e >> 8);
   const int m = (int)(e & 255), L = it.level + 1, pr = m < L ? m : P.k + m - L;
   const int y0 = y, y1 = ysplit ? y + 1 : 2;
-  if (it.a0 && m < L) {
+  if (!SPECIAL && it.a0 && m < L) {
 #define CALL(F) key_body_tensor<F, LOGM>(P, it, m, w % per, y0, y1, lds)
     FZ_FIELD(pr, CALL)
 #undef CALL
@@ -204,9 +212,10 @@ static int log2_of(int n) {
     default: return -1;              \
   }
 
-template <bool ARG>
+template <bool ARG, int FIELD>
 static int fz_rows(const DevParams& P, const FzItem& arg, const FzItem* items, const uint32_t* list, int n, hipStream_t st) {
-#define CALL(LM) k_fz_rows<LM, ARG><<<dim3(n * 16 / RowOf<LM>::ROWS), RowOf<LM>::THREADS, 0, st>>>(P, arg, items, list)
+  if (n <= 0) return 0;
+#define CALL(LM) k_fz_rows<LM, ARG, FIELD><<<dim3(n * 16 / RowOf<LM>::ROWS), RowOf<LM>::THREADS, 0, st>>>(P, arg, items, list)
   FZ_DISPATCH_M(CALL)
 #undef CALL
   return 0;
@@ -214,12 +223,14 @@ static int fz_rows(const DevParams& P, const FzItem& arg, const FzItem* items, c
 
 // One workgroup per key half while both halves together leave the chip
 // partly idle: the forward rows are then done twice, on idle units.
-template <bool ARG>
+template <bool ARG, int FIELD, bool SPECIAL>
 static int fz_key(const DevParams& P, const FzItem& arg, const FzItem* items, const uint32_t* list, int n, hipStream_t st) {
+  if (n <= 0) return 0;
 #define CALL(LM)                                                                                                       \
   {                                                                                                                    \
     const int blocks = n * 16 / RowOf<LM>::ROWS, ysplit = blocks * (RowOf<LM>::THREADS / 64) <= 2048 ? 1 : 0;          \
-    k_fz_key<LM, ARG><<<dim3(blocks << ysplit), RowOf<LM>::THREADS, 0, st>>>(P, arg, items, list, blocks, ysplit);     \
+    k_fz_key<LM, ARG, FIELD, SPECIAL>                                                                                  \
+        <<<dim3(blocks << ysplit), RowOf<LM>::THREADS, 0, st>>>(P, arg, items, list, blocks, ysplit);                  \
   }
   FZ_DISPATCH_M(CALL)
 #undef CALL
@@ -227,16 +238,31 @@ static int fz_key(const DevParams& P, const FzItem& arg, const FzItem* items, co
 }
 
 int fz_rows_item(const DevParams& P, const FzItem& it, hipStream_t st) {
-  return fz_rows<true>(P, it, nullptr, nullptr, it.level + 1, st);
+  return fz_rows<true, FZ_ANY>(P, it, nullptr, nullptr, it.level + 1, st);
 }
 int fz_key_item(const DevParams& P, const FzItem& it, hipStream_t st) {
-  return fz_key<true>(P, it, nullptr, nullptr, it.level + 1 + P.K, st);
+  return fz_key<true, FZ_ANY, false>(P, it, nullptr, nullptr, it.level + 1 + P.K, st);
 }
-int fz_rows_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, hipStream_t st) {
-  return fz_rows<false>(P, FzItem{}, items, list, n, st);
+int fz_rows_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, int nstrict, int field,
+                 hipStream_t st) {
+  const FzItem z{};
+  if (nstrict < 0) return fz_rows<false, FZ_ANY>(P, z, items, list, n, st);
+  if (fz_rows<false, FIELD_STRICT>(P, z, items, list, nstrict, st)) return -1;
+  if (field == FIELD_FP64) return fz_rows<false, FIELD_FP64>(P, z, items, list + nstrict, n - nstrict, st);
+  return fz_rows<false, FIELD_LAZY>(P, z, items, list + nstrict, n - nstrict, st);
 }
-int fz_key_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, hipStream_t st) {
-  return fz_key<false>(P, FzItem{}, items, list, n, st);
+int fz_key_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, int nstrict, int field,
+                hipStream_t st) {
+  const FzItem z{};
+  if (nstrict < 0) return fz_key<false, FZ_ANY, false>(P, z, items, list, n, st);
+  if (fz_key<false, FIELD_STRICT, false>(P, z, items, list, nstrict, st)) return -1;
+  if (field == FIELD_FP64) return fz_key<false, FIELD_FP64, false>(P, z, items, list + nstrict, n - nstrict, st);
+  return fz_key<false, FIELD_LAZY, false>(P, z, items, list + nstrict, n - nstrict, st);
+}
+int fz_key_special_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, int field, hipStream_t st) {
+  const FzItem z{};
+  if (field == FIELD_FP64) return fz_key<false, FIELD_FP64, true>(P, z, items, list, n, st);
+  return fz_key<false, FIELD_LAZY, true>(P, z, items, list, n, st);
 }
 
 }  // namespace aoa

@@ -33,9 +33,14 @@ void fz_up_item(const DevParams& P, const FzItem& it, bool mul, hipStream_t st);
 int fz_key_item(const DevParams& P, const FzItem& it, hipStream_t st);
 void fz_down_item(const DevParams& P, const FzItem& it, hipStream_t st);
 // The same stage by stage over device tables: `list` entries are item << 8 | limb.
-int fz_rows_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, hipStream_t st);
+// nstrict >= 0: the first nstrict entries are of primes wider than 2^56 and the
+// others of form `field`; the special limbs' key products have a list of their own.
+int fz_rows_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, int nstrict, int field,
+                 hipStream_t st);
 void fz_up_desc(const DevParams& P, const FzItem* items, int n, int max_level, bool mul, hipStream_t st);
-int fz_key_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, hipStream_t st);
+int fz_key_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, int nstrict, int field,
+                hipStream_t st);
+int fz_key_special_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, int field, hipStream_t st);
 void fz_down_desc(const DevParams& P, const FzItem* items, int n, int max_level, hipStream_t st);
 
 // out = a op b (out = a*b + c for MULADD) over nlimbs limbs mapped to primes
