@@ -119,13 +119,14 @@ struct FieldLazy {
   // factor of two products: canonical
   __device__ __forceinline__ V factor(V x) const { return out(x); }
   __device__ __forceinline__ V key(V x, uint64_t k) const { return mul_barrett62_lazy(x, k, p, mu2, nb); }
-  // d2 key + (B mod q) d_y, d2 = a1 b1, d_0 = a0 b0, d_1 = a0 b1 + a1 b0
-  template <int Y>
-  __device__ __forceinline__ V tensor(uint64_t a0, uint64_t a1, uint64_t b0, uint64_t b1, uint64_t k, W bq) const {
-    const uint64_t d2 = mul_barrett62(a1, b1, p, mu2, nb);
-    const uint64_t d = Y ? key(a0, b1) + key(a1, b0) : key(a0, b0);
-    return key(d2, k) + mul(d, bq);
+  // HomMul's products d2 = a1 b1, d0 = a0 b0, d1 = a0 b1 + a1 b0 and their
+  // relinearisation d2 key + (B mod q) d
+  __device__ __forceinline__ V d2(uint64_t a1, uint64_t b1) const { return mul_barrett62(a1, b1, p, mu2, nb); }
+  __device__ __forceinline__ V d0(uint64_t a0, uint64_t b0) const { return key(a0, b0); }
+  __device__ __forceinline__ V d1(uint64_t a0, uint64_t a1, uint64_t b0, uint64_t b1) const {
+    return key(a0, b1) + key(a1, b0);
   }
+  __device__ __forceinline__ V relin(V d2, uint64_t k, V d, W bq) const { return key(d2, k) + mul(d, bq); }
 };
 
 struct FieldFp64 {
@@ -188,13 +189,12 @@ struct FieldFp64 {
   }
   __device__ __forceinline__ V factor(V x) const { return red(x); }
   __device__ __forceinline__ V key(V x, uint64_t k) const { return mul(x, in(k)); }
-  template <int Y>
-  __device__ __forceinline__ V tensor(uint64_t a0, uint64_t a1, uint64_t b0, uint64_t b1, uint64_t k, W bq) const {
-    const V A0 = in(a0), A1 = in(a1), B0 = in(b0), B1 = in(b1);
-    const V d2 = mul(A1, B1);
-    const V d = Y ? mul(A0, B1) + mul(A1, B0) : mul(A0, B0);
-    return mul(d2, in(k)) + mul(d, bq);
+  __device__ __forceinline__ V d2(uint64_t a1, uint64_t b1) const { return mul(in(a1), in(b1)); }
+  __device__ __forceinline__ V d0(uint64_t a0, uint64_t b0) const { return mul(in(a0), in(b0)); }
+  __device__ __forceinline__ V d1(uint64_t a0, uint64_t a1, uint64_t b0, uint64_t b1) const {
+    return mul(in(a0), in(b1)) + mul(in(a1), in(b0));
   }
+  __device__ __forceinline__ V relin(V d2, uint64_t k, V d, W bq) const { return mul(d2, in(k)) + mul(d, bq); }
 };
 
 struct FieldStrict {
@@ -253,12 +253,12 @@ struct FieldStrict {
     r += (v >> 31) * c;  // below 2^52
     return r >= p ? r - p : r;
   }
-  template <int Y>
-  __device__ __forceinline__ V tensor(uint64_t a0, uint64_t a1, uint64_t b0, uint64_t b1, uint64_t k, W bq) const {
-    const uint64_t d2 = key(a1, b1);
-    const uint64_t d = Y ? add_mod(key(a0, b1), key(a1, b0), p) : key(a0, b0);
-    return add_mod(key(d2, k), mul(d, bq), p);
+  __device__ __forceinline__ V d2(uint64_t a1, uint64_t b1) const { return key(a1, b1); }
+  __device__ __forceinline__ V d0(uint64_t a0, uint64_t b0) const { return key(a0, b0); }
+  __device__ __forceinline__ V d1(uint64_t a0, uint64_t a1, uint64_t b0, uint64_t b1) const {
+    return add_mod(key(a0, b1), key(a1, b0), p);
   }
+  __device__ __forceinline__ V relin(V d2, uint64_t k, V d, W bq) const { return add_mod(key(d2, k), mul(d, bq), p); }
 };
 
 // Brings the values that an inverse round of NB stages has doubled more than

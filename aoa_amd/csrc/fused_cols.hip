@@ -213,12 +213,12 @@ __global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 
 // ---------------------------------------------------------------- ModDown --
 template <class F>
-__device__ __forceinline__ void down_in(const DevParams& P, const uint64_t* src, int pr, int M, int q, uint64_t* t) {
+__device__ __forceinline__ void down_in(const DevParams& P, const uint64_t (&u)[4], int pr, int q, uint64_t* t) {
   const F f(P.primes[pr]);
   const uint64_t* T = P.fz.tw[1] + (size_t)pr * P.N * 2;
   typename F::V x[4];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) x[k] = f.raw_in(src[(size_t)(4 * q + k) * M]);
+  for (int k = 0; k < 4; ++k) x[k] = f.raw_in(u[k]);
   col_inv_b(f, x, T, q);
   col_turn<true>(f, x, t, q);
   col_inv_a(f, x, T, P.fz.lc_key + 4 * (size_t)pr);
@@ -236,8 +236,8 @@ __device__ __forceinline__ uint64_t down_deviation(const DevParams& P, uint64_t 
   return sub_mod(f, x, dq.p);
 }
 
-// Looks for the products a_j c_ij of the limbs i = g + 4 n, n0 <= n < n0 + NL,
-// whose remainder may lie in the reference's deviation window and takes what
+// Looks for the products a_j c_ij of the limbs i = g + 4 n, n0 <= n < n0 + left
+// (the table goes on to NL limbs: later limbs, or the first one again), whose remainder may lie in the reference's deviation window and takes what
 // they deviate by off x_i.  frac(a c / q) = frac(al c/q + ah frac(2^28 c/q)),
 // a = al + ah 2^28, in two FP64 multiply-adds onto 1.5 2^36 + 2^-15, which leaves
 // its first 16 bits (one unit off at most, two units added) in the low half
@@ -245,7 +245,8 @@ __device__ __forceinline__ uint64_t down_deviation(const DevParams& P, uint64_t 
 // About one wave in a hundred looks closer: to 2^-22 (bias 2^-21, bound 2^-20
 // more), then with the exact formulas.
 template <int NL>
-__device__ __forceinline__ void down_screen(const DevParams& P, const uint64_t* aux, uint64_t* xq, int g, int n0, int c) {
+__device__ __forceinline__ void down_screen(const DevParams& P, const uint64_t* aux, uint64_t* xq, int g, int n0, int left,
+                                            int c) {
   const cptr<double> tab = as_const(P.fz.scr) + (g * 16 + n0) * 2;
   const cptr<double> thr = as_const(P.fz.scr_thr) + g + 4 * n0;
   double widest = thr[0];
@@ -265,7 +266,7 @@ __device__ __forceinline__ void down_screen(const DevParams& P, const uint64_t* 
     }
     if (__builtin_amdgcn_ballot_w64(least <= bound)) {
 #pragma unroll 1
-      for (int n = 0; n < NL; ++n) {
+      for (int n = 0; n < left; ++n) {
         const double s = __builtin_fma(ah, e[2 * n + 1], __builtin_fma(al, e[2 * n], 4.76837158203125e-07));
         if (__builtin_amdgcn_fract(s) < thr[4 * n]) {
           const int i = g + 4 * (n0 + n);
@@ -326,7 +327,7 @@ __device__ __forceinline__ void down_out(const DevParams& P, const FzItem& it, c
       for (int b = 0; b < NB; ++b) {
         const int n = (nb0 + b) * 16 + (lane & 15);
         uint64_t v = conv_join<T, NB>(acc, b, r, o);
-        if constexpr (T == 8) {
+        if (T == 8 && r == 0) {  // q0 is the first row of its block
           v = v >= o.p ? v - o.p : v;
           v = mul_shoup(xq[i * FZ_PITCH + n] + (o.p - v), w.w, w.q, o.p);
         } else {  // primes below 2^56
@@ -358,12 +359,24 @@ __global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
   uint64_t* xq = aux + down_aux_rows(K) * FZ_PITCH;
   uint64_t* part = xq + up8(L) * FZ_PITCH;
   // inverse columns: Q limbs, then from a wave boundary the special limbs
-  const int L2 = (L + 1) & ~1;
-  for (int t = threadIdx.x; t < (L2 + K) * 32; t += FZ_THREADS) {
-    const int m = t / 32, q = t / FZ_COLS % 4, c = t % FZ_COLS;
+  const int L2 = (L + 1) & ~1, tasks = (L2 + K) * 32;
+  const int q = threadIdx.x / FZ_COLS % 4, cc = threadIdx.x % FZ_COLS;
+  // the next round's values are requested before this round's are used
+  auto load = [&](int t, uint64_t (&u)[4]) {
+    const int m = t / 32, row = m < L2 ? min(m, L - 1) : m - L2 + L;
+    const uint64_t* s = p + (size_t)row * P.N + cc;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) u[k] = s[(size_t)(4 * q + k) * M];
+  };
+  uint64_t u[4];
+  if ((int)threadIdx.x < tasks) load(threadIdx.x, u);
+  for (int t = threadIdx.x; t < tasks; t += FZ_THREADS) {
+    uint64_t un[4] = {0, 0, 0, 0};
+    if (t + FZ_THREADS < tasks) load(t + FZ_THREADS, un);
+    const int m = t / 32;
     if (m < L2) {
       if (m < L) {
-#define CALL(F) down_in<F>(P, p + (size_t)m * P.N + c, m, M, q, xq + m * FZ_PITCH + c)
+#define CALL(F) down_in<F>(P, u, m, q, xq + m * FZ_PITCH + cc)
         switch (P.primes[m].field) {
           case FIELD_FP64: CALL(FieldFp64); break;
           case FIELD_LAZY: CALL(FieldLazy); break;
@@ -373,12 +386,13 @@ __global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
       }
     } else {
       const int j = m - L2;
-      const uint64_t* s = p + (size_t)(L + j) * P.N + c;
-      if (P.primes[P.k].field == FIELD_FP64)
-        down_in<FieldFp64>(P, s, P.k + j, M, q, aux + j * FZ_PITCH + c);
+      if (ld_prime_field(P.primes, P.k) == FIELD_FP64)
+        down_in<FieldFp64>(P, u, P.k + j, q, aux + j * FZ_PITCH + cc);
       else
-        down_in<FieldLazy>(P, s, P.k + j, M, q, aux + j * FZ_PITCH + c);
+        down_in<FieldLazy>(P, u, P.k + j, q, aux + j * FZ_PITCH + cc);
     }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) u[k] = un[k];
   }
   if (!rescale && threadIdx.x < FZ_TILE) aux[K * FZ_PITCH + threadIdx.x] = 0;
   __syncthreads();
@@ -389,18 +403,16 @@ __global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
     part[g * FZ_TILE + c] = j1 > j0 ? down_top(P, aux, it.level, j0, j1, c) : 0;
   }
   if (!P.moddown_exact) {
-    int n = 0;
     const int nl = (lout - g + 3) / 4;  // limbs g, g + 4, ... below lout
-    for (; nl - n >= 8; n += 8) down_screen<8>(P, aux, xq, g, n, c);
-    if (nl - n >= 4) {
-      down_screen<4>(P, aux, xq, g, n, c);
-      n += 4;
+    for (int n = 0; n < nl; n += 8) {
+      const int left = min(nl - n, 8);
+      if (left > 4)
+        down_screen<8>(P, aux, xq, g, n, left, c);
+      else if (left > 2)
+        down_screen<4>(P, aux, xq, g, n, left, c);
+      else
+        down_screen<2>(P, aux, xq, g, n, left, c);
     }
-    if (nl - n >= 2) {
-      down_screen<2>(P, aux, xq, g, n, c);
-      n += 2;
-    }
-    if (nl - n >= 1) down_screen<1>(P, aux, xq, g, n, c);
   }
   __syncthreads();
   if (rescale) {

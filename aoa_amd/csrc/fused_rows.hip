@@ -1,7 +1,5 @@
 // Row kernels of the fused key switching (fused.hpp): the forward and inverse
 // row stages with the products between them.
-#include <type_traits>
-
 #include "fused.hpp"
 
 namespace aoa {
@@ -113,26 +111,28 @@ __device__ __forceinline__ void key_body_tensor(const DevParams& P, const FzItem
   const RowId<LOGM> id(tile, lds);
   const size_t o = (size_t)m * P.N;
   const uint64_t *a0 = glob(it.a0) + o, *a1 = glob(it.a1) + o, *b0 = glob(it.b0) + o, *b1 = glob(it.b1) + o;
+  const uint64_t *kb = glob(it.kb) + o, *ka = glob(it.ka) + o;
+  const typename F::W bq = f.tw_u(P.fz.bq + 2 * m, 0);
+  // both halves' products from one reading of the operands; the second waits
+  // in registers while the first is transformed
+  typename F::V x[G::V], x1[G::V];
+#pragma unroll
+  for (int k = 0; k < G::V; ++k) {
+    const uint32_t i = id.off + G::TS * 8 * k;
+    const uint64_t va0 = at_byte<uint64_t>(a0, i), va1 = at_byte<uint64_t>(a1, i);
+    const uint64_t vb0 = at_byte<uint64_t>(b0, i), vb1 = at_byte<uint64_t>(b1, i);
+    const auto d2 = f.d2(va1, vb1);
+    if (y0 == 0) x[k] = f.relin(d2, at_byte<uint64_t>(kb, i), f.d0(va0, vb0), bq);
+    if (y1 == 2) x1[k] = f.relin(d2, at_byte<uint64_t>(ka, i), f.d1(va0, va1, vb0, vb1), bq);
+  }
 #pragma unroll 1
   for (int y = y0; y < y1; ++y) {
-    const uint32_t z = opaque_zero(), off = id.off + z;
-    const typename F::W bq = f.tw_u(P.fz.bq + 2 * m, 0);
-    const uint64_t* kp = glob(y ? it.ka : it.kb) + o;
-    typename F::V x[G::V];
-    auto products = [&](auto half) {
+    if (y) {
 #pragma unroll
-      for (int k = 0; k < G::V; ++k) {
-        const uint32_t i = off + G::TS * 8 * k;
-        x[k] = f.template tensor<half.value>(at_byte<uint64_t>(a0, i), at_byte<uint64_t>(a1, i), at_byte<uint64_t>(b0, i),
-                                             at_byte<uint64_t>(b1, i), at_byte<uint64_t>(kp, i), bq);
-      }
-    };
-    if (y)
-      products(std::integral_constant<int, 1>());
-    else
-      products(std::integral_constant<int, 0>());
+      for (int k = 0; k < G::V; ++k) x[k] = x1[k];
+    }
     row_turn<LOGM, LV, 0, G::ROUNDS - 1>(f, x, id.s, id.L);
-    rows_out<F, LOGM>(f, x, T + z, glob(y ? it.P1 : it.P0) + o, id);
+    rows_out<F, LOGM>(f, x, T + opaque_zero(), glob(y ? it.P1 : it.P0) + o, id);
   }
 }
 

@@ -165,7 +165,7 @@ void build_fused_tables(const HostParams& h, FusedTables* out) {
   }
   // Screen of the ModDown products: frac(a c/q) = frac(al c/q + ah frac(2^28 c/q)), a = al + ah 2^28.
   out->scr.assign((size_t)K * 4 * 16 * 2, 0.0);
-  out->scr_thr.assign(k, 0.0);
+  out->scr_thr.assign(64, 0.0);
   for (int i = 0; i < k; ++i) {
     const uint64_t q = h.primes[i];
     for (int j = 0; j < K; ++j) {
@@ -179,6 +179,14 @@ void build_fused_tables(const HostParams& h, FusedTables* out) {
     const uint64_t thr = d.quirk_thr < q ? d.quirk_thr : q;
     out->scr_thr[i] = (double)((long double)thr / (long double)q) + std::ldexp(1.0, -20);
   }
+  // past the last limb of a group: its first limb again, which adds no hit
+  for (int j = 0; j < K; ++j)
+    for (int g = 0; g < 4 && g < k; ++g)
+      for (int n = (k - g + 3) / 4; n < 16; ++n)
+        for (int h = 0; h < 2; ++h) {
+          double* e = &out->scr[(((size_t)j * 4 + g) * 16) * 2];
+          e[2 * n + h] = e[h];
+        }
 }
 
 }  // namespace aoa

@@ -89,7 +89,7 @@ struct FusedDev {
   const ConvOut* mu_out;   // [k][K] (l, j)
   const ConvOut* md_out;   // [k]
   const double* scr;       // [K][4][16][2]: frac(c/q_i), frac(2^28 c/q_i) for c = (B/b_j) mod q_i, i = g + 4n
-  const double* scr_thr;   // [k]: screen bound of q_i
+  const double* scr_thr;   // [64]: screen bound of q_i (0 from k on)
   uint32_t mu_stride;      // bytes of mu_w per level
   int mu_kb, md_kb;        // steps of 8 inputs the layouts hold
 };
