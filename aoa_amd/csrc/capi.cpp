@@ -97,7 +97,7 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
   secs.push_back({F.tw[0].data(), F.tw[0].size() * 8, 0});
   secs.push_back({F.tw[1].data(), F.tw[1].size() * 8, 0});
   secs.push_back({F.lc.data(), F.lc.size() * 8, 0});
-  secs.push_back({F.lc_key.data(), F.lc_key.size() * 8, 0});
+  secs.push_back({F.lc_b.data(), F.lc_b.size() * 8, 0});
   secs.push_back({F.lc_up.data(), F.lc_up.size() * 8, 0});
   secs.push_back({F.bq.data(), F.bq.size() * 8, 0});
   secs.push_back({F.mu_w.data(), F.mu_w.size(), 0});
@@ -106,6 +106,7 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
   secs.push_back({F.md_out.data(), F.md_out.size() * sizeof(ConvOut), 0});
   secs.push_back({F.scr.data(), F.scr.size() * 8, 0});
   secs.push_back({F.scr_thr.data(), F.scr_thr.size() * 8, 0});
+  secs.push_back({F.lc_down.data(), F.lc_down.size() * 8, 0});
   const int nsec = (int)secs.size();
   size_t total = 0;
   for (int i = 0; i < nsec; ++i) {
@@ -157,7 +158,7 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
   Z.tw[0] = (const uint64_t*)(b + secs[fsec].off);
   Z.tw[1] = (const uint64_t*)(b + secs[fsec + 1].off);
   Z.lc = (const uint64_t*)(b + secs[fsec + 2].off);
-  Z.lc_key = (const uint64_t*)(b + secs[fsec + 3].off);
+  Z.lc_b = (const uint64_t*)(b + secs[fsec + 3].off);
   Z.lc_up = (const uint64_t*)(b + secs[fsec + 4].off);
   Z.bq = (const uint64_t*)(b + secs[fsec + 5].off);
   Z.mu_w = (const uint8_t*)(b + secs[fsec + 6].off);
@@ -166,7 +167,9 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
   Z.md_out = (const ConvOut*)(b + secs[fsec + 9].off);
   Z.scr = (const double*)(b + secs[fsec + 10].off);
   Z.scr_thr = (const double*)(b + secs[fsec + 11].off);
+  Z.lc_down = (const uint64_t*)(b + secs[fsec + 12].off);
   Z.mu_stride = F.mu_stride;
+  Z.md_stride = F.md_stride;
   Z.mu_kb = F.mu_kb;
   Z.md_kb = F.md_kb;
   *out = h;

@@ -54,8 +54,25 @@ __device__ __forceinline__ uint64_t shoup4(uint64_t x, uint64_t w, uint64_t wq, 
   const uint32_t w0 = (uint32_t)w, w1 = (uint32_t)(w >> 32), n0 = (uint32_t)np, n1 = (uint32_t)(np >> 32);
   uint64_t acc = (uint64_t)x0 * w0;
   acc = (uint64_t)q0 * n0 + acc;
-  const uint32_t hi = x0 * w1 + x1 * w0 + q0 * n1 + q1 * n0;
-  return acc + ((uint64_t)hi << 32);
+  // the high words' sum stays in 32 bits (left to itself the compiler widens
+  // it into a 64-bit add of a register pair with a zero)
+  uint32_t hi;
+  asm("v_add3_u32 %0, %1, %2, %3"
+      : "=v"(hi)
+      : "v"((uint32_t)(acc >> 32)), "v"(x0 * w1 + x1 * w0), "v"(q0 * n1 + q1 * n0));
+  return ((uint64_t)hi << 32) | (uint32_t)acc;
+}
+
+// u - v + off, off1 = off + 1: without a borrow chain, whose carry would have
+// to wait two instructions.
+__device__ __forceinline__ uint64_t diff(uint64_t u, uint64_t v, uint64_t off1) { return u + off1 + ~v; }
+
+// x - p where that is not negative, else x: the borrow is the condition.
+__device__ __forceinline__ uint64_t csub(uint64_t x, uint64_t p) {
+  unsigned b0, b1;
+  const uint32_t l = __builtin_subc((uint32_t)x, (uint32_t)p, 0u, &b0);
+  const uint32_t h = __builtin_subc((uint32_t)(x >> 32), (uint32_t)(p >> 32), b0, &b1);
+  return b1 ? x : ((uint64_t)h << 32) | l;
 }
 
 struct FieldLazy {
@@ -89,29 +106,28 @@ struct FieldLazy {
   __device__ __forceinline__ void fwd(V& a, V& b, W w) const {
     const V v = mul(b, w), u = a;
     a = u + v;
-    b = u + 4 * p - v;
+    b = diff(u, v, 4 * p + 1);
   }
   // stage S of an inverse round, values below (8 << S) p
   template <int S>
   __device__ __forceinline__ void inv(V& a, V& b, W w) const {
     const V u = a, v = b;
     a = u + v;
-    b = mul(u + ((8 * p) << S) - v, w);
+    b = mul(diff(u, v, ((8 * p) << S) + 1), w);
   }
   // the last stage, values below 64p: canonical
   __device__ __forceinline__ void inv_last(V& a, V& b, W w0, W w1) const {
     const V u = a, v = b;
     a = fix4(shoup4(u + v, w0.w, w0.q, np));
-    b = fix4(shoup4(u + 64 * p - v, w1.w, w1.q, np));
+    b = fix4(shoup4(diff(u, v, 64 * p + 1), w1.w, w1.q, np));
   }
   __device__ __forceinline__ uint64_t fix4(uint64_t x) const {
-    x = x >= 2 * p ? x - 2 * p : x;
-    return x >= p ? x - p : x;
+    return csub(csub(x, 2 * p), p);
   }
   // any value -> [0, 3p): the quotient from the high word
   __device__ __forceinline__ V red(V x) const {
     const uint32_t q = mulhi32((uint32_t)(x >> 32), mu32);
-    return x - (uint64_t)q * p;
+    return x + (uint64_t)q * np;
   }
   static constexpr int kGrow = 2;  // doublings a value may keep after a round
   __device__ __forceinline__ uint64_t out(V x) const { return fix4(red(x)); }
@@ -219,22 +235,24 @@ struct FieldStrict {
     for (int k = 0; k < C; ++k) t[k] = tw(T, i + k);
   }
   __device__ __forceinline__ W lc(const uint64_t* e, int which) const { return tw(e, which); }
-  __device__ __forceinline__ V mul(V x, W w) const { return mul_shoup(x, w.w, w.q, p); }
+  __device__ __forceinline__ V mul(V x, W w) const {
+    return csub(mul_shoup_lazy(x, w.w, w.q, p), p);
+  }
   __device__ __forceinline__ void fwd(V& a, V& b, W w) const {
     const V v = mul(b, w), u = a;
-    a = add_mod(u, v, p);
-    b = sub_mod(u, v, p);
+    a = csub(u + v, p);
+    b = csub(diff(u, v, p + 1), p);
   }
   template <int S>
   __device__ __forceinline__ void inv(V& a, V& b, W w) const {
     const V u = a, v = b;
-    a = add_mod(u, v, p);
-    b = mul(u + (p - v), w);
+    a = csub(u + v, p);
+    b = mul(diff(u, v, p + 1), w);
   }
   __device__ __forceinline__ void inv_last(V& a, V& b, W w0, W w1) const {
     const V u = a, v = b;
     a = mul(u + v, w0);
-    b = mul(u + (p - v), w1);
+    b = mul(diff(u, v, p + 1), w1);
   }
   __device__ __forceinline__ V red(V x) const { return x; }
   static constexpr int kGrow = 64;
@@ -249,9 +267,8 @@ struct FieldStrict {
     const uint64_t z = (hi << 1) | (lo >> 63);  // x k = z 2^63 + (lo mod 2^63)
     const uint64_t u = (uint64_t)(uint32_t)z * c, v = (z >> 32) * c + (u >> 32);  // z c = v 2^32 + low word of u
     uint64_t r = (lo & M63) + (((v << 32) & M63) | (uint32_t)u);
-    r = r >= p ? r - p : r;
-    r += (v >> 31) * c;  // below 2^52
-    return r >= p ? r - p : r;
+    r = csub(r, p) + (v >> 31) * c;  // the product is below 2^52
+    return csub(r, p);
   }
   __device__ __forceinline__ V d2(uint64_t a1, uint64_t b1) const { return key(a1, b1); }
   __device__ __forceinline__ V d0(uint64_t a0, uint64_t b0) const { return key(a0, b0); }

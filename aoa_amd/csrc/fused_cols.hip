@@ -49,6 +49,7 @@ __device__ __forceinline__ void conv_acc(v4i (&acc)[T][NB], const uint8_t* W, in
     for (int b = 0; b < NB; ++b) acc[t][b] = v4i{0, 0, 0, 0};
   const v4i* w = reinterpret_cast<const v4i*>(W) + lane;
   const int n = lane & 15, g = lane >> 4;
+#pragma unroll 2
   for (int kb = 0; kb < kbn; ++kb) {
     v4i in[NB];
 #pragma unroll
@@ -66,14 +67,16 @@ __device__ __forceinline__ void conv_acc(v4i (&acc)[T][NB], const uint8_t* W, in
   }
 }
 
-// The sum modulo o.p in [0, 1.3 p) from its digit columns (component r).  The
-// columns stay below 2^23 (at most 65 x 7 bytes), pairs of them fit 32 bits.
+// The sum plus z < p modulo p = o.p, in [0, 1.3 p), from its digit columns
+// (component r).  The columns stay below 2^23 (at most 65 x 7 bytes), pairs of
+// them fit 32 bits.
 template <int T, int NB>
-__device__ __forceinline__ uint64_t conv_join(const v4i (&acc)[T][NB], int b, int r, const ConvOut& o) {
+__device__ __forceinline__ uint64_t conv_join(const v4i (&acc)[T][NB], int b, int r, const ConvOut& o, uint64_t z) {
   auto S = [&](int t) -> int { return t < T ? acc[t < T ? t : 0][b][r] : 0; };
   const int A01 = S(0) + (S(1) << 8), A23 = S(2) + (S(3) << 8), A45 = S(4) + (S(5) << 8), A67 = S(6) + (S(7) << 8);
-  float f = __builtin_fmaf((float)A45, o.c_32, __builtin_fmaf((float)A23, o.c_16, o.c_b));
-  uint64_t v = o.off + (uint64_t)((int64_t)A01 + (int64_t)A23 * 65536);
+  // z's high word below 2^31
+  float f = __builtin_fmaf((float)A45 + (float)(int)(z >> 32), o.c_32, __builtin_fmaf((float)A23, o.c_16, o.c_b));
+  uint64_t v = o.off + z + (uint64_t)((int64_t)A01 + (int64_t)A23 * 65536);
   uint32_t hi = (uint32_t)A45;
   if (T > 6) {
     f = __builtin_fmaf((float)A67, o.c_48, f);
@@ -167,7 +170,7 @@ __device__ __forceinline__ void up_conv(const DevParams& P, const FzItem& it, in
       const ConvOut o = ld_conv(Z.mu_out + (size_t)it.level * P.K + j);
 #pragma unroll
       for (int b = 0; b < NB; ++b)
-        to[j * FZ_PITCH + (nb0 + b) * 16 + (lane & 15)] = conv_join<T, NB>(acc, b, r, o);
+        to[j * FZ_PITCH + (nb0 + b) * 16 + (lane & 15)] = conv_join<T, NB>(acc, b, r, o, 0);
     }
   }
 }
@@ -213,7 +216,8 @@ __global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 
 // ---------------------------------------------------------------- ModDown --
 template <class F>
-__device__ __forceinline__ void down_in(const DevParams& P, const uint64_t (&u)[4], int pr, int q, uint64_t* t) {
+__device__ __forceinline__ void down_in(const DevParams& P, const uint64_t (&u)[4], int pr, const uint64_t* lc, int q,
+                                        uint64_t* t) {
   const F f(P.primes[pr]);
   const uint64_t* T = P.fz.tw[1] + (size_t)pr * P.N * 2;
   typename F::V x[4];
@@ -221,123 +225,96 @@ __device__ __forceinline__ void down_in(const DevParams& P, const uint64_t (&u)[
   for (int k = 0; k < 4; ++k) x[k] = f.raw_in(u[k]);
   col_inv_b(f, x, T, q);
   col_turn<true>(f, x, t, q);
-  col_inv_a(f, x, T, P.fz.lc_key + 4 * (size_t)pr);
+  col_inv_a(f, x, T, lc);
 #pragma unroll
   for (int k = 0; k < 4; ++k) t[(q + 4 * k) * FZ_COLS] = f.out_last(x[k]);
 }
 
-// ref(a c) - (a c mod q) mod q of one product, c = (B/b_j) mod q_i: what the
-// reference's reduction of it deviates by.
-__device__ __forceinline__ uint64_t down_deviation(const DevParams& P, uint64_t a, int i, int j) {
+// f_i (ref(a c) - (a c mod q)) mod q of one product, c = (B/b_j) mod q_i: what
+// the reference's reduction of it takes off the result, f_i as in lc_down.
+__device__ __forceinline__ uint64_t down_deviation(const DevParams& P, uint64_t a, int i, int j, int set) {
   const DevPrime dq = ld_prime(P.primes, i);
   const tw2 w = ld_tw2(reinterpret_cast<const tw2*>(P.bhat_mod_q) + (size_t)i * P.K, j);
+  const tw2 f = i < set && set < P.k ? ld_tw2(reinterpret_cast<const tw2*>(P.md_fin) + (size_t)set * P.k, i)
+                                     : ld_tw2(reinterpret_cast<const tw2*>(P.inv_b_mod_q), i);
   const uint64_t x = mul_shoup(a, w.w, w.q, dq.p);
-  const uint64_t f = ref_barrett(mulhi64(a, w.w), a * w.w, dq.p, dq.mu, (int)dq.nb);
-  return sub_mod(f, x, dq.p);
+  const uint64_t r = ref_barrett(mulhi64(a, w.w), a * w.w, dq.p, dq.mu, (int)dq.nb);
+  return mul_shoup(sub_mod(r, x, dq.p), f.w, f.q, dq.p);
 }
 
-// Looks for the products a_j c_ij of the limbs i = g + 4 n, n0 <= n < n0 + left
-// (the table goes on to NL limbs: later limbs, or the first one again), whose remainder may lie in the reference's deviation window and takes what
-// they deviate by off x_i.  frac(a c / q) = frac(al c/q + ah frac(2^28 c/q)),
-// a = al + ah 2^28, in two FP64 multiply-adds onto 1.5 2^36 + 2^-15, which leaves
-// its first 16 bits (one unit off at most, two units added) in the low half
+// Looks for the products a_j c_ij of the limbs i0 <= i < i0 + NL whose
+// remainder may lie in the reference's deviation window and takes what they
+// deviate by off the results.  frac(a c / q) = frac(al c/q + ah frac(2^28 c/q)),
+// a = al + ah 2^28, in two FP64 multiply-adds onto 1.5 2^36 + 2^-16, which leaves
+// its first 16 bits (one unit off at most, one unit added) in the low half
 // word; the least of a term's NL halves is compared with the widest window.
-// About one wave in a hundred looks closer: to 2^-22 (bias 2^-21, bound 2^-20
-// more), then with the exact formulas.
+// About one wave in twenty looks closer: at each limb's half word, then to
+// 2^-22 (bias 2^-21, bound 2^-20 more), then with the exact formulas.
 template <int NL>
-__device__ __forceinline__ void down_screen(const DevParams& P, const uint64_t* aux, uint64_t* xq, int g, int n0, int left,
-                                            int c) {
-  const cptr<double> tab = as_const(P.fz.scr) + (g * 16 + n0) * 2;
-  const cptr<double> thr = as_const(P.fz.scr_thr) + g + 4 * n0;
+__device__ __forceinline__ void down_screen(const DevParams& P, const uint64_t* aux, uint64_t* xq, int i0, int c, int set) {
+  const cptr<double> tab = as_const(P.fz.scr) + i0 * 2;
+  const cptr<double> thr = as_const(P.fz.scr_thr) + i0;
   double widest = thr[0];
 #pragma unroll
-  for (int n = 1; n < NL; ++n) widest = __builtin_fmax(widest, thr[4 * n]);
-  const uint32_t bound = min((uint32_t)(widest * 65536.0) + 4, 65535u);
+  for (int n = 1; n < NL; ++n) widest = __builtin_fmax(widest, thr[n]);
+  const uint32_t bound = __builtin_amdgcn_readfirstlane(min((uint32_t)(widest * 65536.0 + 2.1), 65535u));
   for (int j = 0; j < P.K; ++j) {
     const uint64_t a = aux[j * FZ_PITCH + c];
     const double al = (double)((uint32_t)a & ((1u << 28) - 1)), ah = (double)(uint32_t)(a >> 28);
     const cptr<double> e = tab + (size_t)j * 128;
-    uint16_t least = 65535;
+    uint16_t h[NL], least = 65535;
 #pragma unroll
     for (int n = 0; n < NL; ++n) {
-      const double s = __builtin_fma(ah, e[2 * n + 1], __builtin_fma(al, e[2 * n], 103079215104.000030517578125));
-      const uint16_t h = (uint16_t)(uint32_t)__double_as_longlong(s);
-      least = h < least ? h : least;
+      const double s = __builtin_fma(ah, e[2 * n + 1], __builtin_fma(al, e[2 * n], 103079215104.0000152587890625));
+      h[n] = (uint16_t)(uint32_t)__double_as_longlong(s);
+      least = __builtin_elementwise_min(least, h[n]);
     }
     if (__builtin_amdgcn_ballot_w64(least <= bound)) {
-#pragma unroll 1
-      for (int n = 0; n < left; ++n) {
-        const double s = __builtin_fma(ah, e[2 * n + 1], __builtin_fma(al, e[2 * n], 4.76837158203125e-07));
-        if (__builtin_amdgcn_fract(s) < thr[4 * n]) {
-          const int i = g + 4 * (n0 + n);
-          uint64_t* x = xq + i * FZ_PITCH + c;
-          *x = sub_mod(*x, down_deviation(P, a, i, j), ld_prime_p(P.primes, i));
+      // opaque, so that this branch's addresses are not carried around the loop
+      int jo = j;
+      asm volatile("" : "+s"(jo));
+#pragma unroll
+      for (int n = 0; n < NL; ++n) {
+        if (__builtin_amdgcn_ballot_w64(h[n] <= bound)) {
+          const double s = __builtin_fma(ah, e[2 * n + 1], __builtin_fma(al, e[2 * n], 4.76837158203125e-07));
+          if (__builtin_amdgcn_fract(s) < thr[n]) {
+            const int i = i0 + n;
+            uint64_t* x = xq + i * FZ_PITCH + c;
+            *x = sub_mod(*x, down_deviation(P, a, i, jo, set), ld_prime_p(P.primes, i));
+          }
         }
       }
     }
   }
 }
 
-// The rescale's dropped limb `level` (a prime below 2^57): the conversion's sum
-// over j in [j0, j1), with the deviating products as the reference reduces
-// them, in [0, 5 q) (as moddown_conv in rns.hip).
-__device__ __forceinline__ uint64_t down_top(const DevParams& P, const uint64_t* aux, int level, int j0, int j1, int c) {
-  constexpr uint32_t M28 = (1u << 28) - 1;
-  constexpr int TW = (int)(sizeof(MdTerm) / 4);
-  const cptr<uint32_t> terms = as_const(P.md_terms) + (size_t)level * TW;
-  const uint32_t thr = as_const(P.md_thr)[level];
-  uint64_t s0 = 0, s2 = 0, sm = 0;
-  for (int j = j0; j < j1; ++j) {
-    const uint64_t a = aux[j * FZ_PITCH + c];
-    const uint32_t a0 = (uint32_t)a, a1 = (uint32_t)(a >> 32);
-    const uint32_t al = a0 & M28, ah = (uint32_t)(a >> 28);
-    const cptr<uint32_t> e = terms + (size_t)j * P.k * TW;
-    s0 += (uint64_t)al * e[0];
-    s2 += (uint64_t)ah * e[1];
-    sm += (uint64_t)(al + ah) * e[2];
-    if (!P.moddown_exact && moddown_screen(a0, a1, e[3], e[4], e[5]) <= thr) {
-      const uint64_t d = down_deviation(P, a, level, j);
-      s0 += d;
-      sm += d;
-    }
-  }
-  return reduce_sums_lazy(s0, sm - s0 - s2, s2, ld_prime_p(P.primes, level), as_const(P.md_red)[2 * level],
-                          ld_prime_nb(P.primes, level));
-}
-
-// Limbs 16 ib.. of coefficients 16 nb0..: the conversion and the result,
-// (x_i - sum) B^-1 (+ add_i), or with the rescale, whose dropped limb is input
-// K of the sum, (x_i - sum) B^-1 q_l^-1.
-template <int T, int NB>
-__device__ __forceinline__ void down_out(const DevParams& P, const FzItem& it, const uint64_t* add, uint64_t* out, int ib,
-                                         int nb0, int lout, const uint64_t* aux, const uint64_t* xq, int M, int col0,
-                                         int lane) {
+// Limbs 16 ib.. of coefficients 16 nb0..: the conversion and the result
+// f_i x_i - sum (xq holds f_i x_i; with a rescale the dropped limb is input K of
+// the sum), canonical, + add_i.  TOP: limb `level` alone, into input K.
+template <int T, int NB, bool TOP>
+__device__ __forceinline__ void down_out(const DevParams& P, int set, const uint64_t* add, uint64_t* out, int ib, int nb0,
+                                         int lout, uint64_t* aux, const uint64_t* xq, int M, int col0, int lane) {
   const FusedDev& Z = P.fz;
   v4i acc[T][NB];
-  conv_acc<T, NB>(acc, Z.md_w + (size_t)ib * 8 * Z.md_kb * 1024, Z.md_kb, Z.md_kb, aux, nb0, lane);
-  const tw2* fin = it.rescale ? reinterpret_cast<const tw2*>(P.md_fin) + (size_t)it.level * P.k
-                              : reinterpret_cast<const tw2*>(P.inv_b_mod_q);
+  conv_acc<T, NB>(acc, Z.md_w + (size_t)set * Z.md_stride + (size_t)ib * 8 * Z.md_kb * 1024, Z.md_kb, Z.md_kb, aux, nb0,
+                  lane);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int i = ib * 16 + 4 * (lane >> 4) + r;
-    if (i < lout) {
-      const ConvOut o = ld_conv(Z.md_out + i);
-      const tw2 w = fin[i];
+    if (TOP ? i == lout : i < lout) {
+      const ConvOut o = ld_conv(Z.md_out + (size_t)set * P.k + i);
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         const int n = (nb0 + b) * 16 + (lane & 15);
-        uint64_t v = conv_join<T, NB>(acc, b, r, o);
-        if (T == 8 && r == 0) {  // q0 is the first row of its block
-          v = v >= o.p ? v - o.p : v;
-          v = mul_shoup(xq[i * FZ_PITCH + n] + (o.p - v), w.w, w.q, o.p);
-        } else {  // primes below 2^56
-          v = shoup4(xq[i * FZ_PITCH + n] + (2 * o.p - v), w.w, w.q, 0 - o.p);
-          v = v >= 2 * o.p ? v - 2 * o.p : v;
-          v = v >= o.p ? v - o.p : v;
+        uint64_t v = conv_join<T, NB>(acc, b, r, o, xq[i * FZ_PITCH + n]);
+        v = csub(v, o.p);
+        if (TOP) {
+          aux[P.K * FZ_PITCH + n] = v;
+        } else {
+          const size_t at = (size_t)i * P.N + (size_t)(n / FZ_COLS) * M + col0 + n % FZ_COLS;
+          if (add) v = add_mod(v, add[at], o.p);
+          out[at] = v;
         }
-        const size_t at = (size_t)i * P.N + (size_t)(n / FZ_COLS) * M + col0 + n % FZ_COLS;
-        if (add) v = add_mod(v, add[at], o.p);
-        out[at] = v;
       }
     }
   }
@@ -348,16 +325,15 @@ __host__ __device__ inline int down_aux_rows(int K) { return (K + 8) & ~7; }
 template <bool ARG>
 __global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_fz_down(DevParams P, FzItem arg,
                                                                                                 const FzItem* items) {
-  extern __shared__ uint64_t fz_lds[];  // special limbs (and the dropped limb), Q limbs, partial sums [4][128]
+  extern __shared__ uint64_t fz_lds[];  // special limbs (and the dropped limb), Q limbs
   const int M = P.N / 16, per = M / FZ_COLS, K = P.K;
   const int w = xcd_chunk_id(blockIdx.x, gridDim.x);
   const FzItem it = fz_item<ARG>(arg, items, w / (2 * per));
   const int y = (w / per) & 1, col0 = (w % per) * FZ_COLS, L = it.level + 1;
-  const int rescale = it.rescale, lout = rescale ? it.level : L;
+  const int rescale = it.rescale, lout = rescale ? it.level : L, set = rescale ? it.level : P.k;
   const uint64_t* p = glob(y ? it.P1 : it.P0) + col0;
   uint64_t* aux = fz_lds;
   uint64_t* xq = aux + down_aux_rows(K) * FZ_PITCH;
-  uint64_t* part = xq + up8(L) * FZ_PITCH;
   // inverse columns: Q limbs, then from a wave boundary the special limbs
   const int L2 = (L + 1) & ~1, tasks = (L2 + K) * 32;
   const int q = threadIdx.x / FZ_COLS % 4, cc = threadIdx.x % FZ_COLS;
@@ -376,7 +352,7 @@ __global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
     const int m = t / 32;
     if (m < L2) {
       if (m < L) {
-#define CALL(F) down_in<F>(P, u, m, q, xq + m * FZ_PITCH + cc)
+#define CALL(F) down_in<F>(P, u, m, P.fz.lc_down + 4 * ((size_t)set * P.k + m), q, xq + m * FZ_PITCH + cc)
         switch (P.primes[m].field) {
           case FIELD_FP64: CALL(FieldFp64); break;
           case FIELD_LAZY: CALL(FieldLazy); break;
@@ -387,57 +363,58 @@ __global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
     } else {
       const int j = m - L2;
       if (ld_prime_field(P.primes, P.k) == FIELD_FP64)
-        down_in<FieldFp64>(P, u, P.k + j, q, aux + j * FZ_PITCH + cc);
+        down_in<FieldFp64>(P, u, P.k + j, P.fz.lc_b + 4 * j, q, aux + j * FZ_PITCH + cc);
       else
-        down_in<FieldLazy>(P, u, P.k + j, q, aux + j * FZ_PITCH + cc);
+        down_in<FieldLazy>(P, u, P.k + j, P.fz.lc_b + 4 * j, q, aux + j * FZ_PITCH + cc);
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) u[k] = un[k];
   }
-  if (!rescale && threadIdx.x < FZ_TILE) aux[K * FZ_PITCH + threadIdx.x] = 0;
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  const int g = wave >> 1, c = (wave & 1) * 64 + lane;
-  if (rescale) {
-    const int jq = (K + 3) / 4, j0 = g * jq, j1 = min(K, j0 + jq);
-    part[g * FZ_TILE + c] = j1 > j0 ? down_top(P, aux, it.level, j0, j1, c) : 0;
-  }
   if (!P.moddown_exact) {
-    const int nl = (lout - g + 3) / 4;  // limbs g, g + 4, ... below lout
-    for (int n = 0; n < nl; n += 8) {
-      const int left = min(nl - n, 8);
-      if (left > 4)
-        down_screen<8>(P, aux, xq, g, n, left, c);
-      else if (left > 2)
-        down_screen<4>(P, aux, xq, g, n, left, c);
-      else
-        down_screen<2>(P, aux, xq, g, n, left, c);
-    }
-  }
-  __syncthreads();
-  if (rescale) {
-    if (threadIdx.x < FZ_TILE) {
-      const int l = it.level;
-      const uint64_t q = ld_prime_p(P.primes, l), q5 = as_const(P.md_red)[2 * l + 1];
-      uint64_t s = 0;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) s = add_mod(s, part[t * FZ_TILE + threadIdx.x], q5);
-      const tw2 bi = ld_tw2(reinterpret_cast<const tw2*>(P.inv_b_mod_q), l);
-      aux[K * FZ_PITCH + threadIdx.x] = mul_shoup(xq[l * FZ_PITCH + threadIdx.x] + q5 - s, bi.w, bi.q, q);
+    // two waves of 64 coefficients for each quarter of the limbs
+    const int g = wave >> 1, c = (wave & 1) * 64 + lane, per_g = (L + 3) / 4;
+    const int end = min(L, (g + 1) * per_g);
+    for (int i = g * per_g; i < end;) {
+      const int left = end - i;
+      if (left >= 8) {
+        down_screen<8>(P, aux, xq, i, c, set);
+        i += 8;
+        continue;
+      }
+      switch (left) {
+        case 7: down_screen<7>(P, aux, xq, i, c, set); break;
+        case 6: down_screen<6>(P, aux, xq, i, c, set); break;
+        case 5: down_screen<5>(P, aux, xq, i, c, set); break;
+        case 4: down_screen<4>(P, aux, xq, i, c, set); break;
+        case 3: down_screen<3>(P, aux, xq, i, c, set); break;
+        case 2: down_screen<2>(P, aux, xq, i, c, set); break;
+        default: down_screen<1>(P, aux, xq, i, c, set); break;
+      }
+      break;
     }
     __syncthreads();
   }
   const uint64_t* add = glob(y ? it.add1 : it.add0);
   uint64_t* out = glob(y ? it.out1 : it.out0);
+  if (rescale) {
+    const int ib = it.level / 16, nb = ld_prime_nb(P.primes, ib * 16);
+    if (nb > 56)
+      down_out<8, 1, true>(P, P.k, nullptr, nullptr, ib, wave, it.level, aux, xq, M, col0, lane);
+    else
+      down_out<7, 1, true>(P, P.k, nullptr, nullptr, ib, wave, it.level, aux, xq, M, col0, lane);
+    __syncthreads();
+  }
   const int units = ((lout + 15) / 16) * 4;
   for (int u = wave; u < units; u += FZ_THREADS / 64) {
     const int ib = u / 4, nb0 = (u % 4) * 2, nb = ld_prime_nb(P.primes, ib * 16);
     if (nb > 56)
-      down_out<8, 2>(P, it, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
+      down_out<8, 2, false>(P, set, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
     else if (nb > 48)
-      down_out<7, 2>(P, it, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
+      down_out<7, 2, false>(P, set, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
     else
-      down_out<6, 2>(P, it, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
+      down_out<6, 2, false>(P, set, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
   }
 }
 
@@ -456,7 +433,7 @@ static void fz_up(const DevParams& P, const FzItem& arg, const FzItem* items, in
 
 template <bool ARG>
 static void fz_down(const DevParams& P, const FzItem& arg, const FzItem* items, int n, int max_level, hipStream_t st) {
-  const size_t lds = ((size_t)(down_aux_rows(P.K) + ((max_level + 8) & ~7)) * FZ_PITCH + 4 * FZ_TILE) * 8;
+  const size_t lds = ((size_t)(down_aux_rows(P.K) + ((max_level + 8) & ~7)) * FZ_PITCH) * 8;
   k_fz_down<ARG><<<dim3((unsigned)(2 * n * (P.N / FZ_TILE))), FZ_THREADS, lds, st>>>(P, arg, items);
 }
 

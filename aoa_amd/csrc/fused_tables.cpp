@@ -73,7 +73,8 @@ struct ConvRow {
     }
   }
   // The kernel sums V + off with off = (128 sum) + m p, m p >= |V|, so the
-  // total lies in [0, 2^17 p); its quotient estimate is low by 0.02 to 0.2.
+  // total lies in [0, 2^17 p); its quotient estimate is low by 0.02 to 0.2, which
+  // leaves a remainder below 1.3 p.
   ConvOut finish() const {
     const uint64_t m = (uint64_t)(bound / p) + 2;
     ConvOut o;
@@ -107,13 +108,25 @@ void build_fused_tables(const HostParams& h, FusedTables* out) {
     }
   }
   out->lc.assign((size_t)R * 4, 0);
-  out->lc_key.assign((size_t)R * 4, 0);
+  out->lc_b.assign((size_t)K * 4, 0);
+  out->lc_down.assign((size_t)(k + 1) * k * 4, 0);
   for (int r = 0; r < R; ++r) {
     const DevPrime& d = h.dprimes[r];
     put_lc(&out->lc[4 * r], d.ninv, d.w1ninv, d.p, d.field);
-    const uint64_t s = r < k ? 1 : h.inv_bhat[2 * (r - k)];
-    put_lc(&out->lc_key[4 * r], mulm(d.ninv, s, d.p), mulm(d.w1ninv, s, d.p), d.p, d.field);
+    if (r < k) continue;
+    const uint64_t s = h.inv_bhat[2 * (r - k)];
+    put_lc(&out->lc_b[4 * (r - k)], mulm(d.ninv, s, d.p), mulm(d.w1ninv, s, d.p), d.p, d.field);
   }
+  // ModDown's factor of limb i: B^-1, with a rescale from level l > i also q_l^-1
+  auto down_factor = [&](int l, int i) {
+    return l < k && i < l ? h.md_fin[((size_t)l * k + i) * 2] : h.inv_b_mod_q[2 * i];
+  };
+  for (int l = 0; l <= k; ++l)
+    for (int i = 0; i < k; ++i) {
+      const DevPrime& d = h.dprimes[i];
+      const uint64_t s = down_factor(l, i);
+      put_lc(&out->lc_down[((size_t)l * k + i) * 4], mulm(d.ninv, s, d.p), mulm(d.w1ninv, s, d.p), d.p, d.field);
+    }
   out->lc_up.assign((size_t)k * k * 4, 0);
   for (int l = 0; l < k; ++l)
     for (int i = 0; i <= l; ++i) {
@@ -146,32 +159,38 @@ void build_fused_tables(const HostParams& h, FusedTables* out) {
                  h.qhat_mod_b[((size_t)l * K + j) * k + i]);
       out->mu_out[(size_t)l * K + j] = row.finish();
     }
-  // ModDown: inputs a_j (j < K) and, with the rescale, the dropped limb times B in slot K.
+  // ModDown's result of limb i is f_i x_i - sum_j f_i c_ij a_j - q_l^-1 top (the
+  // last with a rescale from level l, top in slot K); one table per l, and
+  // index k without a rescale.
   const int ib_n = (k + 15) / 16;
   out->md_kb = (K + 8) / 8;
-  out->md_w.assign((size_t)ib_n * 8 * out->md_kb * 1024, 0);
-  out->md_out.assign(k, ConvOut{});
-  for (int i = 0; i < k; ++i) {
-    const int nb = (int)h.dprimes[i].nb;
-    // digits of the widest prime of the block (the first)
-    const int T_blk = conv_digits((int)h.dprimes[i / 16 * 16].nb);
-    ConvRow row;
-    row.p = h.primes[i];
-    row.T = conv_digits(nb);
-    uint8_t* blk = &out->md_w[(size_t)(i / 16) * 8 * out->md_kb * 1024];
-    for (int j = 0; j <= K; ++j)
-      row.slot(blk, i % 16, out->md_kb, T_blk, j, 7, j < K ? h.bhat_mod_q[((size_t)i * K + j) * 2] : h.b_mod_q[2 * i]);
-    out->md_out[i] = row.finish();
-  }
+  out->md_stride = (uint32_t)(ib_n * 8 * out->md_kb * 1024);
+  out->md_w.assign((size_t)(k + 1) * out->md_stride, 0);
+  out->md_out.assign((size_t)(k + 1) * k, ConvOut{});
+  for (int l = 0; l <= k; ++l)
+    for (int i = 0; i < k; ++i) {
+      if (l < k && i >= l) continue;
+      const uint64_t q = h.primes[i], f = down_factor(l, i);
+      // digits of the widest prime of the block (the first)
+      const int T_blk = conv_digits((int)h.dprimes[i / 16 * 16].nb);
+      ConvRow row;
+      row.p = q;
+      row.T = conv_digits((int)h.dprimes[i].nb);
+      uint8_t* blk = &out->md_w[(size_t)l * out->md_stride + (size_t)(i / 16) * 8 * out->md_kb * 1024];
+      for (int j = 0; j < K; ++j)
+        row.slot(blk, i % 16, out->md_kb, T_blk, j, 7, q - mulm(h.bhat_mod_q[((size_t)i * K + j) * 2], f, q));
+      if (l < k) row.slot(blk, i % 16, out->md_kb, T_blk, K, 7, q - h.inv_ql_mod_qi[((size_t)l * k + i) * 2]);
+      out->md_out[(size_t)l * k + i] = row.finish();
+    }
   // Screen of the ModDown products: frac(a c/q) = frac(al c/q + ah frac(2^28 c/q)), a = al + ah 2^28.
-  out->scr.assign((size_t)K * 4 * 16 * 2, 0.0);
+  out->scr.assign((size_t)K * 64 * 2, 0.0);
   out->scr_thr.assign(64, 0.0);
   for (int i = 0; i < k; ++i) {
     const uint64_t q = h.primes[i];
     for (int j = 0; j < K; ++j) {
       const uint64_t c = h.bhat_mod_q[((size_t)i * K + j) * 2];
       const uint64_t c28 = (uint64_t)(((u128)c << 28) % q);
-      double* e = &out->scr[(((size_t)j * 4 + i % 4) * 16 + i / 4) * 2];
+      double* e = &out->scr[((size_t)j * 64 + i) * 2];
       e[0] = (double)((long double)c / (long double)q);
       e[1] = (double)((long double)c28 / (long double)q);
     }
@@ -179,14 +198,6 @@ void build_fused_tables(const HostParams& h, FusedTables* out) {
     const uint64_t thr = d.quirk_thr < q ? d.quirk_thr : q;
     out->scr_thr[i] = (double)((long double)thr / (long double)q) + std::ldexp(1.0, -20);
   }
-  // past the last limb of a group: its first limb again, which adds no hit
-  for (int j = 0; j < K; ++j)
-    for (int g = 0; g < 4 && g < k; ++g)
-      for (int n = (k - g + 3) / 4; n < 16; ++n)
-        for (int h = 0; h < 2; ++h) {
-          double* e = &out->scr[(((size_t)j * 4 + g) * 16) * 2];
-          e[2 * n + h] = e[h];
-        }
 }
 
 }  // namespace aoa

@@ -79,18 +79,19 @@ struct FusedDev {
   const uint64_t* tw[2];
   // last inverse stage's two constants, 4 words per entry ((w, quotient) pairs, or two doubles):
   const uint64_t* lc;      // [k+K]: N^-1, psi^-brev(1) N^-1
-  const uint64_t* lc_key;  // [k+K]: the same, special limbs also times (B/b_j)^-1
+  const uint64_t* lc_b;    // [K]: of special limb j, also times (B/b_j)^-1
+  const uint64_t* lc_down; // [k+1][k] (l, i): also times B^-1 (and q_l^-1 for i < l < k)
   const uint64_t* lc_up;   // [k][k] (l, i): the same times (Q_l/q_i)^-1
   const uint64_t* bq;      // [k][2]: B mod q_i (pair, or one double)
   // ModUp and ModDown as products of signed bytes, in the operand order of
   // the 16x16x64 matrix instruction: [block of 16 outputs][digit][step of 8 inputs][lane][16]
-  const uint8_t* mu_w;     // per level: mu_stride bytes
-  const uint8_t* md_w;
+  const uint8_t* mu_w;     // [k] levels of mu_stride bytes
+  const uint8_t* md_w;     // [k+1] levels rescaled from (k: none) of md_stride bytes
   const ConvOut* mu_out;   // [k][K] (l, j)
-  const ConvOut* md_out;   // [k]
-  const double* scr;       // [K][4][16][2]: frac(c/q_i), frac(2^28 c/q_i) for c = (B/b_j) mod q_i, i = g + 4n
-  const double* scr_thr;   // [64]: screen bound of q_i (0 from k on)
-  uint32_t mu_stride;      // bytes of mu_w per level
+  const ConvOut* md_out;   // [k+1][k] (l, i)
+  const double* scr;       // [K][64][2]: frac(c/q_i), frac(2^28 c/q_i) for c = (B/b_j) mod q_i
+  const double* scr_thr;   // [64]: screen bound of q_i
+  uint32_t mu_stride, md_stride;
   int mu_kb, md_kb;        // steps of 8 inputs the layouts hold
 };
 
@@ -181,11 +182,11 @@ struct HostParams {
 
 // Host tables behind FusedDev.
 struct FusedTables {
-  std::vector<uint64_t> tw[2], lc, lc_key, lc_up, bq;
+  std::vector<uint64_t> tw[2], lc, lc_b, lc_down, lc_up, bq;
   std::vector<uint8_t> mu_w, md_w;
   std::vector<ConvOut> mu_out, md_out;
   std::vector<double> scr, scr_thr;
-  uint32_t mu_stride = 0;
+  uint32_t mu_stride = 0, md_stride = 0;
   int mu_kb = 0, md_kb = 0;
 };
 void build_fused_tables(const HostParams& h, FusedTables* out);
