@@ -290,10 +290,10 @@ __device__ __forceinline__ void down_screen(const DevParams& P, const uint64_t* 
 
 // Limbs 16 ib.. of coefficients 16 nb0..: the conversion and the result
 // f_i x_i - sum (xq holds f_i x_i; with a rescale the dropped limb is input K of
-// the sum), canonical, + add_i.  TOP: limb `level` alone, into input K.
-template <int T, int NB, bool TOP>
+// the sum), canonical, + add_i.
+template <int T, int NB>
 __device__ __forceinline__ void down_out(const DevParams& P, int set, const uint64_t* add, uint64_t* out, int ib, int nb0,
-                                         int lout, uint64_t* aux, const uint64_t* xq, int M, int col0, int lane) {
+                                         int lout, const uint64_t* aux, const uint64_t* xq, int M, int col0, int lane) {
   const FusedDev& Z = P.fz;
   v4i acc[T][NB];
   conv_acc<T, NB>(acc, Z.md_w + (size_t)set * Z.md_stride + (size_t)ib * 8 * Z.md_kb * 1024, Z.md_kb, Z.md_kb, aux, nb0,
@@ -301,22 +301,54 @@ __device__ __forceinline__ void down_out(const DevParams& P, int set, const uint
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int i = ib * 16 + 4 * (lane >> 4) + r;
-    if (TOP ? i == lout : i < lout) {
+    if (i < lout) {
       const ConvOut o = ld_conv(Z.md_out + (size_t)set * P.k + i);
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         const int n = (nb0 + b) * 16 + (lane & 15);
         uint64_t v = conv_join<T, NB>(acc, b, r, o, xq[i * FZ_PITCH + n]);
         v = csub(v, o.p);
-        if (TOP) {
-          aux[P.K * FZ_PITCH + n] = v;
-        } else {
-          const size_t at = (size_t)i * P.N + (size_t)(n / FZ_COLS) * M + col0 + n % FZ_COLS;
-          if (add) v = add_mod(v, add[at], o.p);
-          out[at] = v;
-        }
+        const size_t at = (size_t)i * P.N + (size_t)(n / FZ_COLS) * M + col0 + n % FZ_COLS;
+        if (add) v = add_mod(v, add[at], o.p);
+        out[at] = v;
       }
     }
+  }
+}
+
+// The dropped limb's sum for coefficients 16 nb..: one output, so the rows of a
+// product are its digits (row n: digit n & 7, by the same constants).  Digits 0..3
+// stay in the first 16 lanes, digits 4..7 in the next.
+__device__ __forceinline__ v4i down_top_sum(const DevParams& P, int level, const uint64_t* aux, int nb, int lane) {
+  const FusedDev& Z = P.fz;
+  const int n = lane & 15, g = lane >> 4;
+  const uint8_t* W = Z.md_w + (size_t)P.k * Z.md_stride + ((size_t)(level / 16) * 8 + (n & 7)) * Z.md_kb * 1024;
+  const v4i* w = reinterpret_cast<const v4i*>(W) + (level & 15) + 16 * g;
+  const uint64_t* q = aux + 2 * g * FZ_PITCH + nb * 16 + n;
+  v4i acc{0, 0, 0, 0};
+#pragma unroll 4
+  for (int kb = 0; kb < Z.md_kb; ++kb, q += 8 * FZ_PITCH) {
+    const uint64_t v0 = q[0] ^ 0x8080808080808080ull, v1 = q[FZ_PITCH] ^ 0x8080808080808080ull;
+    const v4i in{(int)(uint32_t)v0, (int)(v0 >> 32), (int)(uint32_t)v1, (int)(v1 >> 32)};
+    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[(size_t)kb * 64], in, acc, 0, 0, 0);
+  }
+  return acc;
+}
+// ... and the limb itself into input K of the other limbs' sums.
+__device__ __forceinline__ void down_top(const DevParams& P, int level, v4i sum, const uint64_t* xq, uint64_t* aux, int nb,
+                                         int lane) {
+  v4i acc[8][1];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    acc[r][0][0] = sum[r];
+    acc[r + 4][0][0] = __shfl(sum[r], (lane & 15) + 16);
+  }
+  if (lane < 16) {
+    const ConvOut o = ld_conv(P.fz.md_out + (size_t)P.k * P.k + level);
+    const int n = nb * 16 + lane;
+    const uint64_t z = xq[level * FZ_PITCH + n];
+    const uint64_t v = conv_join<8, 1>(acc, 0, 0, o, z);  // unused digits are 0
+    aux[P.K * FZ_PITCH + n] = csub(v, o.p);
   }
 }
 
@@ -372,6 +404,8 @@ __global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
   }
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  v4i top{0, 0, 0, 0};
+  if (rescale) top = down_top_sum(P, it.level, aux, wave, lane);
   if (!P.moddown_exact) {
     // two waves of 64 coefficients for each quarter of the limbs
     const int g = wave >> 1, c = (wave & 1) * 64 + lane, per_g = (L + 3) / 4;
@@ -399,22 +433,18 @@ __global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
   const uint64_t* add = glob(y ? it.add1 : it.add0);
   uint64_t* out = glob(y ? it.out1 : it.out0);
   if (rescale) {
-    const int ib = it.level / 16, nb = ld_prime_nb(P.primes, ib * 16);
-    if (nb > 56)
-      down_out<8, 1, true>(P, P.k, nullptr, nullptr, ib, wave, it.level, aux, xq, M, col0, lane);
-    else
-      down_out<7, 1, true>(P, P.k, nullptr, nullptr, ib, wave, it.level, aux, xq, M, col0, lane);
+    down_top(P, it.level, top, xq, aux, wave, lane);
     __syncthreads();
   }
   const int units = ((lout + 15) / 16) * 4;
   for (int u = wave; u < units; u += FZ_THREADS / 64) {
     const int ib = u / 4, nb0 = (u % 4) * 2, nb = ld_prime_nb(P.primes, ib * 16);
     if (nb > 56)
-      down_out<8, 2, false>(P, set, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
+      down_out<8, 2>(P, set, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
     else if (nb > 48)
-      down_out<7, 2, false>(P, set, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
+      down_out<7, 2>(P, set, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
     else
-      down_out<6, 2, false>(P, set, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
+      down_out<6, 2>(P, set, add, out, ib, nb0, lout, aux, xq, M, col0, lane);
   }
 }
 
