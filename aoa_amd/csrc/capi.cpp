@@ -360,7 +360,14 @@ extern "C" int aoa_encrypt(const aoa_params* h, void* stream, uint64_t* c0, uint
   uint64_t* u = (uint64_t*)ws;
   uint64_t* e0 = u + (size_t)k * N;
   uint64_t* e1 = e0 + (size_t)k * N;
-  launch_sample_encrypt(P, u, e0, e1, k, seed, nonce, st);
+  // The fused rows write c0, c1 and m from workgroups of their own, so these
+  // must not overlap each other or what they are formed from.
+  const size_t kN = (size_t)k * N;
+  auto apart = [&](const uint64_t* a, const uint64_t* b, size_t n) { return a + kN <= b || b + n <= a; };
+  const bool fused = nt_default(P) && apart(c0, c1, kN) && apart(c0, m, kN) && apart(c1, m, kN) && apart(c0, u, 3 * kN) &&
+                     apart(c1, u, 3 * kN) && apart(m, u, 3 * kN) && apart(c0, pk_b, kN) && apart(c0, pk_a, kN) &&
+                     apart(c1, pk_b, kN) && apart(c1, pk_a, kN) && apart(m, pk_b, kN) && apart(m, pk_a, kN);
+  launch_sample_encrypt(P, u, e0, e1, fused ? m : nullptr, k, seed, nonce, st);
   LimbMap mm;
   std::memset(&mm, 0, sizeof(mm));
   mm.base[0] = m;
@@ -370,6 +377,13 @@ extern "C" int aoa_encrypt(const aoa_params* h, void* stream, uint64_t* c0, uint
   mm.nlimbs = k;
   mm.qlimbs = k;
   mm.npolys = 4;
+  if (fused) {
+    for (int y = 0; y < 4; ++y) mm.src[y] = mm.base[y];
+    nt_forward_cols(P, mm, st);
+    if (nt_encrypt_rows(P, NtEncrypt{u, e0, e1, pk_b, pk_a, m, c0, c1}, k, st))
+      return fail(AOA_ERR_UNSUPPORTED, "no NTT split for this N");
+    return check_launch("aoa_encrypt");
+  }
   if (ntt_forward(P, mm, 0, st)) return fail(AOA_ERR_UNSUPPORTED, "no NTT split for this N");
   launch_encrypt_combine(P, c0, c1, pk_b, pk_a, u, e0, e1, m, k, st);
   return check_launch("aoa_encrypt");
@@ -382,6 +396,10 @@ extern "C" int aoa_decrypt(const aoa_params* h, void* stream, uint64_t* m, uint6
   const DevParams& P = h->dev;
   hipStream_t st = (hipStream_t)stream;
   const int L = level + 1;
+  if (nt_default(P)) {
+    if (nt_decrypt(P, m, c0, c1, s, L, st)) return fail(AOA_ERR_UNSUPPORTED, "no NTT split for this N");
+    return check_launch("aoa_decrypt");
+  }
   LimbMap mc;
   std::memset(&mc, 0, sizeof(mc));
   mc.base[0] = c0;

@@ -100,8 +100,6 @@ struct FieldLazy {
 #pragma unroll
     for (int c = 0; c < C; ++c) t[c] = tw(T, i + c);
   }
-  // constant `which` of a last-stage entry
-  __device__ __forceinline__ W lc(const uint64_t* e, int which) const { return tw(e, which); }
   __device__ __forceinline__ V mul(V x, W w) const { return shoup4(x, w.w, w.q, np); }
   __device__ __forceinline__ void fwd(V& a, V& b, W w) const {
     const V v = mul(b, w), u = a;
@@ -134,6 +132,7 @@ struct FieldLazy {
   __device__ __forceinline__ uint64_t out_last(V x) const { return x; }  // after inv_last
   // factor of two products: canonical
   __device__ __forceinline__ V factor(V x) const { return out(x); }
+  __device__ __forceinline__ V add(V a, V b) const { return a + b; }  // up to 2^8 p
   __device__ __forceinline__ V key(V x, uint64_t k) const { return mul_barrett62_lazy(x, k, p, mu2, nb); }
   // HomMul's products d2 = a1 b1, d0 = a0 b0, d1 = a0 b1 + a1 b0 and their
   // relinearisation d2 key + (B mod q) d
@@ -173,7 +172,6 @@ struct FieldFp64 {
       }
     }
   }
-  __device__ __forceinline__ W lc(const uint64_t* e, int which) const { return tw(e, which); }
   __device__ __forceinline__ V mul(V x, W w) const {
     const double h = x * w, q = __builtin_rint(h * pinv);
     const double l = __builtin_fma(x, w, -h);
@@ -204,6 +202,7 @@ struct FieldFp64 {
     return (uint64_t)__double_as_longlong(x + 4503599627370496.0) & 0x000fffffffffffffull;
   }
   __device__ __forceinline__ V factor(V x) const { return red(x); }
+  __device__ __forceinline__ V add(V a, V b) const { return a + b; }  // up to 17 p
   __device__ __forceinline__ V key(V x, uint64_t k) const { return mul(x, in(k)); }
   __device__ __forceinline__ V d2(uint64_t a1, uint64_t b1) const { return mul(in(a1), in(b1)); }
   __device__ __forceinline__ V d0(uint64_t a0, uint64_t b0) const { return mul(in(a0), in(b0)); }
@@ -234,7 +233,6 @@ struct FieldStrict {
 #pragma unroll
     for (int k = 0; k < C; ++k) t[k] = tw(T, i + k);
   }
-  __device__ __forceinline__ W lc(const uint64_t* e, int which) const { return tw(e, which); }
   __device__ __forceinline__ V mul(V x, W w) const {
     return csub(mul_shoup_lazy(x, w.w, w.q, p), p);
   }
@@ -259,6 +257,7 @@ struct FieldStrict {
   __device__ __forceinline__ uint64_t out(V x) const { return x; }
   __device__ __forceinline__ uint64_t out_last(V x) const { return x; }
   __device__ __forceinline__ V factor(V x) const { return x; }
+  __device__ __forceinline__ V add(V a, V b) const { return add_mod(a, b, p); }
   // x k mod p by folding at bit 63 twice: 2^63 = c mod p
   __device__ __forceinline__ V key(V x, uint64_t k) const {
     constexpr uint64_t M63 = ~0ull >> 1;
@@ -295,39 +294,53 @@ __device__ __forceinline__ void inv_reduce(const F& f, typename F::V (&x)[V]) {
 // ----------------------------------------------------------------- columns --
 // The 16 rows of a column over four threads q = 0..3 of four values: rows q +
 // 4k for the first two stages, rows 4q + k for the last two.  T: the prime's
-// FusedDev::tw block.
-template <class F>
+// FusedDev::tw block.  U: T and q are the same for a whole wave.
+template <bool U, class F>
+__device__ __forceinline__ typename F::W col_tw(const F& f, const uint64_t* T, int i) {
+  if constexpr (U) return f.tw_u(T, i);
+  return f.tw(T, i);
+}
+template <bool U, class F>
+__device__ __forceinline__ void col_tw2(const F& f, typename F::W (&w)[2], const uint64_t* T, int i) {
+  if constexpr (U) {
+    w[0] = f.tw_u(T, i);
+    w[1] = f.tw_u(T, i + 1);
+  } else {
+    f.tws(w, T, i);
+  }
+}
+template <bool U = false, class F>
 __device__ __forceinline__ void col_fwd_a(const F& f, typename F::V (&x)[4], const uint64_t* T) {
-  const typename F::W w1 = f.tw(T, 1), w2 = f.tw(T, 2), w3 = f.tw(T, 3);
+  const typename F::W w1 = col_tw<U>(f, T, 1), w2 = col_tw<U>(f, T, 2), w3 = col_tw<U>(f, T, 3);
   f.fwd(x[0], x[2], w1);
   f.fwd(x[1], x[3], w1);
   f.fwd(x[0], x[1], w2);
   f.fwd(x[2], x[3], w3);
 }
-template <class F>
+template <bool U = false, class F>
 __device__ __forceinline__ void col_fwd_b(const F& f, typename F::V (&x)[4], const uint64_t* T, int q) {
   typename F::W w[2];
-  const typename F::W w4 = f.tw(T, 4 + q);
-  f.tws(w, T, 8 + 2 * q);
+  const typename F::W w4 = col_tw<U>(f, T, 4 + q);
+  col_tw2<U>(f, w, T, 8 + 2 * q);
   f.fwd(x[0], x[2], w4);
   f.fwd(x[1], x[3], w4);
   f.fwd(x[0], x[1], w[0]);
   f.fwd(x[2], x[3], w[1]);
 }
-template <class F>
+template <bool U = false, class F>
 __device__ __forceinline__ void col_inv_b(const F& f, typename F::V (&x)[4], const uint64_t* T, int q) {
   typename F::W w[2];
-  const typename F::W w4 = f.tw(T, 4 + q);
-  f.tws(w, T, 8 + 2 * q);
+  const typename F::W w4 = col_tw<U>(f, T, 4 + q);
+  col_tw2<U>(f, w, T, 8 + 2 * q);
   f.template inv<0>(x[0], x[1], w[0]);
   f.template inv<0>(x[2], x[3], w[1]);
   f.template inv<1>(x[0], x[2], w4);
   f.template inv<1>(x[1], x[3], w4);
 }
 // Outputs through F::out_last; lc: the last stage's constants.
-template <class F>
+template <bool U = false, class F>
 __device__ __forceinline__ void col_inv_a(const F& f, typename F::V (&x)[4], const uint64_t* T, const uint64_t* lc) {
-  const typename F::W w2 = f.tw(T, 2), w3 = f.tw(T, 3), n0 = f.lc(lc, 0), n1 = f.lc(lc, 1);
+  const typename F::W w2 = col_tw<U>(f, T, 2), w3 = col_tw<U>(f, T, 3), n0 = col_tw<U>(f, lc, 0), n1 = col_tw<U>(f, lc, 1);
   f.template inv<2>(x[0], x[1], w2);
   f.template inv<2>(x[2], x[3], w3);
   f.inv_last(x[0], x[2], n0, n1);

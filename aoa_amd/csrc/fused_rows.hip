@@ -4,53 +4,6 @@
 
 namespace aoa {
 
-// FIELD: the form of every limb of the launch, or FZ_ANY, which looks it up;
-// a kernel of one form holds fewer registers.
-constexpr int FZ_ANY = -1;
-#define FZ_FIELD(pr_, CALL)                                                            \
-  switch (FIELD == FZ_ANY ? (int)ld_prime_field(P.primes, pr_) : FIELD) {              \
-    case FIELD_FP64: if constexpr (FIELD == FZ_ANY || FIELD == FIELD_FP64) CALL(FieldFp64); break;      \
-    case FIELD_LAZY: if constexpr (FIELD == FZ_ANY || FIELD == FIELD_LAZY) CALL(FieldLazy); break;      \
-    default: if constexpr (FIELD == FZ_ANY || FIELD == FIELD_STRICT) CALL(FieldStrict); break;          \
-  }
-
-// Work item of a workgroup: its index, or with P.xcd_chunks the XCD chunk map.
-__device__ __forceinline__ int fz_work(const DevParams& P, int w, int n) { return P.xcd_chunks ? xcd_chunk_id(w, n) : w; }
-
-// Values per thread: four (two stages a round) up to rows of 1024, so that a
-// small call's few rows spread over many waves; eight above.
-template <int LOGM>
-using RowOf = Row<LOGM, (LOGM <= 10 ? 2 : 3)>;
-
-template <int LOGM>
-struct RowId {
-  using G = RowOf<LOGM>;
-  int s, row;
-  uint32_t off;   // byte offset of the thread's first strided element in its limb
-  uint32_t poff;  // of its first packed one
-  uint64_t* L;
-  __device__ __forceinline__ RowId(int tile, uint64_t* lds) {
-    const int rl = G::ROWS == 1 ? 0 : threadIdx.x / G::TS;
-    s = G::ROWS == 1 ? threadIdx.x : threadIdx.x % G::TS;
-    row = tile * G::ROWS + rl;
-    off = (row * G::M + s) * 8;
-    poff = (row * G::M + s * G::V) * 8;
-    L = lds + rl * G::PITCH;
-  }
-};
-
-// The inverse rows of x (packed) and the store.
-template <class F, int LOGM>
-__device__ __forceinline__ void rows_out(const F& f, typename F::V (&x)[RowOf<LOGM>::V], const uint64_t* T, uint64_t* dst,
-                                         const RowId<LOGM>& id) {
-  using G = RowOf<LOGM>;
-  constexpr int LV = LOGM <= 10 ? 2 : 3;
-  const RoundTw<LOGM, LV, G::ROUNDS - 1, F> t(f, T, id.row, id.s);
-  row_inv_from<LOGM, LV, G::ROUNDS - 1>(f, x, t, T, id.row, id.s, id.L);
-#pragma unroll
-  for (int k = 0; k < G::V; ++k) put_byte(dst, id.off + G::TS * 8 * k, f.raw(x[k]));
-}
-
 // ------------------------------------------------------ d2 = a b, its rows --
 template <class F, int LOGM>
 __device__ __forceinline__ void rows_body(const DevParams& P, const uint64_t* a, const uint64_t* b, uint64_t* dst, int pr,
@@ -92,14 +45,6 @@ __global__ __launch_bounds__(RowOf<LOGM>::THREADS) void k_fz_rows(DevParams P, F
 // limbs take their NTT-domain input d2 and addends d0, d1 from the operands;
 // other limbs come as forward columns and take the forward rows here, once for
 // both key halves.  y0..y1: the key halves of this workgroup.
-
-// A zero that the compiler does not see through: what depends on it is formed
-// again for each key half instead of staying in registers from one to the next.
-__device__ __forceinline__ uint32_t opaque_zero() {
-  uint32_t z = 0;
-  asm volatile("" : "+s"(z));
-  return z;
-}
 
 template <class F, int LOGM>
 __device__ __forceinline__ void key_body_tensor(const DevParams& P, const FzItem& it, int m, int tile, int y0, int y1,
@@ -194,23 +139,6 @@ __global__ __launch_bounds__(RowOf<LOGM>::THREADS) __attribute__((amdgpu_waves_p
 }
 
 // ---------------------------------------------------------------- launch ---
-
-static int log2_of(int n) {
-  int g = 0;
-  while ((1 << g) < n) ++g;
-  return g;
-}
-
-#define FZ_DISPATCH_M(CALL)          \
-  switch (log2_of(P.N) - 4) {        \
-    case 7: CALL(7); break;          \
-    case 8: CALL(8); break;          \
-    case 9: CALL(9); break;          \
-    case 10: CALL(10); break;        \
-    case 11: CALL(11); break;        \
-    case 12: CALL(12); break;        \
-    default: return -1;              \
-  }
 
 template <bool ARG, int FIELD>
 static int fz_rows(const DevParams& P, const FzItem& arg, const FzItem* items, const uint32_t* list, int n, hipStream_t st) {

@@ -43,6 +43,23 @@ int fz_key_desc(const DevParams& P, const FzItem* items, const uint32_t* list, i
 int fz_key_special_desc(const DevParams& P, const FzItem* items, const uint32_t* list, int n, int field, hipStream_t st);
 void fz_down_desc(const DevParams& P, const FzItem* items, int n, int max_level, hipStream_t st);
 
+// Plain transforms on the fused kernels' split (fused_ntt.hip), the default
+// where no split was asked for.
+bool nt_default(const DevParams& P);
+int nt_forward(const DevParams& P, const LimbMap& m, hipStream_t st);
+int nt_inverse(const DevParams& P, const LimbMap& m, hipStream_t st);
+int nt_forward_desc(const DevParams& P, const NttDesc* d, int n, hipStream_t st);
+int nt_inverse_desc(const DevParams& P, const NttDesc* d, int n, hipStream_t st);
+// Encryption after the forward columns of m, u, e0 + m and e1 (limbs of N words).
+struct NtEncrypt {
+  const uint64_t *u, *e0, *e1, *pkb, *pka;
+  uint64_t *m, *c0, *c1;
+};
+int nt_encrypt_rows(const DevParams& P, const NtEncrypt& a, int nlimbs, hipStream_t st);
+void nt_forward_cols(const DevParams& P, const LimbMap& m, hipStream_t st);
+// c0, c1 -> NTT domain, m = c0 + c1 s in the coefficient domain.
+int nt_decrypt(const DevParams& P, uint64_t* m, uint64_t* c0, uint64_t* c1, const uint64_t* s, int nlimbs, hipStream_t st);
+
 // out = a op b (out = a*b + c for MULADD) over nlimbs limbs mapped to primes
 // as in LimbMap (qlimbs Q limbs from prime0, then special limbs).
 void launch_encrypt_combine(const DevParams& P, uint64_t* c0, uint64_t* c1, const uint64_t* pkb,
@@ -70,9 +87,9 @@ void launch_conjugate(const DevParams& P, uint64_t* out, const uint64_t* in, int
 void launch_sample(const DevParams& P, uint64_t* out, int res0, int nres, int kind, uint64_t seed, uint64_t nonce,
                    hipStream_t st);
 // u (ZO) at nonce, e0 and e1 (Gaussian) at nonce + 1 and nonce + 2, limbs
-// 0..nres-1, in one launch.
-void launch_sample_encrypt(const DevParams& P, uint64_t* u, uint64_t* e0, uint64_t* e1, int nres, uint64_t seed,
-                           uint64_t nonce, hipStream_t st);
+// 0..nres-1, in one launch; with m, e0 + m.
+void launch_sample_encrypt(const DevParams& P, uint64_t* u, uint64_t* e0, uint64_t* e1, const uint64_t* m, int nres,
+                           uint64_t seed, uint64_t nonce, hipStream_t st);
 
 void launch_special_fft(const DevParams& P, double* vals, int n, int inverse, hipStream_t st);
 void launch_encode_pack(const DevParams& P, uint64_t* out, const double* vals, int slots, double scale, int k,

@@ -15,6 +15,11 @@
 // stages per register round and one LDS exchange between rounds.  Twiddles
 // psi^brev(i) come from a per-prime table with Shoup quotients.
 //
+// These splits run where a caller asks for one (or a tuning run found one
+// faster); the default is N = 16 x M (fused_ntt.hip), faster at every N: 61
+// limbs at N = 2^16 75 us both ways against 100, 4 limbs at N = 2^12 in one
+// workgroup each 11 us against 7.
+//
 // Every pass exists in two launch forms: limbs described by kernel arguments
 // (plain calls) and limbs listed in a device descriptor table (batches).
 #include "device_common.hpp"
@@ -883,11 +888,12 @@ static int pick_n1(const DevParams& P, int N1) {
   }
 
 int ntt_forward(const DevParams& P, LimbMap m, int N1, hipStream_t st) {
+  for (int y = 0; y < m.npolys; ++y)
+    if (!m.src[y]) m.src[y] = m.base[y];
+  if (!N1 && nt_default(P)) return nt_forward(P, m, st);
   N1 = pick_n1(P, N1);
   if (!N1) return -1;
   const int N2 = P.N / N1, g0 = log2i(N1);
-  for (int y = 0; y < m.npolys; ++y)
-    if (!m.src[y]) m.src[y] = m.base[y];
   if (N1 == P.N) {
     dim3 grid(m.nlimbs, m.npolys);
 #define CALL1(L) k_ntt_fwd_single<L><<<grid, SGeo<L>::TH, 0, st>>>(P, m)
@@ -916,12 +922,13 @@ int ntt_forward(const DevParams& P, LimbMap m, int N1, hipStream_t st) {
 
 int ntt_inverse(const DevParams& P, LimbMap m, int N1, const uint64_t* key0, const uint64_t* key1,
                 hipStream_t st, const uint64_t* add0, const uint64_t* add1) {
+  for (int y = 0; y < m.npolys; ++y)
+    if (!m.src[y]) m.src[y] = m.base[y];
+  if (!N1 && !key0 && nt_default(P)) return nt_inverse(P, m, st);
   N1 = pick_n1(P, N1);
   if (!N1) return -1;
   if ((add0 || add1) && (N1 == P.N || !key0)) return -1;  // adds: two-pass key products only
   const int N2 = P.N / N1, g0 = log2i(N1);
-  for (int y = 0; y < m.npolys; ++y)
-    if (!m.src[y]) m.src[y] = m.base[y];
   if (N1 == P.N) {
     dim3 grid(m.nlimbs, m.npolys);
 #define CALL1(L) k_ntt_inv_single<L><<<grid, SGeo<L>::TH, 0, st>>>(P, m, key0, key1)
@@ -963,6 +970,7 @@ int ntt_inverse(const DevParams& P, LimbMap m, int N1, const uint64_t* key0, con
   } while (0)
 
 int ntt_forward_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hipStream_t st, int nstrict) {
+  if (!N1 && nt_default(P)) return nt_forward_desc(P, d, ndesc, st);
   N1 = pick_n1(P, N1);
   if (!N1 || ndesc <= 0) return -1;
   const int N2 = P.N / N1, g0 = log2i(N1);
@@ -988,6 +996,7 @@ int ntt_forward_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hi
 }
 
 int ntt_inverse_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hipStream_t st, int nstrict, bool canon) {
+  if (!N1 && nt_default(P)) return nt_inverse_desc(P, d, ndesc, st);
   N1 = pick_n1(P, N1);
   if (!N1 || ndesc <= 0) return -1;
   const int N2 = P.N / N1, g0 = log2i(N1);

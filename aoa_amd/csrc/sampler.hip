@@ -99,9 +99,10 @@ __global__ __launch_bounds__(256) void k_sample_uniform(DevParams P, uint64_t* o
   out[(size_t)l * P.N + i] = u_hi + (s < u_lo ? 1 : 0);
 }
 
-// Gaussian, ZO and narrow: one value per coefficient, written to every limb.
-__device__ __forceinline__ void sample_small_at(const DevParams& P, uint64_t* out, int res0, int nres, int kind,
-                                                uint64_t seed, uint64_t nonce, uint32_t i) {
+// Gaussian, ZO and narrow: one value per coefficient, written to every limb
+// (plus add's limb, canonical, if there is one).
+__device__ __forceinline__ void sample_small_at(const DevParams& P, uint64_t* out, const uint64_t* add, int res0, int nres,
+                                                int kind, uint64_t seed, uint64_t nonce, uint32_t i) {
   const u32x4 c = draw(seed, nonce, ((uint32_t)kind << 24) | 0xFFFFFFu, i);
   int64_t v;
   if (kind == SAMPLE_GAUSSIAN) {
@@ -116,32 +117,47 @@ __device__ __forceinline__ void sample_small_at(const DevParams& P, uint64_t* ou
   } else {  // narrow
     v = (int64_t)__umul64hi(lo64(c), 3) - 1;
   }
-  for (int l = res0; l < res0 + nres; ++l)
-    out[(size_t)l * P.N + i] = small_residue(v, ld_prime(P.primes, l).p);
+  if (!add) {
+    for (int l = res0; l < res0 + nres; ++l) out[(size_t)l * P.N + i] = small_residue(v, ld_prime_p(P.primes, l));
+    return;
+  }
+  // eight limbs' addends requested together: a store may alias the next load
+  for (int l0 = res0; l0 < res0 + nres; l0 += 8) {
+    uint64_t m[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) m[j] = l0 + j < res0 + nres ? add[(size_t)(l0 + j) * P.N + i] : 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (l0 + j < res0 + nres) {
+        const uint64_t p = ld_prime_p(P.primes, l0 + j);
+        out[(size_t)(l0 + j) * P.N + i] = add_mod(small_residue(v, p), m[j], p);
+      }
+    }
+  }
 }
 
 __global__ __launch_bounds__(256) void k_sample_small(DevParams P, uint64_t* out, int res0, int nres, int kind,
                                                       uint64_t seed, uint64_t nonce) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   if (i >= (uint32_t)P.N) return;
-  sample_small_at(P, out, res0, nres, kind, seed, nonce, i);
+  sample_small_at(P, out, nullptr, res0, nres, kind, seed, nonce, i);
 }
 
 // An encryption's three draws in one launch (blockIdx.y = 0, 1, 2): u (ZO) at
 // nonce, e0 and e1 (Gaussian) at nonce + 1 and nonce + 2, limbs 0..nres-1;
-// the same values as three aoa_sample calls.
+// the same values as three aoa_sample calls; with m, e0 + m.
 __global__ __launch_bounds__(256) void k_sample_encrypt(DevParams P, uint64_t* u, uint64_t* e0, uint64_t* e1,
-                                                        int nres, uint64_t seed, uint64_t nonce) {
+                                                        const uint64_t* m, int nres, uint64_t seed, uint64_t nonce) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   if (i >= (uint32_t)P.N) return;
   const int y = blockIdx.y;
-  sample_small_at(P, y == 0 ? u : (y == 1 ? e0 : e1), 0, nres, y == 0 ? SAMPLE_ZO : SAMPLE_GAUSSIAN, seed,
+  sample_small_at(P, y == 0 ? u : (y == 1 ? e0 : e1), y == 1 ? m : nullptr, 0, nres, y == 0 ? SAMPLE_ZO : SAMPLE_GAUSSIAN, seed,
                   nonce + (uint64_t)y, i);
 }
 
-void launch_sample_encrypt(const DevParams& P, uint64_t* u, uint64_t* e0, uint64_t* e1, int nres, uint64_t seed,
-                           uint64_t nonce, hipStream_t st) {
-  k_sample_encrypt<<<dim3((unsigned)((P.N + 255) / 256), 3), 256, 0, st>>>(P, u, e0, e1, nres, seed, nonce);
+void launch_sample_encrypt(const DevParams& P, uint64_t* u, uint64_t* e0, uint64_t* e1, const uint64_t* m, int nres,
+                           uint64_t seed, uint64_t nonce, hipStream_t st) {
+  k_sample_encrypt<<<dim3((unsigned)((P.N + 255) / 256), 3), 256, 0, st>>>(P, u, e0, e1, m, nres, seed, nonce);
 }
 
 __global__ __launch_bounds__(256) void k_fill_zero(uint64_t* out, size_t n) {
