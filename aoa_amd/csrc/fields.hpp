@@ -9,7 +9,8 @@
 //               with h = a w rounded, l = a w - h exact and q = rint(h / p): exact
 //               while |a| <= 17 p (|h - q p| and the result stay below 2^53).  A
 //               butterfly is eight FP64 instructions and its twiddle one double.
-//  FieldStrict  wider primes (the 63-bit q0): canonical residues.
+//  FieldStrict  wider primes (the 63-bit q0, p = 2^63 - c): 64-bit values, with
+//               2^63 = c and a carry out of 64 bits = 2c; below 2p in the inverse.
 //
 // Bounds.  Forward: every stage adds at most 4p (lazy) or about 0.6 p (FP64):
 // 16 stages stay below 72 p and 12 p.  Inverse: a stage doubles the sums; after
@@ -212,69 +213,87 @@ struct FieldFp64 {
   __device__ __forceinline__ V relin(V d2, uint64_t k, V d, W bq) const { return mul(d2, in(k)) + mul(d, bq); }
 };
 
+// Of a small call's limbs this one ends last: a butterfly is 33 vector
+// instructions (a Shoup product and canonical sums: about 45).
 struct FieldStrict {
   using V = uint64_t;
-  struct W {
-    uint64_t w, q;
-  };
+  using W = uint64_t;
   uint64_t p;
-  uint32_t c;  // p = 2^63 - c, c < 2^26 (build_host_params checks it)
-  __device__ __forceinline__ explicit FieldStrict(const DevPrime& d) : p(d.p), c((uint32_t)d.eps) {}
+  uint32_t c, c2;  // p = 2^63 - c, c < 2^26 (build_host_params checks it); 2c
+  __device__ __forceinline__ explicit FieldStrict(const DevPrime& d) : p(d.p), c((uint32_t)d.eps), c2(2 * (uint32_t)d.eps) {}
   __device__ __forceinline__ V in(uint64_t x) const { return x; }
   __device__ __forceinline__ V raw_in(uint64_t x) const { return x; }
   __device__ __forceinline__ uint64_t raw(V x) const { return x; }
-  __device__ __forceinline__ W tw(const uint64_t* T, uint32_t i) const {
-    const tw2 t = at_byte<tw2>(T, i * 16);
-    return W{t.w, t.q};
-  }
-  __device__ __forceinline__ W tw_u(const uint64_t* T, uint32_t i) const { return at_byte_u<W>(T, i * 16); }
+  __device__ __forceinline__ W tw(const uint64_t* T, uint32_t i) const { return at_byte<uint64_t>(T, i * 16); }
+  __device__ __forceinline__ W tw_u(const uint64_t* T, uint32_t i) const { return at_byte_u<uint64_t>(T, i * 16); }
   template <int C>
   __device__ __forceinline__ void tws(W (&t)[C], const uint64_t* T, uint32_t i) const {
 #pragma unroll
     for (int k = 0; k < C; ++k) t[k] = tw(T, i + k);
   }
+  // x w mod p, any x, w < p: below 2^63 + 2^54, by folding at bit 63 (2^63 = c).
+  // x w = z 2^63 + lo with z c = t 2^63 + m (t < 2^27 + 1), s = lo + m < 2^64.
   __device__ __forceinline__ V mul(V x, W w) const {
-    return csub(mul_shoup_lazy(x, w.w, w.q, p), p);
+    constexpr uint64_t M63 = ~0ull >> 1;
+    uint64_t hi, lo;
+    mul128(x, w, &hi, &lo);
+    const uint64_t z = (hi << 1) | (lo >> 63);
+    const uint64_t u = (uint64_t)(uint32_t)z * c, v = (z >> 32) * c + (u >> 32);  // z c = v 2^32 + low word of u
+    const uint64_t s = (lo & M63) + (((v << 32) & M63) | (uint32_t)u);
+    return (uint64_t)((uint32_t)(v >> 31) + (uint32_t)(s >> 63)) * c + (s & M63);
+  }
+  // u + v and u - v as 64-bit values, v < 2p: a carry is 2^64 = 2c mod p.  No
+  // second one: u + v - 2^64 < 2p and u - v + 2^64 > 2c.
+  __device__ __forceinline__ V plus(V u, V v) const {
+    unsigned b0, b1;
+    const uint32_t l = __builtin_addc((uint32_t)u, (uint32_t)v, 0u, &b0);
+    const uint32_t h = __builtin_addc((uint32_t)(u >> 32), (uint32_t)(v >> 32), b0, &b1);
+    return (((uint64_t)h << 32) | l) + (b1 ? c2 : 0u);
+  }
+  __device__ __forceinline__ V minus(V u, V v) const {
+    unsigned b0, b1;
+    const uint32_t l = __builtin_subc((uint32_t)u, (uint32_t)v, 0u, &b0);
+    const uint32_t h = __builtin_subc((uint32_t)(u >> 32), (uint32_t)(v >> 32), b0, &b1);
+    return (((uint64_t)h << 32) | l) - (b1 ? c2 : 0u);
+  }
+  // u + v below 2p for u, v < 2p
+  __device__ __forceinline__ V add(V u, V v) const {
+    unsigned b0, b1, b2, b3;
+    const uint32_t l = __builtin_addc((uint32_t)u, (uint32_t)v, 0u, &b0);
+    const uint32_t h = __builtin_addc((uint32_t)(u >> 32), (uint32_t)(v >> 32), b0, &b1);
+    const uint32_t tl = __builtin_addc(l, c2, 0u, &b2), th = __builtin_addc(h, 0u, b2, &b3);
+    return b1 | b3 ? ((uint64_t)th << 32) | tl : ((uint64_t)h << 32) | l;
   }
   __device__ __forceinline__ void fwd(V& a, V& b, W w) const {
     const V v = mul(b, w), u = a;
-    a = csub(u + v, p);
-    b = csub(diff(u, v, p + 1), p);
+    a = plus(u, v);
+    b = minus(u, v);
   }
   template <int S>
   __device__ __forceinline__ void inv(V& a, V& b, W w) const {
     const V u = a, v = b;
-    a = csub(u + v, p);
-    b = mul(diff(u, v, p + 1), w);
+    a = add(u, v);
+    b = mul(minus(u, v), w);
   }
   __device__ __forceinline__ void inv_last(V& a, V& b, W w0, W w1) const {
     const V u = a, v = b;
-    a = mul(u + v, w0);
-    b = mul(diff(u, v, p + 1), w1);
+    a = csub(mul(add(u, v), w0), p);
+    b = csub(mul(minus(u, v), w1), p);
   }
   __device__ __forceinline__ V red(V x) const { return x; }
   static constexpr int kGrow = 64;
-  __device__ __forceinline__ uint64_t out(V x) const { return x; }
-  __device__ __forceinline__ uint64_t out_last(V x) const { return x; }
+  __device__ __forceinline__ uint64_t out(V x) const {
+    return csub((x & (~0ull >> 1)) + (x >> 63 ? c : 0u), p);
+  }
+  __device__ __forceinline__ uint64_t out_last(V x) const { return x; }  // after inv_last
   __device__ __forceinline__ V factor(V x) const { return x; }
-  __device__ __forceinline__ V add(V a, V b) const { return add_mod(a, b, p); }
-  // x k mod p by folding at bit 63 twice: 2^63 = c mod p
-  __device__ __forceinline__ V key(V x, uint64_t k) const {
-    constexpr uint64_t M63 = ~0ull >> 1;
-    uint64_t hi, lo;
-    mul128(x, k, &hi, &lo);
-    const uint64_t z = (hi << 1) | (lo >> 63);  // x k = z 2^63 + (lo mod 2^63)
-    const uint64_t u = (uint64_t)(uint32_t)z * c, v = (z >> 32) * c + (u >> 32);  // z c = v 2^32 + low word of u
-    uint64_t r = (lo & M63) + (((v << 32) & M63) | (uint32_t)u);
-    r = csub(r, p) + (v >> 31) * c;  // the product is below 2^52
-    return csub(r, p);
-  }
-  __device__ __forceinline__ V d2(uint64_t a1, uint64_t b1) const { return key(a1, b1); }
-  __device__ __forceinline__ V d0(uint64_t a0, uint64_t b0) const { return key(a0, b0); }
+  __device__ __forceinline__ V key(V x, uint64_t k) const { return mul(x, k); }
+  __device__ __forceinline__ V d2(uint64_t a1, uint64_t b1) const { return mul(a1, b1); }
+  __device__ __forceinline__ V d0(uint64_t a0, uint64_t b0) const { return mul(a0, b0); }
   __device__ __forceinline__ V d1(uint64_t a0, uint64_t a1, uint64_t b0, uint64_t b1) const {
-    return add_mod(key(a0, b1), key(a1, b0), p);
+    return add(mul(a0, b1), mul(a1, b0));
   }
-  __device__ __forceinline__ V relin(V d2, uint64_t k, V d, W bq) const { return add_mod(key(d2, k), mul(d, bq), p); }
+  __device__ __forceinline__ V relin(V d2, uint64_t k, V d, W bq) const { return add(mul(d2, k), mul(d, bq)); }
 };
 
 // Brings the values that an inverse round of NB stages has doubled more than
@@ -447,13 +466,15 @@ __device__ __forceinline__ void row_turn(const F& f, typename F::V (&x)[1 << LOG
 
 // Strided in, packed out.  A thread writes to LDS only where it read last, so
 // one barrier per exchange is enough.  Each round's twiddles are requested
-// before the barrier that leads to it.
+// before the round that precedes it.
 template <int LOGM, int LOGV, int I, class F>
 __device__ __forceinline__ void row_fwd_from(const F& f, typename F::V (&x)[1 << LOGV], const RoundTw<LOGM, LOGV, I, F>& t,
                                              const uint64_t* T, int row, int s, uint64_t* L) {
-  round_fwd<LOGM, LOGV, I>(f, x, t);
-  if constexpr (I + 1 < Row<LOGM, LOGV>::ROUNDS) {
+  if constexpr (I + 1 >= Row<LOGM, LOGV>::ROUNDS) {
+    round_fwd<LOGM, LOGV, I>(f, x, t);
+  } else {
     const RoundTw<LOGM, LOGV, I + 1, F> n(f, T, row, s);
+    round_fwd<LOGM, LOGV, I>(f, x, t);
     row_turn<LOGM, LOGV, I, I + 1>(f, x, s, L);
     row_fwd_from<LOGM, LOGV, I + 1>(f, x, n, T, row, s, L);
   }
@@ -469,9 +490,11 @@ __device__ __forceinline__ void row_fwd(const F& f, typename F::V (&x)[1 << LOGV
 template <int LOGM, int LOGV, int I, class F>
 __device__ __forceinline__ void row_inv_from(const F& f, typename F::V (&x)[1 << LOGV], const RoundTw<LOGM, LOGV, I, F>& t,
                                              const uint64_t* T, int row, int s, uint64_t* L) {
-  round_inv<LOGM, LOGV, I, 0>(f, x, t);
-  if constexpr (I > 0) {
+  if constexpr (I == 0) {
+    round_inv<LOGM, LOGV, I, 0>(f, x, t);
+  } else {
     const RoundTw<LOGM, LOGV, I - 1, F> n(f, T, row, s);
+    round_inv<LOGM, LOGV, I, 0>(f, x, t);
     row_turn<LOGM, LOGV, I, I - 1>(f, x, s, L);
     row_inv_from<LOGM, LOGV, I - 1>(f, x, n, T, row, s, L);
   }

@@ -82,7 +82,7 @@ template <class F, int LOGM, bool INV>
 __device__ __forceinline__ void nt_rows(const DevParams& P, const uint64_t* src, uint64_t* dst, int pr, int tile,
                                         uint64_t* lds) {
   using G = RowOf<LOGM>;
-  constexpr int LV = LOGM <= 10 ? 2 : 3;
+  constexpr int LV = kLogV<LOGM>;
   const RowId<LOGM> id(tile, lds);
   uint64_t u[G::V];
 #pragma unroll
@@ -116,13 +116,13 @@ __global__ __launch_bounds__(RowOf<LOGM>::THREADS) void k_nt_rows(DevParams P, L
 
 // Decryption's rows: both components' forward rows (stored, as the transforms
 // leave them), c0 + c1 s and its inverse rows.  A chain of three row transforms
-// in one launch: 21.6 us at N = 2^15, 12 limbs, for the 31 of two launches of
+// in one launch: 16.9 us at N = 2^15, 12 limbs, for the 31 of two launches of
 // rows and the product between them.
 template <class F, int LOGM>
 __device__ __forceinline__ void nt_decrypt(const DevParams& P, uint64_t* c0, uint64_t* c1, const uint64_t* s, uint64_t* out,
                                            int pr, int tile, uint64_t* lds) {
   using G = RowOf<LOGM>;
-  constexpr int LV = LOGM <= 10 ? 2 : 3;
+  constexpr int LV = kLogV<LOGM>;
   const RowId<LOGM> id(tile, lds);
   const F f(ld_prime(P.primes, pr));
   const uint64_t* T = P.fz.tw[0] + (size_t)pr * P.N * 2;

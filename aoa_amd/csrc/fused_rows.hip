@@ -9,7 +9,7 @@ template <class F, int LOGM>
 __device__ __forceinline__ void rows_body(const DevParams& P, const uint64_t* a, const uint64_t* b, uint64_t* dst, int pr,
                                           int tile, uint64_t* lds) {
   using G = RowOf<LOGM>;
-  constexpr int LV = LOGM <= 10 ? 2 : 3;
+  constexpr int LV = kLogV<LOGM>;
   const F f(ld_prime(P.primes, pr));
   const uint64_t* T = P.fz.tw[1] + (size_t)pr * P.N * 2;
   const RowId<LOGM> id(tile, lds);
@@ -50,7 +50,7 @@ template <class F, int LOGM>
 __device__ __forceinline__ void key_body_tensor(const DevParams& P, const FzItem& it, int m, int tile, int y0, int y1,
                                                 uint64_t* lds) {
   using G = RowOf<LOGM>;
-  constexpr int LV = LOGM <= 10 ? 2 : 3;
+  constexpr int LV = kLogV<LOGM>;
   const F f(ld_prime(P.primes, m));
   const uint64_t* T = P.fz.tw[1] + (size_t)m * P.N * 2;
   const RowId<LOGM> id(tile, lds);
@@ -85,7 +85,7 @@ template <class F, int LOGM>
 __device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, int m, int pr, int tile, int y0, int y1,
                                          uint64_t* lds) {
   using G = RowOf<LOGM>;
-  constexpr int LV = LOGM <= 10 ? 2 : 3;
+  constexpr int LV = kLogV<LOGM>;
   const F f(ld_prime(P.primes, pr));
   const int N = P.N, L = it.level + 1;
   const uint64_t* T = P.fz.tw[1] + (size_t)pr * N * 2;
