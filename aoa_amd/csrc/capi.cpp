@@ -70,8 +70,8 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
       {H.inv_b_mod_q.data(), H.inv_b_mod_q.size() * 8, 0},
       {H.b_mod_q.data(), H.b_mod_q.size() * 8, 0},
       {H.inv_ql_mod_qi.data(), H.inv_ql_mod_qi.size() * 8, 0},
-      {H.enc_w.data(), H.enc_w.size() * 8, 0},
-      {H.rot_group.data(), H.rot_group.size() * 4, 0},
+      {H.enc_t[0].data(), H.enc_t[0].size() * 8, 0},
+      {H.enc_t[1].data(), H.enc_t[1].size() * 8, 0},
       {H.gauss_cdt.data(), H.gauss_cdt.size() * 8, 0},
       {H.md_terms.data(), H.md_terms.size() * sizeof(MdTerm), 0},
       {H.md_thr.data(), H.md_thr.size() * 4, 0},
@@ -141,8 +141,8 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
   D.inv_b_mod_q = (const uint64_t*)(b + secs[7].off);
   D.b_mod_q = (const uint64_t*)(b + secs[8].off);
   D.inv_ql_mod_qi = (const uint64_t*)(b + secs[9].off);
-  D.enc_w = (const double*)(b + secs[10].off);
-  D.rot_group = (const uint32_t*)(b + secs[11].off);
+  D.enc_t[0] = (const double*)(b + secs[10].off);
+  D.enc_t[1] = (const double*)(b + secs[11].off);
   D.gauss_cdt = (const uint64_t*)(b + secs[12].off);
   D.md_terms = (const uint32_t*)(b + secs[13].off);
   D.md_thr = (const uint32_t*)(b + secs[14].off);
@@ -322,8 +322,7 @@ extern "C" int aoa_encode(const aoa_params* h, void* stream, uint64_t* out, doub
   if (scale == 0) return fail(AOA_ERR_ARG, "scale must be positive");
   if (nres <= 0 || nres > h->host.k) return fail(AOA_ERR_ARG, "limb count out of range");
   if (!aligned16(vals)) return fail(AOA_ERR_ARG, "values must be 16-byte aligned");
-  launch_special_fft(h->dev, vals, slots, 1, (hipStream_t)stream);
-  launch_encode_pack(h->dev, out, vals, slots, (double)scale, nres, (hipStream_t)stream);
+  launch_encode(h->dev, out, vals, slots, (double)scale, nres, (hipStream_t)stream);
   return check_launch("aoa_encode");
 }
 
@@ -333,8 +332,7 @@ extern "C" int aoa_decode(const aoa_params* h, void* stream, double* vals, const
   if (!slots_ok(h, slots)) return fail(AOA_ERR_ARG, "slots must be a power of two <= N/2");
   if (scale == 0) return fail(AOA_ERR_ARG, "scale must be positive");
   if (!aligned16(vals)) return fail(AOA_ERR_ARG, "values must be 16-byte aligned");
-  launch_decode_unpack(h->dev, vals, in, slots, (double)scale, (hipStream_t)stream);
-  launch_special_fft(h->dev, vals, slots, 0, (hipStream_t)stream);
+  launch_decode(h->dev, vals, in, slots, (double)scale, (hipStream_t)stream);
   return check_launch("aoa_decode");
 }
 

@@ -4,10 +4,10 @@
 // The FFT follows the reference's loop structure (HEAAN's fftSpecial /
 // fftSpecialInv): a bit reversal and log2(n) radix-2 stages whose twiddle
 // for butterfly j of a block of length len is exp(+-2 pi i (5^j mod 4 len) /
-// (4 len)), read from the parameter set's table of 2N-th roots.  Every
-// stage is one launch of n/2 threads (n <= N/2 slot values); the arithmetic
-// is written operation by operation with contraction off, so each value is
-// rounded exactly as the host loops round it.
+// (4 len)).  Entry len/2 + j of a direction's table holds it (DevParams::enc_t),
+// so a stage's twiddles are consecutive.  The arithmetic is written operation
+// by operation with contraction off, so each value is rounded exactly as the
+// host loops round it.
 #include "device_common.hpp"
 #include "kernels.hpp"
 
@@ -15,7 +15,7 @@
 
 namespace aoa {
 
-struct alignas(16) cplx {
+struct cplx {
   double re, im;
 };
 
@@ -23,10 +23,6 @@ __device__ __forceinline__ cplx cmul(cplx a, cplx b) {
   const double re = a.re * b.re - a.im * b.im;
   const double im = a.re * b.im + a.im * b.re;
   return cplx{re, im};
-}
-
-__device__ __forceinline__ cplx enc_root(const DevParams& P, uint32_t t) {
-  return cplx{P.enc_w[2 * (size_t)t], P.enc_w[2 * (size_t)t + 1]};
 }
 
 // In-place bit reversal: the thread of the smaller index of each pair swaps
@@ -47,28 +43,17 @@ __global__ __launch_bounds__(256) void k_enc_bitrev(cplx* v, int n, int logn, in
   if (i != j) v[j] = a;
 }
 
-// fftSpecial stage (encoder.cu:56-70): u = v[a], t = v[b] * ksi; v[a] = u + t, v[b] = u - t.
-__global__ __launch_bounds__(256) void k_enc_stage_fwd(DevParams P, cplx* v, int n, int len) {
-  const int b = blockIdx.x * 256 + threadIdx.x;
-  if (b >= n / 2) return;
-  const int lenh = len >> 1, lenq = len << 2;
-  const int i = (b / lenh) * len, j = b % lenh;
-  const uint32_t t = (P.rot_group[j] % (uint32_t)lenq) * (uint32_t)(2 * P.N / lenq);
-  const cplx u = v[i + j], w = cmul(v[i + j + lenh], enc_root(P, t));
-  v[i + j] = cplx{u.re + w.re, u.im + w.im};
-  v[i + j + lenh] = cplx{u.re - w.re, u.im - w.im};
+// fftSpecial's butterfly (encoder.cu:56-70): u = v[a], t = v[b] * ksi; v[a] = u + t, v[b] = u - t.
+__device__ __forceinline__ void bfly_fwd(cplx& a, cplx& b, cplx w) {
+  const cplx u = a, t = cmul(b, w);
+  a = cplx{u.re + t.re, u.im + t.im};
+  b = cplx{u.re - t.re, u.im - t.im};
 }
-
-// fftSpecialInv stage (encoder.cu:96-110): u = v[a] + v[b], t = (v[a] - v[b]) * ksi^-1.
-__global__ __launch_bounds__(256) void k_enc_stage_inv(DevParams P, cplx* v, int n, int len) {
-  const int b = blockIdx.x * 256 + threadIdx.x;
-  if (b >= n / 2) return;
-  const int lenh = len >> 1, lenq = len << 2;
-  const int i = (b / lenh) * len, j = b % lenh;
-  const uint32_t t = ((uint32_t)lenq - P.rot_group[j] % (uint32_t)lenq) * (uint32_t)(2 * P.N / lenq);
-  const cplx x = v[i + j], y = v[i + j + lenh];
-  v[i + j] = cplx{x.re + y.re, x.im + y.im};
-  v[i + j + lenh] = cmul(cplx{x.re - y.re, x.im - y.im}, enc_root(P, t));
+// fftSpecialInv's (encoder.cu:96-110): u = v[a] + v[b], t = (v[a] - v[b]) * ksi^-1.
+__device__ __forceinline__ void bfly_inv(cplx& a, cplx& b, cplx w) {
+  const cplx x = a, y = b;
+  a = cplx{x.re + y.re, x.im + y.im};
+  b = cmul(cplx{x.re - y.re, x.im - y.im}, w);
 }
 
 // Residues of the encoded plaintext on limbs 0..k-1 (encoder.cu:166-221):
@@ -97,16 +82,17 @@ __global__ __launch_bounds__(256) void k_enc_pack(DevParams P, uint64_t* out, co
 // Slot values from limb 0 in the coefficient domain (encoder.cu:223-257):
 // the residue x <= p/2 gives x / scale, a larger one (x - p) / scale, both
 // converted to double before the subtraction as the reference does.
-__global__ __launch_bounds__(256) void k_dec_unpack(DevParams P, cplx* out, const uint64_t* in, int slots,
-                                                    double scale) {
-  const int s = blockIdx.x * 256 + threadIdx.x;
-  if (s >= slots) return;
-  const int half = P.N / 2, gap = half / slots;
-  const uint64_t p = P.primes[0].p;
-  const uint64_t a = in[(size_t)s * gap], b = in[(size_t)s * gap + half];
-  const double re = a <= (p >> 1) ? (double)a / scale : ((double)a - (double)p) / scale;
-  const double im = b <= (p >> 1) ? (double)b / scale : ((double)b - (double)p) / scale;
-  out[s] = cplx{re, im};
+struct DecodeIn {
+  const uint64_t* in;  // limb 0, or null: the values are in memory
+  int slots;
+  double scale;
+};
+__device__ __forceinline__ cplx dec_value(const DevParams& P, const DecodeIn& d, int s) {
+  const int half = P.N / 2, gap = half / d.slots;
+  const uint64_t p = ld_prime_p(P.primes, 0);
+  const uint64_t a = d.in[(size_t)s * gap], b = d.in[(size_t)s * gap + half];
+  return cplx{a <= (p >> 1) ? (double)a / d.scale : ((double)a - (double)p) / d.scale,
+              b <= (p >> 1) ? (double)b / d.scale : ((double)b - (double)p) / d.scale};
 }
 
 static int ilog2(int n) {
@@ -117,127 +103,222 @@ static int ilog2(int n) {
 
 static unsigned blocks(size_t n) { return (unsigned)((n + 255) / 256); }
 
-// Stages of length <= B inside aligned blocks of B values, in LDS: one
-// workgroup per block (B <= 4096: 64 KiB of values and 8 KiB of the rotation
-// group).  Forward: stages len = 2..B; inverse: len = B..2.  With whole != 0
-// the block is the whole vector and the bit reversal is folded into the load
-// (forward) or, with the division by n, into the store (inverse).  Each
-// thread takes the butterflies b = t, t + 1024 of every stage and requests
-// the next stage's roots before the barrier, so the table latency overlaps
-// it; the arithmetic of each butterfly is unchanged.
-constexpr int kFftThreads = 1024;
+// The stages of length <= B inside aligned blocks of B <= 4096 values, one
+// workgroup of B / 4 threads per block: four values a thread and two stages a
+// round (after a first, or before a last, round of one stage if log2 B is odd),
+// with one exchange through LDS between rounds, where a thread writes only what
+// it read last; each round's twiddles are requested a round earlier.  Latency
+// bound: the chain of rounds sets the time (2048 values: 12.0 us with a stage a
+// barrier and the twiddles looked up through 5^j, 5.9 now).
+// rev: the bit reversal over n values, on the way in (forward) or out
+// (inverse, with the division by n: a product with 1/n, exact).
 constexpr int kFftBlock = 4096;
-constexpr int kFftPer = kFftBlock / 2 / kFftThreads;  // butterflies per thread and stage
+__device__ __forceinline__ int fft_pad(int i) { return i + (i >> 2); }
+__device__ __forceinline__ int fft_at(int lo, int t, int k) {
+  return ((t >> lo) << (lo + 2)) + (t & ((1 << lo) - 1)) + (k << lo);
+}
+__device__ __forceinline__ int brev(int i, int logn) { return logn ? (int)(__brev((unsigned)i) >> (32 - logn)) : 0; }
 
-__global__ __launch_bounds__(kFftThreads) void k_enc_fft_block(DevParams P, cplx* v, int B, int logB, int inverse,
-                                                               int whole) {
-  extern __shared__ cplx buf[];
-  uint32_t* rot = reinterpret_cast<uint32_t*>(buf + B);  // rotation group 5^j mod 2N, j < B/2
-  const int t = threadIdx.x;
-  cplx* blk = v + (size_t)blockIdx.x * B;
-  if (whole && !inverse) {
-    for (int i = t; i < B; i += kFftThreads) buf[logB ? (__brev((unsigned)i) >> (32 - logB)) : 0] = blk[i];
-  } else {
-    for (int i = t; i < B; i += kFftThreads) buf[i] = blk[i];
-  }
-  for (int i = t; i < B / 2; i += kFftThreads) rot[i] = P.rot_group[i];
-  __syncthreads();
-  // root of butterfly b in the stage of length len
-  auto root = [&](int len, int b) {
-    const int lenh = len >> 1, lenq = len << 2;
-    const uint32_t step = (uint32_t)(2 * P.N / lenq);
-    const uint32_t r = rot[b % lenh] % (uint32_t)lenq;
-    return enc_root(P, (inverse ? (uint32_t)lenq - r : r) * step);
+template <bool INV>
+__global__ __launch_bounds__(kFftBlock / 4) void k_enc_fft(DevParams P, const cplx* src, cplx* dst, int logB, int logn, int rev,
+                                                           DecodeIn d) {
+  extern __shared__ double fft_lds[];
+  const int B = 1 << logB, t = threadIdx.x, base = blockIdx.x << logB;
+  double *re = fft_lds, *im = fft_lds + B + (B >> 2);
+  const cplx* T = reinterpret_cast<const cplx*>(P.enc_t[INV]);
+  const bool on = 4 * t < B;
+  cplx x[4], w[3];
+  // entry of a round's first stage, then the two of its second (double rounds)
+  auto twiddles = [&](int lo, int low) {
+    w[0] = T[(1 << lo) + low];
+    w[1] = T[(2 << lo) + low];
+    w[2] = T[(3 << lo) + low];
   };
-  cplx w[kFftPer];
-  const int first = inverse ? B : 2;
+  auto exchange = [&](int from, int to) {
+    if (on) {
 #pragma unroll
-  for (int q = 0; q < kFftPer; ++q) {
-    const int b = t + q * kFftThreads;
-    if (b < B / 2) w[q] = root(first, b);
-  }
-  if (!inverse) {
-    for (int len = 2; len <= B; len <<= 1) {
-      const int lenh = len >> 1;
-#pragma unroll
-      for (int q = 0; q < kFftPer; ++q) {
-        const int b = t + q * kFftThreads;
-        if (b >= B / 2) continue;
-        const int i = (b / lenh) * len, j = b % lenh;
-        const cplx u = buf[i + j], x = cmul(buf[i + j + lenh], w[q]);
-        buf[i + j] = cplx{u.re + x.re, u.im + x.im};
-        buf[i + j + lenh] = cplx{u.re - x.re, u.im - x.im};
+      for (int k = 0; k < 4; ++k) {
+        const int i = fft_pad(fft_at(from, t, k));
+        re[i] = x[k].re;
+        im[i] = x[k].im;
       }
-      if (len < B) {
+    }
+    __syncthreads();
+    if (on) {
 #pragma unroll
-        for (int q = 0; q < kFftPer; ++q) {
-          const int b = t + q * kFftThreads;
-          if (b < B / 2) w[q] = root(len << 1, b);
+      for (int k = 0; k < 4; ++k) {
+        const int i = fft_pad(fft_at(to, t, k));
+        x[k] = cplx{re[i], im[i]};
+      }
+    }
+  };
+  const bool odd = logB & 1;
+  if (!INV) {
+    if (on) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int i = 4 * t + k;
+        if (i < B) {
+          const int s = rev ? brev(base + i, logn) : base + i;
+          x[k] = d.in ? dec_value(P, d, s) : src[s];
         }
       }
-      __syncthreads();
+    }
+    int lo = 0;
+    if (odd) {
+      const cplx w1 = T[1];
+      if (on && logB > 1) twiddles(1, t & 1);
+      bfly_fwd(x[0], x[1], w1);
+      if (logB > 1) {
+        bfly_fwd(x[2], x[3], w1);
+        exchange(0, 1);
+        lo = 1;
+      }
+    } else if (on && logB > 0) {
+      twiddles(0, 0);
+    }
+    while (logB > 1) {
+      const cplx w0 = w[0], w1 = w[1], w2 = w[2];
+      const bool last = lo + 2 >= logB;
+      if (on && !last) twiddles(lo + 2, t & ((4 << lo) - 1));
+      bfly_fwd(x[0], x[1], w0);
+      bfly_fwd(x[2], x[3], w0);
+      bfly_fwd(x[0], x[2], w1);
+      bfly_fwd(x[1], x[3], w2);
+      if (last) break;
+      exchange(lo, lo + 2);
+      lo += 2;
+    }
+    if (on) {
+      if (logB < 2) lo = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int i = fft_at(lo, t, k);
+        if (i < B) dst[base + i] = x[k];
+      }
     }
   } else {
-    for (int len = B; len >= 2; len >>= 1) {
-      const int lenh = len >> 1;
+    int lo = logB > 2 ? logB - 2 : 0;
+    if (on) {
 #pragma unroll
-      for (int q = 0; q < kFftPer; ++q) {
-        const int b = t + q * kFftThreads;
-        if (b >= B / 2) continue;
-        const int i = (b / lenh) * len, j = b % lenh;
-        const cplx x = buf[i + j], y = buf[i + j + lenh];
-        buf[i + j] = cplx{x.re + y.re, x.im + y.im};
-        buf[i + j + lenh] = cmul(cplx{x.re - y.re, x.im - y.im}, w[q]);
+      for (int k = 0; k < 4; ++k) {
+        const int i = fft_at(lo, t, k);
+        if (i < B) x[k] = src[base + i];
       }
-      if (len > 2) {
+      if (logB > 1) twiddles(lo, t & ((1 << lo) - 1));
+    }
+    while (logB > 1) {
+      const cplx w0 = w[0], w1 = w[1], w2 = w[2];
+      if (on && lo >= 2) twiddles(lo - 2, t & ((1 << (lo - 2)) - 1));
+      bfly_inv(x[0], x[2], w1);
+      bfly_inv(x[1], x[3], w2);
+      bfly_inv(x[0], x[1], w0);
+      bfly_inv(x[2], x[3], w0);
+      if (lo < 2) break;
+      exchange(lo, lo - 2);
+      lo -= 2;
+    }
+    if (odd) {
+      const cplx w1 = T[1];
+      if (logB > 1) {
+        exchange(1, 0);
+        bfly_inv(x[2], x[3], w1);
+      }
+      bfly_inv(x[0], x[1], w1);
+    }
+    if (on) {
+      const double f = rev ? 1.0 / (double)(1 << logn) : 1.0;
 #pragma unroll
-        for (int q = 0; q < kFftPer; ++q) {
-          const int b = t + q * kFftThreads;
-          if (b < B / 2) w[q] = root(len >> 1, b);
+      for (int k = 0; k < 4; ++k) {
+        const int i = 4 * t + k;
+        if (i < B) {
+          if (rev)
+            dst[brev(base + i, logn)] = cplx{x[k].re * f, x[k].im * f};
+          else
+            dst[base + i] = x[k];
         }
       }
-      __syncthreads();
     }
-  }
-  if (whole && inverse) {
-    const double dn = (double)B;
-    for (int i = t; i < B; i += kFftThreads)
-      blk[logB ? (__brev((unsigned)i) >> (32 - logB)) : 0] = cplx{buf[i].re / dn, buf[i].im / dn};
-  } else {
-    for (int i = t; i < B; i += kFftThreads) blk[i] = buf[i];
   }
 }
 
-// The stages of length <= 4096 run in LDS (one launch); a vector longer than
-// 4096 adds one launch per remaining stage and a separate bit reversal.
+// The last (forward) or first (inverse) three stages of n = 8 B values, eight
+// values a thread in registers: a launch for three.  Encoding 2^14 values (with
+// the residues): 15 us in three launches, 38 us in five before; decoding them 14
+// for 40.
+template <bool INV>
+__global__ __launch_bounds__(64) void k_enc_outer(DevParams P, const cplx* src, cplx* dst, int B) {
+  const int j = blockIdx.x * 64 + threadIdx.x;
+  const cplx* T = reinterpret_cast<const cplx*>(P.enc_t[INV]) + j;
+  cplx x[8], w[7];
+#pragma unroll
+  for (int m = 0; m < 8; ++m) x[m] = src[j + (size_t)m * B];
+#pragma unroll
+  for (int m = 0; m < 7; ++m) w[m] = T[(size_t)(m + 1) * B];
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    const int h = INV ? 4 >> s : 1 << s;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      if (m & h) continue;
+      const cplx tw = w[h - 1 + (m & (h - 1))];
+      if (INV)
+        bfly_inv(x[m], x[m + h], tw);
+      else
+        bfly_fwd(x[m], x[m + h], tw);
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < 8; ++m) dst[j + (size_t)m * B] = x[m];
+}
+
+template <bool INV>
+static void fft_blocks(const DevParams& P, const cplx* src, cplx* dst, int n, int rev, const DecodeIn& d, hipStream_t st) {
+  const int B = n <= kFftBlock ? n : n / 8;
+  const int threads = B / 4 < 64 ? 64 : B / 4;
+  k_enc_fft<INV><<<(unsigned)(n / B), threads, (size_t)(B + B / 4) * 16, st>>>(P, src, dst, ilog2(B), ilog2(n), rev, d);
+}
+template <bool INV>
+static void fft_outer(const DevParams& P, const cplx* src, cplx* dst, int n, hipStream_t st) {
+  k_enc_outer<INV><<<(unsigned)(n / 8 / 64), 64, 0, st>>>(P, src, dst, n / 8);
+}
+
+// A vector of at most 4096 values takes one launch; a longer one the blocks,
+// the outer stages and, in place, a bit reversal.
 void launch_special_fft(const DevParams& P, double* vals, int n, int inverse, hipStream_t st) {
   cplx* v = reinterpret_cast<cplx*>(vals);
-  const int logn = ilog2(n);
-  const int B = n < kFftBlock ? n : kFftBlock;
-  const int logB = ilog2(B);
-  const size_t lds = (size_t)B * sizeof(cplx) + (size_t)(B / 2) * sizeof(uint32_t);
-  const unsigned nblk = (unsigned)(n / B);
-  const int whole = n == B;
+  const DecodeIn none{nullptr, 1, 1.0};
+  const bool whole = n <= kFftBlock;
   if (!inverse) {
-    if (!whole) k_enc_bitrev<<<blocks(n), 256, 0, st>>>(v, n, logn, 0);
-    k_enc_fft_block<<<nblk, kFftThreads, lds, st>>>(P, v, B, logB, 0, whole);
-    for (int len = 2 * B; len <= n; len <<= 1) k_enc_stage_fwd<<<blocks(n / 2), 256, 0, st>>>(P, v, n, len);
+    if (!whole) k_enc_bitrev<<<blocks(n), 256, 0, st>>>(v, n, ilog2(n), 0);
+    fft_blocks<false>(P, v, v, n, whole, none, st);
+    if (!whole) fft_outer<false>(P, v, v, n, st);
   } else {
-    for (int len = n; len > B; len >>= 1) k_enc_stage_inv<<<blocks(n / 2), 256, 0, st>>>(P, v, n, len);
-    k_enc_fft_block<<<nblk, kFftThreads, lds, st>>>(P, v, B, logB, 1, whole);
-    if (!whole) k_enc_bitrev<<<blocks(n), 256, 0, st>>>(v, n, logn, 1);
+    if (!whole) fft_outer<true>(P, v, v, n, st);
+    fft_blocks<true>(P, v, v, n, whole, none, st);
+    if (!whole) k_enc_bitrev<<<blocks(n), 256, 0, st>>>(v, n, ilog2(n), 1);
   }
 }
 
-void launch_encode_pack(const DevParams& P, uint64_t* out, const double* vals, int slots, double scale, int k,
-                        hipStream_t st) {
-  k_enc_pack<<<blocks((size_t)k * P.N), 256, 0, st>>>(P, out, reinterpret_cast<const cplx*>(vals), slots, scale,
-                                                       k);
+// The inverse FFT in place and the residues of its values.  A long vector goes
+// through the first limb of the output (at most N/2 values: N words) between
+// its two launches, so that the second one's bit reversal meets no other block.
+void launch_encode(const DevParams& P, uint64_t* out, double* vals, int slots, double scale, int k, hipStream_t st) {
+  cplx* v = reinterpret_cast<cplx*>(vals);
+  cplx* src = v;
+  if (slots > kFftBlock) {
+    src = reinterpret_cast<cplx*>(out);
+    fft_outer<true>(P, v, src, slots, st);
+  }
+  fft_blocks<true>(P, src, v, slots, 1, DecodeIn{nullptr, 1, 1.0}, st);
+  k_enc_pack<<<blocks((size_t)k * P.N), 256, 0, st>>>(P, out, v, slots, scale, k);
 }
 
-void launch_decode_unpack(const DevParams& P, double* vals, const uint64_t* in, int slots, double scale,
-                          hipStream_t st) {
-  k_dec_unpack<<<blocks(slots), 256, 0, st>>>(P, reinterpret_cast<cplx*>(vals), in, slots, scale);
+// The blocks read their values from limb 0 in bit-reversed order.
+void launch_decode(const DevParams& P, double* vals, const uint64_t* in, int slots, double scale, hipStream_t st) {
+  cplx* v = reinterpret_cast<cplx*>(vals);
+  fft_blocks<false>(P, nullptr, v, slots, 1, DecodeIn{in, slots, scale}, st);
+  if (slots > kFftBlock) fft_outer<false>(P, v, v, slots, st);
 }
 
 }  // namespace aoa

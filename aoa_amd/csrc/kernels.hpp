@@ -78,10 +78,6 @@ void launch_eltwise_scalar(const DevParams& P, int op, uint64_t* out, const uint
                            int prime0, hipStream_t st);
 void launch_conjugate(const DevParams& P, uint64_t* out, const uint64_t* in, int nlimbs, hipStream_t st);
 
-// CKKS encoder (FP64).  vals holds n complex values (re, im interleaved);
-// the special FFT runs in place (inverse: encoding direction, with the
-// division by n).  encode_pack writes k limbs of N residues from slots values;
-// decode_unpack reads limb 0 (coefficient domain) into slots values.
 // Sampler: limbs res0..res0+nres-1 of out (poly base pointer, limb r at
 // out + r*N) from distribution `kind`, keyed by (seed, nonce).
 void launch_sample(const DevParams& P, uint64_t* out, int res0, int nres, int kind, uint64_t seed, uint64_t nonce,
@@ -91,11 +87,13 @@ void launch_sample(const DevParams& P, uint64_t* out, int res0, int nres, int ki
 void launch_sample_encrypt(const DevParams& P, uint64_t* u, uint64_t* e0, uint64_t* e1, const uint64_t* m, int nres,
                            uint64_t seed, uint64_t nonce, hipStream_t st);
 
+// CKKS encoder (FP64).  vals holds n complex values (re, im interleaved); the
+// special FFT runs in place (inverse: encoding direction, with the division by
+// n).  encode: the inverse FFT of vals in place and k limbs of N residues of its
+// values; decode: the FFT of limb 0's (coefficient domain) slot values.
 void launch_special_fft(const DevParams& P, double* vals, int n, int inverse, hipStream_t st);
-void launch_encode_pack(const DevParams& P, uint64_t* out, const double* vals, int slots, double scale, int k,
-                        hipStream_t st);
-void launch_decode_unpack(const DevParams& P, double* vals, const uint64_t* in, int slots, double scale,
-                          hipStream_t st);
+void launch_encode(const DevParams& P, uint64_t* out, double* vals, int slots, double scale, int k, hipStream_t st);
+void launch_decode(const DevParams& P, double* vals, const uint64_t* in, int slots, double scale, hipStream_t st);
 void launch_modup(const DevParams& P, const uint64_t* x, uint64_t* outB, int level, hipStream_t st);
 
 // ModDown of npolys polys.  inQ[y] holds Q limbs 0..level, inB[y] the K

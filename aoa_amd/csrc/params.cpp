@@ -455,6 +455,15 @@ std::string build_host_params(int N, int k, int kl, int prec, HostParams* out) {
       P.rot_group[j] = (uint32_t)g;
       g = g * 5 % M;
     }
+    for (int dir = 0; dir < 2; ++dir) {
+      P.enc_t[dir].assign(N, 0.0);
+      for (size_t h = 1; h < (size_t)N / 2; h *= 2)
+        for (size_t j = 0; j < h; ++j) {
+          const size_t r = P.rot_group[j] % (8 * h), t = (dir ? 8 * h - r : r) * (M / (8 * h));
+          P.enc_t[dir][2 * (h + j)] = P.enc_w[2 * t];
+          P.enc_t[dir][2 * (h + j) + 1] = P.enc_w[2 * t + 1];
+        }
+    }
   }
   return "";
 }

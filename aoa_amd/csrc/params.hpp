@@ -124,8 +124,9 @@ struct DevParams {
   const uint64_t* inv_b_mod_q;   // [k][2]: B^-1 mod q_i, Shoup
   const uint64_t* b_mod_q;       // [k][2]: B mod q_i, Shoup
   const uint64_t* inv_ql_mod_qi; // [k][k][2]: (l,i) -> q_l^-1 mod q_i, Shoup
-  const double* enc_w;           // [2N][2]: exp(2 pi i t / 2N), the encoder's roots of unity
-  const uint32_t* rot_group;     // [N/2]: 5^j mod 2N
+  // the encoder's twiddles, [0: forward, 1: inverse][N/2][2]: entry h + j (j < h)
+  // is exp(+-2 pi i (5^j mod 8 h) / (8 h))
+  const double* enc_t[2];
   const uint64_t* gauss_cdt;     // [2 kGaussHalf]: round(2^64 P(e <= j - kGaussHalf)), e = round(3.2 z)
   const uint32_t* md_terms;      // [K][k][6]: ModDown product constants (MdTerm), Q primes below 2^56
   const uint32_t* md_thr;        // [k]: ModDown screen threshold of q_i
@@ -170,6 +171,7 @@ struct HostParams {
   std::vector<uint64_t> bscale;     // K * 4
   std::vector<double> enc_w;        // 2N complex roots, interleaved (re, im)
   std::vector<uint32_t> rot_group;  // N/2 entries
+  std::vector<double> enc_t[2];     // DevParams::enc_t, taken from enc_w
   std::vector<uint64_t> gauss_cdt;  // 2 kGaussHalf entries
   std::vector<MdConst> md_const;    // k * K entries, [i][j]
   std::vector<MdTerm> md_terms;     // K * k entries, [j][i]

@@ -117,20 +117,22 @@ __device__ __forceinline__ void sample_small_at(const DevParams& P, uint64_t* ou
   } else {  // narrow
     v = (int64_t)__umul64hi(lo64(c), 3) - 1;
   }
-  if (!add) {
-    for (int l = res0; l < res0 + nres; ++l) out[(size_t)l * P.N + i] = small_residue(v, ld_prime_p(P.primes, l));
-    return;
-  }
-  // eight limbs' addends requested together: a store may alias the next load
+  // eight limbs' primes and addends requested together: a store may alias the
+  // next load
   for (int l0 = res0; l0 < res0 + nres; l0 += 8) {
-    uint64_t m[8];
+    uint64_t p[8], m[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) m[j] = l0 + j < res0 + nres ? add[(size_t)(l0 + j) * P.N + i] : 0;
+    for (int j = 0; j < 8; ++j) {
+      const int l = min(l0 + j, res0 + nres - 1);
+      p[j] = ld_prime_p(P.primes, l);
+      if (add) m[j] = add[(size_t)l * P.N + i];
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       if (l0 + j < res0 + nres) {
-        const uint64_t p = ld_prime_p(P.primes, l0 + j);
-        out[(size_t)(l0 + j) * P.N + i] = add_mod(small_residue(v, p), m[j], p);
+        uint64_t r = small_residue(v, p[j]);
+        if (add) r = add_mod(r, m[j], p[j]);
+        out[(size_t)(l0 + j) * P.N + i] = r;
       }
     }
   }

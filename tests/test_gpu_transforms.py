@@ -62,3 +62,35 @@ def test_encrypt_decrypt_match_splits(gpu, shape, alias):
         got.append(enc + d + [t])
     for name, a, b in zip(("c0", "c1", "m", "d0", "d1", "plain"), *got):
         assert (a == b).all(), name
+
+
+@pytest.mark.parametrize("logn", range(16))
+def test_encoder_sizes_bitexact(gpu, logn):
+    """Both directions of the special FFT, encode and decode at every slot
+    count of N = 2^16: equal to the oracle's bit for bit."""
+    import ctypes
+    import torch
+    import orc
+    from aoa_amd import FORWARD, INVERSE, Params
+    N, n, scale = 65536, 1 << logn, 1 << 48
+    P, O = Params(N, 2, 0, 48), orc.Oracle(N, 2, 0, 48)
+    rng = np.random.default_rng(logn)
+    z = rng.uniform(-1, 1, n) + 1j * rng.uniform(-1, 1, n)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.complex128).view(np.float64).copy()).cuda()
+    bits = lambda a: np.ascontiguousarray(a).view(np.uint64)
+    print("encoder n=%d" % n, flush=True)
+    for dirn in (FORWARD, INVERSE):
+        t, ref = dev(z), np.ascontiguousarray(z).view(np.float64).copy()
+        P.special_fft(t, n, dirn)
+        orc.load().orc_fft_special(ref.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), n, N, int(dirn == INVERSE))
+        assert np.array_equal(bits(t.cpu().numpy()), bits(ref)), dirn
+    out, vals = P.zeros(2), dev(z)
+    P.encode(out, vals, n, scale)
+    assert np.array_equal(bits(vals.cpu().numpy()), bits(ref))  # left in place
+    want = O.encode(z, scale).reshape(2, N)
+    got = P.to_host(out).reshape(2, N)
+    for r in range(2):
+        assert np.array_equal(got[r], want[r] % np.uint64(O.primes[r])), r
+    back = dev(np.zeros(n))
+    P.decode(back, out, n, scale)
+    assert np.array_equal(bits(back.cpu().numpy()), bits(O.decode(want[0], n, scale)))
