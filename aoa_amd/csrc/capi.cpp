@@ -603,8 +603,7 @@ extern "C" int aoa_rotate_left(const aoa_params* h, void* stream, uint64_t* out0
   uint64_t* kws = R1 + (size_t)L * N;  // 3(L+K) limbs
   (void)K;
   const uint64_t g = galois_of(rot_slots, P.N);
-  launch_automorphism(P, R0, c0, L, g, st);
-  launch_automorphism(P, R1, c1, L, g, st);
+  launch_automorphism2(P, R0, R1, c0, c1, L, g, st);
   int rc = keyswitch_core(h, st, out0, out1, R0, R1, rtk_b, rtk_a, level, kws);
   if (rc) return rc;
   return check_launch("aoa_rotate_left");

@@ -81,6 +81,11 @@ __device__ __forceinline__ void key_body_tensor(const DevParams& P, const FzItem
   }
 }
 
+// Two words of a key, which need no more than a word's alignment.
+struct KeyPair {
+  uint64_t a, b;
+};
+
 template <class F, int LOGM>
 __device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, int m, int pr, int tile, int y0, int y1,
                                          uint64_t* lds) {
@@ -105,9 +110,9 @@ __device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, i
     typename F::V x[G::V];
 #pragma unroll
     for (int k = 0; k < G::V; k += 2) {
-      const tw2 v = at_byte<tw2>(kp, id.poff + 8 * k);
-      x[k] = f.key(x0[k], v.w);
-      x[k + 1] = f.key(x0[k + 1], v.q);
+      const KeyPair v = at_byte<KeyPair>(kp, id.poff + 8 * k);
+      x[k] = f.key(x0[k], v.a);
+      x[k + 1] = f.key(x0[k + 1], v.b);
     }
     if (y > y0) __syncthreads();  // the first half's last exchange has been read
     rows_out<F, LOGM>(f, x, T + z, glob(y ? it.P1 : it.P0) + (size_t)m * N, id);

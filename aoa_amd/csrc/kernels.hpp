@@ -119,6 +119,9 @@ void launch_checksum(const uint64_t* x, size_t n, uint64_t off, uint64_t* acc, h
 // Galois automorphism X -> X^g (g odd) in the coefficient domain, gather form.
 void launch_automorphism(const DevParams& P, uint64_t* out, const uint64_t* in, int nlimbs,
                          uint64_t galois, hipStream_t st);
+// Both polynomials of a rotation in one launch.
+void launch_automorphism2(const DevParams& P, uint64_t* out0, uint64_t* out1, const uint64_t* in0, const uint64_t* in1,
+                          int nlimbs, uint64_t galois, hipStream_t st);
 uint64_t galois_inverse(uint64_t galois, int N);
 
 // rho of a QB polynomial: Q limbs times (B mod q_i), special limbs zero.

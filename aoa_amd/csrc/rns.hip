@@ -810,18 +810,18 @@ void launch_dr2(const DevParams& P, uint64_t* c21, uint64_t* c22, uint64_t* c23,
 // to stay in L2 while its workgroups run.  Workgroups take their block of the
 // output through xcd_chunk_id, so the blocks of one limb run on one XCD (one
 // L2) one after another instead of on all eight.
-__global__ __launch_bounds__(256) void k_automorphism(DevParams P, uint64_t* out, const uint64_t* in,
-                                                      uint64_t ginv) {
+// blockIdx.y: the polynomial (a rotation's two in one launch).
+__global__ __launch_bounds__(256) void k_automorphism(DevParams P, uint64_t* out0, uint64_t* out1, const uint64_t* in0,
+                                                      const uint64_t* in1, uint64_t ginv) {
   const size_t N = (size_t)P.N;
   const size_t blk = (size_t)xcd_chunk_id(blockIdx.x, gridDim.x);
   const size_t e = blk * 256 + threadIdx.x;
   const int li = (int)((blk * 256) >> P.logN);
   const uint64_t j = e & (N - 1);
-  const uint64_t p = P.primes[li].p;
   const uint64_t t = (j * ginv) & (2 * N - 1);
-  const uint64_t* src = in + (size_t)li * N;
-  uint64_t v = t < N ? src[t] : neg_mod(src[t - N], p);
-  out[e] = v;
+  const uint64_t* src = (blockIdx.y ? in1 : in0) + (size_t)li * N;
+  const uint64_t v = src[t & (N - 1)], p = ld_prime_p(P.primes, li);
+  (blockIdx.y ? out1 : out0)[e] = t < N ? v : neg_mod(v, p);
 }
 
 uint64_t galois_inverse(uint64_t galois, int N) {
@@ -839,7 +839,12 @@ uint64_t galois_inverse(uint64_t galois, int N) {
 void launch_automorphism(const DevParams& P, uint64_t* out, const uint64_t* in, int nlimbs,
                          uint64_t galois, hipStream_t st) {
   const size_t total = (size_t)nlimbs * P.N;
-  k_automorphism<<<dim3((unsigned)(total / 256)), 256, 0, st>>>(P, out, in, galois_inverse(galois, P.N));
+  k_automorphism<<<dim3((unsigned)(total / 256)), 256, 0, st>>>(P, out, out, in, in, galois_inverse(galois, P.N));
+}
+void launch_automorphism2(const DevParams& P, uint64_t* out0, uint64_t* out1, const uint64_t* in0, const uint64_t* in1,
+                          int nlimbs, uint64_t galois, hipStream_t st) {
+  const size_t total = (size_t)nlimbs * P.N;
+  k_automorphism<<<dim3((unsigned)(total / 256), 2), 256, 0, st>>>(P, out0, out1, in0, in1, galois_inverse(galois, P.N));
 }
 
 // Descriptor form, one entry per limb: out = sigma(in) (+ addsrc when set).
