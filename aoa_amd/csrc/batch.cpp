@@ -245,7 +245,7 @@ size_t batch_fill(aoa_batch* b, uint64_t* ws, char* host, char* dev, size_t desc
         return n;
       };
       g.field_q = (int)g.params->host.dprimes[k > 1 ? 1 : 0].field;
-      g.field_b = (int)g.params->host.dprimes[k].field;
+      g.field_b = g.params->host.K ? (int)g.params->host.dprimes[k].field : FIELD_LAZY;
       g.ns_rows = split_at(rows);
       g.ns_keyq = split_at(keyq);
       g.n_rows = (int)rows.size();

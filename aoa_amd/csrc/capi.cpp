@@ -85,9 +85,11 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
   // (device only: the host keeps the natural tables).
   std::vector<uint64_t> rowtw[3][2];
   int rowsec[3][2];
+  parallel_for(6, (size_t)(H.k + H.K) * H.N, [&](int t) {
+    row_twiddle_order(t & 1 ? H.tw_inv : H.tw_fwd, H.N, H.k + H.K, 64 << (t >> 1), &rowtw[t >> 1][t & 1]);
+  });
   for (int si = 0; si < 3; ++si)
     for (int dir = 0; dir < 2; ++dir) {
-      row_twiddle_order(dir ? H.tw_inv : H.tw_fwd, H.N, H.k + H.K, 64 << si, &rowtw[si][dir]);
       rowsec[si][dir] = rowtw[si][dir].empty() ? -1 : (int)secs.size();
       if (!rowtw[si][dir].empty()) secs.push_back({rowtw[si][dir].data(), rowtw[si][dir].size() * 8, 0});
     }

@@ -96,7 +96,7 @@ void build_fused_tables(const HostParams& h, FusedTables* out) {
     const std::vector<uint64_t>& tw = dir ? h.tw_inv : h.tw_fwd;
     std::vector<uint64_t>& o = out->tw[dir];
     o.assign((size_t)R * N * 2, 0);
-    for (int r = 0; r < R; ++r) {
+    parallel_for(R, (size_t)N, [&](int r) {
       const uint64_t p = h.primes[r];
       const uint64_t* src = &tw[(size_t)r * N * 2];
       uint64_t* dst = &o[(size_t)r * N * 2];
@@ -105,7 +105,7 @@ void build_fused_tables(const HostParams& h, FusedTables* out) {
       } else {
         std::memcpy(dst, src, (size_t)N * 16);
       }
-    }
+    });
   }
   out->lc.assign((size_t)R * 4, 0);
   out->lc_b.assign((size_t)K * 4, 0);
@@ -143,12 +143,12 @@ void build_fused_tables(const HostParams& h, FusedTables* out) {
   }
   // ModUp at level l: inputs v_i (i <= l), outputs j.
   const int jb_n = (K + 15) / 16;
-  const int Tb = conv_digits((int)h.dprimes[k].nb);  // special primes share their bit length
+  const int Tb = K ? conv_digits((int)h.dprimes[k].nb) : 0;  // special primes share their bit length
   out->mu_kb = (k + 7) / 8;
   out->mu_stride = (uint32_t)(jb_n * Tb * out->mu_kb * 1024);
   out->mu_w.assign((size_t)k * out->mu_stride, 0);
   out->mu_out.assign((size_t)k * K, ConvOut{});
-  for (int l = 0; l < k; ++l)
+  parallel_for(k, (size_t)k * K * 64, [&](int l) {
     for (int j = 0; j < K; ++j) {
       ConvRow row;
       row.p = h.primes[k + j];
@@ -159,6 +159,7 @@ void build_fused_tables(const HostParams& h, FusedTables* out) {
                  h.qhat_mod_b[((size_t)l * K + j) * k + i]);
       out->mu_out[(size_t)l * K + j] = row.finish();
     }
+  });
   // ModDown's result of limb i is f_i x_i - sum_j f_i c_ij a_j - q_l^-1 top (the
   // last with a rescale from level l, top in slot K); one table per l, and
   // index k without a rescale.
@@ -167,7 +168,7 @@ void build_fused_tables(const HostParams& h, FusedTables* out) {
   out->md_stride = (uint32_t)(ib_n * 8 * out->md_kb * 1024);
   out->md_w.assign((size_t)(k + 1) * out->md_stride, 0);
   out->md_out.assign((size_t)(k + 1) * k, ConvOut{});
-  for (int l = 0; l <= k; ++l)
+  parallel_for(k + 1, (size_t)k * K * 64, [&](int l) {
     for (int i = 0; i < k; ++i) {
       if (l < k && i >= l) continue;
       const uint64_t q = h.primes[i], f = down_factor(l, i);
@@ -182,6 +183,7 @@ void build_fused_tables(const HostParams& h, FusedTables* out) {
       if (l < k) row.slot(blk, i % 16, out->md_kb, T_blk, K, 7, q - h.inv_ql_mod_qi[((size_t)l * k + i) * 2]);
       out->md_out[(size_t)l * k + i] = row.finish();
     }
+  });
   // Screen of the ModDown products: frac(a c/q) = frac(al c/q + ah frac(2^28 c/q)), a = al + ah 2^28.
   out->scr.assign((size_t)K * 64 * 2, 0.0);
   out->scr_thr.assign(64, 0.0);

@@ -1,8 +1,14 @@
 // Host-side construction of a parameter set (primes, twiddles, RNS constants).
 #include "params.hpp"
 
+#include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
+#include <exception>
+#include <mutex>
+#include <system_error>
+#include <thread>
 
 namespace aoa {
 
@@ -137,6 +143,31 @@ uint32_t moddown_screen_thr(uint64_t thr, uint64_t p) {
   return t > 0xFFFFFFFFu ? 0xFFFFFFFFu : (uint32_t)t;
 }
 
+void parallel_for(int n, size_t cost, const std::function<void(int)>& f) {
+  std::atomic<int> next{0};
+  std::mutex m;
+  std::exception_ptr error;
+  auto work = [&] {
+    try {
+      for (int i; (i = next.fetch_add(1)) < n;) f(i);
+    } catch (...) {
+      std::lock_guard<std::mutex> lock(m);
+      error = std::current_exception();
+      next = n;
+    }
+  };
+  std::vector<std::thread> ts;
+  ts.reserve(8);
+  try {
+    const size_t want = std::min<size_t>({(size_t)n, 8, std::thread::hardware_concurrency(), n * cost / 65536 + 1});
+    for (size_t t = 1; t < want; ++t) ts.emplace_back(work);
+  } catch (const std::system_error&) {  // no more threads: the others do it
+  }
+  work();
+  for (std::thread& t : ts) t.join();
+  if (error) std::rethrow_exception(error);
+}
+
 void row_twiddle_order(const std::vector<uint64_t>& tw, int N, int R, int S, std::vector<uint64_t>* out) {
   out->clear();
   const int N1 = S > 0 ? N / S : 0;
@@ -210,30 +241,25 @@ std::string build_host_params(int N, int k, int kl, int prec, HostParams* out) {
   // Twiddles: psi = g^((p-1)/2N); forward table psi^brev(i), inverse psi^-brev(i).
   P.tw_fwd.assign((size_t)R * N * 2, 0);
   P.tw_inv.assign((size_t)R * N * 2, 0);
-  std::vector<uint64_t> pw(N), ipw(N);
-  for (int r = 0; r < R; ++r) {
-    uint64_t p = P.primes[r];
-    uint64_t psi = powm(P.roots[r], (p - 1) / (2 * (uint64_t)N), p);
-    uint64_t ipsi = inv_mod(psi, p);
-    pw[0] = 1;
-    ipw[0] = 1;
-    for (int i = 1; i < N; ++i) {
-      pw[i] = mulm(pw[i - 1], psi, p);
-      ipw[i] = mulm(ipw[i - 1], ipsi, p);
-    }
+  parallel_for(R, 2 * (size_t)N, [&](int r) {
+    const uint64_t p = P.primes[r];
+    const uint64_t psi = powm(P.roots[r], (p - 1) / (2 * (uint64_t)N), p), ipsi = inv_mod(psi, p);
     uint64_t* tf = &P.tw_fwd[(size_t)r * N * 2];
     uint64_t* ti = &P.tw_inv[(size_t)r * N * 2];
-    for (int i = 0; i < N; ++i) {
-      uint32_t e = bit_reverse((uint32_t)i, P.logN);
-      tf[2 * i] = pw[e];
-      tf[2 * i + 1] = shoup_quot(pw[e], p);
-      ti[2 * i] = ipw[e];
-      ti[2 * i + 1] = shoup_quot(ipw[e], p);
+    uint64_t pw = 1, ipw = 1;
+    for (int e = 0; e < N; ++e) {
+      const uint32_t i = bit_reverse((uint32_t)e, P.logN);
+      tf[2 * i] = pw;
+      tf[2 * i + 1] = shoup_quot(pw, p);
+      ti[2 * i] = ipw;
+      ti[2 * i + 1] = shoup_quot(ipw, p);
+      pw = mulm(pw, psi, p);
+      ipw = mulm(ipw, ipsi, p);
     }
     DevPrime& d = P.dprimes[r];
     d.w1ninv = mulm(ti[2], d.ninv, p);
     d.w1ninv_q = shoup_quot(d.w1ninv, p);
-  }
+  });
 
   // RNS constants (aoa-ntt/src/cuda/manager.cu:566-759), as residues of
   // products of primes; no big integers are needed.
@@ -242,7 +268,7 @@ std::string build_host_params(int N, int k, int kl, int prec, HostParams* out) {
   P.inv_qhat.assign((size_t)k * k * 2, 0);
   P.qhat_mod_b.assign((size_t)k * kl * k, 0);
   P.inv_ql_mod_qi.assign((size_t)k * k * 2, 0);
-  for (int l = 0; l < k; ++l) {
+  parallel_for(k, (size_t)k * kl, [&](int l) {
     for (int i = 0; i <= l; ++i) {
       // (Q_l / q_i) mod q_i, Q_l = q_0 ... q_l
       uint64_t qi = Qp[i];
@@ -266,7 +292,7 @@ std::string build_host_params(int N, int k, int kl, int prec, HostParams* out) {
       P.inv_ql_mod_qi[((size_t)l * k + i) * 2] = v;
       P.inv_ql_mod_qi[((size_t)l * k + i) * 2 + 1] = shoup_quot(v, Qp[i]);
     }
-  }
+  });
   // ModUp's constants (Q_l/q_i) mod b_j split at bit 28, in the order the
   // kernel reads them: one block of kp = K rounded up to 16 entries per (l, i),
   // special limb j = g + 4t (g = j % 4) at position (t / 4) 16 + 4 g + t % 4,

@@ -54,3 +54,52 @@ def test_fused_parity(gpu, shape, exact):
         n = level * N
         for y in range(2):
             assert np.array_equal(P.to_host(out[y])[:n], ref[y][:n]), "product c%d level %d" % (y, level)
+
+
+def _ref_barrett(x, p):
+    """The reference's reduction of x < 2^128 (aoa-ntt/src/cuda/htrans/common.cu:257-291)."""
+    nb = p.bit_length()
+    mu = (1 << 2 * nb) // p
+    A = x - ((x >> (2 * nb - 64)) * mu >> 64) * p
+    r = ((A & ((1 << nb) - 1)) - (A >> nb) * p) & ((1 << nb) - 1)
+    return r - p if r >= p else r
+
+
+def test_many_deviating_products(gpu):
+    """Every coefficient of every special limb in the deviation window of one
+    limb's product, so that a workgroup finds more of them than its list holds:
+    the key's special limbs are made for it from the ModUp of the polynomial 1."""
+    from aoa_amd import FORWARD, Params
+    N, k, kl, prec = 2048, 4, 5, 48
+    P, O = Params(N, k, kl, prec), Oracle(N, k, kl, prec)
+    q, b = [int(p) for p in P.primes[:k]], [int(p) for p in P.primes[k:]]
+    B, Q = 1, 1
+    for x in b:
+        B *= x
+    for x in q:
+        Q *= x
+    rng = np.random.default_rng(5)
+    key = [O.random_poly(rng, k + kl) for _ in range(2)]
+    special = np.zeros((k + kl, N), dtype=np.uint64)
+    for j in range(kl):
+        i = 1 + j % (k - 1)
+        c = (B // b[j]) % q[i]
+        inv, eps = pow(c, -1, q[i]), (1 << q[i].bit_length()) - q[i]
+        tries = ((eps + r) * inv % q[i] + n * q[i] for r in range(20000) for n in range(b[j] // q[i]))
+        a = next(x for x in tries if _ref_barrett(x * c, q[i]) != x * c % q[i])
+        v = sum(pow(Q // x, -1, x) * (Q // x) for x in q) % b[j]
+        special[k + j, :] = a * (B // b[j]) * pow(v, -1, b[j]) % b[j]
+    d = P.to_device(special.reshape(-1))
+    P.ntt(d, 0, k + kl, FORWARD)
+    key[0].reshape(k + kl, N)[k:] = P.to_host(d).reshape(k + kl, N)[k:]
+    one = np.zeros((k, N), dtype=np.uint64)
+    one[:, 0] = 1
+    c1 = [O.random_poly(rng, k), one.reshape(-1)]
+    ref = O.rotate_left(c1, key, 0, k - 1)
+    O.set_moddown_exact(True)
+    plain = O.rotate_left(c1, key, 0, k - 1)
+    assert (ref[0] != plain[0]).sum() > 2 * N  # three limbs deviate
+    out, dk = [P.zeros(k), P.zeros(k)], [P.to_device(x) for x in key]
+    P.rotate_left(out, [P.to_device(x) for x in c1], dk, 0, k - 1, P.workspace(k - 1))
+    for y in range(2):
+        assert np.array_equal(P.to_host(out[y]), ref[y]), y
