@@ -146,7 +146,7 @@ size_t batch_fill(aoa_batch* b, uint64_t* ws, char* host, char* dev, size_t desc
         for (int y = 0; y < 2; ++y)
           for (int i = 0; i <= it.level; ++i) {
             uint64_t* l = it.poly[y] + (size_t)i * N;
-            (it.dir == AOA_FORWARD ? prefwd : preinv).push_back({l, l, nullptr, i, 0});
+            (it.dir == AOA_FORWARD ? prefwd : preinv).push_back({l, l, i, 0});
           }
       auto key_entries = [&](uint32_t item, int Lq) {
         for (int m = 0; m < Lq; ++m) keyq.push_back(item << 8 | m);
@@ -592,8 +592,8 @@ extern "C" int aoa_batch_autotune(aoa_batch* b, void* stream, int reps, aoa_tune
   int rc = aoa_batch_build(b);
   if (rc) return -rc;
   hipStream_t st = (hipStream_t)stream;
-  // NTT splits valid for every ring of the batch (0: each handle's own)
-  std::vector<int> splits;
+  // the handles' own transforms (0) and the splits valid for every ring of the batch
+  std::vector<int> splits{0};
   for (int n1 : {64, 128, 256, 2048, 4096}) {
     bool ok = true, any = false;
     for (auto& L : b->layers)
@@ -603,7 +603,6 @@ extern "C" int aoa_batch_autotune(aoa_batch* b, void* stream, int reps, aoa_tune
       }
     if (ok && any) splits.push_back(n1);
   }
-  if (splits.size() < 2) splits.assign(1, 0);
   std::vector<aoa_batch_options> cand;
   for (int n1 : splits)
     for (int xcd = 0; xcd < 2; ++xcd) {

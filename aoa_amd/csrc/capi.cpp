@@ -79,7 +79,6 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
       {H.md_fin.data(), H.md_fin.size() * 8, 0},
       {H.md_negb.data(), H.md_negb.size() * 4, 0},
       {H.mu_terms.data(), H.mu_terms.size() * 4, 0},
-      {H.bscale.data(), H.bscale.size() * 8, 0},
   };
   // Row-pass twiddle orders, one per two-pass split of N and direction
   // (device only: the host keeps the natural tables).
@@ -152,7 +151,6 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
   D.md_fin = (const uint64_t*)(b + secs[16].off);
   D.md_negb = (const uint32_t*)(b + secs[17].off);
   D.mu_terms = (const uint32_t*)(b + secs[18].off);
-  D.bscale = (const uint64_t*)(b + secs[19].off);
   for (int si = 0; si < 3; ++si)
     for (int dir = 0; dir < 2; ++dir)
       D.tw_row[si][dir] = rowsec[si][dir] < 0 ? nullptr : (const uint64_t*)(b + secs[rowsec[si][dir]].off);
@@ -266,7 +264,7 @@ extern "C" int aoa_ntt(const aoa_params* h, void* stream, uint64_t* d, int res0,
   if (res0 < 0 || nres <= 0 || res0 + nres > R) return fail(AOA_ERR_ARG, "limb range out of bounds");
   LimbMap m = limbs_of(d + (size_t)res0 * h->host.N, res0, nres, h->host.k);
   hipStream_t st = (hipStream_t)stream;
-  int rc = dir == AOA_FORWARD ? ntt_forward(h->dev, m, 0, st) : ntt_inverse(h->dev, m, 0, nullptr, nullptr, st);
+  int rc = dir == AOA_FORWARD ? ntt_forward(h->dev, m, 0, st) : ntt_inverse(h->dev, m, 0, st);
   if (rc) return fail(AOA_ERR_UNSUPPORTED, "no NTT split for this N");
   return check_launch("aoa_ntt");
 }
@@ -410,7 +408,7 @@ extern "C" int aoa_decrypt(const aoa_params* h, void* stream, uint64_t* m, uint6
   if (ntt_forward(P, mc, 0, st)) return fail(AOA_ERR_UNSUPPORTED, "no NTT split for this N");
   launch_eltwise(P, ELT_MULADD, m, c1, s, c0, L, L, 0, st);
   LimbMap mo = limbs_of(m, 0, L, h->host.k);
-  if (ntt_inverse(P, mo, 0, nullptr, nullptr, st)) return fail(AOA_ERR_UNSUPPORTED, "no NTT split for this N");
+  if (ntt_inverse(P, mo, 0, st)) return fail(AOA_ERR_UNSUPPORTED, "no NTT split for this N");
   return check_launch("aoa_decrypt");
 }
 
@@ -480,7 +478,6 @@ extern "C" int aoa_moddown(const aoa_params* h, void* stream, uint64_t* d_q_out,
   a.out[0] = d_q_out;
   a.npolys = 1;
   a.level = level;
-  a.rescale = 0;
   launch_moddown(h->dev, a, (hipStream_t)stream);
   return check_launch("aoa_moddown");
 }

@@ -84,60 +84,12 @@ __device__ __forceinline__ int limb_prime(const LimbMap& m, int k, int li) {
 }
 
 // Descriptor tables of the batched (stage-fused) launches: one entry per
-// limb (NTT, tensor) or per polynomial (ModUp, ModDown).
+// limb.
 struct NttDesc {
   const uint64_t* src;  // first-pass input limb (== dst for in place)
   uint64_t* dst;        // output limb
-  const uint64_t* key;  // inverse only: key limb to multiply by first (or null)
   int prime;
   int pad;
-};
-
-// Key switching's inverse first pass with both key halves: dst[y] = first
-// inverse pass of (src * key[y] + (B mod q) add[y]) for y = 0, 1 (the column
-// pass then runs on dst[0] and dst[1] as ordinary NttDesc entries).  add is
-// null, or (Q limbs of a two-pass transform only) NTT-domain limbs whose
-// ModDown-scaled sum joins the product: ModDown(X + B d) = ModDown(X) + d.
-// With ab[0] set (HomMul's Q limbs, two-pass transforms), ab = a0, a1, b0,
-// b1 (NTT domain, canonical) stand for src and add: the input is d2 = a1 b1
-// and add[y] is d0 = a0 b0 for y = 0, d1 = a0 b1 + a1 b0 for y = 1, computed
-// in the pass from the operands, so that the tensor product is never stored.
-struct KeyDesc2 {
-  const uint64_t* src;
-  uint64_t* dst[2];
-  const uint64_t* key[2];
-  const uint64_t* add[2];
-  const uint64_t* ab[4];
-  int prime;
-  int pad;
-};
-
-struct TensorDesc {
-  const uint64_t* a0;
-  const uint64_t* a1;
-  const uint64_t* b0;
-  const uint64_t* b1;
-  uint64_t* d0;
-  uint64_t* d1;
-  uint64_t* d2;
-  int prime;
-  int pad;
-};
-
-struct ModUpDesc {
-  const uint64_t* x;  // Q limbs 0..level, stride N
-  uint64_t* outB;     // K special limbs, stride N
-  int level;
-  int pad;
-};
-
-struct ModDownDesc {
-  const uint64_t* inQ;
-  const uint64_t* inB;
-  const uint64_t* add;
-  uint64_t* out;
-  int level;
-  int rescale;
 };
 
 struct AutoDesc {
@@ -149,7 +101,7 @@ struct AutoDesc {
   int pad;
 };
 
-// One HomMul (a0 set) or key switching of the fused kernels (fused.hip).
+// One HomMul (a0 set) or key switching of the fused kernels (fused.hpp).
 // Limb-major buffers, stride N; P0 and P1 hold level + 1 + K limbs.
 struct FzItem {
   const uint64_t *a0, *a1, *b0, *b1;  // HomMul's operands (NTT domain)

@@ -14,7 +14,7 @@ struct NtLimb {
 template <bool FIRST>
 __device__ __forceinline__ NtLimb nt_table(const NttDesc* d, int l) {
   const cptr<uint64_t> w = as_const(reinterpret_cast<const uint64_t*>(d + l));
-  return NtLimb{glob((const uint64_t*)w[FIRST ? 0 : 1]), glob((uint64_t*)w[1]), (int)(uint32_t)w[3]};
+  return NtLimb{glob((const uint64_t*)w[FIRST ? 0 : 1]), glob((uint64_t*)w[1]), (int)(uint32_t)w[2]};
 }
 #define NT_LIMB(FIRST, l_)                                                                                  \
   ARG ? NtLimb{(FIRST ? m.src[blockIdx.y] : m.base[blockIdx.y]) + (size_t)(l_) * P.N,                       \

@@ -15,16 +15,12 @@ constexpr int kHwMaxAttempts = 4096;
 
 int ntt_default_n1(int N);
 bool ntt_valid_split(int N, int N1);
-// Forward / inverse NTT of every limb in `m`.  N1 = 0 picks the default split.
-// With key0/key1 set, the inverse multiplies limb li of m.src[0] by limb
-// prime_of(li) of key y before transforming into m.base[y] (y = 0, 1); with
-// add0/add1 also set (two-pass splits only; -1 otherwise), (B mod q) times
-// limb li of add y joins the product of each Q limb (li < m.qlimbs).
+// Forward / inverse NTT of every limb in `m`.  N1 = 0: the set's split, or
+// without one nt_forward / nt_inverse.
 int ntt_forward(const DevParams& P, LimbMap m, int N1, hipStream_t st);
-int ntt_inverse(const DevParams& P, LimbMap m, int N1, const uint64_t* key0, const uint64_t* key1,
-                hipStream_t st, const uint64_t* add0 = nullptr, const uint64_t* add1 = nullptr);
+int ntt_inverse(const DevParams& P, LimbMap m, int N1, hipStream_t st);
 
-// Fused key switching (fused.hip).  fz_mul: HomMul + relinearisation (+ rescale)
+// Fused key switching (fused.hpp).  fz_mul: HomMul + relinearisation (+ rescale)
 // of one item; fz_switch: key switching of one item.  Workspace in the item.
 int fz_mul(const DevParams& P, const FzItem& it, hipStream_t st);
 int fz_switch(const DevParams& P, const FzItem& it, hipStream_t st);
@@ -68,12 +64,6 @@ void launch_encrypt_combine(const DevParams& P, uint64_t* c0, uint64_t* c1, cons
 void launch_eltwise(const DevParams& P, int op, uint64_t* out, const uint64_t* a, const uint64_t* b,
                     const uint64_t* c, int nlimbs, int qlimbs, int prime0, hipStream_t st);
 
-// d0 = a0*b0, d1 = a0*b1 + a1*b0, d2 = a1*b1 on L Q-limbs (NTT domain).
-void launch_tensor(const DevParams& P, uint64_t* d0, uint64_t* d1, uint64_t* d2, const uint64_t* a0,
-                   const uint64_t* a1, const uint64_t* b0, const uint64_t* b1, int L, hipStream_t st);
-
-// ModUp: x holds Q limbs 0..level (coefficient domain, stride N); writes K
-// special limbs to outB (stride N).
 void launch_eltwise_scalar(const DevParams& P, int op, uint64_t* out, const uint64_t* a, uint64_t b, int nlimbs,
                            int prime0, hipStream_t st);
 void launch_conjugate(const DevParams& P, uint64_t* out, const uint64_t* in, int nlimbs, hipStream_t st);
@@ -94,12 +84,13 @@ void launch_sample_encrypt(const DevParams& P, uint64_t* u, uint64_t* e0, uint64
 void launch_special_fft(const DevParams& P, double* vals, int n, int inverse, hipStream_t st);
 void launch_encode(const DevParams& P, uint64_t* out, double* vals, int slots, double scale, int k, hipStream_t st);
 void launch_decode(const DevParams& P, double* vals, const uint64_t* in, int slots, double scale, hipStream_t st);
+// ModUp: x holds Q limbs 0..level (coefficient domain, stride N); writes K
+// special limbs to outB (stride N).
 void launch_modup(const DevParams& P, const uint64_t* x, uint64_t* outB, int level, hipStream_t st);
 
 // ModDown of npolys polys.  inQ[y] holds Q limbs 0..level, inB[y] the K
 // special limbs (coefficient domain).  out[y] limb i = (inQ_i - conv_i(inB)) *
-// B^-1 mod q_i (+ add[y] limb i when add[y] != null).  With rescale, the
-// result is further rescaled by q_level and only limbs 0..level-1 are written.
+// B^-1 mod q_i (+ add[y] limb i when add[y] != null).
 struct ModDownArgs {
   const uint64_t* inQ[2];
   const uint64_t* inB[2];
@@ -107,7 +98,6 @@ struct ModDownArgs {
   uint64_t* out[2];
   int npolys;
   int level;
-  int rescale;
 };
 void launch_moddown(const DevParams& P, const ModDownArgs& a, hipStream_t st);
 
@@ -133,29 +123,8 @@ void launch_dr2(const DevParams& P, uint64_t* c21, uint64_t* c22, uint64_t* c23,
 
 // Descriptor-driven (stage-fused) forms used by batches: one launch covers
 // every descriptor of the table (device memory).
-// nstrict: the first nstrict descriptors use primes of 2^61 and above and
-// the rest do not (a prime-major list); -1 when not known.
-int ntt_forward_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hipStream_t st, int nstrict = -1);
-// canon = false: the two-pass form's lazy limbs may end in [0, 2p) (for
-// ModUp and ModDown, which take them so); q0 and the single-workgroup form
-// stay canonical.
-int ntt_inverse_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hipStream_t st, int nstrict = -1,
-                     bool canon = true);
-// Key-switching inverse NTT: first pass from KeyDesc2 entries (one input limb,
-// two keys, two outputs), second pass over the NttDesc list of outputs.
-// canon = false as above, and in the two-pass form the special limbs (prime
-// index k + j) come out multiplied by (B/b_j)^-1 mod b_j, in [0, 2 b_j), for
-// a ModDown that takes them so (ModDownDesc::bscaled).
-int ntt_inverse_key2_desc(const DevParams& P, const KeyDesc2* d2, int n2, const NttDesc* dcol, int ncol, int N1,
-                          hipStream_t st, int n2strict = -1, int ncolstrict = -1, bool canon = true);
-// Whether ntt_inverse_key2_desc(..., N1, ..., canon = false) scales the
-// special limbs (the two-pass form).
-bool ntt_key2_bscaled(const DevParams& P, int N1);
-void launch_tensor_desc(const DevParams& P, const TensorDesc* d, int ndesc, hipStream_t st);
-void launch_modup_desc(const DevParams& P, const ModUpDesc* d, int ndesc, int max_level, hipStream_t st);
-// bscaled: every descriptor's special limbs come from ntt_inverse_key2_desc's
-// scaled form (already multiplied by (B/b_j)^-1 mod b_j, in [0, 2 b_j)).
-void launch_moddown_desc(const DevParams& P, const ModDownDesc* d, int ndesc, bool bscaled, hipStream_t st);
+int ntt_forward_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hipStream_t st);
+int ntt_inverse_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hipStream_t st);
 void launch_automorphism_desc(const DevParams& P, const AutoDesc* d, int ndesc, hipStream_t st);
 
 }  // namespace aoa

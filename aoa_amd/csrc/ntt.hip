@@ -210,9 +210,6 @@ __device__ __forceinline__ void fwd_row_body(const DevParams& P, const uint64_t*
   for (int k = 0; k < 16; ++k) dst[sl + TS * k] = L[swz(sl + TS * k)];
 }
 
-// Row pass of the inverse: global stages g0+log2(S)-1 .. g0.  With a key, the
-// input limb is first multiplied by the key limb (key switching:
-// INTT(x * key_b), INTT(x * key_a) from one input).
 // The inverse row pass after the input limb is in registers (x[k] = element
 // sl + TS*k of the thread's row): stages g0+log2(S)-1 .. g0, result to dst.
 // T is the prime's inverse table, TR its row-ordered copy (row_twiddle_order)
@@ -279,43 +276,12 @@ __device__ __forceinline__ void inv_row_core(const DevParams& P, uint64_t (&x)[1
   for (int k = 0; k < 16; ++k) dst[sl + TS * k] = x[k];
 }
 
-// x * key mod p for a key-switching product (LZ: result in [0, 2p), which the
-// lazy inverse butterflies accept).
-template <bool LZ>
-__device__ __forceinline__ uint64_t key_mul(uint64_t x, uint64_t k, const DevPrime& dp) {
-  return LZ ? mul_barrett62_lazy(x, k, dp.p, dp.mu2, (int)dp.nb) : mul_barrett(x, k, dp.p, dp.mu, (int)dp.nb);
-}
-
-// Same, canonical: the operand of a further product.
-template <bool LZ>
-__device__ __forceinline__ uint64_t key_mul_canon(uint64_t x, uint64_t k, const DevPrime& dp) {
-  return LZ ? mul_barrett62(x, k, dp.p, dp.mu2, (int)dp.nb) : mul_barrett(x, k, dp.p, dp.mu, (int)dp.nb);
-}
-
-// x (products in [0, 2p) when LZ, else canonical) plus (B mod q) times the
-// NTT-domain addend of a Q limb pr, left in the same range.
-template <bool LZ>
-__device__ __forceinline__ void add_bscaled(uint64_t (&x)[16], const uint64_t* ap, int stride, const DevParams& P,
-                                            int pr, uint64_t p) {
-  const tw2 bq = reinterpret_cast<const tw2*>(P.b_mod_q)[pr];
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const uint64_t t = x[k] + mul_shoup(ap[stride * k], bq.w, bq.q, p);
-    // lazy: [0, 3p) -> [0, 2p); strict: canonical sum
-    x[k] = LZ ? (t >= 2 * p ? t - 2 * p : t) : (t >= p ? t - p : t);
-  }
-}
-
-// Row pass of the inverse: global stages g0+log2(S)-1 .. g0.  With a key, the
-// input limb is first multiplied by the key limb, and then (if add is set,
-// for Q limbs) (B mod q) times the add limb joins the product.
+// Row pass of the inverse: global stages g0+log2(S)-1 .. g0.
 template <int S, bool LZ>
-__device__ __forceinline__ void inv_row_body(const DevParams& P, const uint64_t* src, uint64_t* dst,
-                                             const uint64_t* key, const uint64_t* add, int pr, int tile, int g0,
-                                             uint64_t* lds) {
+__device__ __forceinline__ void inv_row_body(const DevParams& P, const uint64_t* src, uint64_t* dst, int pr, int tile,
+                                             int g0, uint64_t* lds) {
   using G = Geo<S>;
   constexpr int C = G::C, TS = G::TS, PS = S + S / 16;
-  const DevPrime dp = P.primes[pr];
   const uint64_t* T = P.tw_inv + (size_t)pr * P.N * 2;
   const uint64_t* TR = P.tw_row[G::LOGS - 6][1] + (size_t)pr * P.N * 2;
   const int rl = threadIdx.x / TS, sl = threadIdx.x % TS;
@@ -324,74 +290,12 @@ __device__ __forceinline__ void inv_row_body(const DevParams& P, const uint64_t*
   uint64_t x[16];
 #pragma unroll
   for (int k = 0; k < 16; ++k) x[k] = src[sl + TS * k];
-  if (key) {
-    const uint64_t* kp = key + (size_t)row * S;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) x[k] = key_mul<LZ>(x[k], kp[sl + TS * k], dp);
-    if (add) add_bscaled<LZ>(x, add + (size_t)row * S + sl, TS, P, pr, dp.p);
-  }
-  inv_row_core<S, LZ>(P, x, dst + (size_t)row * S, dp.p, T, TR, row, sl, g0, lds + rl * PS);
-}
-
-// Key switching's two products from one input limb: dst0 = first inverse
-// pass of (src * key0 + (B mod q) add0), dst1 = same with key1 and add1 (the
-// adds may be null).  The workgroup reads its src tile twice; the second read
-// is served by the L2 cache, so HBM sees the input once while the registers
-// hold one tile at a time.  With HomMul's operands (a0 set: Q limbs of the
-// batched form) the input is d2 = a1 b1 and the adds are d0 = a0 b0 and
-// d1 = a0 b1 + a1 b0 (congruent to the reference's (a0+a1)(b0+b1) - d0 - d2),
-// formed here from the four operand tiles, which the two key halves' workgroups
-// of a tile read from HBM once between them (the second from L2).
-template <int S, bool LZ>
-__device__ __forceinline__ void inv_row_key2_body(const DevParams& P, const uint64_t* src, uint64_t* dst0,
-                                                  uint64_t* dst1, const uint64_t* key0, const uint64_t* key1,
-                                                  const uint64_t* add0, const uint64_t* add1, const uint64_t* a0,
-                                                  const uint64_t* a1, const uint64_t* b0, const uint64_t* b1, int pr,
-                                                  int tile, int g0, uint64_t* lds, int ysel) {
-  using G = Geo<S>;
-  constexpr int C = G::C, TS = G::TS, PS = S + S / 16;
-  const DevPrime dp = P.primes[pr];
-  const uint64_t p = dp.p;
-  const uint64_t* T = P.tw_inv + (size_t)pr * P.N * 2;
-  const uint64_t* TR = P.tw_row[G::LOGS - 6][1] + (size_t)pr * P.N * 2;
-  const int rl = threadIdx.x / TS, sl = threadIdx.x % TS;
-  const int row = tile * C + rl;
-  const size_t off = (size_t)row * S;
-#pragma unroll
-  for (int y = 0; y < 2; ++y) {
-    if (ysel >= 0 && y != ysel) continue;
-    const uint64_t* kp = (y ? key1 : key0) + off;
-    uint64_t x[16];
-    if (a0) {
-      const tw2 bq = reinterpret_cast<const tw2*>(P.b_mod_q)[pr];
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        const size_t i = off + sl + TS * k;
-        const uint64_t A0 = a0[i], A1 = a1[i], B0 = b0[i], B1 = b1[i];
-        const uint64_t d2 = key_mul_canon<LZ>(A1, B1, dp);
-        // lazy: d in [0, 4p), the sum in [0, 3p) -> [0, 2p); strict: below 2p, then canonical
-        const uint64_t d = y ? key_mul<LZ>(A0, B1, dp) + key_mul<LZ>(A1, B0, dp) : key_mul<LZ>(A0, B0, dp);
-        const uint64_t t = key_mul<LZ>(d2, kp[sl + TS * k], dp) + mul_shoup(d, bq.w, bq.q, p);
-        x[k] = LZ ? (t >= 2 * p ? t - 2 * p : t) : (t >= p ? t - p : t);
-      }
-    } else {
-      const uint64_t* ap = y ? add1 : add0;
-#pragma unroll
-      for (int k = 0; k < 16; ++k) x[k] = key_mul<LZ>(src[off + sl + TS * k], kp[sl + TS * k], dp);
-      if (ap) add_bscaled<LZ>(x, ap + off + sl, TS, P, pr, p);  // set for Q limbs only
-    }
-    if (y && ysel < 0) __syncthreads();  // the row's LDS block is reused
-    inv_row_core<S, LZ>(P, x, (y ? dst1 : dst0) + off, p, T, TR, row, sl, g0, lds + rl * PS);
-  }
+  inv_row_core<S, LZ>(P, x, dst + (size_t)row * S, P.primes[pr].p, T, TR, row, sl, g0, lds + rl * PS);
 }
 
 // Column pass of the inverse: global stages log2(S)-1 .. 0, N^-1 folded into
 // stage 0.
-// CANON = false (lazy primes only) leaves the outputs in [0, 2p) for a
-// consumer that takes them so (ModUp, ModDown).  BS (with CANON = false):
-// the special limbs (pr >= k) also take ModDown's factor (B/b_j)^-1 mod b_j
-// in this stage (bscale), so that ModDown does not multiply them again.
-template <int S, bool LZ, bool CANON = true, bool BS = false>
+template <int S, bool LZ>
 __device__ __forceinline__ void inv_col_body(const DevParams& P, const uint64_t* src, uint64_t* dst, int pr,
                                              int tile, int N2, uint64_t* lds) {
   using G = Geo<S>;
@@ -435,24 +339,11 @@ __device__ __forceinline__ void inv_col_body(const DevParams& P, const uint64_t*
     }
   }
   // stage 0 with N^-1: a' = (u+v) N^-1, b' = (u-v) psi^-brev(1) N^-1
-  uint64_t n0 = dp.ninv, n0q = dp.ninv_q, n1 = dp.w1ninv, n1q = dp.w1ninv_q;
-  if (BS && pr >= P.k) {
-    const cptr<uint64_t> bs = as_const(P.bscale) + 4 * (pr - P.k);
-    n0 = bs[0];
-    n0q = bs[1];
-    n1 = bs[2];
-    n1q = bs[3];
-  }
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     uint64_t u = x[k], v = x[k + 8];
-    if (LZ && !CANON) {
-      x[k] = mul_shoup_lazy(u + v, n0, n0q, p);
-      x[k + 8] = mul_shoup_lazy(u + 2 * p - v, n1, n1q, p);
-    } else {
-      x[k] = mul_shoup(u + v, dp.ninv, dp.ninv_q, p);
-      x[k + 8] = mul_shoup(LZ ? u + 2 * p - v : u + (p - v), dp.w1ninv, dp.w1ninv_q, p);
-    }
+    x[k] = mul_shoup(u + v, dp.ninv, dp.ninv_q, p);
+    x[k + 8] = mul_shoup(LZ ? u + 2 * p - v : u + (p - v), dp.w1ninv, dp.w1ninv_q, p);
   }
 #pragma unroll
   for (int k = 0; k < 16; ++k) dst[(size_t)(sl + TS * k) * N2 + c] = x[k];
@@ -492,23 +383,17 @@ __global__ __launch_bounds__(256) void k_ntt_fwd_row(DevParams P, LimbMap m, int
 }
 
 template <int S>
-__global__ __launch_bounds__(256) void k_ntt_inv_row(DevParams P, LimbMap m, int g0, const uint64_t* key0,
-                                                      const uint64_t* key1, const uint64_t* add0,
-                                                      const uint64_t* add1) {
+__global__ __launch_bounds__(256) void k_ntt_inv_row(DevParams P, LimbMap m, int g0) {
   __shared__ uint64_t lds[Geo<S>::ROW_LDS];
   const int tiles = (P.N / S) / Geo<S>::C;
   const int li = blockIdx.x / tiles;
   const int y = blockIdx.y;
   const size_t off = (size_t)li * P.N;
   const int pr = limb_prime(m, P.k, li);
-  const uint64_t* key = key0 ? (y == 0 ? key0 : key1) + (size_t)pr * P.N : nullptr;
-  const uint64_t* addy = y == 0 ? add0 : add1;
-  const uint64_t* add = addy && li < m.qlimbs ? addy + off : nullptr;
-  const uint64_t* src = (key0 ? m.src[0] : m.src[y]) + off;
   if (lazy_prime(P, pr))
-    inv_row_body<S, true>(P, src, m.base[y] + off, key, add, pr, blockIdx.x % tiles, g0, lds);
+    inv_row_body<S, true>(P, m.src[y] + off, m.base[y] + off, pr, blockIdx.x % tiles, g0, lds);
   else
-    inv_row_body<S, false>(P, src, m.base[y] + off, key, add, pr, blockIdx.x % tiles, g0, lds);
+    inv_row_body<S, false>(P, m.src[y] + off, m.base[y] + off, pr, blockIdx.x % tiles, g0, lds);
 }
 
 template <int S>
@@ -526,15 +411,6 @@ __global__ __launch_bounds__(256) void k_ntt_inv_col(DevParams P, LimbMap m, int
 
 // ----------------------------------------------- descriptor-driven kernels --
 
-// MODE: 0 decides lazy or strict butterflies per descriptor; 1 (every
-// descriptor's prime is below 2^61) and 2 (none is) compile one form only,
-// which keeps the register count of the lazy form (launchers split a
-// prime-major descriptor list at the first lazy prime).
-template <int MODE>
-__device__ __forceinline__ bool use_lazy(const DevParams& P, int pr) {
-  return MODE == 1 ? true : (MODE == 2 ? false : lazy_prime(P, pr));
-}
-
 // Work item of this workgroup: blockIdx.x, or with P.xcd_chunks its XCD
 // chunk id (xcd_chunk_id), so that neighbouring items -- in a prime-major
 // descriptor list, the tiles of one prime -- share an XCD and its L2.
@@ -542,95 +418,52 @@ __device__ __forceinline__ int work_id(const DevParams& P) {
   return P.xcd_chunks ? xcd_chunk_id(blockIdx.x, gridDim.x) : (int)blockIdx.x;
 }
 
-template <int S, int MODE>
+template <int S>
 __global__ __launch_bounds__(256) void k_ntt_fwd_col_d(DevParams P, const NttDesc* d, int N2) {
   __shared__ uint64_t lds[Geo<S>::COL_LDS];
   const int wid = work_id(P);
   const int tiles = N2 / Geo<S>::C;
   const NttDesc e = d[wid / tiles];
-  if (use_lazy<MODE>(P, e.prime))
+  if (lazy_prime(P, e.prime))
     fwd_col_body<S, true>(P, glob(e.src), glob(e.dst), e.prime, wid % tiles, N2, lds);
-  else if (MODE != 1)
+  else
     fwd_col_body<S, false>(P, glob(e.src), glob(e.dst), e.prime, wid % tiles, N2, lds);
 }
 
-template <int S, int MODE>
+template <int S>
 __global__ __launch_bounds__(256) void k_ntt_fwd_row_d(DevParams P, const NttDesc* d, int g0) {
   __shared__ uint64_t lds[Geo<S>::ROW_LDS];
   const int wid = work_id(P);
   const int tiles = (P.N / S) / Geo<S>::C;
   const NttDesc e = d[wid / tiles];
-  if (use_lazy<MODE>(P, e.prime))
+  if (lazy_prime(P, e.prime))
     fwd_row_body<S, true>(P, glob(e.dst), glob(e.dst), e.prime, wid % tiles, g0, lds);
-  else if (MODE != 1)
+  else
     fwd_row_body<S, false>(P, glob(e.dst), glob(e.dst), e.prime, wid % tiles, g0, lds);
 }
 
-template <int S, int MODE>
+template <int S>
 __global__ __launch_bounds__(256) void k_ntt_inv_row_d(DevParams P, const NttDesc* d, int g0) {
   __shared__ uint64_t lds[Geo<S>::ROW_LDS];
   const int wid = work_id(P);
   const int tiles = (P.N / S) / Geo<S>::C;
   const NttDesc e = d[wid / tiles];
-  if (use_lazy<MODE>(P, e.prime))
-    inv_row_body<S, true>(P, glob(e.src), glob(e.dst), glob(e.key), nullptr, e.prime, wid % tiles, g0, lds);
-  else if (MODE != 1)
-    inv_row_body<S, false>(P, glob(e.src), glob(e.dst), glob(e.key), nullptr, e.prime, wid % tiles, g0, lds);
+  if (lazy_prime(P, e.prime))
+    inv_row_body<S, true>(P, glob(e.src), glob(e.dst), e.prime, wid % tiles, g0, lds);
+  else
+    inv_row_body<S, false>(P, glob(e.src), glob(e.dst), e.prime, wid % tiles, g0, lds);
 }
 
-// One workgroup per tile and key half: workgroups w and w + 8 take the two
-// halves of one tile; as workgroups are dispatched round-robin over the 8
-// XCDs, both run on one XCD and the second read of the input tile comes from
-// its L2.  `ntiles` = descriptors x tiles per limb; the grid is rounded up to
-// a multiple of 16.
-template <int S, int MODE>
-__global__ __launch_bounds__(256) void k_ntt_inv_row_key2_d(DevParams P, const KeyDesc2* d, int g0, int ntiles) {
-  __shared__ uint64_t lds[Geo<S>::ROW_LDS];
-  const int tiles = (P.N / S) / Geo<S>::C;
-  const int w = blockIdx.x;
-  const int y = (w >> 3) & 1, b = ((w >> 4) << 3) | (w & 7);
-  if (b >= ntiles) return;
-  const KeyDesc2& e = d[b / tiles];
-  const uint64_t* src = glob(e.src);
-  uint64_t *d0 = glob(e.dst[0]), *d1 = glob(e.dst[1]);
-  const uint64_t *k0 = glob(e.key[0]), *k1 = glob(e.key[1]), *a0 = glob(e.add[0]), *a1 = glob(e.add[1]);
-  const uint64_t *t0 = glob(e.ab[0]), *t1 = glob(e.ab[1]), *t2 = glob(e.ab[2]), *t3 = glob(e.ab[3]);
-  const int pr = e.prime;
-  if (use_lazy<MODE>(P, pr))
-    inv_row_key2_body<S, true>(P, src, d0, d1, k0, k1, a0, a1, t0, t1, t2, t3, pr, b % tiles, g0, lds, y);
-  else if (MODE != 1)
-    inv_row_key2_body<S, false>(P, src, d0, d1, k0, k1, a0, a1, t0, t1, t2, t3, pr, b % tiles, g0, lds, y);
-}
-
-template <int S, int MODE, bool CANON, bool BS = false>
-__device__ __forceinline__ void inv_col_d(const DevParams& P, const NttDesc* d, int N2, uint64_t* lds) {
+template <int S>
+__global__ __launch_bounds__(256) void k_ntt_inv_col_d(DevParams P, const NttDesc* d, int N2) {
+  __shared__ uint64_t lds[Geo<S>::COL_LDS];
   const int wid = work_id(P);
   const int tiles = N2 / Geo<S>::C;
   const NttDesc e = d[wid / tiles];
-  if (use_lazy<MODE>(P, e.prime))
-    inv_col_body<S, true, CANON, BS>(P, glob(e.dst), glob(e.dst), e.prime, wid % tiles, N2, lds);
-  else if (MODE != 1)
+  if (lazy_prime(P, e.prime))
+    inv_col_body<S, true>(P, glob(e.dst), glob(e.dst), e.prime, wid % tiles, N2, lds);
+  else
     inv_col_body<S, false>(P, glob(e.dst), glob(e.dst), e.prime, wid % tiles, N2, lds);
-}
-
-template <int S, int MODE>
-__global__ __launch_bounds__(256) void k_ntt_inv_col_d(DevParams P, const NttDesc* d, int N2) {
-  __shared__ uint64_t lds[Geo<S>::COL_LDS];
-  inv_col_d<S, MODE, true>(P, d, N2, lds);
-}
-
-// Same, the lazy limbs' outputs left in [0, 2p) (the q0 limbs stay canonical).
-template <int S, int MODE>
-__global__ __launch_bounds__(256) void k_ntt_inv_col_lazy_d(DevParams P, const NttDesc* d, int N2) {
-  __shared__ uint64_t lds[Geo<S>::COL_LDS];
-  inv_col_d<S, MODE, false>(P, d, N2, lds);
-}
-
-// Same, the special limbs also multiplied by (B/b_j)^-1 mod b_j for ModDown.
-template <int S, int MODE>
-__global__ __launch_bounds__(256) void k_ntt_inv_col_bscale_d(DevParams P, const NttDesc* d, int N2) {
-  __shared__ uint64_t lds[Geo<S>::COL_LDS];
-  inv_col_d<S, MODE, false, true>(P, d, N2, lds);
 }
 
 // ------------------------------------------- single-workgroup transform --
@@ -661,18 +494,15 @@ struct SGeo {
   static constexpr int N = 1 << LOGN, TH = N / 4, V = 4, R = 2, LDS = N + N / 32;
 };
 
-// Coalesced load of a limb (optionally times a key limb) into LDS.
-template <int LOGN, bool LZ>
-__device__ __forceinline__ void sp_load(const uint64_t* src, const uint64_t* key, const DevPrime& dp,
-                                        uint64_t* lds) {
+// Coalesced load of a limb into LDS.
+template <int LOGN>
+__device__ __forceinline__ void sp_load(const uint64_t* src, uint64_t* lds) {
   constexpr int V = SGeo<LOGN>::V, TH = SGeo<LOGN>::TH;
   const int t = threadIdx.x;
 #pragma unroll
   for (int m = 0; m < V; ++m) {
     const int i = t + TH * m;
-    uint64_t v = src[i];
-    if (key) v = key_mul<LZ>(v, key[i], dp);
-    lds[spz(i)] = v;
+    lds[spz(i)] = src[i];
   }
   __syncthreads();
 }
@@ -694,7 +524,7 @@ __device__ __forceinline__ void fwd_single_body(const DevParams& P, const uint64
   const uint64_t p = dp.p;
   const uint64_t* T = P.tw_fwd + (size_t)pr * G::N * 2;
   const int t = threadIdx.x;
-  sp_load<LOGN, LZ>(src, nullptr, dp, lds);
+  sp_load<LOGN>(src, lds);
   uint64_t x[V];
 #pragma unroll
   for (int s0 = 0; s0 < LOGN; s0 += R) {
@@ -725,18 +555,17 @@ __device__ __forceinline__ void fwd_single_body(const DevParams& P, const uint64
   sp_store<LOGN>(dst, lds);
 }
 
-// Inverse: stages LOGN-1 .. 0 (Gentleman-Sande), N^-1 folded into stage 0;
-// with a key the input limb is first multiplied by the key limb.
+// Inverse: stages LOGN-1 .. 0 (Gentleman-Sande), N^-1 folded into stage 0.
 template <int LOGN, bool LZ>
-__device__ __forceinline__ void inv_single_body(const DevParams& P, const uint64_t* src, uint64_t* dst,
-                                                const uint64_t* key, int pr, uint64_t* lds) {
+__device__ __forceinline__ void inv_single_body(const DevParams& P, const uint64_t* src, uint64_t* dst, int pr,
+                                                uint64_t* lds) {
   using G = SGeo<LOGN>;
   constexpr int V = G::V, R = G::R;
   const DevPrime dp = P.primes[pr];
   const uint64_t p = dp.p;
   const uint64_t* T = P.tw_inv + (size_t)pr * G::N * 2;
   const int t = threadIdx.x;
-  sp_load<LOGN, LZ>(src, key, dp, lds);
+  sp_load<LOGN>(src, lds);
   uint64_t x[V];
 #pragma unroll
   for (int done = 0; done < LOGN; done += R) {
@@ -782,17 +611,14 @@ __global__ __launch_bounds__(SGeo<LOGN>::TH) void k_ntt_fwd_single(DevParams P, 
 }
 
 template <int LOGN>
-__global__ __launch_bounds__(SGeo<LOGN>::TH) void k_ntt_inv_single(DevParams P, LimbMap m, const uint64_t* key0,
-                                                         const uint64_t* key1) {
+__global__ __launch_bounds__(SGeo<LOGN>::TH) void k_ntt_inv_single(DevParams P, LimbMap m) {
   __shared__ uint64_t lds[SGeo<LOGN>::LDS];
   const int li = blockIdx.x, y = blockIdx.y, pr = limb_prime(m, P.k, li);
   const size_t off = (size_t)li * P.N;
-  const uint64_t* key = key0 ? (y == 0 ? key0 : key1) + (size_t)pr * P.N : nullptr;
-  const uint64_t* src = (key0 ? m.src[0] : m.src[y]) + off;
   if (lazy_prime(P, pr))
-    inv_single_body<LOGN, true>(P, src, m.base[y] + off, key, pr, lds);
+    inv_single_body<LOGN, true>(P, m.src[y] + off, m.base[y] + off, pr, lds);
   else
-    inv_single_body<LOGN, false>(P, src, m.base[y] + off, key, pr, lds);
+    inv_single_body<LOGN, false>(P, m.src[y] + off, m.base[y] + off, pr, lds);
 }
 
 template <int LOGN>
@@ -814,28 +640,11 @@ __global__ __launch_bounds__(SGeo<LOGN>::TH) void k_ntt_inv_single_d(DevParams P
   const NttDesc& e = d[blockIdx.x];
   const uint64_t* src = glob(e.src);
   uint64_t* dst = glob(e.dst);
-  const uint64_t* key = glob(e.key);
   const int pr = e.prime;
   if (lazy_prime(P, pr))
-    inv_single_body<LOGN, true>(P, src, dst, key, pr, lds);
+    inv_single_body<LOGN, true>(P, src, dst, pr, lds);
   else
-    inv_single_body<LOGN, false>(P, src, dst, key, pr, lds);
-}
-
-// Both key products of one input limb, one workgroup per (limb, key half).
-template <int LOGN>
-__global__ __launch_bounds__(SGeo<LOGN>::TH) void k_ntt_inv_single_key2_d(DevParams P, const KeyDesc2* d) {
-  __shared__ uint64_t lds[SGeo<LOGN>::LDS];
-  const KeyDesc2& e = d[blockIdx.x >> 1];
-  const int y = blockIdx.x & 1;
-  const uint64_t* src = glob(e.src);
-  uint64_t* dst = glob(y ? e.dst[1] : e.dst[0]);
-  const uint64_t* key = glob(y ? e.key[1] : e.key[0]);
-  const int pr = e.prime;
-  if (lazy_prime(P, pr))
-    inv_single_body<LOGN, true>(P, src, dst, key, pr, lds);
-  else
-    inv_single_body<LOGN, false>(P, src, dst, key, pr, lds);
+    inv_single_body<LOGN, false>(P, src, dst, pr, lds);
 }
 
 // ---------------------------------------------------------------- launch ---
@@ -876,7 +685,7 @@ static int log2i(int n) {
   }
 
 static int pick_n1(const DevParams& P, int N1) {
-  if (N1 == 0) N1 = P.ntt_n1 ? P.ntt_n1 : ntt_default_n1(P.N);
+  if (N1 == 0) N1 = P.ntt_n1;
   return ntt_valid_split(P.N, N1) ? N1 : 0;
 }
 
@@ -920,18 +729,16 @@ int ntt_forward(const DevParams& P, LimbMap m, int N1, hipStream_t st) {
   return 0;
 }
 
-int ntt_inverse(const DevParams& P, LimbMap m, int N1, const uint64_t* key0, const uint64_t* key1,
-                hipStream_t st, const uint64_t* add0, const uint64_t* add1) {
+int ntt_inverse(const DevParams& P, LimbMap m, int N1, hipStream_t st) {
   for (int y = 0; y < m.npolys; ++y)
     if (!m.src[y]) m.src[y] = m.base[y];
-  if (!N1 && !key0 && nt_default(P)) return nt_inverse(P, m, st);
+  if (!N1 && nt_default(P)) return nt_inverse(P, m, st);
   N1 = pick_n1(P, N1);
   if (!N1) return -1;
-  if ((add0 || add1) && (N1 == P.N || !key0)) return -1;  // adds: two-pass key products only
   const int N2 = P.N / N1, g0 = log2i(N1);
   if (N1 == P.N) {
     dim3 grid(m.nlimbs, m.npolys);
-#define CALL1(L) k_ntt_inv_single<L><<<grid, SGeo<L>::TH, 0, st>>>(P, m, key0, key1)
+#define CALL1(L) k_ntt_inv_single<L><<<grid, SGeo<L>::TH, 0, st>>>(P, m)
     AOA_DISPATCH_LOGN(P.N, CALL1)
 #undef CALL1
     return 0;
@@ -939,7 +746,7 @@ int ntt_inverse(const DevParams& P, LimbMap m, int N1, const uint64_t* key0, con
   {
     const int tiles = N1 / (4096 / N2);
     dim3 grid(tiles * m.nlimbs, m.npolys);
-#define CALLR(S) k_ntt_inv_row<S><<<grid, 256, 0, st>>>(P, m, g0, key0, key1, add0, add1)
+#define CALLR(S) k_ntt_inv_row<S><<<grid, 256, 0, st>>>(P, m, g0)
     AOA_DISPATCH_S(N2, CALLR)
 #undef CALLR
   }
@@ -955,21 +762,7 @@ int ntt_inverse(const DevParams& P, LimbMap m, int N1, const uint64_t* key0, con
   return 0;
 }
 
-// Launches kernel K<S, MODE> over `n` descriptors of which the first
-// `strict` use primes of 2^61 and above (strict < 0: not known, one launch
-// deciding per descriptor).
-#define AOA_SPLIT_LAUNCH(K, S, GRIDPER, DESC, N_, STRICT, ...)                                          \
-  do {                                                                                                  \
-    if ((STRICT) < 0) {                                                                                 \
-      K<S, 0><<<dim3((GRIDPER) * (N_)), 256, 0, st>>>(P, DESC, __VA_ARGS__);                           \
-    } else {                                                                                            \
-      if ((STRICT) > 0) K<S, 2><<<dim3((GRIDPER) * (STRICT)), 256, 0, st>>>(P, DESC, __VA_ARGS__);     \
-      if ((N_) > (STRICT))                                                                              \
-        K<S, 1><<<dim3((GRIDPER) * ((N_) - (STRICT))), 256, 0, st>>>(P, (DESC) + (STRICT), __VA_ARGS__); \
-    }                                                                                                   \
-  } while (0)
-
-int ntt_forward_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hipStream_t st, int nstrict) {
+int ntt_forward_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hipStream_t st) {
   if (!N1 && nt_default(P)) return nt_forward_desc(P, d, ndesc, st);
   N1 = pick_n1(P, N1);
   if (!N1 || ndesc <= 0) return -1;
@@ -982,20 +775,20 @@ int ntt_forward_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hi
   }
   {
     const int tiles = N2 / (4096 / N1);
-#define CALLC(S) AOA_SPLIT_LAUNCH(k_ntt_fwd_col_d, S, tiles, d, ndesc, nstrict, N2)
+#define CALLC(S) k_ntt_fwd_col_d<S><<<dim3(tiles * ndesc), 256, 0, st>>>(P, d, N2)
     AOA_DISPATCH_S(N1, CALLC)
 #undef CALLC
   }
   {
     const int tiles = N1 / (4096 / N2);
-#define CALLR(S) AOA_SPLIT_LAUNCH(k_ntt_fwd_row_d, S, tiles, d, ndesc, nstrict, g0)
+#define CALLR(S) k_ntt_fwd_row_d<S><<<dim3(tiles * ndesc), 256, 0, st>>>(P, d, g0)
     AOA_DISPATCH_S(N2, CALLR)
 #undef CALLR
   }
   return 0;
 }
 
-int ntt_inverse_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hipStream_t st, int nstrict, bool canon) {
+int ntt_inverse_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hipStream_t st) {
   if (!N1 && nt_default(P)) return nt_inverse_desc(P, d, ndesc, st);
   N1 = pick_n1(P, N1);
   if (!N1 || ndesc <= 0) return -1;
@@ -1008,57 +801,13 @@ int ntt_inverse_desc(const DevParams& P, const NttDesc* d, int ndesc, int N1, hi
   }
   {
     const int tiles = N1 / (4096 / N2);
-#define CALLR(S) AOA_SPLIT_LAUNCH(k_ntt_inv_row_d, S, tiles, d, ndesc, nstrict, g0)
+#define CALLR(S) k_ntt_inv_row_d<S><<<dim3(tiles * ndesc), 256, 0, st>>>(P, d, g0)
     AOA_DISPATCH_S(N2, CALLR)
 #undef CALLR
   }
   {
     const int tiles = N2 / (4096 / N1);
-#define CALLC(S)                                                              \
-  if (canon) AOA_SPLIT_LAUNCH(k_ntt_inv_col_d, S, tiles, d, ndesc, nstrict, N2); \
-  else AOA_SPLIT_LAUNCH(k_ntt_inv_col_lazy_d, S, tiles, d, ndesc, nstrict, N2)
-    AOA_DISPATCH_S(N1, CALLC)
-#undef CALLC
-  }
-  return 0;
-}
-
-bool ntt_key2_bscaled(const DevParams& P, int N1) {
-  N1 = pick_n1(P, N1);
-  return N1 != 0 && N1 != P.N;
-}
-
-int ntt_inverse_key2_desc(const DevParams& P, const KeyDesc2* d2, int n2, const NttDesc* dcol, int ncol, int N1,
-                          hipStream_t st, int n2strict, int ncolstrict, bool canon) {
-  N1 = pick_n1(P, N1);
-  if (!N1 || n2 <= 0 || ncol <= 0) return -1;
-  const int N2 = P.N / N1, g0 = log2i(N1);
-  if (N1 == P.N) {
-#define CALL1(L) k_ntt_inv_single_key2_d<L><<<dim3(2 * n2), SGeo<L>::TH, 0, st>>>(P, d2)
-    AOA_DISPATCH_LOGN(P.N, CALL1)
-#undef CALL1
-    return 0;
-  }
-  {
-    const int tiles = N1 / (4096 / N2);
-    auto grid = [&](int n) { return dim3((unsigned)((2 * tiles * n + 15) / 16 * 16)); };
-    const int nlazy = n2strict < 0 ? 0 : n2 - n2strict;
-#define CALLR(S)                                                                                          \
-  if (n2strict < 0) {                                                                                     \
-    k_ntt_inv_row_key2_d<S, 0><<<grid(n2), 256, 0, st>>>(P, d2, g0, tiles * n2);                          \
-  } else {                                                                                                \
-    if (n2strict > 0) k_ntt_inv_row_key2_d<S, 2><<<grid(n2strict), 256, 0, st>>>(P, d2, g0, tiles * n2strict); \
-    if (nlazy > 0)                                                                                        \
-      k_ntt_inv_row_key2_d<S, 1><<<grid(nlazy), 256, 0, st>>>(P, d2 + n2strict, g0, tiles * nlazy);        \
-  }
-    AOA_DISPATCH_S(N2, CALLR)
-#undef CALLR
-  }
-  {
-    const int tiles = N2 / (4096 / N1);
-#define CALLC(S)                                                                    \
-  if (canon) AOA_SPLIT_LAUNCH(k_ntt_inv_col_d, S, tiles, dcol, ncol, ncolstrict, N2); \
-  else AOA_SPLIT_LAUNCH(k_ntt_inv_col_bscale_d, S, tiles, dcol, ncol, ncolstrict, N2)
+#define CALLC(S) k_ntt_inv_col_d<S><<<dim3(tiles * ndesc), 256, 0, st>>>(P, d, N2)
     AOA_DISPATCH_S(N1, CALLC)
 #undef CALLC
   }

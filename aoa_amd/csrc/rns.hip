@@ -132,59 +132,6 @@ void launch_conjugate(const DevParams& P, uint64_t* out, const uint64_t* in, int
   k_conjugate<<<dim3((unsigned)(total / 256)), 256, 0, st>>>(P, out, in);
 }
 
-// d0 = a0 b0, d2 = a1 b1, d1 = (a0 + a1)(b0 + b1) - d0 - d2 (= a0 b1 + a1 b0),
-// two adjacent elements per thread of one limb (pointers at element e of the
-// limb, e even), moved as 16-byte vectors.
-struct alignas(16) u64x2 {
-  uint64_t v[2];
-};
-
-__device__ __forceinline__ void tensor_body(const DevPrime& d, uint64_t* d0, uint64_t* d1, uint64_t* d2,
-                                            const uint64_t* a0, const uint64_t* a1, const uint64_t* b0,
-                                            const uint64_t* b1, size_t e) {
-  const u64x2 X0 = *reinterpret_cast<const u64x2*>(a0 + e), X1 = *reinterpret_cast<const u64x2*>(a1 + e);
-  const u64x2 Y0 = *reinterpret_cast<const u64x2*>(b0 + e), Y1 = *reinterpret_cast<const u64x2*>(b1 + e);
-  u64x2 R0, R1, R2;
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const uint64_t x0 = X0.v[t], x1 = X1.v[t], y0 = Y0.v[t], y1 = Y1.v[t];
-    const uint64_t p0 = mul_var(x0, y0, d.p, d.mu, d.mu2, (int)d.nb);
-    const uint64_t p2 = mul_var(x1, y1, d.p, d.mu, d.mu2, (int)d.nb);
-    const uint64_t s = mul_var(add_mod(x0, x1, d.p), add_mod(y0, y1, d.p), d.p, d.mu, d.mu2, (int)d.nb);
-    R0.v[t] = p0;
-    R2.v[t] = p2;
-    R1.v[t] = sub_mod(sub_mod(s, p0, d.p), p2, d.p);
-  }
-  *reinterpret_cast<u64x2*>(d0 + e) = R0;
-  *reinterpret_cast<u64x2*>(d1 + e) = R1;
-  *reinterpret_cast<u64x2*>(d2 + e) = R2;
-}
-
-__global__ __launch_bounds__(256) void k_tensor(DevParams P, uint64_t* d0, uint64_t* d1, uint64_t* d2,
-                                                const uint64_t* a0, const uint64_t* a1,
-                                                const uint64_t* b0, const uint64_t* b1) {
-  const size_t e0 = (size_t)blockIdx.x * 512;
-  const int li = (int)(e0 >> P.logN);
-  tensor_body(P.primes[li], d0, d1, d2, a0, a1, b0, b1, e0 + (size_t)threadIdx.x * 2);
-}
-
-void launch_tensor(const DevParams& P, uint64_t* d0, uint64_t* d1, uint64_t* d2, const uint64_t* a0,
-                   const uint64_t* a1, const uint64_t* b0, const uint64_t* b1, int L, hipStream_t st) {
-  const size_t total = (size_t)L * P.N;
-  k_tensor<<<dim3((unsigned)(total / 512)), 256, 0, st>>>(P, d0, d1, d2, a0, a1, b0, b1);
-}
-
-__global__ __launch_bounds__(256) void k_tensor_d(DevParams P, const TensorDesc* dd) {
-  const int per = P.N / 512;
-  const TensorDesc t = dd[blockIdx.x / per];
-  const size_t e = (size_t)(blockIdx.x % per) * 512 + (size_t)threadIdx.x * 2;
-  tensor_body(P.primes[t.prime], glob(t.d0), glob(t.d1), glob(t.d2), glob(t.a0), glob(t.a1), glob(t.b0), glob(t.b1), e);
-}
-
-void launch_tensor_desc(const DevParams& P, const TensorDesc* d, int ndesc, hipStream_t st) {
-  k_tensor_d<<<dim3((unsigned)(ndesc * (P.N / 512))), 256, 0, st>>>(P, d);
-}
-
 // Basis conversion workgroups: 64 consecutive coefficients x 4 limb groups
 // (wave g of the workgroup handles limbs g, g+4, g+8, ...), so a launch has
 // N/64 workgroups per polynomial and each wave reads 512 contiguous bytes.
@@ -206,7 +153,7 @@ constexpr int BC_GROUPS = 4;
 // (reduce_sums_lazy; the host checks its bound).  The halves of w come split
 // from the mu_terms table, the NL limbs' entries side by side, so that a term
 // takes one scalar load and no scalar ALU work.
-template <int NL, bool LAZY>
+template <int NL>
 __device__ __forceinline__ void modup_pass(const DevParams& P, const uint64_t* tl, int c, const int* jl, int level,
                                            uint64_t* outB, size_t cid) {
   constexpr uint32_t M28 = (1u << 28) - 1;
@@ -272,19 +219,17 @@ __device__ __forceinline__ void modup_pass(const DevParams& P, const uint64_t* t
       }
     }
   }
-  // one lazy reduction per limb (below 5 b_j), then down to [0, b_j), or with
-  // LAZY to [0, 4 b_j), which the forward NTT's lazy butterflies take
+  // one lazy reduction per limb (below 5 b_j), then down to [0, b_j)
 #pragma unroll
   for (int n = 0; n < NL; ++n) {
     const uint64_t b = d[n].p;
     uint64_t r = reduce_sums_lazy(s0[n], sm[n] - s0[n] - s2[n], s2[n], b, as_const(P.md_red)[2 * (k + jl[n])],
                                   (int)d[n].nb);
-    for (uint64_t m = 4 * b; m >= (LAZY ? 4 * b : b); m >>= 1) r = r >= m ? r - m : r;
+    for (uint64_t m = 4 * b; m >= b; m >>= 1) r = r >= m ? r - m : r;
     outB[(size_t)jl[n] * P.N + cid] = r;
   }
 }
 
-template <bool LAZY>
 __device__ __forceinline__ void modup_body(const DevParams& P, const uint64_t* x, uint64_t* outB, int level,
                                            int blk, uint64_t* tl) {
   const int L = level + 1;
@@ -306,13 +251,13 @@ __device__ __forceinline__ void modup_body(const DevParams& P, const uint64_t* x
     const int left = (P.K - j + BC_GROUPS - 1) / BC_GROUPS;
     const int jl[4] = {j, j + BC_GROUPS, j + 2 * BC_GROUPS, j + 3 * BC_GROUPS};
     if (left >= 4) {
-      modup_pass<4, LAZY>(P, tl, c, jl, level, outB, cid);
+      modup_pass<4>(P, tl, c, jl, level, outB, cid);
       j += 4 * BC_GROUPS;
     } else if (left >= 2) {
-      modup_pass<2, LAZY>(P, tl, c, jl, level, outB, cid);
+      modup_pass<2>(P, tl, c, jl, level, outB, cid);
       j += 2 * BC_GROUPS;
     } else {
-      modup_pass<1, LAZY>(P, tl, c, jl, level, outB, cid);
+      modup_pass<1>(P, tl, c, jl, level, outB, cid);
       j += BC_GROUPS;
     }
   }
@@ -321,7 +266,7 @@ __device__ __forceinline__ void modup_body(const DevParams& P, const uint64_t* x
 // Seven waves per SIMD (72 registers, one spilled): 3 % faster than six.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_modup(DevParams P, const uint64_t* x, uint64_t* outB, int level) {
   extern __shared__ uint64_t tl[];  // [L][64]
-  modup_body<false>(P, x, outB, level, blockIdx.x, tl);
+  modup_body(P, x, outB, level, blockIdx.x, tl);
 }
 
 void launch_modup(const DevParams& P, const uint64_t* x, uint64_t* outB, int level, hipStream_t st) {
@@ -329,24 +274,9 @@ void launch_modup(const DevParams& P, const uint64_t* x, uint64_t* outB, int lev
   k_modup<<<dim3(P.N / BC_COEF), 256, lds, st>>>(P, x, outB, level);
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_modup_d(DevParams P, const ModUpDesc* dd) {
-  extern __shared__ uint64_t tl[];
-  const int per = P.N / BC_COEF;
-  const ModUpDesc u = dd[blockIdx.x / per];
-  // the batched form's outputs go only to the forward NTT: left in [0, 4 b_j)
-  modup_body<true>(P, glob(u.x), glob(u.outB), u.level, blockIdx.x % per, tl);
-}
-
-void launch_modup_desc(const DevParams& P, const ModUpDesc* d, int ndesc, int max_level, hipStream_t st) {
-  const size_t lds = (size_t)(max_level + 1) * BC_COEF * sizeof(uint64_t);
-  k_modup_d<<<dim3((unsigned)(ndesc * (P.N / BC_COEF))), 256, lds, st>>>(P, d);
-}
-
 // --------------------------------------------------------------- ModDown ----
 // out_i = (x_i - sum_j ref([x_bj (B/b_j)^-1]_bj * (B/b_j mod q_i))) B^-1 mod q_i
-// (aoa-ntt/src/cuda/manager.cu:312-341), optionally + add_i (rotations, and
-// HomMul with the single-workgroup transform), optionally rescaled:
-// out_i <- (out_i - out_l) q_l^-1 mod q_i (manager.cu:90-118).
+// (aoa-ntt/src/cuda/manager.cu:312-341), optionally + add_i.
 //
 // ref(a*c) is the reference's Barrett reduction of the product (ref_barrett).
 // With A = a*c - qhat*p = delta*p + r (r the exact remainder, delta the
@@ -373,7 +303,7 @@ void launch_modup_desc(const DevParams& P, const ModUpDesc* d, int ndesc, int ma
 // term lies outside the deviation window, where the two agree.  The pass/fail
 // masks come straight from the compares and are not carried across
 // iterations.  fold(i, &z) may add one more term z (-B mod q_i), z < 2^57
-// (the caller's addend and the rescale's dropped limb), so that the caller
+// (the caller's addend), so that the caller
 // finishes the limb with one Shoup product.  The host checks that K products,
 // the folded term and K corrections stay below 2^(62+nb) (build_host_params).
 template <int NL, bool SCREEN, class Fold>
@@ -498,15 +428,9 @@ __device__ __forceinline__ uint64_t moddown_wide(const DevParams& P, const uint6
   return wide_reduce(s, dq.p, dq.mu, (int)dq.nb);
 }
 
-// No folded term.
-struct NoFold {
-  __device__ bool operator()(int, uint64_t*) const { return false; }
-};
-
-// bscaled: inB's limbs already carry (B/b_j)^-1 and lie in [0, 2 b_j).
 __device__ __forceinline__ void moddown_body(const DevParams& P, const uint64_t* inQ, const uint64_t* inB,
-                                             const uint64_t* add, uint64_t* out, int level, int rescale,
-                                             int bscaled, int blk, uint64_t* aux) {
+                                             const uint64_t* add, uint64_t* out, int level, int blk,
+                                             uint64_t* aux) {
   const size_t N = (size_t)P.N;
   const int c = threadIdx.x % BC_COEF;
   // wave-uniform limb group: keeps limb indices and constant loads scalar
@@ -514,18 +438,10 @@ __device__ __forceinline__ void moddown_body(const DevParams& P, const uint64_t*
   const size_t cid = (size_t)blk * BC_COEF + c;
   const int K = P.K, k = P.k;
   const tw2* ib = reinterpret_cast<const tw2*>(P.inv_bhat);
-  if (bscaled) {
-    for (int j = g; j < K; j += BC_GROUPS) {
-      const uint64_t bp = P.primes[k + j].p;
-      const uint64_t x = inB[(size_t)j * N + cid];
-      aux[j * BC_COEF + c] = x >= bp ? x - bp : x;
-    }
-  } else {
-    for (int j = g; j < K; j += BC_GROUPS) {
-      const uint64_t bp = P.primes[k + j].p;
-      const tw2 w = ib[j];
-      aux[j * BC_COEF + c] = mul_shoup(inB[(size_t)j * N + cid], w.w, w.q, bp);
-    }
+  for (int j = g; j < K; j += BC_GROUPS) {
+    const uint64_t bp = P.primes[k + j].p;
+    const tw2 w = ib[j];
+    aux[j * BC_COEF + c] = mul_shoup(inB[(size_t)j * N + cid], w.w, w.q, bp);
   }
   __syncthreads();
   const tw2* ibq = reinterpret_cast<const tw2*>(P.inv_b_mod_q);
@@ -554,11 +470,10 @@ __device__ __forceinline__ void moddown_body(const DevParams& P, const uint64_t*
   // moddown_convs, with the term z (-B) when fold(i, &z) says so, and are
   // written by narrow(i, acc).
   // q0's sum (a 63-bit prime's terms cost about 1.4 times a narrow limb's)
-  // is split over the four waves, as the rescale's top limb is below, so that
+  // is split over the four waves, so that
   // the wave that writes limb 0 carries no more than the others: the partial
   // sums meet in LDS and acc0 is their total, valid after the next barrier.
-  uint64_t* part = aux + (size_t)K * BC_COEF;            // [4][64]: the top limb's partial sums
-  uint64_t* part0 = part + (size_t)BC_GROUPS * BC_COEF;  // [4][64]: q0's
+  uint64_t* part0 = aux + (size_t)K * BC_COEF;  // [4][64]: q0's partial sums
   const int jq = (K + BC_GROUPS - 1) / BC_GROUPS;
   const int j0 = g * jq, j1 = min(K, j0 + jq);
   const bool wide0 = ld_prime_nb(P.primes, 0) > 56;
@@ -606,94 +521,31 @@ __device__ __forceinline__ void moddown_body(const DevParams& P, const uint64_t*
       }
     }
   };
-  if (!rescale) {
-    if (wide0) __syncthreads();
-    // add_i joins the sums as z = add_i: (x_i - acc + add_i B) B^-1 = (x_i - acc) B^-1 + add_i
-    limbs(
-        level + 1, [&](int i, uint64_t acc) { out[(size_t)i * N + cid] = finish(i, acc); },
-        [&](int i, uint64_t* z) {
-          if (!add) return false;
-          *z = add[(size_t)i * N + cid];
-          return true;
-        },
-        [&](int i, uint64_t acc) {
-          const tw2 bi = ld_tw2(ibq, i);
-          out[(size_t)i * N + cid] = mul_shoup(lift(i, acc), bi.w, bi.q, ld_prime_p(P.primes, i));
-        });
-    return;
-  }
-  // Rescale needs limb `level` everywhere: its sum over j is split across the
-  // four groups and combined through LDS.
-  {
-    uint64_t r = 0;
-    if (ld_prime_nb(P.primes, level) > 56) {
-      r = conv(level, j0, j1 > j0 ? j1 : j0);
-    } else if (j1 > j0) {
-      moddown_convs<1>(P, aux, c, level, j0, j1, &r, NoFold());
-    }
-    part[g * BC_COEF + c] = r;
-  }
-  __syncthreads();
-  const uint64_t ml = as_const(P.md_red)[2 * level + 1];
-  uint64_t acc = 0;
-  // four partial sums below ml each: their sum stays below 2^64 and below ml
-  // once reduced by the multiples of pl that ml allows
-#pragma unroll
-  for (int t = 0; t < BC_GROUPS; ++t) acc = add_mod(acc, part[t * BC_COEF + c], ml);
-  const uint64_t top = finish(level, acc);
-  // out_i = ((x_i - acc_i) B^-1 + add_i - top) q_l^-1
-  //       = (x_i - acc_i + z_i B) (B^-1 q_l^-1),  z_i = q_i + add_i - top  (mod q_i)
-  // with top < q_l < q_i (the Q primes decrease): 0 < z_i < 2 q_i.  The
-  // narrow limbs add the term z_i (-B) to their sums and take one Shoup
-  // product; q0 (summed by moddown_wide) multiplies both parts.
-  const tw2* iql = reinterpret_cast<const tw2*>(P.inv_ql_mod_qi) + (size_t)level * k;
-  const tw2* fin = reinterpret_cast<const tw2*>(P.md_fin) + (size_t)level * k;
-  auto zval = [&](int i) { return ld_prime_p(P.primes, i) + (add ? add[(size_t)i * N + cid] : 0) - top; };
+  if (wide0) __syncthreads();
+  // add_i joins the sums as z = add_i: (x_i - acc + add_i B) B^-1 = (x_i - acc) B^-1 + add_i
   limbs(
-      level,
-      [&](int i, uint64_t acc) {
-        const uint64_t p = ld_prime_p(P.primes, i);
-        const tw2 f = ld_tw2(fin, i), sq = ld_tw2(iql, i);
-        out[(size_t)i * N + cid] = add_mod(mul_shoup(lift(i, acc), f.w, f.q, p), mul_shoup(zval(i), sq.w, sq.q, p), p);
-      },
+      level + 1, [&](int i, uint64_t acc) { out[(size_t)i * N + cid] = finish(i, acc); },
       [&](int i, uint64_t* z) {
-        *z = zval(i);
+        if (!add) return false;
+        *z = add[(size_t)i * N + cid];
         return true;
       },
       [&](int i, uint64_t acc) {
-        const tw2 f = ld_tw2(fin, i);
-        out[(size_t)i * N + cid] = mul_shoup(lift(i, acc), f.w, f.q, ld_prime_p(P.primes, i));
+        const tw2 bi = ld_tw2(ibq, i);
+        out[(size_t)i * N + cid] = mul_shoup(lift(i, acc), bi.w, bi.q, ld_prime_p(P.primes, i));
       });
 }
 
-// Eight waves per SIMD, as k_moddown_d: 2.5 % more plain HomMuls per second.
+// Eight waves per SIMD hide the product loop's table loads: 4 % faster than seven.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_moddown(DevParams P, ModDownArgs A) {
-  extern __shared__ uint64_t aux[];  // [K][64], then [4][64] partial sums of the top limb and of q0
+  extern __shared__ uint64_t aux[];  // [K][64], then [4][64] partial sums of q0
   const int y = blockIdx.y;
-  moddown_body(P, A.inQ[y], A.inB[y], A.add[y], A.out[y], A.level, A.rescale, 0, blockIdx.x, aux);
+  moddown_body(P, A.inQ[y], A.inB[y], A.add[y], A.out[y], A.level, blockIdx.x, aux);
 }
 
 void launch_moddown(const DevParams& P, const ModDownArgs& a, hipStream_t st) {
-  const size_t lds = (size_t)(P.K + 2 * BC_GROUPS) * BC_COEF * sizeof(uint64_t);
+  const size_t lds = (size_t)(P.K + BC_GROUPS) * BC_COEF * sizeof(uint64_t);
   k_moddown<<<dim3(P.N / BC_COEF, a.npolys), 256, lds, st>>>(P, a);
-}
-
-// Eight waves per SIMD (58 registers): the batched grid is many times the
-// machine, and more waves hide the product loop's table loads; 4 % faster
-// than seven waves (70 registers) and than five (81, the default).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_moddown_d(DevParams P, const ModDownDesc* dd,
-                                                                                           int bscaled) {
-  extern __shared__ uint64_t aux[];
-  const int per = P.N / BC_COEF;
-  const ModDownDesc m = dd[blockIdx.x / per];
-  // generic (flat) accesses here: the global form ran 1 % slower (more
-  // scalar registers held for the bases, which this kernel already spills)
-  moddown_body(P, m.inQ, m.inB, m.add, m.out, m.level, m.rescale, bscaled, blockIdx.x % per, aux);
-}
-
-void launch_moddown_desc(const DevParams& P, const ModDownDesc* d, int ndesc, bool bscaled, hipStream_t st) {
-  const size_t lds = (size_t)(P.K + 2 * BC_GROUPS) * BC_COEF * sizeof(uint64_t);
-  k_moddown_d<<<dim3((unsigned)(ndesc * (P.N / BC_COEF))), 256, lds, st>>>(P, d, bscaled ? 1 : 0);
 }
 
 // -------------------------------------------------------------- checksum ----

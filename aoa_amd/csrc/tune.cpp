@@ -59,29 +59,32 @@ extern "C" int aoa_autotune_ntt(aoa_params* h, void* stream, int nlimbs, int rep
   (void)hipEventCreate(&e1);
   int best = 0, count = 0;
   double best_us = 1e30;
-  for (int n1 : {64, 128, 256, h->host.N}) {
-    if (!ntt_valid_split(h->host.N, n1)) continue;
+  // the splits, and the default (0), which is kept where none beats it
+  for (int n1 : {64, 128, 256, h->host.N, 0}) {
+    if (n1 && !ntt_valid_split(h->host.N, n1)) continue;
     DevParams P = h->dev;
     P.ntt_n1 = n1;
     for (int w = 0; w < 2; ++w) {
       ntt_forward(P, m, n1, st);
-      ntt_inverse(P, m, n1, nullptr, nullptr, st);
+      ntt_inverse(P, m, n1, st);
     }
     (void)hipEventRecord(e0, st);
     for (int r = 0; r < reps; ++r) {
       ntt_forward(P, m, n1, st);
-      ntt_inverse(P, m, n1, nullptr, nullptr, st);
+      ntt_inverse(P, m, n1, st);
     }
     (void)hipEventRecord(e1, st);
     (void)hipEventSynchronize(e1);
     float ms = 0;
     (void)hipEventElapsedTime(&ms, e0, e1);
     const double us = 1000.0 * ms / reps;
-    if (count < max && out_n1 && out_us) {
-      out_n1[count] = n1;
-      out_us[count] = us;
+    if (n1) {
+      if (count < max && out_n1 && out_us) {
+        out_n1[count] = n1;
+        out_us[count] = us;
+      }
+      ++count;
     }
-    ++count;
     if (us < best_us) {
       best_us = us;
       best = n1;

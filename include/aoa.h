@@ -284,7 +284,8 @@ int aoa_rotate_right(const aoa_params* params, void* stream, uint64_t* out0, uin
 
 /* ---------------------------------------------------------------- tuning --
  * NTT split N = N1 x (N/N1) of a parameter set (N1 in {64, 128, 256}, N/N1 in
- * the same set).  No counterpart in the reference, whose split is fixed per N
+ * the same set, or N1 = N <= 4096) for its plain transforms; 0: the default,
+ * which shares its form (16 x N/16) with the key switching kernels.  No counterpart in the reference, whose split is fixed per N
  * at compile time (aoa-ntt/include/newckks/cuda/htrans/ntt.h:24-44; every
  * split gives the same residues).  Set before issuing work with the handle. */
 int aoa_params_set_ntt_split(aoa_params* params, int n1);
@@ -302,8 +303,9 @@ int aoa_params_set_moddown_exact(aoa_params* params, int exact);
 int aoa_params_get_moddown_exact(const aoa_params* params);
 
 /* Autotuner: times forward+inverse NTTs of `nlimbs` limbs for every valid
- * split (reps repetitions each, on the given stream, allocating a scratch
- * buffer), stores the fastest split in the handle and writes up to `max`
+ * split and for the default transforms (reps repetitions each, on the given
+ * stream, allocating a scratch buffer), stores the fastest split in the handle,
+ * or none where the default is faster, and writes the splits' up to `max`
  * (n1, microseconds) pairs to out_n1/out_us.  Returns the number of
  * candidates, or a negative status. */
 int aoa_autotune_ntt(aoa_params* params, void* stream, int nlimbs, int reps, int* out_n1, double* out_us, int max);
@@ -366,7 +368,7 @@ void aoa_batch_destroy(aoa_batch* batch);
  * factorisation is a fixed table, aoa-ntt/include/newckks/cuda/htrans/ntt.h:13-44).
  * Every choice gives the same residues; aoa_batch_autotune times them. */
 typedef struct {
-  int ntt_split;    /* N1 of the two-pass NTT for the groups whose ring admits it (0: the handle's split) */
+  int ntt_split;    /* N1 of the plain transforms for the groups whose ring admits it (0: as the handle) */
   int prime_major;  /* 1: the descriptors of a stage sorted by prime (default); 0: item after item */
   int xcd_chunks;   /* 1: the NTT passes deal their tiles out to the 8 XCDs in contiguous chunks */
   int strict_split; /* limbs of the 63-bit q0 in a launch of their own: -1 never, 0 from 256
@@ -402,13 +404,13 @@ int aoa_batch_autotune(aoa_batch* batch, void* stream, int reps, aoa_tune_result
 enum {
   AOA_STAGE_PRE_FWD = 0,      /* forward NTT of inputs given in the coefficient domain */
   AOA_STAGE_PRE_INV = 1,      /* inverse NTT of inputs given in the NTT domain */
-  AOA_STAGE_TENSOR = 2,       /* d0, d1, d2 of HomMul (N <= 4096; from N = 8192 up inside AOA_STAGE_INTT) */
+  AOA_STAGE_TENSOR = 2,       /* unused: HomMul's products are formed in stages 4 and 7 */
   AOA_STAGE_AUTOMORPHISM = 3, /* rotation's Galois map */
-  AOA_STAGE_INTT = 4,         /* inverse NTT of d0, d1, d2 (from N = 8192 up: of d2 only, with the tensor product) */
-  AOA_STAGE_MODUP = 5,
-  AOA_STAGE_NTT = 6,          /* forward NTT of the ModUp output */
-  AOA_STAGE_KEY_INTT = 7,     /* key product fused into the inverse NTT */
-  AOA_STAGE_MODDOWN = 8,      /* ModDown (+ rescale, + the additions of rotations and of HomMul below N = 8192) */
+  AOA_STAGE_INTT = 4,         /* HomMul's d2 and the rows of its inverse NTT */
+  AOA_STAGE_MODUP = 5,        /* the columns of that, ModUp, the forward columns of its output */
+  AOA_STAGE_NTT = 6,          /* special limbs: forward rows, both key products, inverse rows */
+  AOA_STAGE_KEY_INTT = 7,     /* Q limbs: the same, for HomMul from the operands with d0 and d1 added */
+  AOA_STAGE_MODDOWN = 8,      /* inverse columns, ModDown (+ rescale, + the additions of rotations) */
   AOA_NSTAGES = 9
 };
 
