@@ -231,8 +231,9 @@ size_t batch_fill(aoa_batch* b, uint64_t* ws, char* host, char* dev, size_t desc
       // The limbs of primes wider than 2^56 (q0), which sort first, take another
       // form of arithmetic; with them in a launch of their own the others'
       // launch compiles for its form alone and holds fewer registers.  Small
-      // stages (a serving step of a few requests) keep one launch by default:
-      // the split pays only where a launch fills the GPU.
+      // stages (a serving step of a few requests) keep one launch by default: 60
+      // entries at N = 2^16 0.356 ms in one launch, 0.383 in two; 960 entries
+      // 4.32 and 4.31.
       constexpr size_t kSplitMin = 256;
       auto split_at = [&](const std::vector<uint32_t>& v) -> int {
         if (b->opt.strict_split < 0 || !pm) return -1;

@@ -5,6 +5,9 @@
 namespace aoa {
 
 // ------------------------------------------------------ d2 = a b, its rows --
+// Memory bound: two operands in, one out.  960 limbs at N = 2^16: 325 us, 4.9
+// TB/s of counter traffic (a tensor pass and the inverse pass of d2 before: 370
+// and more traffic).
 template <class F, int LOGM>
 __device__ __forceinline__ void rows_body(const DevParams& P, const uint64_t* a, const uint64_t* b, uint64_t* dst, int pr,
                                           int tile, uint64_t* lds) {
@@ -119,6 +122,11 @@ __device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, i
   }
 }
 
+// Special limbs at N = 2^16 (992 of 55 bits): 840 us, 0.90 vector instructions a
+// busy CU and cycle: issue bound.  Q limbs (928 of 48 bits): 795 us, 3.7 TB/s, 53
+// for the 32 of q0.  (The split form's row pass took 1.6 ms for all of them and its
+// columns 1.0, now in k_fz_down.)
+//
 // ysplit: one workgroup per key half (the two halves of a tile `n` blocks
 // apart).  SPECIAL: every limb is a special one.
 template <int LOGM, bool ARG, int FIELD, bool SPECIAL>
@@ -155,7 +163,9 @@ static int fz_rows(const DevParams& P, const FzItem& arg, const FzItem* items, c
 }
 
 // One workgroup per key half while both halves together leave the chip
-// partly idle: the forward rows are then done twice, on idle units.
+// partly idle: the forward rows are then done twice, on idle units.  With and
+// without: 7.3 and 10.3 us (N = 2^13, 288 waves), 10.2 and 12.7 (N = 2^14, 1088),
+// 24.6 and 21.2 (N = 2^15, 3584), 90 and 74 (N = 2^16, 7808).
 template <bool ARG, int FIELD, bool SPECIAL>
 static int fz_key(const DevParams& P, const FzItem& arg, const FzItem* items, const uint32_t* list, int n, hipStream_t st) {
   if (n <= 0) return 0;

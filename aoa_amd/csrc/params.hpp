@@ -32,7 +32,7 @@ struct DevPrime {
   uint64_t r64_q;    // its Shoup quotient
   // ModDown cross-base products a*c (a < max special prime, c < p): the
   // reference's Barrett result equals the exact remainder r unless
-  // quirk_lo <= r < quirk_thr (see k_moddown); quirk_lo = eps and
+  // quirk_lo <= r < quirk_thr (see ref_barrett); quirk_lo = eps and
   // quirk_thr = delta_max * eps, or [0, 2^64) when that bound is not usable.
   uint64_t quirk_lo;
   uint64_t quirk_thr;

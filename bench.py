@@ -31,20 +31,18 @@ sys.path.insert(0, ROOT)
 
 N, K_Q, K_B, PREC = 65536, 30, 31, 48
 HBM_PEAK_GBS = 8000.0
-# HBM bytes per k_moddown_d launch at 32 pairs, from two rocprofv3 --pmc runs of
-# `bench.py --profile` (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0; the factors make a
-# 1 GiB device copy read 1 GiB and write 1 GiB); the run is summarised in
-# profiles/moddown_pmc_traffic_n16_k30.md.
-MODDOWN_TRAFFIC_BYTES = {32: 3025902773}
-# VALU wave-instructions per k_moddown_d launch at 32 pairs (SQ_INSTS_VALU summed
-# over the counter instances of one dispatch, rocprofv3 --pmc of
-# `bench.py --profile`; profiles/hommul_batched_n16_k30_valu.md), and a
+# HBM bytes per k_fz_down launch at 32 pairs, from two rocprofv3 --pmc runs
+# (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0; the factors make a 1 GiB device copy
+# read 1 GiB and write 1 GiB); profiles/hommul_batched_n16_k30_counters.md.
+MODDOWN_TRAFFIC_BYTES = {32: 3039468749}
+# VALU wave-instructions per k_fz_down launch at 32 pairs (SQ_INSTS_VALU summed
+# over the counter instances of one dispatch, same file), and a
 # reference issue rate: MI355X's vector FP64 FMA peak (78.6 TFLOP/s = 2 flops x
 # 64 lanes x 256 CUs x 2.4 GHz) counted in wave instructions, one per CU per
 # cycle.  64-bit integer multiply-adds issue at about this rate; 32-bit adds
 # and logic issue faster (about 1.6 times), so the fraction is a proxy that a
 # mix of both can exceed.
-MODDOWN_VALU_INSTS = {32: 9.186e8}
+MODDOWN_VALU_INSTS = {32: 6.978e8}
 VALU_PEAK_INSTS_S = 256 * 2.4e9
 
 
@@ -658,7 +656,7 @@ def main():
         "wall_s": round(wall, 3),
         "roofline": {"bound": "hbm", "achieved": round(md_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(md_gbs / HBM_PEAK_GBS, 4), "traffic": MODDOWN_TRAFFIC_BYTES.get(B),
-                     "kernel": "aoa::k_moddown_d (ModDown + rescale, %d items x 2 polys)" % B,
+                     "kernel": "aoa::k_fz_down (inverse columns + ModDown + rescale, %d items x 2 polys)" % B,
                      "launch_ms": round(md_launch_ms, 4), "algorithmic_bytes": md_bytes,
                      "limiter": "valu",
                      "valu": valu_issue(MODDOWN_VALU_INSTS.get(B), md_launch_ms)},
