@@ -76,7 +76,54 @@ __device__ __forceinline__ uint64_t csub(uint64_t x, uint64_t p) {
   return b1 ? x : ((uint64_t)h << 32) | l;
 }
 
+// Words of caller data.  The forms below take values of up to the prime's nb
+// bits; aoa_eltwise_scalar leaves wider ones, since it uses its scalar as given.
+struct Words {
+  uint32_t hi = 0;
+  __device__ __forceinline__ uint64_t operator()(uint64_t x) {
+    hi |= (uint32_t)(x >> 32);
+    return x;
+  }
+};
+// Canonical residues of such words, one from 2^63 up read as that minus 2^64 (a
+// constant above the prime subtracted from a smaller residue).
+struct Residues {
+  uint64_t p, wq;  // floor(2^64 / p)
+  __device__ __forceinline__ explicit Residues(const DevPrime& d) : p(d.p), wq(d.mu >> (2 * (int)d.nb - 64)) {}
+  __device__ __forceinline__ uint64_t operator()(uint64_t x) const {
+    const bool neg = x >> 63;
+    const uint64_t r = mul_shoup(neg ? 0 - x : x, 1, wq, p);
+    return neg ? neg_mod(r, p) : r;
+  }
+};
+
+// form(w, k, set) for each of a thread's V values, which reads caller data of
+// prime pr through w and keeps what it makes of it by set(array, value): with
+// Words and, where one of the wave was too wide, again with Residues.  That rare
+// loop stays rolled and its results are selected into place: unrolled, its
+// registers cost the key products of 928 limbs of 48 bits at N = 2^16 754 us
+// instead of 682.  U: pr is the same for the whole wave.
+template <int V, bool U = true, class F, class Form>
+__device__ __forceinline__ void with_caller_words(const F& f, const DevPrime* primes, int pr, Form&& form) {
+  Words w;
+#pragma unroll
+  for (int k = 0; k < V; ++k) form(w, k, [&](auto& x, auto v) { x[k] = v; });
+  if constexpr (!F::kAnyWord) {
+    if (__builtin_amdgcn_ballot_w64(w.hi >> (f.bits() - 32) != 0)) {
+      const Residues r(U ? ld_prime(primes, pr) : primes[pr]);
+#pragma unroll 1
+      for (int k = 0; k < V; ++k) {
+        form(r, k, [&](auto& x, auto v) {
+#pragma unroll
+          for (int c = 0; c < V; ++c) x[c] = c == k ? v : x[c];
+        });
+      }
+    }
+  }
+}
+
 struct FieldLazy {
+  static constexpr bool kAnyWord = false;
   using V = uint64_t;
   struct W {
     uint64_t w, q;
@@ -86,6 +133,7 @@ struct FieldLazy {
   int nb;
   __device__ __forceinline__ explicit FieldLazy(const DevPrime& d)
       : p(d.p), np(0 - d.p), mu2(d.mu2), mu32((uint32_t)(d.mu >> (2 * (int)d.nb - 64))), nb((int)d.nb) {}
+  __device__ __forceinline__ int bits() const { return nb; }
   // canonical residue in; raw / raw_in: the 64-bit pattern between two kernels of one path
   __device__ __forceinline__ V in(uint64_t x) const { return x; }
   __device__ __forceinline__ V raw_in(uint64_t x) const { return x; }
@@ -146,10 +194,12 @@ struct FieldLazy {
 };
 
 struct FieldFp64 {
+  static constexpr bool kAnyWord = false;
   using V = double;
   using W = double;
   double p, pinv;
   __device__ __forceinline__ explicit FieldFp64(const DevPrime& d) : p(d.fp), pinv(d.fpinv) {}
+  __device__ __forceinline__ int bits() const { return __builtin_amdgcn_frexp_exp(p); }
   __device__ __forceinline__ V in(uint64_t x) const {  // x < 2^52
     return __longlong_as_double((long long)(x | 0x4330000000000000ull)) - 4503599627370496.0;
   }
@@ -216,6 +266,7 @@ struct FieldFp64 {
 // Of a small call's limbs this one ends last: a butterfly is 33 vector
 // instructions (a Shoup product and canonical sums: about 45).
 struct FieldStrict {
+  static constexpr bool kAnyWord = true;
   using V = uint64_t;
   using W = uint64_t;
   uint64_t p;

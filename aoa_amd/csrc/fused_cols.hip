@@ -126,12 +126,11 @@ __device__ __forceinline__ void up_in(const DevParams& P, const FzItem& it, int 
     const uint64_t* T = P.fz.tw[0] + (size_t)i * P.N * 2;
     const tw2 w = reinterpret_cast<const tw2*>(P.inv_qhat)[(size_t)it.level * P.k + i];
     uint64_t v[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint64_t u = src[(size_t)(q + 4 * k) * M];
-      v[k] = mul_shoup(u, w.w, w.q, dp.p);
-      x[k] = f.in(u);
-    }
+    with_caller_words<4, false>(f, P.primes, i, [&](auto& words, int k, auto set) {
+      const uint64_t u = words(src[(size_t)(q + 4 * k) * M]);
+      set(v, mul_shoup(u, w.w, w.q, dp.p));
+      set(x, f.in(u));
+    });
     col_fwd_a(f, x, T);
     col_turn<false>(f, x, t, q);
     wave_order();

@@ -32,10 +32,14 @@ template <class F, bool INV>
 __device__ __forceinline__ void nt_cols(const DevParams& P, const uint64_t* src, uint64_t* dst, int pr, int q, int c,
                                         uint64_t* lds) {
   const int M = P.N / 16;
-  uint64_t u[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) u[k] = src[(size_t)(INV ? 4 * q + k : q + 4 * k) * M];
   const F f(ld_prime(P.primes, pr));
+  uint64_t u[4];
+  if constexpr (INV) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) u[k] = src[(size_t)(4 * q + k) * M];
+  } else {
+    with_caller_words<4>(f, P.primes, pr, [&](auto& w, int k, auto set) { set(u, w(src[(size_t)(q + 4 * k) * M])); });
+  }
   const uint64_t* T = P.fz.tw[INV ? 1 : 0] + (size_t)pr * P.N * 2;
   uint64_t* t = lds + c;
   typename F::V x[4];
@@ -84,10 +88,16 @@ __device__ __forceinline__ void nt_rows(const DevParams& P, const uint64_t* src,
   using G = RowOf<LOGM>;
   constexpr int LV = kLogV<LOGM>;
   const RowId<LOGM> id(tile, lds);
-  uint64_t u[G::V];
-#pragma unroll
-  for (int k = 0; k < G::V; ++k) u[k] = at_byte<uint64_t>(src, id.off + G::TS * 8 * k);
   const F f(ld_prime(P.primes, pr));
+  uint64_t u[G::V];
+  if constexpr (INV) {
+    with_caller_words<G::V>(f, P.primes, pr, [&](auto& w, int k, auto set) {
+      set(u, w(at_byte<uint64_t>(src, id.off + G::TS * 8 * k)));
+    });
+  } else {
+#pragma unroll
+    for (int k = 0; k < G::V; ++k) u[k] = at_byte<uint64_t>(src, id.off + G::TS * 8 * k);
+  }
   const uint64_t* T = P.fz.tw[INV ? 1 : 0] + (size_t)pr * P.N * 2;
   typename F::V x[G::V];
 #pragma unroll
@@ -135,10 +145,13 @@ __device__ __forceinline__ void nt_decrypt(const DevParams& P, uint64_t* c0, uin
   }
   rows_fwd_all<F, LOGM>(f, z, u, T, id);
 #pragma unroll
-  for (int k = 0; k < G::V; ++k) {
-    put_byte(c1, id.off + G::TS * 8 * k, u[k]);
-    z[k] = f.key(f.in(u[k]), at_byte<uint64_t>(s, id.off + G::TS * 8 * k));
-  }
+  for (int k = 0; k < G::V; ++k) put_byte(c1, id.off + G::TS * 8 * k, u[k]);
+  uint64_t v[G::V];
+  with_caller_words<G::V>(f, P.primes, pr, [&](auto& w, int k, auto set) {
+    set(v, w(at_byte<uint64_t>(s, id.off + G::TS * 8 * k)));
+  });
+#pragma unroll
+  for (int k = 0; k < G::V; ++k) z[k] = f.key(f.in(u[k]), v[k]);
   rows_fwd_all<F, LOGM>(f, x, u, T + opaque_zero(), id);
 #pragma unroll
   for (int k = 0; k < G::V; ++k) {
@@ -182,8 +195,12 @@ __device__ __forceinline__ void nt_encrypt(const DevParams& P, const NtEncrypt& 
     for (int k = 0; k < G::V; ++k) z[k] = f.raw_in(at_byte<uint64_t>(a.u + o, id.off + G::TS * 8 * k));
     rows_fwd_all<F, LOGM>(f, z, u, T, id);
     const uint64_t* pk = (y == 0 ? a.pkb : a.pka) + o;
+    uint64_t v[G::V];
+    with_caller_words<G::V>(f, P.primes, i, [&](auto& w, int k, auto set) {
+      set(v, w(at_byte<uint64_t>(pk, id.off + G::TS * 8 * k)));
+    });
 #pragma unroll
-    for (int k = 0; k < G::V; ++k) z[k] = f.key(f.in(u[k]), at_byte<uint64_t>(pk, id.off + G::TS * 8 * k));
+    for (int k = 0; k < G::V; ++k) z[k] = f.key(f.in(u[k]), v[k]);
   }
   rows_fwd_all<F, LOGM>(f, x, u, T + opaque_zero(), id);
   uint64_t* out = (y == 0 ? a.c0 : y == 1 ? a.c1 : a.m) + o;

@@ -1,5 +1,7 @@
 // Row kernels of the fused key switching (fused.hpp): the forward and inverse
 // row stages with the products between them.
+#include <type_traits>
+
 #include "fused.hpp"
 
 namespace aoa {
@@ -17,11 +19,10 @@ __device__ __forceinline__ void rows_body(const DevParams& P, const uint64_t* a,
   const uint64_t* T = P.fz.tw[1] + (size_t)pr * P.N * 2;
   const RowId<LOGM> id(tile, lds);
   typename F::V x[G::V];
-#pragma unroll
-  for (int k = 0; k < G::V; ++k) {
+  with_caller_words<G::V>(f, P.primes, pr, [&](auto& w, int k, auto set) {
     const uint32_t o = id.off + G::TS * 8 * k;
-    x[k] = f.key(f.in(at_byte<uint64_t>(a, o)), at_byte<uint64_t>(b, o));
-  }
+    set(x, f.key(f.in(w(at_byte<uint64_t>(a, o))), w(at_byte<uint64_t>(b, o))));
+  });
   row_turn<LOGM, LV, 0, G::ROUNDS - 1>(f, x, id.s, id.L);
   rows_out<F, LOGM>(f, x, T, dst, id);
 }
@@ -64,15 +65,24 @@ __device__ __forceinline__ void key_body_tensor(const DevParams& P, const FzItem
   // both halves' products from one reading of the operands; the second waits
   // in registers while the first is transformed
   typename F::V x[G::V], x1[G::V];
-#pragma unroll
-  for (int k = 0; k < G::V; ++k) {
-    const uint32_t i = id.off + G::TS * 8 * k;
-    const uint64_t va0 = at_byte<uint64_t>(a0, i), va1 = at_byte<uint64_t>(a1, i);
-    const uint64_t vb0 = at_byte<uint64_t>(b0, i), vb1 = at_byte<uint64_t>(b1, i);
-    const auto d2 = f.d2(va1, vb1);
-    if (y0 == 0) x[k] = f.relin(d2, at_byte<uint64_t>(kb, i), f.d0(va0, vb0), bq);
-    if (y1 == 2) x1[k] = f.relin(d2, at_byte<uint64_t>(ka, i), f.d1(va0, va1, vb0, vb1), bq);
-  }
+  auto form = [&](auto first, auto second) {
+    with_caller_words<G::V>(f, P.primes, m, [&](auto& w, int k, auto set) {
+      const uint32_t i = id.off + G::TS * 8 * k;
+      const uint64_t va0 = w(at_byte<uint64_t>(a0, i)), va1 = w(at_byte<uint64_t>(a1, i));
+      const uint64_t vb0 = w(at_byte<uint64_t>(b0, i)), vb1 = w(at_byte<uint64_t>(b1, i));
+      const auto d2 = f.d2(va1, vb1);
+      if (first) set(x, f.relin(d2, at_byte<uint64_t>(kb, i), f.d0(va0, vb0), bq));
+      if (second) set(x1, f.relin(d2, at_byte<uint64_t>(ka, i), f.d1(va0, va1, vb0, vb1), bq));
+    });
+  };
+  // Which halves, decided once: with a branch per value the loads went out a
+  // value at a time (928 limbs of 48 bits at N = 2^16 796 us, now 682).
+  if (y1 - y0 == 2)
+    form(std::true_type(), std::true_type());
+  else if (y0 == 0)
+    form(std::true_type(), std::false_type());
+  else
+    form(std::false_type(), std::true_type());
 #pragma unroll 1
   for (int y = y0; y < y1; ++y) {
     if (y) {
@@ -123,7 +133,7 @@ __device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, i
 }
 
 // Special limbs at N = 2^16 (992 of 55 bits): 840 us, 0.90 vector instructions a
-// busy CU and cycle: issue bound.  Q limbs (928 of 48 bits): 795 us, 3.7 TB/s, 53
+// busy CU and cycle: issue bound.  Q limbs (928 of 48 bits): 682 us, 4.3 TB/s, 53
 // for the 32 of q0.  (The split form's row pass took 1.6 ms for all of them and its
 // columns 1.0, now in k_fz_down.)
 //

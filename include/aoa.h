@@ -93,7 +93,15 @@ int aoa_eltwise(const aoa_params* params, void* stream, int op, uint64_t* out, c
  * correction for add/sub, its Barrett reduction for mul).  Replaces
  * NTTEngine::execute_op_by_uint (aoa-ntt/src/cuda/htrans/ntt.cu:531-580), the
  * kernel under poly_add / poly_sub / poly_mul by a uint64_t
- * (aoa-ntt/src/arithmetic/poly_t.cpp:157-235). */
+ * (aoa-ntt/src/arithmetic/poly_t.cpp:157-235).
+ *
+ * Its results may thus lie outside [0, q_r).  aoa_ntt, aoa_encrypt, aoa_decrypt,
+ * the products, aoa_keyswitch's d and the batches take such residues: a word
+ * stands for its value mod q_r, one from 2^63 up for that minus 2^64 (q0's words
+ * below 2^63), and their results are those of the reduced residues.  With an
+ * explicit split (aoa_params_set_ntt_split) transforms, encryption and decryption
+ * are exact for words below 2 q_r; what a rotation or add0 adds is added with one
+ * correction; switching keys are canonical. */
 int aoa_eltwise_scalar(const aoa_params* params, void* stream, int op, uint64_t* out, const uint64_t* a, uint64_t b,
                        int res0, int nres);
 
