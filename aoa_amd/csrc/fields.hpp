@@ -102,12 +102,15 @@ struct Residues {
 // Words and, where one of the wave was too wide, again with Residues.  That rare
 // loop stays rolled and its results are selected into place: unrolled, its
 // registers cost the key products of 928 limbs of 48 bits at N = 2^16 754 us
-// instead of 682.  U: pr is the same for the whole wave.
-template <int V, bool U = true, class F, class Form>
-__device__ __forceinline__ void with_caller_words(const F& f, const DevPrime* primes, int pr, Form&& form) {
+// instead of 682.  then() follows either way, the first time before the test, so
+// that what it loads is requested with the words.  U: pr is the same for the whole
+// wave.
+template <int V, bool U = true, class F, class Form, class Then>
+__device__ __forceinline__ void with_caller_words(const F& f, const DevPrime* primes, int pr, Form&& form, Then&& then) {
   Words w;
 #pragma unroll
   for (int k = 0; k < V; ++k) form(w, k, [&](auto& x, auto v) { x[k] = v; });
+  then();
   if constexpr (!F::kAnyWord) {
     if (__builtin_amdgcn_ballot_w64(w.hi >> (f.bits() - 32) != 0)) {
       const Residues r(U ? ld_prime(primes, pr) : primes[pr]);
@@ -118,8 +121,13 @@ __device__ __forceinline__ void with_caller_words(const F& f, const DevPrime* pr
           for (int c = 0; c < V; ++c) x[c] = c == k ? v : x[c];
         });
       }
+      then();
     }
   }
+}
+template <int V, bool U = true, class F, class Form>
+__device__ __forceinline__ void with_caller_words(const F& f, const DevPrime* primes, int pr, Form&& form) {
+  with_caller_words<V, U>(f, primes, pr, form, [] {});
 }
 
 struct FieldLazy {

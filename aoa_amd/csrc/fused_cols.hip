@@ -130,8 +130,7 @@ __device__ __forceinline__ void up_in(const DevParams& P, const FzItem& it, int 
       const uint64_t u = words(src[(size_t)(q + 4 * k) * M]);
       set(v, mul_shoup(u, w.w, w.q, dp.p));
       set(x, f.in(u));
-    });
-    col_fwd_a(f, x, T);
+    }, [&] { col_fwd_a(f, x, T); });
     col_turn<false>(f, x, t, q);
     wave_order();
 #pragma unroll

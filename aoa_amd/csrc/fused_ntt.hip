@@ -33,22 +33,18 @@ __device__ __forceinline__ void nt_cols(const DevParams& P, const uint64_t* src,
                                         uint64_t* lds) {
   const int M = P.N / 16;
   const F f(ld_prime(P.primes, pr));
-  uint64_t u[4];
-  if constexpr (INV) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) u[k] = src[(size_t)(4 * q + k) * M];
-  } else {
-    with_caller_words<4>(f, P.primes, pr, [&](auto& w, int k, auto set) { set(u, w(src[(size_t)(q + 4 * k) * M])); });
-  }
   const uint64_t* T = P.fz.tw[INV ? 1 : 0] + (size_t)pr * P.N * 2;
   uint64_t* t = lds + c;
   typename F::V x[4];
+  if constexpr (INV) {
 #pragma unroll
-  for (int k = 0; k < 4; ++k) x[k] = INV ? f.raw_in(u[k]) : f.in(u[k]);
-  if constexpr (INV)
+    for (int k = 0; k < 4; ++k) x[k] = f.raw_in(src[(size_t)(4 * q + k) * M]);
     col_inv_b<true>(f, x, T, q);
-  else
-    col_fwd_a<true>(f, x, T);
+  } else {
+    with_caller_words<4>(
+        f, P.primes, pr, [&](auto& w, int k, auto set) { set(x, f.in(w(src[(size_t)(q + 4 * k) * M]))); },
+        [&] { col_fwd_a<true>(f, x, T); });
+  }
 #pragma unroll
   for (int k = 0; k < 4; ++k) t[(INV ? 4 * q + k : q + 4 * k) * NT_COLS] = f.raw(x[k]);
   __syncthreads();

@@ -48,10 +48,13 @@ __global__ __launch_bounds__(RowOf<LOGM>::THREADS) void k_fz_rows(DevParams P, F
 // Limb m of an item: Q limbs 0..level, then the special limbs.  HomMul's Q
 // limbs take their NTT-domain input d2 and addends d0, d1 from the operands;
 // other limbs come as forward columns and take the forward rows here, once for
-// both key halves.  y0..y1: the key halves of this workgroup.
+// both key halves.  BOTH: this
+// workgroup forms both key halves, otherwise half y0; a kernel each, since with
+// the choice at run time the halves' code and registers added up (hommul at
+// N = 2^16, k = 30: 199 us, now 190).
 
-template <class F, int LOGM>
-__device__ __forceinline__ void key_body_tensor(const DevParams& P, const FzItem& it, int m, int tile, int y0, int y1,
+template <class F, int LOGM, bool BOTH>
+__device__ __forceinline__ void key_body_tensor(const DevParams& P, const FzItem& it, int m, int tile, int y0,
                                                 uint64_t* lds) {
   using G = RowOf<LOGM>;
   constexpr int LV = kLogV<LOGM>;
@@ -77,14 +80,14 @@ __device__ __forceinline__ void key_body_tensor(const DevParams& P, const FzItem
   };
   // Which halves, decided once: with a branch per value the loads went out a
   // value at a time (928 limbs of 48 bits at N = 2^16 796 us, now 682).
-  if (y1 - y0 == 2)
+  if constexpr (BOTH)
     form(std::true_type(), std::true_type());
   else if (y0 == 0)
     form(std::true_type(), std::false_type());
   else
     form(std::false_type(), std::true_type());
 #pragma unroll 1
-  for (int y = y0; y < y1; ++y) {
+  for (int y = BOTH ? 0 : y0; y < (BOTH ? 2 : y0 + 1); ++y) {
     if (y) {
 #pragma unroll
       for (int k = 0; k < G::V; ++k) x[k] = x1[k];
@@ -99,8 +102,8 @@ struct KeyPair {
   uint64_t a, b;
 };
 
-template <class F, int LOGM>
-__device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, int m, int pr, int tile, int y0, int y1,
+template <class F, int LOGM, bool BOTH>
+__device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, int m, int pr, int tile, int y0,
                                          uint64_t* lds) {
   using G = RowOf<LOGM>;
   constexpr int LV = kLogV<LOGM>;
@@ -116,7 +119,7 @@ __device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, i
 #pragma unroll
   for (int k = 0; k < G::V; ++k) x0[k] = f.factor(x0[k]);
 #pragma unroll 1
-  for (int y = y0; y < y1; ++y) {
+  for (int y = BOTH ? 0 : y0; y < (BOTH ? 2 : y0 + 1); ++y) {
     const uint32_t z = opaque_zero();
     // packed, as the inverse rows begin: a thread's values are 16-byte loads
     const uint64_t* kp = glob(y ? it.ka : it.kb) + (size_t)pr * N;
@@ -127,7 +130,7 @@ __device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, i
       x[k] = f.key(x0[k], v.a);
       x[k + 1] = f.key(x0[k + 1], v.b);
     }
-    if (y > y0) __syncthreads();  // the first half's last exchange has been read
+    if (BOTH && y) __syncthreads();  // the first half's last exchange has been read
     rows_out<F, LOGM>(f, x, T + z, glob(y ? it.P1 : it.P0) + (size_t)m * N, id);
   }
 }
@@ -137,25 +140,24 @@ __device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, i
 // for the 32 of q0.  (The split form's row pass took 1.6 ms for all of them and its
 // columns 1.0, now in k_fz_down.)
 //
-// ysplit: one workgroup per key half (the two halves of a tile `n` blocks
-// apart).  SPECIAL: every limb is a special one.
-template <int LOGM, bool ARG, int FIELD, bool SPECIAL>
+// !BOTH: one workgroup per key half (the two halves of a tile `n` blocks apart).
+// SPECIAL: every limb is a special one.
+template <int LOGM, bool ARG, int FIELD, bool SPECIAL, bool BOTH>
 __global__ __launch_bounds__(RowOf<LOGM>::THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_fz_key(
-    DevParams P, FzItem arg, const FzItem* items, const uint32_t* list, int n, int ysplit) {
+    DevParams P, FzItem arg, const FzItem* items, const uint32_t* list, int n) {
   __shared__ uint64_t lds[RowOf<LOGM>::LDS];
   constexpr int per = 16 / RowOf<LOGM>::ROWS;
-  const int y = ysplit ? (int)blockIdx.x / n : 0;
-  const int w = fz_work(P, ysplit ? (int)blockIdx.x % n : (int)blockIdx.x, n);
+  const int y = BOTH ? 0 : (int)blockIdx.x / n;
+  const int w = fz_work(P, BOTH ? (int)blockIdx.x : (int)blockIdx.x % n, n);
   const uint32_t e = fz_entry<ARG>(list, w / per);
   const FzItem it = fz_item<ARG>(arg, items, e >> 8);
   const int m = (int)(e & 255), L = it.level + 1, pr = m < L ? m : P.k + m - L;
-  const int y0 = y, y1 = ysplit ? y + 1 : 2;
   if (!SPECIAL && it.a0 && m < L) {
-#define CALL(F) key_body_tensor<F, LOGM>(P, it, m, w % per, y0, y1, lds)
+#define CALL(F) key_body_tensor<F, LOGM, BOTH>(P, it, m, w % per, y, lds)
     FZ_FIELD(pr, CALL)
 #undef CALL
   } else {
-#define CALL(F) key_body<F, LOGM>(P, it, m, pr, w % per, y0, y1, lds)
+#define CALL(F) key_body<F, LOGM, BOTH>(P, it, m, pr, w % per, y, lds)
     FZ_FIELD(pr, CALL)
 #undef CALL
   }
@@ -181,9 +183,13 @@ static int fz_key(const DevParams& P, const FzItem& arg, const FzItem* items, co
   if (n <= 0) return 0;
 #define CALL(LM)                                                                                                       \
   {                                                                                                                    \
-    const int blocks = n * 16 / RowOf<LM>::ROWS, ysplit = blocks * (RowOf<LM>::THREADS / 64) <= 2048 ? 1 : 0;          \
-    k_fz_key<LM, ARG, FIELD, SPECIAL>                                                                                  \
-        <<<dim3(blocks << ysplit), RowOf<LM>::THREADS, 0, st>>>(P, arg, items, list, blocks, ysplit);                  \
+    const int blocks = n * 16 / RowOf<LM>::ROWS;                                                                       \
+    if (blocks * (RowOf<LM>::THREADS / 64) <= 2048)                                                                    \
+      k_fz_key<LM, ARG, FIELD, SPECIAL, false>                                                                         \
+          <<<dim3(2 * blocks), RowOf<LM>::THREADS, 0, st>>>(P, arg, items, list, blocks);                              \
+    else                                                                                                               \
+      k_fz_key<LM, ARG, FIELD, SPECIAL, true>                                                                          \
+          <<<dim3(blocks), RowOf<LM>::THREADS, 0, st>>>(P, arg, items, list, blocks);                                  \
   }
   FZ_DISPATCH_M(CALL)
 #undef CALL
