@@ -5,19 +5,18 @@
 //               takes any 64-bit value and drops the lowest of the quotient's
 //               four partial products (result below 4p), so a butterfly needs no
 //               conditional correction: 17 vector instructions instead of 27.
-//  FieldFp64    p <= 2^48: signed FP64 integers.  a w mod p = fma(-q, p, h) + l
-//               with h = a w rounded, l = a w - h exact and q = rint(h / p): exact
-//               while |a| <= 17 p (|h - q p| and the result stay below 2^53).  A
-//               butterfly is eight FP64 instructions and its twiddle one double.
+//  FieldFp64    p <= 2^48: signed FP64 integers (exact.hpp).  A butterfly is eight
+//               FP64 instructions and its twiddle one double.
 //  FieldStrict  wider primes (the 63-bit q0, p = 2^63 - c): 64-bit values, with
 //               2^63 = c and a carry out of 64 bits = 2c; below 2p in the inverse.
 //
-// Bounds.  Forward: every stage adds at most 4p (lazy) or about 0.6 p (FP64):
-// 16 stages stay below 72 p and 12 p.  Inverse: a stage doubles the sums; after
-// each register round inv_reduce brings the grown values back (below 8p, and to
-// about p), so that the next four stages stay below 128 p and 17 p.
+// Bounds (FP64: exact.hpp).  Forward: every stage adds at most 4p, 16 stages stay
+// below 72 p.  Inverse: a stage doubles the sums; after each register round
+// inv_reduce brings the grown values back below 8p, so that the next four stages
+// stay below 128 p.
 #pragma once
 #include "device_common.hpp"
+#include "exact.hpp"
 
 namespace aoa {
 
@@ -170,6 +169,7 @@ struct FieldLazy {
     a = u + v;
     b = mul(diff(u, v, ((8 * p) << S) + 1), w);
   }
+  __device__ __forceinline__ V before_last(V x) const { return x; }
   // the last stage, values below 64p: canonical
   __device__ __forceinline__ void inv_last(V& a, V& b, W w0, W w1) const {
     const V u = a, v = b;
@@ -201,16 +201,12 @@ struct FieldLazy {
   __device__ __forceinline__ V relin(V d2, uint64_t k, V d, W bq) const { return key(d2, k) + mul(d, bq); }
 };
 
-struct FieldFp64 {
+struct FieldFp64 : Fp64 {
   static constexpr bool kAnyWord = false;
   using V = double;
   using W = double;
-  double p, pinv;
-  __device__ __forceinline__ explicit FieldFp64(const DevPrime& d) : p(d.fp), pinv(d.fpinv) {}
+  __device__ __forceinline__ explicit FieldFp64(const DevPrime& d) : Fp64(d.fp, d.fpinv) {}
   __device__ __forceinline__ int bits() const { return __builtin_amdgcn_frexp_exp(p); }
-  __device__ __forceinline__ V in(uint64_t x) const {  // x < 2^52
-    return __longlong_as_double((long long)(x | 0x4330000000000000ull)) - 4503599627370496.0;
-  }
   __device__ __forceinline__ V raw_in(uint64_t x) const { return __longlong_as_double((long long)x); }
   __device__ __forceinline__ uint64_t raw(V x) const { return (uint64_t)__double_as_longlong(x); }
   __device__ __forceinline__ W tw(const uint64_t* T, uint32_t i) const { return at_byte<double>(T, i * 8); }
@@ -231,35 +227,7 @@ struct FieldFp64 {
       }
     }
   }
-  __device__ __forceinline__ V mul(V x, W w) const {
-    const double h = x * w, q = __builtin_rint(h * pinv);
-    const double l = __builtin_fma(x, w, -h);
-    return __builtin_fma(-q, p, h) + l;
-  }
-  __device__ __forceinline__ void fwd(V& a, V& b, W w) const {
-    const V v = mul(b, w), u = a;
-    a = u + v;
-    b = u - v;
-  }
-  template <int S>
-  __device__ __forceinline__ void inv(V& a, V& b, W w) const {
-    const V u = a, v = b;
-    a = u + v;
-    b = mul(u - v, w);
-  }
-  __device__ __forceinline__ void inv_last(V& a, V& b, W w0, W w1) const {
-    const V u = a, v = b;
-    a = mul(u + v, w0);
-    b = mul(u - v, w1);
-  }
-  __device__ __forceinline__ V red(V x) const { return __builtin_fma(-__builtin_rint(x * pinv), p, x); }
   static constexpr int kGrow = 1;
-  __device__ __forceinline__ uint64_t out(V x) const { return out_last(red(x)); }
-  // |x| < p -> canonical
-  __device__ __forceinline__ uint64_t out_last(V x) const {
-    x = x < 0 ? x + p : x;
-    return (uint64_t)__double_as_longlong(x + 4503599627370496.0) & 0x000fffffffffffffull;
-  }
   __device__ __forceinline__ V factor(V x) const { return red(x); }
   __device__ __forceinline__ V add(V a, V b) const { return a + b; }  // up to 17 p
   __device__ __forceinline__ V key(V x, uint64_t k) const { return mul(x, in(k)); }
@@ -334,6 +302,7 @@ struct FieldStrict {
     a = add(u, v);
     b = mul(minus(u, v), w);
   }
+  __device__ __forceinline__ V before_last(V x) const { return x; }
   __device__ __forceinline__ void inv_last(V& a, V& b, W w0, W w1) const {
     const V u = a, v = b;
     a = csub(mul(add(u, v), w0), p);
@@ -421,6 +390,7 @@ __device__ __forceinline__ void col_inv_a(const F& f, typename F::V (&x)[4], con
   const typename F::W w2 = col_tw<U>(f, T, 2), w3 = col_tw<U>(f, T, 3), n0 = col_tw<U>(f, lc, 0), n1 = col_tw<U>(f, lc, 1);
   f.template inv<2>(x[0], x[1], w2);
   f.template inv<2>(x[2], x[3], w3);
+  x[0] = f.before_last(x[0]);
   f.inv_last(x[0], x[2], n0, n1);
   f.inv_last(x[1], x[3], n0, n1);
 }
