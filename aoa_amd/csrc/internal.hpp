@@ -12,6 +12,10 @@ struct aoa_params {
   aoa::HostParams host;
   aoa::DevParams dev;
   void* dmem = nullptr;
+  int split = 0;  // the split as set or tuned
+  // the split that stands for the default transforms, once aoa_autotune_ntt has
+  // found them faster than it and every other
+  int default_as = 0;
 };
 
 namespace aoa {

@@ -13,7 +13,6 @@ enum EltOp { ELT_ADD = 0, ELT_SUB = 1, ELT_MUL = 2, ELT_NEG = 3, ELT_MULADD = 5 
 enum SampleKind { SAMPLE_UNIFORM = 0, SAMPLE_GAUSSIAN = 1, SAMPLE_ZO = 2, SAMPLE_HW = 3, SAMPLE_NARROW = 4 };
 constexpr int kHwMaxAttempts = 4096;
 
-int ntt_default_n1(int N);
 bool ntt_valid_split(int N, int N1);
 // Forward / inverse NTT of every limb in `m`.  N1 = 0: the set's split, or
 // without one nt_forward / nt_inverse.

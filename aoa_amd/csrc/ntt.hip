@@ -658,18 +658,6 @@ bool ntt_valid_split(int N, int N1) {
   return N2 == 64 || N2 == 128 || N2 == 256;
 }
 
-int ntt_default_n1(int N) {
-  switch (N) {
-    case 2048: return 2048;
-    case 4096: return 4096;
-    case 8192: return 128;
-    case 16384: return 128;
-    case 32768: return 128;
-    case 65536: return 256;
-    default: return 0;
-  }
-}
-
 static int log2i(int n) {
   int g = 0;
   while ((1 << g) < n) ++g;

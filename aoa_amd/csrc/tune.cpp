@@ -11,7 +11,8 @@ using namespace aoa;
 extern "C" int aoa_params_set_ntt_split(aoa_params* h, int n1) {
   if (!h) return set_error(AOA_ERR_ARG, "null params");
   if (n1 != 0 && !ntt_valid_split(h->host.N, n1)) return set_error(AOA_ERR_ARG, "invalid NTT split");
-  h->dev.ntt_n1 = n1;
+  h->split = n1;
+  h->dev.ntt_n1 = n1 == h->default_as ? 0 : n1;
   return AOA_OK;
 }
 
@@ -28,7 +29,7 @@ extern "C" int aoa_params_get_moddown_exact(const aoa_params* h) {
 
 extern "C" int aoa_params_get_ntt_split(const aoa_params* h) {
   if (!h) return -set_error(AOA_ERR_ARG, "null params");
-  return h->dev.ntt_n1 ? h->dev.ntt_n1 : ntt_default_n1(h->host.N);
+  return h->split;
 }
 
 extern "C" int aoa_autotune_ntt(aoa_params* h, void* stream, int nlimbs, int reps, int* out_n1, double* out_us,
@@ -58,8 +59,8 @@ extern "C" int aoa_autotune_ntt(aoa_params* h, void* stream, int nlimbs, int rep
   (void)hipEventCreate(&e0);
   (void)hipEventCreate(&e1);
   int best = 0, count = 0;
-  double best_us = 1e30;
-  // the splits, and the default (0), which is kept where none beats it
+  double best_us = 1e30, default_us = 1e30;
+  // the splits, and the default (0), which stays in use where none beats it
   for (int n1 : {64, 128, 256, h->host.N, 0}) {
     if (n1 && !ntt_valid_split(h->host.N, n1)) continue;
     DevParams P = h->dev;
@@ -78,13 +79,15 @@ extern "C" int aoa_autotune_ntt(aoa_params* h, void* stream, int nlimbs, int rep
     float ms = 0;
     (void)hipEventElapsedTime(&ms, e0, e1);
     const double us = 1000.0 * ms / reps;
-    if (n1) {
-      if (count < max && out_n1 && out_us) {
-        out_n1[count] = n1;
-        out_us[count] = us;
-      }
-      ++count;
+    if (!n1) {
+      default_us = us;
+      continue;
     }
+    if (count < max && out_n1 && out_us) {
+      out_n1[count] = n1;
+      out_us[count] = us;
+    }
+    ++count;
     if (us < best_us) {
       best_us = us;
       best = n1;
@@ -95,6 +98,8 @@ extern "C" int aoa_autotune_ntt(aoa_params* h, void* stream, int nlimbs, int rep
   (void)hipFree(buf);
   int rc = check_launch("aoa_autotune_ntt");
   if (rc) return -rc;
-  h->dev.ntt_n1 = best;
+  h->split = best;
+  h->default_as = default_us < best_us ? best : 0;
+  h->dev.ntt_n1 = h->default_as ? 0 : best;
   return count;
 }

@@ -292,10 +292,12 @@ int aoa_rotate_right(const aoa_params* params, void* stream, uint64_t* out0, uin
 
 /* ---------------------------------------------------------------- tuning --
  * NTT split N = N1 x (N/N1) of a parameter set (N1 in {64, 128, 256}, N/N1 in
- * the same set, or N1 = N <= 4096) for its plain transforms; 0: the default,
- * which shares its form (16 x N/16) with the key switching kernels.  No counterpart in the reference, whose split is fixed per N
- * at compile time (aoa-ntt/include/newckks/cuda/htrans/ntt.h:24-44; every
- * split gives the same residues).  Set before issuing work with the handle. */
+ * the same set, or N1 = N <= 4096) for its plain transforms; 0 (a new handle's):
+ * the default, which shares its form (16 x N/16) with the key switching kernels
+ * and is the faster at every N.  Setting what the getter returned restores the
+ * handle.  No counterpart in the reference, whose split is fixed per N at compile
+ * time (aoa-ntt/include/newckks/cuda/htrans/ntt.h:24-44; every split gives the
+ * same residues).  Set before issuing work with the handle. */
 int aoa_params_set_ntt_split(aoa_params* params, int n1);
 int aoa_params_get_ntt_split(const aoa_params* params);
 
@@ -312,10 +314,11 @@ int aoa_params_get_moddown_exact(const aoa_params* params);
 
 /* Autotuner: times forward+inverse NTTs of `nlimbs` limbs for every valid
  * split and for the default transforms (reps repetitions each, on the given
- * stream, allocating a scratch buffer), stores the fastest split in the handle,
- * or none where the default is faster, and writes the splits' up to `max`
- * (n1, microseconds) pairs to out_n1/out_us.  Returns the number of
- * candidates, or a negative status. */
+ * stream, allocating a scratch buffer), stores the fastest split in the handle
+ * and writes the splits' up to `max` (n1, microseconds) pairs to out_n1/out_us.
+ * Where the default is faster still, the stored split stands for it from then on:
+ * the handle runs the default transforms while that split is set.  Returns the
+ * number of candidates, or a negative status. */
 int aoa_autotune_ntt(aoa_params* params, void* stream, int nlimbs, int reps, int* out_n1, double* out_us, int max);
 
 /* ---------------------------------------------------------------- batches --
