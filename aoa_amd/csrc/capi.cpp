@@ -394,7 +394,11 @@ extern "C" int aoa_decrypt(const aoa_params* h, void* stream, uint64_t* m, uint6
   const DevParams& P = h->dev;
   hipStream_t st = (hipStream_t)stream;
   const int L = level + 1;
-  if (nt_default(P)) {
+  // The fused rows read s while other workgroups transform c0 and c1, so it must
+  // not overlap them.
+  const size_t LN = (size_t)L * P.N;
+  auto apart = [&](const uint64_t* c) { return s + LN <= c || c + LN <= s; };
+  if (nt_default(P) && apart(c0) && apart(c1)) {
     if (nt_decrypt(P, m, c0, c1, s, L, st)) return fail(AOA_ERR_UNSUPPORTED, "no NTT split for this N");
     return check_launch("aoa_decrypt");
   }
