@@ -2,6 +2,8 @@
 // the kernel sequences of the plain (one ciphertext per call) form.
 #include <algorithm>
 #include <cstring>
+#include <exception>
+#include <memory>
 #include <string>
 
 #include "internal.hpp"
@@ -43,15 +45,10 @@ static int fail(int code, const std::string& msg) { return set_error(code, msg);
 
 extern "C" const char* aoa_last_error(void) { return g_err.c_str(); }
 
-extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** out) {
-  if (!out) return fail(AOA_ERR_ARG, "null output handle");
-  *out = nullptr;
-  aoa_params* h = new aoa_params();
+static int create_params(int N, int k, int kl, int prec, aoa_params** out) {
+  std::unique_ptr<aoa_params, decltype(&aoa_params_destroy)> h(new aoa_params(), aoa_params_destroy);
   std::string err = build_host_params(N, k, kl, prec, &h->host);
-  if (!err.empty()) {
-    delete h;
-    return fail(AOA_ERR_UNSUPPORTED, err);
-  }
+  if (!err.empty()) return fail(AOA_ERR_UNSUPPORTED, err);
   const HostParams& H = h->host;
   // One allocation, 256-byte aligned sections.
   struct Sec {
@@ -114,17 +111,11 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
     secs[i].off = total;
     total += (secs[i].bytes + 255) & ~(size_t)255;
   }
-  if (hipMalloc(&h->dmem, total) != hipSuccess) {
-    delete h;
-    return fail(AOA_ERR_HIP, "hipMalloc of parameter tables failed");
-  }
+  if (hipMalloc(&h->dmem, total) != hipSuccess) return fail(AOA_ERR_HIP, "hipMalloc of parameter tables failed");
   for (int i = 0; i < nsec; ++i) {
     if (hipMemcpy((char*)h->dmem + secs[i].off, secs[i].src, secs[i].bytes, hipMemcpyHostToDevice) !=
-        hipSuccess) {
-      (void)hipFree(h->dmem);
-      delete h;
+        hipSuccess)
       return fail(AOA_ERR_HIP, "hipMemcpy of parameter tables failed");
-    }
   }
   char* b = (char*)h->dmem;
   DevParams& D = h->dev;
@@ -172,8 +163,18 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
   Z.md_stride = F.md_stride;
   Z.mu_kb = F.mu_kb;
   Z.md_kb = F.md_kb;
-  *out = h;
+  *out = h.release();
   return AOA_OK;
+}
+
+extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** out) {
+  if (!out) return fail(AOA_ERR_ARG, "null output handle");
+  *out = nullptr;
+  try {
+    return create_params(N, k, kl, prec, out);
+  } catch (const std::exception&) {
+    return fail(AOA_ERR_HIP, "no memory for the parameter tables");
+  }
 }
 
 extern "C" void aoa_params_destroy(aoa_params* h) {

@@ -7,7 +7,6 @@
 #include <cstring>
 #include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 namespace aoa {
@@ -161,7 +160,7 @@ void parallel_for(int n, size_t cost, const std::function<void(int)>& f) {
   try {
     const size_t want = std::min<size_t>({(size_t)n, 8, std::thread::hardware_concurrency(), n * cost / 65536 + 1});
     for (size_t t = 1; t < want; ++t) ts.emplace_back(work);
-  } catch (const std::system_error&) {  // no more threads: the others do it
+  } catch (const std::exception&) {  // no more threads, or no memory for one: the others do it
   }
   work();
   for (std::thread& t : ts) t.join();

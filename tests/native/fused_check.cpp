@@ -3,9 +3,11 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <new>
 #include <random>
 
 #include "exact.hpp"
@@ -13,6 +15,16 @@
 
 using namespace aoa;
 typedef __int128 i128;
+
+// The fail_in-th allocation of this thread from now on throws (0: none).
+static thread_local int fail_in = 0;
+void* operator new(size_t n) {
+  if (fail_in && --fail_in == 0) throw std::bad_alloc();
+  if (void* p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 static int failures = 0;
 static void expect(bool ok, const char* what, const char* where = "") {
@@ -90,8 +102,28 @@ static void fp64_forms() {
   }
 }
 
+// parallel_for where the calling thread runs out of memory at its i-th allocation,
+// the creation of threads among them: every call is made once, or the exception
+// comes back; threads that were created are joined.
+static void parallel_for_without_memory() {
+  for (int i = 1; i <= 12; ++i) {
+    std::atomic<int> calls{0};
+    const std::function<void(int)> f = [&](int) { ++calls; };
+    bool thrown = false;
+    fail_in = i;
+    try {
+      parallel_for(64, 65536, f);
+    } catch (const std::bad_alloc&) {
+      thrown = true;
+    }
+    fail_in = 0;
+    expect(thrown || calls == 64, "parallel_for without memory");
+  }
+}
+
 int main() {
   chains();
+  parallel_for_without_memory();
   fp64_forms();
   std::printf("fused host checks: %d failure(s)\n", failures);
   return failures ? 1 : 0;
