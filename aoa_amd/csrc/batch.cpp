@@ -293,18 +293,34 @@ struct StageTimer {
   }
 };
 
-// Issues every stage launch of the batch on stream st (stage order
-// AOA_STAGE_*); with a timer, each (layer, stage) launch run is bracketed by
-// an event pair.
+// The batch's NTT split where the group's ring admits it and the group has
+// transforms of its own (nothing else uses one), else 0.
+static int group_split(const aoa_batch* b, const BatchGroup& g) {
+  return !g.ntts.empty() && b->opt.ntt_split && ntt_valid_split(g.params->host.N, b->opt.ntt_split) ? b->opt.ntt_split : 0;
+}
+// Builds the tables of the batch's split, so that a launch (or a capture) does not.
+static int prepare_splits(const aoa_batch* b) {
+  for (auto& L : b->layers)
+    for (auto& g : L.groups)
+      if (const int n1 = group_split(b, g)) {
+        DevParams P = g.params->dev;
+        if (const int rc = use_split(g.params, n1, &P)) return rc;
+      }
+  return AOA_OK;
+}
+
 // The parameters a group's launches use: its handle's, with the batch's NTT
-// split (when the group's ring admits it) and XCD mapping.
+// split and XCD mapping.
 static DevParams launch_params(const aoa_batch* b, const BatchGroup& g) {
   DevParams P = g.params->dev;
-  if (b->opt.ntt_split && ntt_valid_split(P.N, b->opt.ntt_split)) P.ntt_n1 = b->opt.ntt_split;
+  if (const int n1 = group_split(b, g)) (void)use_split(g.params, n1, &P);
   P.xcd_chunks = b->opt.xcd_chunks ? 1 : 0;
   return P;
 }
 
+// Issues every stage launch of the batch on stream st (stage order
+// AOA_STAGE_*); with a timer, each (layer, stage) launch run is bracketed by
+// an event pair.
 int batch_enqueue(aoa_batch* b, hipStream_t st, StageTimer* tm) {
   int rc = AOA_OK;
   auto run = [&](int s, auto&& has, auto&& go) {
@@ -458,6 +474,7 @@ extern "C" int aoa_batch_barrier(aoa_batch* b) {
 extern "C" int aoa_batch_build(aoa_batch* b) {
   if (!b) return set_error(AOA_ERR_ARG, "null batch");
   if (b->built) return AOA_OK;
+  if (const int rc = prepare_splits(b)) return rc;
   size_t ws = 0, desc = 0;
   batch_sizes(b, &ws, &desc);
   b->ws_bytes = ws;
@@ -505,6 +522,7 @@ extern "C" int aoa_batch_set_options(aoa_batch* b, const aoa_batch_options* o) {
   b->opt.prime_major = o->prime_major ? 1 : 0;
   b->opt.xcd_chunks = o->xcd_chunks ? 1 : 0;
   if (!b->built) return AOA_OK;
+  if (const int rc = prepare_splits(b)) return rc;
   // same descriptors in another order: refill the tables in place
   if (hipDeviceSynchronize() != hipSuccess) return set_error(AOA_ERR_HIP, "hipDeviceSynchronize failed");
   drop_graph(b);

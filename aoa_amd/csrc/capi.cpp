@@ -45,126 +45,135 @@ static int fail(int code, const std::string& msg) { return set_error(code, msg);
 
 extern "C" const char* aoa_last_error(void) { return g_err.c_str(); }
 
-static int create_params(int N, int k, int kl, int prec, aoa_params** out) {
+namespace {
+
+// A table on its way to the device: *at becomes its address.
+struct Section {
+  const void* src;
+  size_t bytes;
+  const void** at;
+};
+template <class T, class D>
+Section section(const std::vector<T>& v, const D** at) {
+  return Section{v.data(), v.size() * sizeof(T), (const void**)at};
+}
+
+// One allocation of 256-byte aligned sections.  Those below 1 MiB go up in one
+// copy: a copy takes 8 us or more, and small rings have some thirty.
+int upload(std::vector<Section>& secs, void** mem) {
+  std::stable_partition(secs.begin(), secs.end(), [](const Section& s) { return s.bytes < ((size_t)1 << 20); });
+  size_t total = 0, small = 0;
+  std::vector<size_t> off;
+  for (const Section& s : secs) {
+    off.push_back(total);
+    total += (s.bytes + 255) & ~(size_t)255;
+    if (s.bytes < ((size_t)1 << 20)) small = total;
+  }
+  std::vector<char> stage(small);
+  if (hipMalloc(mem, total) != hipSuccess) return fail(AOA_ERR_HIP, "hipMalloc of parameter tables failed");
+  char* b = (char*)*mem;
+  bool ok = true;
+  for (size_t i = 0; i < secs.size(); ++i) {
+    if (off[i] < small)
+      std::memcpy(&stage[off[i]], secs[i].src, secs[i].bytes);
+    else
+      ok = ok && hipMemcpy(b + off[i], secs[i].src, secs[i].bytes, hipMemcpyHostToDevice) == hipSuccess;
+    *secs[i].at = b + off[i];
+  }
+  ok = ok && (!small || hipMemcpy(b, stage.data(), small, hipMemcpyHostToDevice) == hipSuccess);
+  return ok ? AOA_OK : fail(AOA_ERR_HIP, "hipMemcpy of parameter tables failed");
+}
+
+int create_params(int N, int k, int kl, int prec, aoa_params** out) {
   std::unique_ptr<aoa_params, decltype(&aoa_params_destroy)> h(new aoa_params(), aoa_params_destroy);
   std::string err = build_host_params(N, k, kl, prec, &h->host);
   if (!err.empty()) return fail(AOA_ERR_UNSUPPORTED, err);
   const HostParams& H = h->host;
-  // One allocation, 256-byte aligned sections.
-  struct Sec {
-    const void* src;
-    size_t bytes;
-    size_t off;
-  };
-  std::vector<Sec> secs = {
-      {H.dprimes.data(), H.dprimes.size() * sizeof(DevPrime), 0},
-      {H.tw_fwd.data(), H.tw_fwd.size() * 8, 0},
-      {H.tw_inv.data(), H.tw_inv.size() * 8, 0},
-      {H.inv_qhat.data(), H.inv_qhat.size() * 8, 0},
-      {H.qhat_mod_b.data(), H.qhat_mod_b.size() * 8, 0},
-      {H.inv_bhat.data(), H.inv_bhat.size() * 8, 0},
-      {H.bhat_mod_q.data(), H.bhat_mod_q.size() * 8, 0},
-      {H.inv_b_mod_q.data(), H.inv_b_mod_q.size() * 8, 0},
-      {H.b_mod_q.data(), H.b_mod_q.size() * 8, 0},
-      {H.inv_ql_mod_qi.data(), H.inv_ql_mod_qi.size() * 8, 0},
-      {H.enc_t[0].data(), H.enc_t[0].size() * 8, 0},
-      {H.enc_t[1].data(), H.enc_t[1].size() * 8, 0},
-      {H.gauss_cdt.data(), H.gauss_cdt.size() * 8, 0},
-      {H.md_terms.data(), H.md_terms.size() * sizeof(MdTerm), 0},
-      {H.md_thr.data(), H.md_thr.size() * 4, 0},
-      {H.md_red.data(), H.md_red.size() * 8, 0},
-      {H.md_fin.data(), H.md_fin.size() * 8, 0},
-      {H.md_negb.data(), H.md_negb.size() * 4, 0},
-      {H.mu_terms.data(), H.mu_terms.size() * 4, 0},
-  };
-  // Row-pass twiddle orders, one per two-pass split of N and direction
-  // (device only: the host keeps the natural tables).
-  std::vector<uint64_t> rowtw[3][2];
-  int rowsec[3][2];
-  parallel_for(6, (size_t)(H.k + H.K) * H.N, [&](int t) {
-    row_twiddle_order(t & 1 ? H.tw_inv : H.tw_fwd, H.N, H.k + H.K, 64 << (t >> 1), &rowtw[t >> 1][t & 1]);
-  });
-  for (int si = 0; si < 3; ++si)
-    for (int dir = 0; dir < 2; ++dir) {
-      rowsec[si][dir] = rowtw[si][dir].empty() ? -1 : (int)secs.size();
-      if (!rowtw[si][dir].empty()) secs.push_back({rowtw[si][dir].data(), rowtw[si][dir].size() * 8, 0});
-    }
   FusedTables F;
   build_fused_tables(H, &F);
-  const int fsec = (int)secs.size();
-  secs.push_back({F.tw[0].data(), F.tw[0].size() * 8, 0});
-  secs.push_back({F.tw[1].data(), F.tw[1].size() * 8, 0});
-  secs.push_back({F.lc.data(), F.lc.size() * 8, 0});
-  secs.push_back({F.lc_b.data(), F.lc_b.size() * 8, 0});
-  secs.push_back({F.lc_up.data(), F.lc_up.size() * 8, 0});
-  secs.push_back({F.bq.data(), F.bq.size() * 8, 0});
-  secs.push_back({F.mu_w.data(), F.mu_w.size(), 0});
-  secs.push_back({F.md_w.data(), F.md_w.size(), 0});
-  secs.push_back({F.mu_out.data(), F.mu_out.size() * sizeof(ConvOut), 0});
-  secs.push_back({F.md_out.data(), F.md_out.size() * sizeof(ConvOut), 0});
-  secs.push_back({F.scr.data(), F.scr.size() * 8, 0});
-  secs.push_back({F.scr_thr.data(), F.scr_thr.size() * 8, 0});
-  secs.push_back({F.lc_down.data(), F.lc_down.size() * 8, 0});
-  const int nsec = (int)secs.size();
-  size_t total = 0;
-  for (int i = 0; i < nsec; ++i) {
-    secs[i].off = total;
-    total += (secs[i].bytes + 255) & ~(size_t)255;
-  }
-  if (hipMalloc(&h->dmem, total) != hipSuccess) return fail(AOA_ERR_HIP, "hipMalloc of parameter tables failed");
-  for (int i = 0; i < nsec; ++i) {
-    if (hipMemcpy((char*)h->dmem + secs[i].off, secs[i].src, secs[i].bytes, hipMemcpyHostToDevice) !=
-        hipSuccess)
-      return fail(AOA_ERR_HIP, "hipMemcpy of parameter tables failed");
-  }
-  char* b = (char*)h->dmem;
+  if (hipGetDevice(&h->device) != hipSuccess) return fail(AOA_ERR_HIP, "no current device");
   DevParams& D = h->dev;
+  FusedDev& Z = D.fz;
+  std::vector<Section> secs = {
+      section(H.dprimes, &D.primes),
+      section(H.inv_qhat, &D.inv_qhat),
+      section(H.qhat_mod_b, &D.qhat_mod_b),
+      section(H.inv_bhat, &D.inv_bhat),
+      section(H.bhat_mod_q, &D.bhat_mod_q),
+      section(H.inv_b_mod_q, &D.inv_b_mod_q),
+      section(H.b_mod_q, &D.b_mod_q),
+      section(H.inv_ql_mod_qi, &D.inv_ql_mod_qi),
+      section(H.enc_t[0], &D.enc_t[0]),
+      section(H.enc_t[1], &D.enc_t[1]),
+      section(H.gauss_cdt, &D.gauss_cdt),
+      section(H.md_terms, &D.md_terms),
+      section(H.md_thr, &D.md_thr),
+      section(H.md_red, &D.md_red),
+      section(H.md_fin, &D.md_fin),
+      section(H.md_negb, &D.md_negb),
+      section(H.mu_terms, &D.mu_terms),
+      section(F.tw[0], &Z.tw[0]),
+      section(F.tw[1], &Z.tw[1]),
+      section(F.lc, &Z.lc),
+      section(F.lc_b, &Z.lc_b),
+      section(F.lc_up, &Z.lc_up),
+      section(F.lc_down, &Z.lc_down),
+      section(F.bq, &Z.bq),
+      section(F.mu_w, &Z.mu_w),
+      section(F.md_w, &Z.md_w),
+      section(F.mu_out, &Z.mu_out),
+      section(F.md_out, &Z.md_out),
+      section(F.scr, &Z.scr),
+      section(F.scr_thr, &Z.scr_thr),
+  };
+  const int rc = upload(secs, &h->dmem);
+  if (rc) return rc;
   D.N = H.N;
   D.logN = H.logN;
   D.k = H.k;
   D.K = H.K;
-  D.primes = (const DevPrime*)(b + secs[0].off);
-  D.tw_fwd = (const uint64_t*)(b + secs[1].off);
-  D.tw_inv = (const uint64_t*)(b + secs[2].off);
-  D.inv_qhat = (const uint64_t*)(b + secs[3].off);
-  D.qhat_mod_b = (const uint64_t*)(b + secs[4].off);
-  D.inv_bhat = (const uint64_t*)(b + secs[5].off);
-  D.bhat_mod_q = (const uint64_t*)(b + secs[6].off);
-  D.inv_b_mod_q = (const uint64_t*)(b + secs[7].off);
-  D.b_mod_q = (const uint64_t*)(b + secs[8].off);
-  D.inv_ql_mod_qi = (const uint64_t*)(b + secs[9].off);
-  D.enc_t[0] = (const double*)(b + secs[10].off);
-  D.enc_t[1] = (const double*)(b + secs[11].off);
-  D.gauss_cdt = (const uint64_t*)(b + secs[12].off);
-  D.md_terms = (const uint32_t*)(b + secs[13].off);
-  D.md_thr = (const uint32_t*)(b + secs[14].off);
-  D.md_red = (const uint64_t*)(b + secs[15].off);
-  D.md_fin = (const uint64_t*)(b + secs[16].off);
-  D.md_negb = (const uint32_t*)(b + secs[17].off);
-  D.mu_terms = (const uint32_t*)(b + secs[18].off);
-  for (int si = 0; si < 3; ++si)
-    for (int dir = 0; dir < 2; ++dir)
-      D.tw_row[si][dir] = rowsec[si][dir] < 0 ? nullptr : (const uint64_t*)(b + secs[rowsec[si][dir]].off);
-  FusedDev& Z = D.fz;
-  Z.tw[0] = (const uint64_t*)(b + secs[fsec].off);
-  Z.tw[1] = (const uint64_t*)(b + secs[fsec + 1].off);
-  Z.lc = (const uint64_t*)(b + secs[fsec + 2].off);
-  Z.lc_b = (const uint64_t*)(b + secs[fsec + 3].off);
-  Z.lc_up = (const uint64_t*)(b + secs[fsec + 4].off);
-  Z.bq = (const uint64_t*)(b + secs[fsec + 5].off);
-  Z.mu_w = (const uint8_t*)(b + secs[fsec + 6].off);
-  Z.md_w = (const uint8_t*)(b + secs[fsec + 7].off);
-  Z.mu_out = (const ConvOut*)(b + secs[fsec + 8].off);
-  Z.md_out = (const ConvOut*)(b + secs[fsec + 9].off);
-  Z.scr = (const double*)(b + secs[fsec + 10].off);
-  Z.scr_thr = (const double*)(b + secs[fsec + 11].off);
-  Z.lc_down = (const uint64_t*)(b + secs[fsec + 12].off);
   Z.mu_stride = F.mu_stride;
   Z.md_stride = F.md_stride;
   Z.mu_kb = F.mu_kb;
   Z.md_kb = F.md_kb;
   *out = h.release();
   return AOA_OK;
+}
+
+}  // namespace
+
+int aoa::use_split(const aoa_params* h, int n1, DevParams* P) try {
+  if (n1) {
+    std::lock_guard<std::mutex> lock(h->split_mu);
+    if (!h->split_mem) {
+      const HostParams& H = h->host;
+      std::vector<uint64_t> row[3][2];
+      parallel_for(6, (size_t)(H.k + H.K) * H.N, [&](int t) {
+        row_twiddle_order(t & 1 ? H.tw_inv : H.tw_fwd, H.N, H.k + H.K, 64 << (t >> 1), &row[t >> 1][t & 1]);
+      });
+      SplitTables t{};
+      std::vector<Section> secs = {section(H.tw_fwd, &t.tw_fwd), section(H.tw_inv, &t.tw_inv)};
+      for (int i = 0; i < 6; ++i)
+        if (!row[i >> 1][i & 1].empty()) secs.push_back(section(row[i >> 1][i & 1], &t.tw_row[i >> 1][i & 1]));
+      int prev = 0;
+      void* mem = nullptr;
+      if (hipGetDevice(&prev) != hipSuccess || hipSetDevice(h->device) != hipSuccess)
+        return fail(AOA_ERR_HIP, "the parameter set's device is not usable");
+      const int rc = upload(secs, &mem);
+      (void)hipSetDevice(prev);
+      if (rc) {
+        if (mem) (void)hipFree(mem);
+        return rc;
+      }
+      h->split_tables = t;
+      h->split_mem = mem;
+    }
+    P->split = h->split_tables;
+  }
+  P->ntt_n1 = n1;
+  return AOA_OK;
+} catch (const std::exception&) {
+  return fail(AOA_ERR_HIP, "no memory for a split's tables");
 }
 
 extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** out) {
@@ -180,6 +189,7 @@ extern "C" int aoa_params_create(int N, int k, int kl, int prec, aoa_params** ou
 extern "C" void aoa_params_destroy(aoa_params* h) {
   if (!h) return;
   if (h->dmem) (void)hipFree(h->dmem);
+  if (h->split_mem) (void)hipFree(h->split_mem);
   delete h;
 }
 

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 
 #include "../../include/aoa.h"
@@ -10,8 +11,13 @@
 
 struct aoa_params {
   aoa::HostParams host;
-  aoa::DevParams dev;
+  aoa::DevParams dev{};
   void* dmem = nullptr;
+  int device = 0;
+  // tables of the explicit splits, shared by every user of the handle
+  mutable std::mutex split_mu;
+  mutable void* split_mem = nullptr;
+  mutable aoa::SplitTables split_tables{};
   int split = 0;  // the split as set or tuned
   // the split that stands for the default transforms, once aoa_autotune_ntt has
   // found them faster than it and every other
@@ -26,6 +32,10 @@ int set_error(int code, const std::string& msg);
 int check_launch(const char* what);
 // 5^rot mod 2N: the Galois element of a left rotation by rot slots.
 uint64_t galois_of(int rot_slots, int N);
+
+// Makes P, a copy of h's parameters or h's own, use the split n1 (0: the default),
+// whose tables are built on the first use of a split with h: not during a capture.
+int use_split(const aoa_params* h, int n1, DevParams* P);
 
 // HomMul + relinearisation (+ rescale when rescale != 0) of (a0, a1) and
 // (b0, b1) at `level` into (c3_0, c3_1), with ws_bytes of caller workspace.

@@ -94,7 +94,7 @@ __device__ __forceinline__ void fwd_col_body(const DevParams& P, const uint64_t*
   constexpr int C = G::C, TS = G::TS, LOGS = G::LOGS, LDW = C + 1;
   const int col0 = tile * C;
   const uint64_t p = P.primes[pr].p;
-  const uint64_t* T = P.tw_fwd + (size_t)pr * P.N * 2;
+  const uint64_t* T = P.split.tw_fwd + (size_t)pr * P.N * 2;
   src += col0;
   dst += col0;
   const int tid = threadIdx.x;
@@ -141,9 +141,9 @@ __device__ __forceinline__ void fwd_row_body(const DevParams& P, const uint64_t*
   constexpr int C = G::C, TS = G::TS, LOGS = G::LOGS, PS = S + S / 16;
   const int row0 = tile * C;
   const uint64_t p = P.primes[pr].p;
-  const uint64_t* T = P.tw_fwd + (size_t)pr * P.N * 2;
+  const uint64_t* T = P.split.tw_fwd + (size_t)pr * P.N * 2;
   // the second round's stages: entries in row order (row_twiddle_order)
-  const uint64_t* TR = P.tw_row[LOGS - 6][0] + (size_t)pr * P.N * 2;
+  const uint64_t* TR = P.split.tw_row[LOGS - 6][0] + (size_t)pr * P.N * 2;
   const int tid = threadIdx.x;
   const int rl = tid / TS;
   const int sl = tid % TS;
@@ -282,8 +282,8 @@ __device__ __forceinline__ void inv_row_body(const DevParams& P, const uint64_t*
                                              int g0, uint64_t* lds) {
   using G = Geo<S>;
   constexpr int C = G::C, TS = G::TS, PS = S + S / 16;
-  const uint64_t* T = P.tw_inv + (size_t)pr * P.N * 2;
-  const uint64_t* TR = P.tw_row[G::LOGS - 6][1] + (size_t)pr * P.N * 2;
+  const uint64_t* T = P.split.tw_inv + (size_t)pr * P.N * 2;
+  const uint64_t* TR = P.split.tw_row[G::LOGS - 6][1] + (size_t)pr * P.N * 2;
   const int rl = threadIdx.x / TS, sl = threadIdx.x % TS;
   const int row = tile * C + rl;
   src += (size_t)row * S;
@@ -303,7 +303,7 @@ __device__ __forceinline__ void inv_col_body(const DevParams& P, const uint64_t*
   const int col0 = tile * C;
   const DevPrime dp = P.primes[pr];
   const uint64_t p = dp.p;
-  const uint64_t* T = P.tw_inv + (size_t)pr * P.N * 2;
+  const uint64_t* T = P.split.tw_inv + (size_t)pr * P.N * 2;
   src += col0;
   dst += col0;
   const int tid = threadIdx.x;
@@ -522,7 +522,7 @@ __device__ __forceinline__ void fwd_single_body(const DevParams& P, const uint64
   constexpr int V = G::V, R = G::R;
   const DevPrime dp = P.primes[pr];
   const uint64_t p = dp.p;
-  const uint64_t* T = P.tw_fwd + (size_t)pr * G::N * 2;
+  const uint64_t* T = P.split.tw_fwd + (size_t)pr * G::N * 2;
   const int t = threadIdx.x;
   sp_load<LOGN>(src, lds);
   uint64_t x[V];
@@ -563,7 +563,7 @@ __device__ __forceinline__ void inv_single_body(const DevParams& P, const uint64
   constexpr int V = G::V, R = G::R;
   const DevPrime dp = P.primes[pr];
   const uint64_t p = dp.p;
-  const uint64_t* T = P.tw_inv + (size_t)pr * G::N * 2;
+  const uint64_t* T = P.split.tw_inv + (size_t)pr * G::N * 2;
   const int t = threadIdx.x;
   sp_load<LOGN>(src, lds);
   uint64_t x[V];

@@ -96,9 +96,22 @@ struct FusedDev {
   int mu_kb, md_kb;        // steps of 8 inputs the layouts hold
 };
 
+// Twiddles of the transforms by an explicit split, built when one is first used
+// (use_split).
+struct SplitTables {
+  const uint64_t* tw_fwd;  // [k+K][N][2]: psi^brev(i) and Shoup quotient
+  const uint64_t* tw_inv;  // [k+K][N][2]: psi^-brev(i) and Shoup quotient
+  // [log2(S) - 6][0: forward, 1: inverse]: for the row pass of the split
+  // N = (N/S) x S, the twiddle table with the entries of the stages done on
+  // 16 consecutive values per thread reordered (row_twiddle_order), so that
+  // the S/16 threads of a row load adjacent entries; null where N/S is not a
+  // valid split
+  const uint64_t* tw_row[3][2];
+};
+
 struct DevParams {
   int N, logN, k, K;
-  int ntt_n1;  // NTT split N = N1 x (N/N1); 0 = built-in default (autotuner sets it)
+  int ntt_n1;  // NTT split N = N1 x (N/N1); 0: the default, 16 x N/16 (set by use_split)
   // 0: ModDown reproduces the reference's Barrett reduction of its
   // cross-base products (bit-exact residues); 1: exact reduction.
   int moddown_exact;
@@ -106,14 +119,7 @@ struct DevParams {
   // in contiguous chunks (work_id); 0: workgroup id order
   int xcd_chunks;
   const DevPrime* primes;        // [k+K]: Q primes then B primes
-  const uint64_t* tw_fwd;        // [k+K][N][2]: psi^brev(i) and Shoup quotient
-  const uint64_t* tw_inv;        // [k+K][N][2]: psi^-brev(i) and Shoup quotient
-  // [log2(S) - 6][0: forward, 1: inverse]: for the row pass of the split
-  // N = (N/S) x S, the twiddle table with the entries of the stages done on
-  // 16 consecutive values per thread reordered (row_twiddle_order), so that
-  // the S/16 threads of a row load adjacent entries; null where N/S is not a
-  // valid split
-  const uint64_t* tw_row[3][2];
+  SplitTables split;             // where ntt_n1 is set
   const uint64_t* inv_qhat;      // [k][k][2]: (l,i) -> (Q_l/q_i)^-1 mod q_i, Shoup
   const uint64_t* qhat_mod_b;    // [k][K][k]: (l,j,i) -> (Q_l/q_i) mod b_j
   const uint64_t* inv_bhat;      // [K][2]: (B/b_j)^-1 mod b_j, Shoup

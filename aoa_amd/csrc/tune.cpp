@@ -11,9 +11,9 @@ using namespace aoa;
 extern "C" int aoa_params_set_ntt_split(aoa_params* h, int n1) {
   if (!h) return set_error(AOA_ERR_ARG, "null params");
   if (n1 != 0 && !ntt_valid_split(h->host.N, n1)) return set_error(AOA_ERR_ARG, "invalid NTT split");
-  h->split = n1;
-  h->dev.ntt_n1 = n1 == h->default_as ? 0 : n1;
-  return AOA_OK;
+  const int rc = use_split(h, n1 == h->default_as ? 0 : n1, &h->dev);
+  if (!rc) h->split = n1;
+  return rc;
 }
 
 extern "C" int aoa_params_set_moddown_exact(aoa_params* h, int exact) {
@@ -58,13 +58,13 @@ extern "C" int aoa_autotune_ntt(aoa_params* h, void* stream, int nlimbs, int rep
   hipEvent_t e0, e1;
   (void)hipEventCreate(&e0);
   (void)hipEventCreate(&e1);
-  int best = 0, count = 0;
+  int best = 0, count = 0, rc = AOA_OK;
   double best_us = 1e30, default_us = 1e30;
   // the splits, and the default (0), which stays in use where none beats it
   for (int n1 : {64, 128, 256, h->host.N, 0}) {
     if (n1 && !ntt_valid_split(h->host.N, n1)) continue;
     DevParams P = h->dev;
-    P.ntt_n1 = n1;
+    if ((rc = use_split(h, n1, &P))) break;
     for (int w = 0; w < 2; ++w) {
       ntt_forward(P, m, n1, st);
       ntt_inverse(P, m, n1, st);
@@ -96,10 +96,10 @@ extern "C" int aoa_autotune_ntt(aoa_params* h, void* stream, int nlimbs, int rep
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   (void)hipFree(buf);
-  int rc = check_launch("aoa_autotune_ntt");
+  if (!rc) rc = check_launch("aoa_autotune_ntt");
   if (rc) return -rc;
   h->split = best;
   h->default_as = default_us < best_us ? best : 0;
-  h->dev.ntt_n1 = h->default_as ? 0 : best;
+  if ((rc = use_split(h, h->default_as ? 0 : best, &h->dev))) return -rc;
   return count;
 }

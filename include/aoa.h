@@ -297,7 +297,9 @@ int aoa_rotate_right(const aoa_params* params, void* stream, uint64_t* out0, uin
  * and is the faster at every N.  Setting what the getter returned restores the
  * handle.  No counterpart in the reference, whose split is fixed per N at compile
  * time (aoa-ntt/include/newckks/cuda/htrans/ntt.h:24-44; every split gives the
- * same residues).  Set before issuing work with the handle. */
+ * same residues).  Set before issuing work with the handle.  The first split used
+ * with a handle (set, tuned, or a batch's option) allocates and uploads its
+ * twiddles, 8 (k + kl) N words at most: not during a capture. */
 int aoa_params_set_ntt_split(aoa_params* params, int n1);
 int aoa_params_get_ntt_split(const aoa_params* params);
 
