@@ -52,12 +52,6 @@ struct BatchLayer {
   std::vector<BatchGroup> groups;
 };
 
-// Workspace limbs of one HomMul item: d2 after its inverse rows (L), the
-// special limbs (K), P0, P1 (L + K each); of a rotation: the rotated
-// polynomials (L each), the forward columns of the second (L + K), P0, P1.
-size_t mul_ws_limbs(int L, int K) { return 3 * (size_t)L + 3 * (size_t)K; }
-size_t rot_ws_limbs(int L, int K) { return 5 * (size_t)L + 3 * (size_t)K; }
-
 }  // namespace aoa
 
 struct aoa_batch {

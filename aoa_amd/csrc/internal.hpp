@@ -43,6 +43,12 @@ int hommul_core(const aoa_params* h, void* stream, uint64_t* c3_0, uint64_t* c3_
                 const uint64_t* a1, const uint64_t* b0, const uint64_t* b1, const uint64_t* evk_b,
                 const uint64_t* evk_a, int level, void* ws, size_t ws_bytes, int rescale);
 
+// Workspace limbs of one HomMul item of a batch: d2 after its inverse rows (L), the
+// special limbs (K), P0, P1 (L + K each); of a rotation: the rotated
+// polynomials (L each), the forward columns of the second (L + K), P0, P1.
+inline size_t mul_ws_limbs(int L, int K) { return 3 * (size_t)L + 3 * (size_t)K; }
+inline size_t rot_ws_limbs(int L, int K) { return 5 * (size_t)L + 3 * (size_t)K; }
+
 // Batch planning with caller-provided memory (the serving loop rebuilds a
 // batch every step from preallocated workspace and descriptor buffers).
 void batch_sizes(const aoa_batch* b, size_t* ws_bytes, size_t* desc_bytes);

@@ -166,9 +166,8 @@ static size_t ct_bytes(const KeySet& ks, int level) {
 }
 
 static size_t op_ws_bytes(const KeySet& ks, const aoa_op& op, int level) {
-  const size_t N = ks.params->host.N, K = ks.params->host.K, L = level + 1;
-  const size_t limbs = op.kind == AOA_OP_MUL ? 6 * L + 3 * K : 5 * L + 3 * K;
-  return limbs * N * 8 + 256;
+  const int K = ks.params->host.K, L = level + 1;
+  return (op.kind == AOA_OP_MUL ? mul_ws_limbs(L, K) : rot_ws_limbs(L, K)) * ks.params->host.N * 8 + 256;
 }
 
 extern "C" int aoa_server_create(size_t pool_bytes, size_t step_ws_bytes, int max_active, aoa_server** out) {
