@@ -616,6 +616,11 @@ extern "C" int aoa_batch_autotune(aoa_batch* b, void* stream, int reps, aoa_tune
       }
     if (ok && any) splits.push_back(n1);
   }
+  // a split is for the batch's own transforms: without any its candidates are the
+  // first one's programs, whose results they get
+  bool split_matters = false;
+  for (auto& L : b->layers)
+    for (auto& g : L.groups) split_matters = split_matters || !g.ntts.empty();
   std::vector<aoa_batch_options> cand;
   for (int n1 : splits)
     for (int xcd = 0; xcd < 2; ++xcd) {
@@ -646,7 +651,16 @@ extern "C" int aoa_batch_autotune(aoa_batch* b, void* stream, int reps, aoa_tune
   double best_ms = 1e30;
   uint64_t base_sum = 0;
   bool reproducible = true;
+  const size_t distinct = split_matters ? cand.size() : cand.size() / splits.size();
+  std::vector<aoa_tune_result> found;
   for (size_t c = 0; c < cand.size() && !rc; ++c) {
+    if (c >= distinct) {
+      aoa_tune_result r = found[c % distinct];
+      r.opt = cand[c];
+      if (count < max && results) results[count] = r;
+      ++count;
+      continue;
+    }
     rc = aoa_batch_set_options(b, &cand[c]);
     if (rc) break;
     rc = aoa_batch_launch(b, st, 1);  // warm-up (captures the graph)
@@ -676,7 +690,8 @@ extern "C" int aoa_batch_autotune(aoa_batch* b, void* stream, int reps, aoa_tune
     }
     const bool exact = reproducible && sum == base_sum;
     const double t = ms / reps;
-    if (count < max && results) results[count] = aoa_tune_result{cand[c], t, sum, exact ? 1 : 0};
+    found.push_back(aoa_tune_result{cand[c], t, sum, exact ? 1 : 0});
+    if (count < max && results) results[count] = found.back();
     ++count;
     if ((exact || !reproducible) && t < best_ms) {
       best_ms = t;

@@ -115,8 +115,9 @@ struct DevParams {
   // 0: ModDown reproduces the reference's Barrett reduction of its
   // cross-base products (bit-exact residues); 1: exact reduction.
   int moddown_exact;
-  // 1: descriptor-driven NTT passes deal their work items out to the 8 XCDs
-  // in contiguous chunks (work_id); 0: workgroup id order
+  // 1: the fused row kernels and descriptor-driven transforms by an explicit split
+  // deal their work items out to the 8 XCDs in contiguous chunks (fz_work,
+  // work_id); 0: workgroup id order
   int xcd_chunks;
   const DevPrime* primes;        // [k+K]: Q primes then B primes
   SplitTables split;             // where ntt_n1 is set

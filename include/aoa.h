@@ -383,7 +383,9 @@ void aoa_batch_destroy(aoa_batch* batch);
 typedef struct {
   int ntt_split;    /* N1 of the plain transforms for the groups whose ring admits it (0: as the handle) */
   int prime_major;  /* 1: the descriptors of a stage sorted by prime (default); 0: item after item */
-  int xcd_chunks;   /* 1: the NTT passes deal their tiles out to the 8 XCDs in contiguous chunks */
+  int xcd_chunks;   /* 1: the row kernels of products and key switching, and transforms by an explicit
+                       split, deal their tiles out to the 8 XCDs in contiguous chunks (the column
+                       kernels always do, the default transforms never) */
   int strict_split; /* limbs of the 63-bit q0 in a launch of their own: -1 never, 0 from 256
                        descriptors per stage up (default), 1 always */
 } aoa_batch_options;
@@ -407,7 +409,8 @@ typedef struct {
  * the batch, x prime-major or item order, x XCD chunks off / on, x the three
  * strict-split rules), each as `reps` graph replays after one warm-up
  * replay, keeps the fastest candidate whose outputs equal the first
- * candidate's and sets it on the batch.  Writes up to max results; returns
+ * candidate's and sets it on the batch.  In a batch without transforms of its own
+ * the splits change nothing: their candidates repeat the first one's results.  Writes up to max results; returns
  * the number of candidates, or -status.  Allocates a few bytes of device
  * memory for the checksums; synchronises `stream`. */
 int aoa_batch_autotune(aoa_batch* batch, void* stream, int reps, aoa_tune_result* results, int max);
