@@ -110,7 +110,6 @@ int create_params(int N, int k, int kl, int prec, aoa_params** out) {
       section(H.md_thr, &D.md_thr),
       section(H.md_red, &D.md_red),
       section(H.md_fin, &D.md_fin),
-      section(H.md_negb, &D.md_negb),
       section(H.mu_terms, &D.mu_terms),
       section(F.tw[0], &Z.tw[0]),
       section(F.tw[1], &Z.tw[1]),
@@ -486,14 +485,7 @@ extern "C" int aoa_moddown(const aoa_params* h, void* stream, uint64_t* d_q_out,
                            int level) {
   if (!h || !d_q_out || !d_qb_in) return fail(AOA_ERR_ARG, "null argument");
   if (level < 0 || level >= h->host.k) return fail(AOA_ERR_ARG, "level out of range");
-  ModDownArgs a;
-  std::memset(&a, 0, sizeof(a));
-  a.inQ[0] = d_qb_in;
-  a.inB[0] = d_qb_in + (size_t)h->host.k * h->host.N;
-  a.out[0] = d_q_out;
-  a.npolys = 1;
-  a.level = level;
-  launch_moddown(h->dev, a, (hipStream_t)stream);
+  launch_moddown(h->dev, d_qb_in, d_qb_in + (size_t)h->host.k * h->host.N, d_q_out, level, (hipStream_t)stream);
   return check_launch("aoa_moddown");
 }
 

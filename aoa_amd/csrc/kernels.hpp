@@ -87,18 +87,10 @@ void launch_decode(const DevParams& P, double* vals, const uint64_t* in, int slo
 // special limbs to outB (stride N).
 void launch_modup(const DevParams& P, const uint64_t* x, uint64_t* outB, int level, hipStream_t st);
 
-// ModDown of npolys polys.  inQ[y] holds Q limbs 0..level, inB[y] the K
-// special limbs (coefficient domain).  out[y] limb i = (inQ_i - conv_i(inB)) *
-// B^-1 mod q_i (+ add[y] limb i when add[y] != null).
-struct ModDownArgs {
-  const uint64_t* inQ[2];
-  const uint64_t* inB[2];
-  const uint64_t* add[2];
-  uint64_t* out[2];
-  int npolys;
-  int level;
-};
-void launch_moddown(const DevParams& P, const ModDownArgs& a, hipStream_t st);
+// ModDown: inQ holds Q limbs 0..level, inB the K special limbs (coefficient
+// domain).  out limb i = (inQ_i - conv_i(inB)) B^-1 mod q_i.
+void launch_moddown(const DevParams& P, const uint64_t* inQ, const uint64_t* inB, uint64_t* out, int level,
+                    hipStream_t st);
 
 // Rescale c0 and c1 in place (coefficient domain) from `level`.
 void launch_rescale(const DevParams& P, uint64_t* c0, uint64_t* c1, int level, hipStream_t st);

@@ -139,9 +139,6 @@ struct DevParams {
   // primes for ModDown, special primes for ModUp
   const uint64_t* md_red;
   const uint64_t* md_fin;        // [k][k][2]: (l,i) -> B^-1 q_l^-1 mod q_i, Shoup
-  // [k][4]: 28-bit halves (low, high, their sum, 0) of (-B) mod q_i, Q primes
-  // below 2^57: ModDown adds z (-B) to its lazy sums as one more term
-  const uint32_t* md_negb;
   // [k][k+1][kp][4], kp = K rounded up to 16: (l, i, position of j) -> 28-bit
   // halves of (Q_l/q_i) mod b_j and their sum, row i = k: of
   // (2^56 Q_l/q_0) mod b_j; positions as in build_host_params
@@ -173,7 +170,7 @@ struct HostParams {
   std::vector<uint64_t> tw_fwd, tw_inv, inv_qhat, qhat_mod_b, inv_bhat, bhat_mod_q,
       inv_b_mod_q, b_mod_q, inv_ql_mod_qi;
   // K * 4: N^-1 (B/b_j)^-1 and psi^-brev(1) N^-1 (B/b_j)^-1 mod b_j, each with its
-  // Shoup quotient (table 15)
+  // Shoup quotient (table 15; the device's form is FusedTables::lc_b)
   std::vector<uint64_t> bscale;
   std::vector<double> enc_w;        // 2N complex roots, interleaved (re, im)
   std::vector<uint32_t> rot_group;  // N/2 entries
@@ -184,7 +181,9 @@ struct HostParams {
   std::vector<uint32_t> md_thr;     // k entries
   std::vector<uint64_t> md_red;     // (k + K) * 2
   std::vector<uint64_t> md_fin;     // k * k * 2
-  std::vector<uint32_t> md_negb;    // k * 4
+  // k * 4: 28-bit halves (low, high, their sum, 0) of (-B) mod q_i, Q primes below
+  // 2^57 (host checks of a term z (-B) in ModDown's lazy sums)
+  std::vector<uint32_t> md_negb;
   std::vector<uint32_t> mu_terms;   // k * (k + 1) * kp * 4
 };
 

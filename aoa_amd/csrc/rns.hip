@@ -276,7 +276,8 @@ void launch_modup(const DevParams& P, const uint64_t* x, uint64_t* outB, int lev
 
 // --------------------------------------------------------------- ModDown ----
 // out_i = (x_i - sum_j ref([x_bj (B/b_j)^-1]_bj * (B/b_j mod q_i))) B^-1 mod q_i
-// (aoa-ntt/src/cuda/manager.cu:312-341), optionally + add_i.
+// (aoa-ntt/src/cuda/manager.cu:312-341): the stand-alone entry point's; products and
+// rotations use k_fz_down.
 //
 // ref(a*c) is the reference's Barrett reduction of the product (ref_barrett).
 // With A = a*c - qhat*p = delta*p + r (r the exact remainder, delta the
@@ -302,13 +303,11 @@ void launch_modup(const DevParams& P, const uint64_t* x, uint64_t* outB, int lev
 // their low sum (and to sm, so the middle sum keeps its value): every other
 // term lies outside the deviation window, where the two agree.  The pass/fail
 // masks come straight from the compares and are not carried across
-// iterations.  fold(i, &z) may add one more term z (-B mod q_i), z < 2^57
-// (the caller's addend), so that the caller
-// finishes the limb with one Shoup product.  The host checks that K products,
-// the folded term and K corrections stay below 2^(62+nb) (build_host_params).
-template <int NL, bool SCREEN, class Fold>
+// iterations.  The host checks that K products and K corrections stay below
+// 2^(62+nb) (build_host_params).
+template <int NL, bool SCREEN>
 __device__ __forceinline__ void moddown_conv(const DevParams& P, const uint64_t* aux, int c, int i0,
-                                             int j0, int j1, uint64_t* res, Fold fold) {
+                                             int j0, int j1, uint64_t* res) {
   constexpr uint32_t M28 = (1u << 28) - 1;
   constexpr int TW = (int)(sizeof(MdTerm) / 4);
   const int k = P.k, K = P.K;
@@ -366,28 +365,19 @@ __device__ __forceinline__ void moddown_conv(const DevParams& P, const uint64_t*
 #pragma unroll
   for (int n = 0; n < NL; ++n) {
     const int i = i0 + n * BC_GROUPS;
-    uint64_t z;
-    if (fold(i, &z)) {
-      // one more term z (-B mod q_i), z < 2^57: halves below 2^29
-      const cptr<uint32_t> e = as_const(P.md_negb) + 4 * i;
-      const uint32_t zl = (uint32_t)z & M28, zh = (uint32_t)(z >> 28), zs = zl + zh;
-      s0[n] += (uint64_t)zl * e[0];
-      s2[n] += (uint64_t)zh * e[1];
-      sm[n] += (uint64_t)zs * e[2];
-    }
     const cptr<uint64_t> red = as_const(P.md_red) + 2 * i;
     res[n] = reduce_sums_lazy(s0[n], sm[n] - s0[n] - s2[n], s2[n], ld_prime_p(P.primes, i), red[0],
                               ld_prime_nb(P.primes, i));
   }
 }
 
-template <int NL, class Fold>
+template <int NL>
 __device__ __forceinline__ void moddown_convs(const DevParams& P, const uint64_t* aux, int c, int i0,
-                                              int j0, int j1, uint64_t* res, Fold fold) {
+                                              int j0, int j1, uint64_t* res) {
   if (P.moddown_exact)
-    moddown_conv<NL, false>(P, aux, c, i0, j0, j1, res, fold);
+    moddown_conv<NL, false>(P, aux, c, i0, j0, j1, res);
   else
-    moddown_conv<NL, true>(P, aux, c, i0, j0, j1, res, fold);
+    moddown_conv<NL, true>(P, aux, c, i0, j0, j1, res);
 }
 
 // Sum over j in [j0, j1) of the ModDown products of limb i of a prime wider
@@ -429,8 +419,7 @@ __device__ __forceinline__ uint64_t moddown_wide(const DevParams& P, const uint6
 }
 
 __device__ __forceinline__ void moddown_body(const DevParams& P, const uint64_t* inQ, const uint64_t* inB,
-                                             const uint64_t* add, uint64_t* out, int level, int blk,
-                                             uint64_t* aux) {
+                                             uint64_t* out, int level, int blk, uint64_t* aux) {
   const size_t N = (size_t)P.N;
   const int c = threadIdx.x % BC_COEF;
   // wave-uniform limb group: keeps limb indices and constant loads scalar
@@ -450,25 +439,16 @@ __device__ __forceinline__ void moddown_body(const DevParams& P, const uint64_t*
   auto conv = [&](int i, int j0, int j1) -> uint64_t {
     return P.moddown_exact ? moddown_wide<false>(P, aux, c, i, j0, j1) : moddown_wide<true>(P, aux, c, i, j0, j1);
   };
-  // (x_i - acc) B^-1 (+ add_i) mod q_i from the sum acc of limb i, which is
-  // below md_red[i][1] (5 q_i, or q0 for the canonical q0 sums).
-  auto finish = [&](int i, uint64_t acc) -> uint64_t {
-    const uint64_t p = ld_prime_p(P.primes, i);
+  // (x_i - acc) B^-1 mod q_i from the sum acc of limb i, which is below
+  // md_red[i][1] (5 q_i, or q0 for the canonical q0 sums).
+  auto finish = [&](int i, uint64_t acc) {
     const tw2 bi = ld_tw2(ibq, i);
     const uint64_t y = inQ[(size_t)i * N + cid] + as_const(P.md_red)[2 * i + 1] - acc;
-    uint64_t v = mul_shoup(y, bi.w, bi.q, p);
-    if (add) v = add_mod(v, add[(size_t)i * N + cid], p);
-    return v;
+    out[(size_t)i * N + cid] = mul_shoup(y, bi.w, bi.q, ld_prime_p(P.primes, i));
   };
-  // x_i + md_red[i][1] - acc: (x_i - acc) mod q_i as a value below 2^64
-  auto lift = [&](int i, uint64_t acc) -> uint64_t {
-    return inQ[(size_t)i * N + cid] + as_const(P.md_red)[2 * i + 1] - acc;
-  };
-  // This wave's limbs g, g+4, ... below iend, in passes of four, three, two or one.
-  // A limb of a prime wider than 56 bits (q0) is summed exactly by conv
-  // (canonical) and written by wide(i, acc); the others take the lazy sums of
-  // moddown_convs, with the term z (-B) when fold(i, &z) says so, and are
-  // written by narrow(i, acc).
+  // This wave's limbs g, g+4, ... in passes of four, three, two or one.  A limb of
+  // a prime wider than 56 bits (q0) is summed exactly by conv (canonical); the
+  // others take the lazy sums of moddown_convs.
   // q0's sum (a 63-bit prime's terms cost about 1.4 times a narrow limb's)
   // is split over the four waves, so that
   // the wave that writes limb 0 carries no more than the others: the partial
@@ -485,67 +465,54 @@ __device__ __forceinline__ void moddown_body(const DevParams& P, const uint64_t*
     for (int t = 0; t < BC_GROUPS; ++t) a = add_mod(a, part0[t * BC_COEF + c], q0);
     return a;
   };
-  auto limbs = [&](int iend, auto wide, auto fold, auto narrow) {
-    int i = g;
-    while (i < iend) {
-      const int left = (iend - i + BC_GROUPS - 1) / BC_GROUPS;
-      if (ld_prime_nb(P.primes, i) > 56) {
-        wide(i, i == 0 ? acc0() : conv(i, 0, K));
-        i += BC_GROUPS;
-        continue;
-      }
-      int li[4] = {i, i + BC_GROUPS, i + 2 * BC_GROUPS, i + 3 * BC_GROUPS};
-      // the first n limbs of li all have primes below 2^57
-      auto is_narrow = [&](int n) {
-        bool ok = true;
-        for (int t = 1; t < n; ++t) ok &= ld_prime_nb(P.primes, li[t]) <= 56;
-        return ok;
-      };
-      uint64_t r[4];
-      if (left >= 4 && is_narrow(4)) {
-        moddown_convs<4>(P, aux, c, i, 0, K, r, fold);
-        for (int n = 0; n < 4; ++n) narrow(li[n], r[n]);
-        i += 4 * BC_GROUPS;
-      } else if (left == 3 && is_narrow(3)) {
-        moddown_convs<3>(P, aux, c, i, 0, K, r, fold);
-        for (int n = 0; n < 3; ++n) narrow(li[n], r[n]);
-        i += 3 * BC_GROUPS;
-      } else if (left >= 2 && is_narrow(2)) {
-        moddown_convs<2>(P, aux, c, i, 0, K, r, fold);
-        for (int n = 0; n < 2; ++n) narrow(li[n], r[n]);
-        i += 2 * BC_GROUPS;
-      } else {
-        moddown_convs<1>(P, aux, c, i, 0, K, r, fold);
-        narrow(i, r[0]);
-        i += BC_GROUPS;
-      }
-    }
-  };
   if (wide0) __syncthreads();
-  // add_i joins the sums as z = add_i: (x_i - acc + add_i B) B^-1 = (x_i - acc) B^-1 + add_i
-  limbs(
-      level + 1, [&](int i, uint64_t acc) { out[(size_t)i * N + cid] = finish(i, acc); },
-      [&](int i, uint64_t* z) {
-        if (!add) return false;
-        *z = add[(size_t)i * N + cid];
-        return true;
-      },
-      [&](int i, uint64_t acc) {
-        const tw2 bi = ld_tw2(ibq, i);
-        out[(size_t)i * N + cid] = mul_shoup(lift(i, acc), bi.w, bi.q, ld_prime_p(P.primes, i));
-      });
+  int i = g;
+  while (i <= level) {
+    const int left = (level - i) / BC_GROUPS + 1;
+    if (ld_prime_nb(P.primes, i) > 56) {
+      finish(i, i == 0 ? acc0() : conv(i, 0, K));
+      i += BC_GROUPS;
+      continue;
+    }
+    int li[4] = {i, i + BC_GROUPS, i + 2 * BC_GROUPS, i + 3 * BC_GROUPS};
+    // the first n limbs of li all have primes below 2^57
+    auto is_narrow = [&](int n) {
+      bool ok = true;
+      for (int t = 1; t < n; ++t) ok &= ld_prime_nb(P.primes, li[t]) <= 56;
+      return ok;
+    };
+    uint64_t r[4];
+    if (left >= 4 && is_narrow(4)) {
+      moddown_convs<4>(P, aux, c, i, 0, K, r);
+      for (int n = 0; n < 4; ++n) finish(li[n], r[n]);
+      i += 4 * BC_GROUPS;
+    } else if (left == 3 && is_narrow(3)) {
+      moddown_convs<3>(P, aux, c, i, 0, K, r);
+      for (int n = 0; n < 3; ++n) finish(li[n], r[n]);
+      i += 3 * BC_GROUPS;
+    } else if (left >= 2 && is_narrow(2)) {
+      moddown_convs<2>(P, aux, c, i, 0, K, r);
+      for (int n = 0; n < 2; ++n) finish(li[n], r[n]);
+      i += 2 * BC_GROUPS;
+    } else {
+      moddown_convs<1>(P, aux, c, i, 0, K, r);
+      finish(i, r[0]);
+      i += BC_GROUPS;
+    }
+  }
 }
 
 // Eight waves per SIMD hide the product loop's table loads: 4 % faster than seven.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_moddown(DevParams P, ModDownArgs A) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_moddown(
+    DevParams P, const uint64_t* inQ, const uint64_t* inB, uint64_t* out, int level) {
   extern __shared__ uint64_t aux[];  // [K][64], then [4][64] partial sums of q0
-  const int y = blockIdx.y;
-  moddown_body(P, A.inQ[y], A.inB[y], A.add[y], A.out[y], A.level, blockIdx.x, aux);
+  moddown_body(P, inQ, inB, out, level, blockIdx.x, aux);
 }
 
-void launch_moddown(const DevParams& P, const ModDownArgs& a, hipStream_t st) {
+void launch_moddown(const DevParams& P, const uint64_t* inQ, const uint64_t* inB, uint64_t* out, int level,
+                    hipStream_t st) {
   const size_t lds = (size_t)(P.K + BC_GROUPS) * BC_COEF * sizeof(uint64_t);
-  k_moddown<<<dim3(P.N / BC_COEF, a.npolys), 256, lds, st>>>(P, a);
+  k_moddown<<<dim3(P.N / BC_COEF), 256, lds, st>>>(P, inQ, inB, out, level);
 }
 
 // -------------------------------------------------------------- checksum ----

@@ -70,8 +70,8 @@ int aoa_params_primes(const aoa_params* params, uint64_t* out, int n);
  * c >> 28, their sum, the 32-bit words w0 w1 w2 of floor(c 2^96 / q_i), q_i's
  * screen threshold, 2 (the high word of the screen's bias 2^33); all zero for
  * primes of 57 bits or more), 15 [kl][2]: N^-1 (B/b_j)^-1 and psi^-brev(1) N^-1
- * (B/b_j)^-1 mod b_j (the last inverse stage of the special limbs of a batch's
- * key products).
+ * (B/b_j)^-1 mod b_j (what the last inverse stage of the special limbs' key
+ * products multiplies by).
  * Returns the number of words written (or needed, if out is NULL). */
 int64_t aoa_params_table(const aoa_params* params, int which, uint64_t* out, int64_t n);
 
