@@ -1,7 +1,9 @@
-// FP64 residue arithmetic of the transforms and key products (FieldFp64), in a
-// form that the host checks compile too: its exactness rests on bounds.
+// Arithmetic of the fused kernels whose exactness rests on bounds, in a form that
+// the host checks compile too: the FP64 residues of the transforms and key
+// products (FieldFp64), the join of a basis conversion's digit columns and the
+// screen of ModDown's products.
 //
-// A residue modulo p <= 2^48 is a signed integer in a double.  a w mod p =
+// FP64.  A residue modulo p <= 2^48 is a signed integer in a double.  a w mod p =
 // fma(-q, p, h) + l with h = a w rounded, l = a w - h exact, q = rint(h / p).  For
 // |a| <= A p and |w| <= p / 2 the quotient is off by at most A p 2^-53 (1/p and
 // the product, rounded) and l is at most A p^2 2^-54, so that the result stays within
@@ -17,7 +19,7 @@
 // M(13.4) is above 1: out_last needs |x| < p.  before_last brings the first of its
 // operands below 0.51, and M(7.2) = 0.84.
 #pragma once
-#include "modarith.hpp"
+#include "params.hpp"
 
 #if defined(__HIPCC__)
 #define AOA_HDM __host__ __device__ __forceinline__
@@ -74,5 +76,43 @@ struct Fp64 {
     return double_to_bits(x + 4503599627370496.0) & 0x000fffffffffffffull;
   }
 };
+
+// A basis conversion's sum plus z < p modulo p = o.p, in [0, 1.3 p), from its T
+// digit columns S(t).  The columns stay below 2^23 (at most 65 x 7 bytes, or 63 x
+// 7 + 8, of products of two signed bytes), pairs of them fit 32 bits; z's high word
+// is below 2^31.
+template <int T, class Columns>
+AOA_HD uint64_t conv_value(const Columns& column, const ConvOut& o, uint64_t z) {
+  auto S = [&](int t) -> int { return t < T ? column(t < T ? t : 0) : 0; };
+  const int A01 = S(0) + S(1) * 256, A23 = S(2) + S(3) * 256, A45 = S(4) + S(5) * 256, A67 = S(6) + S(7) * 256;
+  float f = __builtin_fmaf((float)A45 + (float)(int)(z >> 32), o.c_32, __builtin_fmaf((float)A23, o.c_16, o.c_b));
+  uint64_t v = o.off + z + (uint64_t)((int64_t)A01 + (int64_t)A23 * 65536);
+  uint32_t hi = (uint32_t)A45;
+  if (T > 6) {
+    f = __builtin_fmaf((float)A67, o.c_48, f);
+    hi += (uint32_t)A67 << 16;
+  }
+  v += (uint64_t)hi << 32;
+  return v - (uint64_t)(uint32_t)f * o.p;
+}
+
+// The screen of ModDown's products a c mod q, a = al + ah 2^28 < 2^56, for
+// remainders below thr q: frac(a c / q) = frac(al c/q + ah frac(2^28 c/q)), e0 and
+// e1 the two constants (FusedDev::scr).  Onto 1.5 2^36 + 2^-16 the sum's first 16
+// bits (one unit off at most, one unit added) end up in the low half word, which
+// is at most screen_bound where the remainder is below thr q.
+AOA_HD uint16_t screen_half(double al, double ah, double e0, double e1) {
+  return (uint16_t)(uint32_t)double_to_bits(
+      __builtin_fma(ah, e1, __builtin_fma(al, e0, 103079215104.0000152587890625)));
+}
+AOA_HD uint32_t screen_bound(double thr) {
+  const uint32_t b = (uint32_t)(thr * 65536.0 + 2.1);
+  return b < 65535u ? b : 65535u;
+}
+// The same to 2^-22 (bias 2^-21; FusedDev::scr_thr holds thr + 2^-20): its fraction
+// is below scr_thr there.
+AOA_HD double screen_fine(double al, double ah, double e0, double e1) {
+  return __builtin_fma(ah, e1, __builtin_fma(al, e0, 4.76837158203125e-07));
+}
 
 }  // namespace aoa

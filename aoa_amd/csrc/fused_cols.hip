@@ -71,23 +71,10 @@ __device__ __forceinline__ void conv_acc(v4i (&acc)[T][NB], const uint8_t* W, in
   }
 }
 
-// The sum plus z < p modulo p = o.p, in [0, 1.3 p), from its digit columns
-// (component r).  The columns stay below 2^23 (at most 65 x 7 bytes), pairs of
-// them fit 32 bits.
+// conv_value of component r.
 template <int T, int NB>
 __device__ __forceinline__ uint64_t conv_join(const v4i (&acc)[T][NB], int b, int r, const ConvOut& o, uint64_t z) {
-  auto S = [&](int t) -> int { return t < T ? acc[t < T ? t : 0][b][r] : 0; };
-  const int A01 = S(0) + (S(1) << 8), A23 = S(2) + (S(3) << 8), A45 = S(4) + (S(5) << 8), A67 = S(6) + (S(7) << 8);
-  // z's high word below 2^31
-  float f = __builtin_fmaf((float)A45 + (float)(int)(z >> 32), o.c_32, __builtin_fmaf((float)A23, o.c_16, o.c_b));
-  uint64_t v = o.off + z + (uint64_t)((int64_t)A01 + (int64_t)A23 * 65536);
-  uint32_t hi = (uint32_t)A45;
-  if (T > 6) {
-    f = __builtin_fmaf((float)A67, o.c_48, f);
-    hi += (uint32_t)A67 << 16;
-  }
-  v += (uint64_t)hi << 32;
-  return v - (uint64_t)(uint32_t)f * o.p;
+  return conv_value<T>([&](int t) { return acc[t][b][r]; }, o, z);
 }
 
 __device__ __forceinline__ ConvOut ld_conv(const ConvOut* t) {
@@ -253,12 +240,10 @@ __device__ __forceinline__ uint64_t down_deviation(const DevParams& P, uint64_t 
 
 // Looks for the products a_j c_ij of the limbs i0 <= i < i0 + NL whose
 // remainder may lie in the reference's deviation window and takes what they
-// deviate by off the results.  frac(a c / q) = frac(al c/q + ah frac(2^28 c/q)),
-// a = al + ah 2^28, in two FP64 multiply-adds onto 1.5 2^36 + 2^-16, which leaves
-// its first 16 bits (one unit off at most, one unit added) in the low half
-// word; the least of a term's NL halves is compared with the widest window.
-// About one wave in twenty looks closer: at each limb's half word, then to
-// 2^-22 (bias 2^-21, bound 2^-20 more), then with the exact formulas.
+// deviate by off the results.  Each product takes two FP64 multiply-adds
+// (screen_half); the least of a term's NL halves is compared with the widest
+// window.  About one wave in twenty looks closer: at each limb's half word, then
+// to 2^-22 (screen_fine), then with the exact formulas.
 template <int NL>
 __device__ __forceinline__ void down_screen(const DevParams& P, const uint64_t* aux, uint64_t* xq, int i0, int c, int set) {
   const cptr<double> tab = as_const(P.fz.scr) + i0 * 2;
@@ -266,7 +251,7 @@ __device__ __forceinline__ void down_screen(const DevParams& P, const uint64_t* 
   double widest = thr[0];
 #pragma unroll
   for (int n = 1; n < NL; ++n) widest = __builtin_fmax(widest, thr[n]);
-  const uint32_t bound = __builtin_amdgcn_readfirstlane(min((uint32_t)(widest * 65536.0 + 2.1), 65535u));
+  const uint32_t bound = __builtin_amdgcn_readfirstlane(screen_bound(widest));
   for (int j = 0; j < P.K; ++j) {
     const uint64_t a = aux[j * FZ_PITCH + c];
     const double al = (double)((uint32_t)a & ((1u << 28) - 1)), ah = (double)(uint32_t)(a >> 28);
@@ -274,8 +259,7 @@ __device__ __forceinline__ void down_screen(const DevParams& P, const uint64_t* 
     uint16_t h[NL], least = 65535;
 #pragma unroll
     for (int n = 0; n < NL; ++n) {
-      const double s = __builtin_fma(ah, e[2 * n + 1], __builtin_fma(al, e[2 * n], 103079215104.0000152587890625));
-      h[n] = (uint16_t)(uint32_t)__double_as_longlong(s);
+      h[n] = screen_half(al, ah, e[2 * n], e[2 * n + 1]);
       least = __builtin_elementwise_min(least, h[n]);
     }
     if (__builtin_amdgcn_ballot_w64(least <= bound)) {
@@ -285,8 +269,7 @@ __device__ __forceinline__ void down_screen(const DevParams& P, const uint64_t* 
 #pragma unroll
       for (int n = 0; n < NL; ++n) {
         if (__builtin_amdgcn_ballot_w64(h[n] <= bound)) {
-          const double s = __builtin_fma(ah, e[2 * n + 1], __builtin_fma(al, e[2 * n], 4.76837158203125e-07));
-          if (__builtin_amdgcn_fract(s) < thr[n]) {
+          if (__builtin_amdgcn_fract(screen_fine(al, ah, e[2 * n], e[2 * n + 1])) < thr[n]) {
             const int i = i0 + n;
             uint64_t* x = xq + i * FZ_PITCH + c;
             *x = sub_mod(*x, down_deviation(P, a, i, jo, set), ld_prime_p(P.primes, i));

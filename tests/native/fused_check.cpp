@@ -102,6 +102,161 @@ static void fp64_forms() {
   }
 }
 
+struct Shape {
+  int N, k, kl, prec;
+};
+static uint64_t mulm(uint64_t a, uint64_t b, uint64_t p) { return (uint64_t)((unsigned __int128)a * b % p); }
+
+// The digit columns of output row m of block `blk` (T digits, kbs steps of 8
+// inputs, of which kbn are used) for the input words in[], as the matrix
+// instruction sums them.
+static void columns(const uint8_t* blk, int T, int kbs, int kbn, int m, const uint64_t* in, int* S) {
+  for (int t = 0; t < 8; ++t) S[t] = 0;
+  for (int t = 0; t < T; ++t)
+    for (int s = 0; s < 8 * kbn; ++s)
+      for (int b = 0; b < 8; ++b) {
+        const int lane = m + 16 * (s % 8 / 2), at = s % 2 * 8 + b;
+        const int w = (int8_t)blk[(((size_t)t * kbs + s / 8) * 64 + lane) * 16 + at];
+        S[t] += w * (int)(int8_t)(uint8_t)((in[s] >> (8 * b)) ^ 0x80);
+        expect(S[t] > -(1 << 23) && S[t] < (1 << 23), "digit columns below 2^23");
+      }
+}
+static uint64_t join(int T, const int* S, const ConvOut& o, uint64_t z) {
+  auto c = [&](int t) { return S[t]; };
+  return T == 6 ? conv_value<6>(c, o, z) : T == 7 ? conv_value<7>(c, o, z) : conv_value<8>(c, o, z);
+}
+static void conv_is(int T, const int* S, const ConvOut& o, uint64_t z, uint64_t want, const char* what) {
+  const uint64_t v = join(T, S, o, z);
+  expect(v % o.p == want % o.p, what, "congruent");
+  expect((double)v < 1.3 * (double)o.p, what, "below 1.3 p");
+  expect(join(8, S, o, z) == v, what, "in eight digits");
+}
+// Residues below p: random, at the ends, or of bytes at the ends.
+static uint64_t sample(std::mt19937_64& rng, uint64_t p, int mode) {
+  switch (mode) {
+    case 0: return 0;
+    case 1: return p - 1;
+    case 2: return 0x8080808080808080ull % p;
+    case 3: {
+      uint64_t v = 0;
+      for (int b = 0; b < 8; ++b) v |= (rng() & 1 ? 0xffull : 0) << (8 * b);
+      return v % p;
+    }
+    default: return rng() % p;
+  }
+}
+
+// ModUp's and ModDown's tables through conv_value against modular sums.
+static void conversions(const Shape& sh, const HostParams& H, const FusedTables& F, std::mt19937_64& rng) {
+  const int k = H.k, K = H.K;
+  const uint64_t* q = H.primes.data();
+  int S[8];
+  std::vector<uint64_t> in(8 * (size_t)std::max(F.mu_kb, F.md_kb) + 8);
+  auto garbage = [&] { for (uint64_t& x : in) x = rng(); };  // rows that no constant meets
+  const int Tb = conv_digits((int)H.dprimes[k].nb);
+  for (int l : {0, 1, 6, 7, 8, k / 2, k - 1}) {
+    if (l >= k) continue;
+    for (int mode = 0; mode < 6; ++mode) {
+      garbage();
+      for (int i = 0; i <= l; ++i) in[i] = sample(rng, q[i], mode);
+      for (int j = 0; j < K; ++j) {
+        uint64_t want = 0;
+        for (int i = 0; i <= l; ++i)
+          want = (want + mulm(in[i] % q[k + j], H.qhat_mod_b[((size_t)l * K + j) * k + i], q[k + j])) % q[k + j];
+        columns(&F.mu_w[(size_t)l * F.mu_stride + (size_t)(j / 16) * Tb * F.mu_kb * 1024], Tb, F.mu_kb, (l + 8) / 8, j % 16,
+                in.data(), S);
+        conv_is(Tb, S, F.mu_out[(size_t)l * K + j], 0, want, "ModUp");
+      }
+    }
+  }
+  // set k: no rescale; set l: from level l, with the dropped limb as input K
+  for (int set : {k, 1, 7, 16, k - 1}) {
+    if (set < 1 || set > k) continue;
+    for (int mode = 0; mode < 6; ++mode) {
+      garbage();
+      for (int j = 0; j < K; ++j) in[j] = sample(rng, q[k + j], mode);
+      if (set < k) in[K] = sample(rng, q[set], mode);
+      for (int i = 0; i < (set < k ? set : k); ++i) {
+        const uint64_t p = q[i], f = set < k ? H.md_fin[((size_t)set * k + i) * 2] : H.inv_b_mod_q[2 * i];
+        const uint64_t z = sample(rng, p, (mode + i) % 6);
+        uint64_t take = set < k ? mulm(in[K] % p, H.inv_ql_mod_qi[((size_t)set * k + i) * 2], p) : 0;
+        for (int j = 0; j < K; ++j)
+          take = (take + mulm(in[j] % p, mulm(H.bhat_mod_q[((size_t)i * K + j) * 2], f, p), p)) % p;
+        columns(&F.md_w[(size_t)set * F.md_stride + (size_t)(i / 16) * 8 * F.md_kb * 1024],
+                conv_digits((int)H.dprimes[i / 16 * 16].nb), F.md_kb, F.md_kb, i % 16, in.data(), S);
+        conv_is(conv_digits((int)H.dprimes[i / 16 * 16].nb), S, F.md_out[(size_t)set * k + i], z, (z + (p - take)) % p,
+                "ModDown");
+      }
+    }
+  }
+  // twiddles and the last stage's constants, as the prime's form reads them
+  for (int r = 0; r < k + K; ++r) {
+    const DevPrime& d = H.dprimes[r];
+    for (int dir = 0; dir < 2; ++dir)
+      for (int n = 0; n < 50; ++n) {
+        const size_t e = (size_t)r * sh.N + rng() % sh.N;
+        const uint64_t want = (dir ? H.tw_inv : H.tw_fwd)[2 * e];
+        const uint64_t* t = &F.tw[dir][(size_t)r * sh.N * 2];
+        if (d.field == FIELD_FP64) {
+          const double w = bits_to_double(t[e - (size_t)r * sh.N]);
+          expect(std::fabs(w) <= d.fp / 2 && residue((i128)w, d.p) == want, "balanced twiddle");
+        } else {
+          expect(t[2 * (e - (size_t)r * sh.N)] == want, "twiddle");
+        }
+      }
+  }
+}
+
+// Every product whose reduction deviates passes the screen, at the window's edges
+// and inside it; products built as in chk_moddown_terms.
+static void screen(const HostParams& H, const FusedTables& F, std::mt19937_64& rng) {
+  const int k = H.k, K = H.K;
+  int deviating = 0;
+  for (int i = 0; i < k; ++i) {
+    const DevPrime& d = H.dprimes[i];
+    const uint64_t thr = d.quirk_thr < d.p ? d.quirk_thr : d.p;
+    for (int t = 0; t < 3000; ++t) {
+      const int j = (int)(rng() % K);
+      const uint64_t b = H.primes[k + j], c = H.bhat_mod_q[((size_t)i * K + j) * 2];
+      uint64_t a = rng() % b;
+      if (t % 4 && c) {
+        const uint64_t edge[4] = {0, d.quirk_lo + rng() % 3 - 1, thr + rng() % 3 - 1,
+                                  d.quirk_lo + rng() % (thr > d.quirk_lo ? thr - d.quirk_lo : 1)};
+        const uint64_t base = mulm(edge[t % 4] % d.p, inv_mod(c, d.p), d.p);
+        const uint64_t most = base < b ? (b - 1 - base) / d.p : 0;
+        a = base < b ? base + (t & 8 ? most : most ? rng() % (most + 1) : 0) * d.p : base % b;
+      }
+      const double al = (double)(a & ((1u << 28) - 1)), ah = (double)(a >> 28);
+      const double* e = &F.scr[((size_t)j * 64 + i) * 2];
+      const double fine = screen_fine(al, ah, e[0], e[1]);
+      const bool half = screen_half(al, ah, e[0], e[1]) <= screen_bound(F.scr_thr[i]);
+      const bool in = half && fine - std::floor(fine) < F.scr_thr[i];
+      const uint64_t exact = mulm(a, c, d.p);
+      const bool dev = ref_barrett(mulhi64(a, c), a * c, d.p, d.mu, (int)d.nb) != exact;
+      deviating += dev;
+      expect(in || !dev, "deviating product passes the screen");
+      expect(in || exact >= thr, "remainder below the threshold passes the screen");
+    }
+  }
+  if (H.prec == 48 || H.prec == 52) expect(deviating > 0, "products that deviate");
+}
+
+static void tables() {
+  std::mt19937_64 rng(2);
+  for (const Shape& s : {Shape{2048, 2, 1, 55}, Shape{2048, 4, 5, 48}, Shape{4096, 9, 7, 52}, Shape{2048, 18, 16, 48},
+                         Shape{2048, 30, 31, 48}, Shape{2048, 48, 52, 45}, Shape{2048, 64, 64, 55}, Shape{16384, 10, 15, 45}}) {
+    HostParams H;
+    FusedTables F;
+    if (!build_host_params(s.N, s.k, s.kl, s.prec, &H).empty()) {
+      expect(false, "build_host_params");
+      continue;
+    }
+    build_fused_tables(H, &F);
+    conversions(s, H, F, rng);
+    screen(H, F, rng);
+  }
+}
+
 // parallel_for where the calling thread runs out of memory at its i-th allocation,
 // the creation of threads among them: every call is made once, or the exception
 // comes back; threads that were created are joined.
@@ -125,6 +280,7 @@ int main() {
   chains();
   parallel_for_without_memory();
   fp64_forms();
+  tables();
   std::printf("fused host checks: %d failure(s)\n", failures);
   return failures ? 1 : 0;
 }

@@ -1,6 +1,7 @@
-"""The fused kernels' host-checkable parts (exact.hpp) at the ends of their
-ranges, built with g++ under AddressSanitizer and UndefinedBehaviorSanitizer
-(tests/native/fused_check.cpp): every check holds, no report."""
+"""The fused kernels' host-checkable parts (exact.hpp) and host tables
+(fused_tables.cpp) at the ends of their ranges, built with g++ under
+AddressSanitizer and UndefinedBehaviorSanitizer (tests/native/fused_check.cpp):
+every check holds, no report."""
 import os
 import shutil
 import subprocess
@@ -18,7 +19,8 @@ def test_fused_host_checks():
     os.makedirs(os.path.dirname(OUT), exist_ok=True)
     subprocess.run(["g++", "-O1", "-g", "-std=c++17", "-ffp-contract=off", "-fno-omit-frame-pointer", "-pthread",
                     "-fsanitize=address,undefined", "-fno-sanitize-recover=all", "-I" + CSRC,
-                    os.path.join(HERE, "native", "fused_check.cpp"), os.path.join(CSRC, "params.cpp"), "-o", OUT],
+                    os.path.join(HERE, "native", "fused_check.cpp"), os.path.join(CSRC, "params.cpp"), os.path.join(CSRC, "fused_tables.cpp"),
+                    "-o", OUT],
                    check=True, capture_output=True, text=True)
     r = subprocess.run([OUT], capture_output=True, text=True, timeout=600,
                        env=dict(os.environ, ASAN_OPTIONS="detect_leaks=1:halt_on_error=1"))
