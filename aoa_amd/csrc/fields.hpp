@@ -482,15 +482,24 @@ __device__ __forceinline__ void round_inv(const F& f, typename F::V (&x)[1 << LO
   }
 }
 
-// From round A's layout to round B's.
-template <int LOGM, int LOGV, int A, int B, class F>
-__device__ __forceinline__ void row_turn(const F& f, typename F::V (&x)[1 << LOGV], int s, uint64_t* L) {
+// From round A's layout to round B's: out, and in after a barrier.
+template <int LOGM, int LOGV, int A, class F>
+__device__ __forceinline__ void row_put(const F& f, const typename F::V (&x)[1 << LOGV], int s, uint64_t* L) {
   using G = Row<LOGM, LOGV>;
 #pragma unroll
   for (int k = 0; k < G::V; ++k) L[G::template Round<A>::at(s, k)] = f.raw(x[k]);
+}
+template <int LOGM, int LOGV, int B, class F>
+__device__ __forceinline__ void row_get(const F& f, typename F::V (&x)[1 << LOGV], int s, const uint64_t* L) {
+  using G = Row<LOGM, LOGV>;
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < G::V; ++k) x[k] = f.raw_in(L[G::template Round<B>::at(s, k)]);
+}
+template <int LOGM, int LOGV, int A, int B, class F>
+__device__ __forceinline__ void row_turn(const F& f, typename F::V (&x)[1 << LOGV], int s, uint64_t* L) {
+  row_put<LOGM, LOGV, A>(f, x, s, L);
+  row_get<LOGM, LOGV, B>(f, x, s, L);
 }
 
 // Strided in, packed out.  A thread writes to LDS only where it read last, so

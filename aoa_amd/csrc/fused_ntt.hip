@@ -85,23 +85,19 @@ __device__ __forceinline__ void nt_rows(const DevParams& P, const uint64_t* src,
   constexpr int LV = kLogV<LOGM>;
   const RowId<LOGM> id(tile, lds);
   const F f(ld_prime(P.primes, pr));
-  uint64_t u[G::V];
-  if constexpr (INV) {
-    with_caller_words<G::V>(f, P.primes, pr, [&](auto& w, int k, auto set) {
-      set(u, w(at_byte<uint64_t>(src, id.off + G::TS * 8 * k)));
-    });
-  } else {
-#pragma unroll
-    for (int k = 0; k < G::V; ++k) u[k] = at_byte<uint64_t>(src, id.off + G::TS * 8 * k);
-  }
   const uint64_t* T = P.fz.tw[INV ? 1 : 0] + (size_t)pr * P.N * 2;
   typename F::V x[G::V];
-#pragma unroll
-  for (int k = 0; k < G::V; ++k) x[k] = INV ? f.in(u[k]) : f.raw_in(u[k]);
   if constexpr (INV) {
-    row_turn<LOGM, LV, 0, G::ROUNDS - 1>(f, x, id.s, id.L);
+    with_caller_words<G::V>(
+        f, P.primes, pr,
+        [&](auto& w, int k, auto set) { set(x, f.in(w(at_byte<uint64_t>(src, id.off + G::TS * 8 * k)))); },
+        [&] { row_put<LOGM, LV, 0>(f, x, id.s, id.L); });
+    row_get<LOGM, LV, G::ROUNDS - 1>(f, x, id.s, id.L);
     rows_out<F, LOGM>(f, x, T, dst, id);
   } else {
+    uint64_t u[G::V];
+#pragma unroll
+    for (int k = 0; k < G::V; ++k) x[k] = f.raw_in(at_byte<uint64_t>(src, id.off + G::TS * 8 * k));
     rows_fwd_all<F, LOGM>(f, x, u, T, id);
 #pragma unroll
     for (int k = 0; k < G::V; ++k) put_byte(dst, id.off + G::TS * 8 * k, u[k]);
