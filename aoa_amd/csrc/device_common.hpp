@@ -66,6 +66,18 @@ __device__ __forceinline__ DevPrime ld_prime(const DevPrime* base, int i) {
   return d;
 }
 
+// Canonical residues of any words, one from 2^63 up read as that minus 2^64: what
+// aoa_eltwise_scalar leaves of a residue smaller than a constant above the prime.
+struct Residues {
+  uint64_t p, wq;  // floor(2^64 / p)
+  __device__ __forceinline__ explicit Residues(const DevPrime& d) : p(d.p), wq(d.mu >> (2 * (int)d.nb - 64)) {}
+  __device__ __forceinline__ uint64_t operator()(uint64_t x) const {
+    const bool neg = x >> 63;
+    const uint64_t r = mul_shoup(neg ? 0 - x : x, 1, wq, p);
+    return neg ? neg_mod(r, p) : r;
+  }
+};
+
 // Where the limbs of one launch live.  Limb li of poly y is at
 // base[y] + li * N and uses prime index prime_of(li): the first `qlimbs`
 // limbs are Q limbs prime0, prime0+1, ..., the rest are special limbs

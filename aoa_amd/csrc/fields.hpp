@@ -84,18 +84,6 @@ struct Words {
     return x;
   }
 };
-// Canonical residues of such words, one from 2^63 up read as that minus 2^64 (a
-// constant above the prime subtracted from a smaller residue).
-struct Residues {
-  uint64_t p, wq;  // floor(2^64 / p)
-  __device__ __forceinline__ explicit Residues(const DevPrime& d) : p(d.p), wq(d.mu >> (2 * (int)d.nb - 64)) {}
-  __device__ __forceinline__ uint64_t operator()(uint64_t x) const {
-    const bool neg = x >> 63;
-    const uint64_t r = mul_shoup(neg ? 0 - x : x, 1, wq, p);
-    return neg ? neg_mod(r, p) : r;
-  }
-};
-
 // form(w, k, set) for each of a thread's V values, which reads caller data of
 // prime pr through w and keeps what it makes of it by set(array, value): with
 // Words and, where one of the wave was too wide, again with Residues.  That rare

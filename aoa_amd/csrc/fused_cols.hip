@@ -282,7 +282,8 @@ __device__ __forceinline__ void down_screen(const DevParams& P, const uint64_t* 
 
 // Limbs 16 ib.. of coefficients 16 nb0..: the conversion and the result
 // f_i x_i - sum (xq holds f_i x_i; with a rescale the dropped limb is input K of
-// the sum), canonical, + add_i.
+// the sum), canonical, + add_i
+// (caller data, canonical or not).
 template <int T, int NB>
 __device__ __forceinline__ void down_out(const DevParams& P, int set, const uint64_t* add, uint64_t* out, int ib, int nb0,
                                          int lout, const uint64_t* aux, const uint64_t* xq, int M, int col0, int lane) {
@@ -290,6 +291,19 @@ __device__ __forceinline__ void down_out(const DevParams& P, int set, const uint
   v4i acc[T][NB];
   conv_acc<T, NB>(acc, Z.md_w + (size_t)set * Z.md_stride + (size_t)ib * 8 * Z.md_kb * 1024, Z.md_kb, Z.md_kb, aux, nb0,
                   lane);
+  // addends requested together (none with a rescale)
+  uint64_t w[4][NB];
+  if (add) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = min(ib * 16 + 4 * (lane >> 4) + r, lout - 1);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const int n = (nb0 + b) * 16 + (lane & 15);
+        w[r][b] = add[(size_t)i * P.N + (size_t)(n / FZ_COLS) * M + col0 + n % FZ_COLS];
+      }
+    }
+  }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int i = ib * 16 + 4 * (lane >> 4) + r;
@@ -301,7 +315,11 @@ __device__ __forceinline__ void down_out(const DevParams& P, int set, const uint
         uint64_t v = conv_join<T, NB>(acc, b, r, o, xq[i * FZ_PITCH + n]);
         v = csub(v, o.p);
         const size_t at = (size_t)i * P.N + (size_t)(n / FZ_COLS) * M + col0 + n % FZ_COLS;
-        if (add) v = add_mod(v, add[at], o.p);
+        if (add) {
+          uint64_t a = w[r][b];
+          if (__builtin_amdgcn_ballot_w64(a >= o.p)) a = Residues(P.primes[i])(a);
+          v = add_mod(v, a, o.p);
+        }
         out[at] = v;
       }
     }

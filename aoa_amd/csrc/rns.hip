@@ -679,7 +679,15 @@ __global__ __launch_bounds__(256) void k_automorphism_d(DevParams P, const AutoD
   const uint64_t* in = glob(a.in);
   const uint64_t* addsrc = glob(a.addsrc);
   uint64_t v = t < N ? in[t] : neg_mod(in[t - N], p);
-  if (addsrc) v = add_mod(v, addsrc[j], p);
+  if (addsrc) {
+    uint64_t w = addsrc[j];
+    if (__builtin_amdgcn_ballot_w64(v >= p || w >= p)) {  // caller data
+      const Residues r(P.primes[a.prime]);
+      v = r(v);
+      w = r(w);
+    }
+    v = add_mod(v, w, p);
+  }
   glob(a.out)[j] = v;
 }
 

@@ -96,12 +96,11 @@ int aoa_eltwise(const aoa_params* params, void* stream, int op, uint64_t* out, c
  * (aoa-ntt/src/arithmetic/poly_t.cpp:157-235).
  *
  * Its results may thus lie outside [0, q_r).  aoa_ntt, aoa_encrypt, aoa_decrypt,
- * the products, aoa_keyswitch's d and the batches take such residues: a word
- * stands for its value mod q_r, one from 2^63 up for that minus 2^64 (q0's words
- * below 2^63), and their results are those of the reduced residues.  With an
+ * the products, aoa_keyswitch, the rotations and the batches take such residues: a
+ * word stands for its value mod q_r, one from 2^63 up for that minus 2^64 (q0's
+ * words below 2^63), and their results are those of the reduced residues.  With an
  * explicit split (aoa_params_set_ntt_split) transforms, encryption and decryption
- * are exact for words below 2 q_r; what a rotation or add0 adds is added with one
- * correction; switching keys are canonical. */
+ * are exact for words below 2 q_r; switching keys are canonical. */
 int aoa_eltwise_scalar(const aoa_params* params, void* stream, int op, uint64_t* out, const uint64_t* a, uint64_t b,
                        int res0, int nres);
 

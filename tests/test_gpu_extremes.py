@@ -8,7 +8,8 @@ from orc import Oracle
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(2048, 3, 4, 48), (4096, 3, 4, 45), (16384, 3, 3, 48), (32768, 2, 3, 45), (65536, 3, 4, 48), (65536, 2, 2, 45)]
+SHAPES = [(2048, 3, 4, 48), (4096, 3, 4, 45), (16384, 3, 3, 48), (32768, 2, 3, 45), (65536, 3, 4, 48), (65536, 2, 2, 45),
+          (65536, 10, 9, 48)]
 
 
 def _poly(O, rng, nlimbs, kind):

@@ -12,7 +12,8 @@ from orc import Oracle
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(2048, 4, 5, 45), (4096, 4, 5, 48), (4096, 3, 4, 52), (8192, 3, 4, 45), (65536, 3, 2, 48), (32768, 2, 3, 55)]
+SHAPES = [(2048, 4, 5, 45), (4096, 4, 5, 48), (4096, 3, 4, 52), (8192, 3, 4, 45), (65536, 3, 2, 48), (32768, 2, 3, 55),
+          (65536, 10, 9, 48), (32768, 10, 9, 52)]  # the last two: both key halves in a workgroup
 
 
 def _cases(O, rng, nlimbs):
@@ -72,20 +73,26 @@ def test_products(gpu, shape):
             ref = O.hommul(host[:2], host[2:], evk, level)
             out = [P.zeros(k), P.zeros(k)]
             P.hommul(out, dev[:2], dev[2:], dk, level, P.workspace(level))
-            bout = [P.zeros(k), P.zeros(k)]
-            B = Batch()
-            B.add_mul(P, dk, [(dev[:2], dev[2:], bout, level)])
-            B.launch()
-            torch.cuda.synchronize()
-            for name, o in (("plain", out), ("batch", bout)):
+            outs = {"plain": out}
+            # one launch for all forms of arithmetic, and one for each
+            for ss in (-1, 1):
+                two = [[P.zeros(k), P.zeros(k)] for _ in range(2)]
+                B = Batch()
+                B.add_mul(P, dk, [(dev[:2], dev[2:], o, level) for o in two])
+                B.set_options(strict_split=ss)
+                B.launch()
+                torch.cuda.synchronize()
+                B.close()
+                outs.update({("batch", ss, i): o for i, o in enumerate(two)})
+            for name, o in outs.items():
                 for y in range(2):
                     assert np.array_equal(P.to_host(o[y])[:level * N], ref[y][:level * N]), (name, y, op, c)
-            B.close()
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "N%d_k%d_K%d_p%d" % s)
 def test_transforms_rotation_and_client_side(gpu, shape):
-    from aoa_amd import FORWARD, INVERSE
+    import torch
+    from aoa_amd import FORWARD, INVERSE, Batch
     P, O, rng = _setup(shape)
     k, N, level = P.k, P.N, P.k - 1
     rtk = [O.random_poly(rng, k + P.kl) for _ in range(2)]
@@ -106,11 +113,25 @@ def test_transforms_rotation_and_client_side(gpu, shape):
         exp = O.rotate_left([ref, other], rtk, 3, level)
         for y in range(2):
             assert np.array_equal(P.to_host(got[y]), exp[y]), ("rotation", y, op, c)
-        P.keyswitch(got[0], got[1], _raise(P, O, op, c, x), dk[0], dk[1], level, P.workspace(level))
+        P.keyswitch(got[0], got[1], _raise(P, O, op, c, x), dk[0], dk[1], level, P.workspace(level),
+                    add0=_raise(P, O, op, c, x))
         canon = [P.zeros(k), P.zeros(k)]
-        P.keyswitch(canon[0], canon[1], P.to_device(want), dk[0], dk[1], level, P.workspace(level))
+        P.keyswitch(canon[0], canon[1], P.to_device(want), dk[0], dk[1], level, P.workspace(level), add0=P.to_device(want))
         for y in range(2):
             assert (got[y] == canon[y]).all(), ("key switch", y, op, c)
+        # rotations of the residues themselves, plain and accumulated in a batch
+        exp = O.rotate_left([want, want], rtk, 3, level)
+        raised = [_raise(P, O, op, c, x) for _ in range(2)]
+        P.rotate_left(got, raised, dk, 3, level, P.workspace(level))
+        B, bout = Batch(), [P.zeros(k), P.zeros(k)]
+        B.add_rotate(P, [(raised, bout, dk, 3, level, True)])
+        B.launch()
+        torch.cuda.synchronize()
+        B.close()
+        p = np.repeat(np.array(O.primes[:k], dtype=np.uint64), N)
+        for y in range(2):
+            assert np.array_equal(P.to_host(got[y]), exp[y]), ("rotation of residues", y, op, c)
+            assert np.array_equal(P.to_host(bout[y]), (exp[y] + want) % p), ("rotate and add", y, op, c)
         # encryption of the message and under the key, decryption of the component and under the key
         outs = []
         for v in (P.to_device(want), _raise(P, O, op, c, x)):
