@@ -1,10 +1,11 @@
 // Residue arithmetic of the 16 x M transforms and the key products
-// (fused.hip): one form per size of prime, behind one interface.
+// (fused_rows.hip, fused_cols.hip, fused_ntt.hip): one form per size of prime,
+// behind one interface.
 //
 //  FieldLazy    p < 2^56: 64-bit residues left below 2^8 p.  A Shoup product
 //               takes any 64-bit value and drops the lowest of the quotient's
 //               four partial products (result below 4p), so a butterfly needs no
-//               conditional correction: 17 vector instructions instead of 27.
+//               conditional correction: 15 vector instructions (compiled alone).
 //  FieldFp64    p <= 2^48: signed FP64 integers (exact.hpp).  A butterfly is eight
 //               FP64 instructions and its twiddle one double.
 //  FieldStrict  wider primes (the 63-bit q0, p = 2^63 - c): 64-bit values, with
@@ -227,8 +228,8 @@ struct FieldFp64 : Fp64 {
   __device__ __forceinline__ V relin(V d2, uint64_t k, V d, W bq) const { return mul(d2, in(k)) + mul(d, bq); }
 };
 
-// Of a small call's limbs this one ends last: a butterfly is 33 vector
-// instructions (a Shoup product and canonical sums: about 45).
+// Of a small call's limbs this one ends last: a butterfly is 32 vector
+// instructions compiled alone (a Shoup product and canonical sums: about 45).
 struct FieldStrict {
   static constexpr bool kAnyWord = true;
   using V = uint64_t;

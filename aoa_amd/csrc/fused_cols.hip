@@ -89,7 +89,7 @@ __device__ __forceinline__ ConvOut ld_conv(const ConvOut* t) {
 // MUL: the item's D (inverse rows of d2) is brought to coefficients; otherwise
 // the item's d holds coefficients, whose Q limbs also start their forward NTT
 // here.  v_i = x_i (Q_l/q_i)^-1 into LDS, the conversion, the forward columns
-// of the special limbs.  32 items at N = 2^16: 550 us (ModUp alone 430 before, the
+// of the special limbs.  32 items at N = 2^16: 540 us (ModUp alone 430 before, the
 // inverse and forward column passes 240 and 260); the chain of a workgroup's
 // phases bounds it, 0.47 vector instructions a busy CU and cycle.
 template <class F, bool MUL>
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(FZ_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 
 // ---------------------------------------------------------------- ModDown --
 // Inverse columns of every limb into LDS, the screen, the dropped limb, the
-// conversion.  64 polynomials at N = 2^16, L = 30, K = 31: 1.755 ms, 7.0e8 vector
+// conversion.  64 polynomials at N = 2^16, L = 30, K = 31: 1.711 ms, 7.0e8 vector
 // instructions, 0.72 a busy CU and cycle: issue bound (integer sums before: 1.75 ms
 // for ModDown and 1.0 for the column pass).  Of a workgroup's cycles about a third
 // each are the columns, the screen and the conversion.

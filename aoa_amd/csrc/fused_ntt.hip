@@ -24,7 +24,7 @@ __device__ __forceinline__ NtLimb nt_table(const NttDesc* d, int l) {
 // ----------------------------------------------------------------- columns --
 // Memory bound: 64 columns on 256 threads, where a wave holds one quarter of
 // the rows of all of them, so its loads are whole 512-byte row segments and its
-// twiddles scalar; the quarters change hands in LDS.  61 limbs at N = 2^16: 13.7
+// twiddles scalar; the quarters change hands in LDS.  61 limbs at N = 2^16: 13.3
 // us, the time of a copy (the split by 256: 22.1 forward, 24.2 inverse).
 constexpr int NT_COLS = 64;
 
@@ -76,8 +76,8 @@ __global__ __launch_bounds__(256) void k_nt_cols(DevParams P, LimbMap m, const N
 
 // -------------------------------------------------------------------- rows --
 // Rows as in the key products' kernel, here between two passes over memory;
-// vector work and twiddle latency bound.  61 limbs at N = 2^16: 22.7 us forward
-// and 25.2 inverse (25.1 and 28.6 for rows of 256).
+// vector work and twiddle latency bound.  61 limbs at N = 2^16: 21.6 us forward
+// and 23.1 inverse (25.1 and 28.6 for rows of 256).
 template <class F, int LOGM, bool INV>
 __device__ __forceinline__ void nt_rows(const DevParams& P, const uint64_t* src, uint64_t* dst, int pr, int tile,
                                         uint64_t* lds) {
@@ -118,7 +118,7 @@ __global__ __launch_bounds__(RowOf<LOGM>::THREADS) void k_nt_rows(DevParams P, L
 
 // Decryption's rows: both components' forward rows (stored, as the transforms
 // leave them), c0 + c1 s and its inverse rows.  A chain of three row transforms
-// in one launch: 16.9 us at N = 2^15, 12 limbs, for the 31 of two launches of
+// in one launch: 16.4 us at N = 2^15, 12 limbs, for the 31 of two launches of
 // rows and the product between them.
 template <class F, int LOGM>
 __device__ __forceinline__ void nt_decrypt(const DevParams& P, uint64_t* c0, uint64_t* c1, const uint64_t* s, uint64_t* out,

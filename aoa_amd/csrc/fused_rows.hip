@@ -7,7 +7,7 @@
 namespace aoa {
 
 // ------------------------------------------------------ d2 = a b, its rows --
-// Memory bound: two operands in, one out.  960 limbs at N = 2^16: 325 us, 4.9
+// Memory bound: two operands in, one out.  960 limbs at N = 2^16: 321 us, 4.8
 // TB/s of counter traffic (a tensor pass and the inverse pass of d2 before: 370
 // and more traffic).
 template <class F, int LOGM>
@@ -79,7 +79,7 @@ __device__ __forceinline__ void key_body_tensor(const DevParams& P, const FzItem
     });
   };
   // Which halves, decided once: with a branch per value the loads went out a
-  // value at a time (928 limbs of 48 bits at N = 2^16 796 us, now 682).
+  // value at a time (928 limbs of 48 bits at N = 2^16 796 us against 682).
   if constexpr (BOTH)
     form(std::true_type(), std::true_type());
   else if (y0 == 0)
@@ -135,8 +135,8 @@ __device__ __forceinline__ void key_body(const DevParams& P, const FzItem& it, i
   }
 }
 
-// Special limbs at N = 2^16 (992 of 55 bits): 840 us, 0.90 vector instructions a
-// busy CU and cycle: issue bound.  Q limbs (928 of 48 bits): 682 us, 4.3 TB/s, 53
+// Special limbs at N = 2^16 (992 of 55 bits): 826 us, 0.90 vector instructions a
+// busy CU and cycle: issue bound.  Q limbs (928 of 48 bits): 667 us, 4.8 TB/s, 47
 // for the 32 of q0.  (The split form's row pass took 1.6 ms for all of them and its
 // columns 1.0, now in k_fz_down.)
 //

@@ -1,4 +1,4 @@
-// Host tables of the fused key-switching kernels (fused.hip).
+// Host tables of the fused kernels (fused.hpp).
 #include <cmath>
 #include <cstring>
 

@@ -143,7 +143,7 @@ struct DevParams {
   // halves of (Q_l/q_i) mod b_j and their sum, row i = k: of
   // (2^56 Q_l/q_0) mod b_j; positions as in build_host_params
   const uint32_t* mu_terms;
-  FusedDev fz;  // tables of the fused key-switching kernels (fused.hip)
+  FusedDev fz;  // tables of the fused kernels (build_fused_tables)
 };
 
 // The device layout of the ModDown product constants: MdConst's first six

@@ -33,8 +33,8 @@ N, K_Q, K_B, PREC = 65536, 30, 31, 48
 HBM_PEAK_GBS = 8000.0
 # HBM bytes per k_fz_down launch at 32 pairs, from two rocprofv3 --pmc runs
 # (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0; the factors make a 1 GiB device copy
-# read 1 GiB and write 1 GiB); profiles/hommul_batched_n16_k30_counters.md.
-MODDOWN_TRAFFIC_BYTES = {32: 3039468749}
+# read 1 GiB and write 1 GiB); profiles/counters.md.
+MODDOWN_TRAFFIC_BYTES = {32: 3039302432}
 # VALU wave-instructions per k_fz_down launch at 32 pairs (SQ_INSTS_VALU summed
 # over the counter instances of one dispatch, same file), and a
 # reference issue rate: MI355X's vector FP64 FMA peak (78.6 TFLOP/s = 2 flops x
@@ -42,7 +42,7 @@ MODDOWN_TRAFFIC_BYTES = {32: 3039468749}
 # cycle.  64-bit integer multiply-adds issue at about this rate; 32-bit adds
 # and logic issue faster (about 1.6 times), so the fraction is a proxy that a
 # mix of both can exceed.
-MODDOWN_VALU_INSTS = {32: 6.978e8}
+MODDOWN_VALU_INSTS = {32: 7.030e8}
 VALU_PEAK_INSTS_S = 256 * 2.4e9
 
 

@@ -74,8 +74,7 @@ def test_batch_mixed_ring_dimensions(gpu):
     rng = np.random.default_rng(32)
     B = Batch()
     checks = []
-    # N <= 4096: tensor kernel + single-workgroup transforms; from 8192 up: the
-    # tensor product fused into the two-pass inverse transform
+    # every row length but two, one group each
     for N, k, prec in ((2048, 2, 55), (4096, 3, 52), (8192, 4, 48), (16384, 8, 48), (65536, 3, 48)):
         P = Params(N, k, 0, prec)
         evk = [P.to_device(_rand(P, rng, P.k + P.kl)) for _ in range(2)]
@@ -151,8 +150,8 @@ def test_autotuner_splits_agree(gpu):
 
 def test_stage_times_runs_the_batch(gpu):
     """The stage-timing run is an ordinary eager run of the batch: outputs equal
-    the plain form, every stage of HomMul is timed once per layer (from
-    N = 8192 up the tensor product runs inside the inverse-NTT stage)."""
+    the plain form, every stage of HomMul is timed once per layer (the
+    tensor product runs inside the inverse-NTT and key stages)."""
     import torch
     from aoa_amd import Batch, Params
     P = Params(16384, 6, 0, 48)
@@ -234,10 +233,9 @@ def test_batch_c4_full_size_equals_plain(gpu):
 
 
 def test_batch_fused_every_level_equals_oracle(gpu):
-    """The batched HomMul at the smallest two-pass size (N=2^13, k=8, prec 48),
-    one item at every level 1..k-1: the tensor pass of d2, d0 and d1 folded
-    into the key products and ModDown without addends give the oracle's
-    residues for every item."""
+    """The batched HomMul at N=2^13, k=8, prec 48, one item at every level
+    1..k-1: d2, d0 and d1 formed in the key products and ModDown without
+    addends give the oracle's residues for every item."""
     import torch
     from aoa_amd import Batch, Params
     N, k = 8192, 8

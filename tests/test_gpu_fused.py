@@ -67,8 +67,9 @@ def _ref_barrett(x, p):
 
 def test_many_deviating_products(gpu):
     """Every coefficient of every special limb in the deviation window of one
-    limb's product, so that a workgroup finds more of them than its list holds:
-    the key's special limbs are made for it from the ModUp of the polynomial 1."""
+    limb's product, so that every coefficient is corrected in place several
+    times: the key's special limbs are made for it from the ModUp of the
+    polynomial 1."""
     from aoa_amd import FORWARD, Params
     N, k, kl, prec = 2048, 4, 5, 48
     P, O = Params(N, k, kl, prec), Oracle(N, k, kl, prec)

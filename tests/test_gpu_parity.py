@@ -14,7 +14,7 @@ from orc import Oracle
 pytestmark = pytest.mark.gpu
 
 # (N, k, kl, prec): N=4096 k=4 prec 52, small/medium shapes, and the reference's test params
-# (N=2048 and 4096 run the single-workgroup transform, larger N the two-pass one).
+# (explicit splits: a workgroup a limb at N=2048 and 4096, two passes at larger N).
 SMALL = [(4096, 4, 5, 52), (8192, 6, 0, 48), (16384, 5, 5, 55), (32768, 4, 0, 48), (4096, 3, 3, 45),
          (2048, 2, 2, 55)]
 
@@ -192,10 +192,9 @@ def test_hommul_parity(gpu, shape):
 
 @pytest.mark.parametrize("n1", [64, 4096])
 def test_hommul_split_parity(gpu, n1):
-    """HomMul at N=4096 with the two-pass split (the additions of d0 and d1
-    join the key products before the inverse NTT) and with the
-    single-workgroup transform (the additions stay in ModDown): both give the
-    oracle's residues, at the top level and at level 1."""
+    """HomMul at N=4096 on handles with a split set, which is for the plain
+    transforms and leaves the product's kernels as they are: the oracle's
+    residues, at the top level and at level 1."""
     P, O = _params(4096, 4, 5, 52)
     P.set_ntt_split(n1)
     rng = np.random.default_rng(17)

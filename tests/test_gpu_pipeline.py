@@ -82,8 +82,7 @@ def test_pipeline_graph_replays(gpu):
 @pytest.mark.parametrize("N,k,kl,prec", [(4096, 4, 5, 52), (16384, 5, 5, 55)])
 def test_encrypt_decrypt_entry_points_match_primitives(gpu, N, k, kl, prec):
     """aoa_encrypt and aoa_decrypt equal the primitive calls they replace
-    (aoa_sample, aoa_ntt, aoa_eltwise), bit for bit, with the single-workgroup
-    transform (N = 4096) and the two-pass one."""
+    (aoa_sample, aoa_ntt, aoa_eltwise), bit for bit, at two row lengths."""
     import torch
     from aoa_amd import Params
     from aoa_amd.core import ADD, FORWARD, INVERSE, MULADD, SAMPLE_GAUSSIAN, SAMPLE_ZO

@@ -88,8 +88,8 @@ def test_rotate_n16_parity(gpu, rot):
 def test_hommul_window_aimed_keys(gpu, shape):
     """HomMul+relin+rescale with keys chosen so that the special limbs of both
     key products put many ModDown products in the reference's deviation
-    window: the plain form (k_moddown, rescale fused) and a batch of the same
-    item at two levels (k_moddown_d) give the oracle's residues, and the
+    window: the plain form and a batch of the same item at two levels
+    (k_fz_down, rescale in it) give the oracle's residues, and the
     window is really hit (the oracle's exact mode differs)."""
     import torch
     from aoa_amd import Batch, Params
